@@ -940,8 +940,8 @@ def moe_router_topk(logits, top_k, norm_topk_prob, shared_gate=True, per_expert_
 
 def quantize(w, kquant_type, imatrix=None, *, stream=None):
     """Encode float weights [..., K] to wire bytes; returns (wq uint8 [..., bytes_per_row], scales uint8 [1]) on w's
-    device.  A tensor on the GPU is encoded there for the legacy and K-quant codecs (one thread per block running
-    the host encoder's code: same bytes); the IQ codecs, CPU tensors and stream="cpu" take the host encoder, as the
+    device.  A tensor on the GPU is encoded there for the legacy and K-quant codecs (the host
+    encoder's arithmetic in its order: same bytes); the IQ codecs, CPU tensors and stream="cpu" take the host encoder, as the
     reference keeps its IQ encoders on the CPU.  Mirrors quantize, src/kquant_ops.cpp:550-631."""
     op = "quantize"
     cid, (wpb, bpb) = _codec(op, kquant_type)

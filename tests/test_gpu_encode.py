@@ -126,3 +126,26 @@ def test_device_encoder_large_matrix_speed_sanity(kq):
     t_host = time.perf_counter() - t0
     print(f"q4_k 2048 x 4096: device {t_dev * 1e3:.1f} ms, host {t_host * 1e3:.1f} ms")
     assert torch.equal(dev.cpu(), host)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("codec", DEV_CODECS)
+def test_device_encoder_both_lane_splits_and_ragged_ends(kq, codec, dtype):
+    """Bytes equal the host's on a matrix large enough for one lane per sub-block and on ones that end inside a
+    workgroup, from aligned and unaligned addresses, with signed zeros, constant blocks and one-sided ones."""
+    gen = torch.Generator().manual_seed(11)
+    wpb = kq.CODEC_GEOMETRY[codec][3]
+    for rows, K in ((2051, 1024), (1, wpb), (3, 3 * wpb)):
+        w = torch.randn((rows, K), generator=gen) * 0.05
+        w[0, : wpb // 2] = 0.0
+        w[0, 1] = -0.0
+        w[rows // 2] = w[rows // 2].abs()
+        w[rows - 1, -wpb:] = -0.25
+        w = w.to(dtype)
+        im = torch.rand(K, generator=gen) + 0.1 if codec in kq.codec_geometry.IMATRIX_CODECS else None
+        host = kq.quantize(w, codec, im)[0]
+        flat = torch.empty(rows * K + 1, dtype=dtype, device="cuda")
+        for off in (0, 1):  # an odd element offset: no four-element loads
+            wd = flat[off:off + rows * K].copy_(w.reshape(-1)).reshape(rows, K)
+            dev = kq.quantize(wd, codec, None if im is None else im.cuda())[0]
+            assert torch.equal(dev.cpu(), host), (codec, rows, K, off)
