@@ -1,5 +1,6 @@
 // C ABI of libkq (declared in include/kq.h): argument validation, error reporting, the device copy of the
 // IQ codebooks and routing to the HIP launchers.  Compiled by hipcc as HIP (the codebooks are a __device__ array).
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -121,10 +122,12 @@ size_t kq_qmm_workspace_size(int M, int N, int K, int transpose, int codec, int 
   (void)dtype;
   if (!codec_ok(codec)) return 0;
   if (!transpose) return kq_nt_workspace_bytes(M, N, K);  // optional: partial sums of a K range cut over the grid
-  if (kq_gemm_supported(M, N, K, codec)) return kq_gemm_workspace_bytes(M, N, K);
+  const size_t mid = kq_mid_supported(M, N, K, codec) ? kq_mid_workspace_bytes(M, N, K) : 0;
+  if (kq_gemm_supported(M, N, K, codec)) return std::max(mid, kq_gemm_workspace_bytes(M, N, K));
   // split-K partial sums (optional) of whichever skinny kernel takes the call
   const size_t tuned = kq_qmm_tuned_workspace_bytes(M, N, K, codec);
   size_t any = (M > 8 && kq_anymma_supported(M, N, K, codec)) ? kq_anymma_dense_workspace_bytes(M, N, K, dtype) : 0;
+  if (mid > any) any = mid;
   if (kq_gemm2_low_supported(M, N, K, codec) && kq_gemm2_low_workspace_bytes(M, K) > any) any = kq_gemm2_low_workspace_bytes(M, K);
   if (kq_gemm3b_supported(M, N, K, codec) && kq_gemm3b_workspace_bytes(M, K) > any) any = kq_gemm3b_workspace_bytes(M, K);
   if (kq_gemm3f_supported(M, N, K, codec) && kq_gemm3f_workspace_bytes(M, K) > any) any = kq_gemm3f_workspace_bytes(M, K);
@@ -151,6 +154,10 @@ int kq_qmm(const void* x_dev, const void* w_dev, void* y_dev, int M, int N, int 
                                       0, 0, codec, dtype, workspace_dev, workspace_bytes, s);
     if (rcn != KQ_ERR_UNSUPPORTED) return rcn;
     return kq_launch_gemm_nt_generic(x_dev, static_cast<const uint8_t*>(w_dev), y_dev, M, N, K, codec, dtype, s);
+  }
+  if (kq_mid_supported(M, N, K, codec) && workspace_dev && workspace_bytes >= kq_mid_workspace_bytes(M, N, K)) {
+    const int rcm = kq_launch_mid(x_dev, static_cast<const uint8_t*>(w_dev), y_dev, M, N, K, codec, dtype, workspace_dev, s);
+    if (rcm != KQ_ERR_UNSUPPORTED) return rcm;
   }
   if (kq_gemm_supported(M, N, K, codec)) {
     const size_t need = kq_gemm_workspace_min_bytes(M, K);

@@ -136,6 +136,13 @@ int kq_launch_gather_tuned(const void* x, const uint8_t* w, const uint8_t* w2, c
                            const uint32_t* rhs, void* out, int B, int M, int N, int K, int x_div,
                            int64_t x_batch_stride, int64_t w_expert_stride, int glu, int act, float limit, int codec,
                            int dtype, int E, KqOutMap om, hipStream_t s);
+// Every codec, 9 ... KQ_MID_MAX_ROWS activation rows: waves stream the weights, one launch behind a prepass that puts the
+// activations into ws (kq_mid_workspace_bytes) in matrix-operand order (kq_mid.hip).
+#define KQ_MID_MAX_ROWS 128
+bool kq_mid_supported(int M, int N, int K, int codec);
+size_t kq_mid_workspace_bytes(int M, int N, int K);
+void kq_mid_force_tile(int rows);
+int kq_launch_mid(const void* x, const uint8_t* w, void* y, int M, int N, int K, int codec, int dtype, void* ws, hipStream_t s);
 // Prefill GEMM (q4_k / q5_k / q6_k, M > 8): needs kq_gemm_workspace_min_bytes(M, K) bytes of device workspace
 // (converted activations); with kq_gemm_workspace_bytes(M, N, K) a call with few tiles cuts K over the grid.
 size_t kq_gemm_workspace_min_bytes(int M, int K);

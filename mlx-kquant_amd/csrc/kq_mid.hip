@@ -1,0 +1,644 @@
+// Matmul of 9 ... a few dozen activation rows, every codec: y[M,N] = x[M,K] . W^T between the streamed skinny kernel
+// (M <= 8) and the tile GEMMs.
+//
+// What bounds it: the weight bytes (HBM).  A call of 32 rows does 64 operations per weight, a tenth of what the matrix
+// cores could do in the time the weights take to arrive, so the kernel is built like the skinny ones: every wave streams
+// wire bytes on its own, and no barrier sits in the stream.
+//   * Workgroup = 8 waves on one tile of up to 32 weight rows; wave w takes the 256-weight steps w, w + 8, ...; the
+//     waves' sums meet in LDS at the end of the tile.  Workgroups are persistent (one per CU) and a wave's next step,
+//     of this tile or the next one, is already on its way while one is multiplied.
+//   * A matrix of fewer tiles than CUs cuts its steps into ranges of eight or more, one workgroup each.  The workgroup
+//     of a tile that finishes last adds the others' sums, in the order of the ranges (finish_tile): no launch behind.
+//   * Wire bytes go to wave-private LDS with direct-to-LDS loads, two slots per wave.
+//   * Activations: a prepass writes them as f16 in matrix-operand order, 1 KiB per (32 rows, 16 weights of K), so a
+//     fragment is one coalesced 16-byte load per lane straight into registers (L2 serves every tile after the first).
+//     Loads of a wave return in order, so fragments and wire bytes of the next step are requested together and waited
+//     for together.
+//   * 33 rows and more run as blocks of 32 rows: the blocks of a tile are neighbours in launch order on one XCD, so that
+//     the second one finds the wire bytes in its L2.
+// Measured: see the routing in kq_mid_supported.
+#include <algorithm>
+
+#include "kq_codes.h"
+#include "kq_dma.h"
+#include "kq_kfrag.h"
+
+namespace {
+
+using namespace kqcodes;
+using namespace kqdma;
+using kqmma::u32x4;
+
+template <int C>
+constexpr bool k_quant() { return C <= KQ_Q6_K; }
+template <int C>
+constexpr bool fp4() { return C == KQ_MXFP4 || C == KQ_NVFP4; }
+
+// Wire geometry of a step (256 weights of a row) in LDS: piece p < PIECES - 1 holds bytes 16 p .., the last one the step's
+// last 16 bytes.  Rows are an odd number of pieces apart (a dummy piece where needed): conflict-free row-per-lane reads.
+template <int C>
+struct MidGeom {
+  static constexpr int WPB = kq_geom(C).wpb, BPB = kq_geom(C).bpb;
+  static constexpr int BYTES = CK_STEP / WPB * BPB;
+  static constexpr int PIECES = (BYTES + 15) / 16, LP = PIECES | 1, LROW = 16 * LP;
+  static constexpr int LOADS = (32 * LP + 63) / 64;
+  // activation order (see mid_prepass_kernel) and sum fragments per step
+  static constexpr int ORD = C == KQ_Q4_K || C == KQ_Q5_K || C == KQ_Q6_K                       ? 0
+                             : C == KQ_IQ4_NL || C == KQ_IQ4_XS || C == KQ_MXFP4 ? 2
+                             : C == KQ_NVFP4                                     ? 3
+                                                                                 : 1;
+  static constexpr int NSUM = C == KQ_Q2_K || C == KQ_Q3_K ? 2 : C == KQ_Q4_K || C == KQ_Q5_K || C == KQ_Q4_1 || C == KQ_Q5_1 ? 1 : 0;
+  static constexpr int NF = 16 + NSUM;  // fragments per step
+};
+template <int C>
+constexpr int mid_slot_bytes() { return MidGeom<C>::LROW * 32 > 4096 ? MidGeom<C>::LROW * 32 : 4096; }
+template <int C>
+constexpr int mid_table_bytes() {
+  if constexpr (k_quant<C>() || fp4<C>()) return 0;
+  else return CodeGeom<C>::GROUPED_GRID_BYTES + CodeGeom<C>::SPREAD_BYTES;
+}
+
+// ------------------------------------------------------------------ activation prepass
+// One workgroup per activation row m: f16 values scaled by the row's power of two (rs[m]) into fragment order,
+//   xf[(m / 32 * nsteps + step) * NF + J][lane = 32 kg + m % 32][8 halves]
+// ORD 0 (q4_k / q5_k / q6_k): fragment 2 j + s, half kg = weights 32 j + 16 kg + 8 s .. of the step; ORD 1: fragment J,
+// half kg = weights 16 J + 8 kg ..; both k0 k2 k1 k3 k4 k6 k5 k7 inside the eight; ORD 2: as ORD 1 with the positions of
+// x[j], x[j + 16] interleaved over every 32 (ORD 3: x[j], x[j + 8] over every 16).  NSUM 1: fragment 16 = sums of the eight 32-wide blocks, kg 0 the f16 part hi,
+// kg 1 the remainder lo, X = 32 (hi + lo); NSUM 2: fragments 16 / 17 = hi / lo of the sixteen 16-wide sums, X = 16 (hi + lo).
+// Rows past M are not written: what they hold reaches output rows that are not stored.
+constexpr int MP_THREADS = 512, MP_REGS = 4;
+
+template <int DT, int ORD, int NSUM>
+__global__ __launch_bounds__(MP_THREADS) void mid_prepass_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ xf,
+                                                                 float* __restrict__ rs, int K, int nsteps,
+                                                                 int* __restrict__ counters, int ncounters) {
+  constexpr int NF = 16 + NSUM;
+  __shared__ float red[MP_THREADS / 64];
+  const int m = blockIdx.x, tid = threadIdx.x;
+  // arrival counters of the main kernel's cut tiles
+  for (int i = m * MP_THREADS + tid; i < ncounters; i += gridDim.x * MP_THREADS) counters[i] = 0;
+  const uint16_t* xi = x + (size_t)m * K;
+  const int ngroups = 32 * nsteps;  // 8-weight groups, the step K ends in zero-filled
+  auto fetch = [&](int g) -> u32x4 {
+    return 8 * g < K ? *reinterpret_cast<const u32x4*>(xi + 8 * g) : u32x4{0, 0, 0, 0};
+  };
+  u32x4 keep[MP_REGS];
+#pragma unroll
+  for (int r = 0; r < MP_REGS; r++) {
+    const int g = tid + MP_THREADS * r;
+    keep[r] = g < ngroups ? fetch(g) : u32x4{0, 0, 0, 0};
+  }
+  float inv = 1.f, scale = 1.f;
+  if constexpr (DT == KQ_BF16) {
+    float amax = 0.f;
+    auto take = [&](u32x4 v) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] << 16)));
+        amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] & 0xffff0000u)));
+      }
+    };
+#pragma unroll
+    for (int r = 0; r < MP_REGS; r++) take(keep[r]);
+    for (int g = tid + MP_THREADS * MP_REGS; g < ngroups; g += MP_THREADS) take(fetch(g));
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    if ((tid & 63) == 0) red[tid >> 6] = amax;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < MP_THREADS / 64; w++) amax = fmaxf(amax, red[w]);
+    const uint32_t eb = (__builtin_bit_cast(uint32_t, amax) >> 23) & 0xff;
+    if (eb != 0 && eb != 0xff) {
+      int e = (int)eb - 127 - 14;  // the largest magnitude lands in [2^14, 2^15)
+      if (e < -100) e = -100;
+      scale = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
+      inv = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23);
+    }
+  }
+  if (tid == 0) rs[m] = scale;
+  uint8_t* base = xf + (size_t)(m >> 5) * nsteps * NF * 1024 + 16 * (m & 31);
+  auto convert = [&](int g, u32x4 v) {  // whole octets of lanes stay together
+    _Float16 h[8];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      if constexpr (DT == KQ_BF16) {
+        h[2 * e] = (_Float16)(__builtin_bit_cast(float, v[e] << 16) * inv);
+        h[2 * e + 1] = (_Float16)(__builtin_bit_cast(float, v[e] & 0xffff0000u) * inv);
+      } else {
+        h[2 * e] = __builtin_bit_cast(_Float16, (uint16_t)(v[e] & 0xffff));
+        h[2 * e + 1] = __builtin_bit_cast(_Float16, (uint16_t)(v[e] >> 16));
+      }
+    }
+    const int st = g >> 5, pc = g & 31;
+    uint8_t* step = base + (size_t)st * NF * 1024;
+    if constexpr (ORD >= 2) {
+      uint32_t own[4], par[4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        own[e] = (uint32_t)__builtin_bit_cast(uint16_t, h[2 * e]) | ((uint32_t)__builtin_bit_cast(uint16_t, h[2 * e + 1]) << 16);
+        // the neighbour two (ORD 3: one) groups on: quad_perm [2,3,0,1] or [1,0,3,2]
+        par[e] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)own[e], ORD == 2 ? 0x4E : 0xB1, 0xf, 0xf, true);
+      }
+      const bool high = (pc & (ORD == 2 ? 2 : 1)) != 0;
+      const uint32_t a0 = high ? par[2] : own[0], a1 = high ? par[3] : own[1];
+      const uint32_t b0 = high ? own[2] : par[0], b1 = high ? own[3] : par[1];
+      const u32x4 o = {(a0 & 0xffffu) | (b0 << 16), (a0 >> 16) | (b0 & 0xffff0000u), (a1 & 0xffffu) | (b1 << 16),
+                       (a1 >> 16) | (b1 & 0xffff0000u)};
+      const int pos = ORD == 2 ? 4 * (pc >> 2) + 2 * (pc & 1) + (high ? 1 : 0) : pc;
+      *reinterpret_cast<u32x4*>(step + (pos >> 1) * 1024 + (pos & 1) * 512) = o;
+    } else {
+      const int J = ORD == 0 ? 2 * (pc >> 2) + (pc & 1) : pc >> 1, kg = ORD == 0 ? (pc >> 1) & 1 : pc & 1;
+      *reinterpret_cast<f16x8*>(step + J * 1024 + kg * 512) = f16x8{h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
+    }
+    if constexpr (NSUM > 0) {
+      float s = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; e++) s += (float)h[e];
+      s += __shfl_xor(s, 1);
+      if constexpr (NSUM == 1) s += __shfl_xor(s, 2);
+      constexpr float unit = NSUM == 1 ? 32.0f : 16.0f;
+      const _Float16 hi = (_Float16)(s * (1.0f / unit)), lo = (_Float16)((s - unit * (float)hi) * (1.0f / unit));
+      if constexpr (NSUM == 1) {
+        if ((pc & 3) == 0) {
+          *reinterpret_cast<_Float16*>(step + 16 * 1024 + 2 * (pc >> 2)) = hi;
+          *reinterpret_cast<_Float16*>(step + 16 * 1024 + 512 + 2 * (pc >> 2)) = lo;
+        }
+      } else if ((pc & 1) == 0) {
+        const int sb = pc >> 1;
+        *reinterpret_cast<_Float16*>(step + 16 * 1024 + 512 * (sb >> 3) + 2 * (sb & 7)) = hi;
+        *reinterpret_cast<_Float16*>(step + 17 * 1024 + 512 * (sb >> 3) + 2 * (sb & 7)) = lo;
+      }
+    }
+  };
+#pragma unroll
+  for (int r = 0; r < MP_REGS; r++) {
+    const int g = tid + MP_THREADS * r;
+    if (g < ngroups) convert(g, keep[r]);
+  }
+  for (int g = tid + MP_THREADS * MP_REGS; g < ngroups; g += MP_THREADS) convert(g, fetch(g));
+}
+
+// ------------------------------------------------------------------ main kernel
+constexpr int MID_WAVES = 8;
+
+struct MidArgs {
+  const uint8_t* xf;
+  const float* rs;
+  const uint8_t* w;
+  uint16_t* y;
+  const uint8_t* grids;
+  int M, N, K;
+  int rpt;       // weight rows per tile (<= 32): fewer than 32 levels the rows over the workgroups
+  int items;     // tiles x 32-row blocks of activations x ranges of steps
+  int mblocks;
+  int splits, steps_per_split;
+  float* part;    // splits > 1: the ranges' sums, [item][1024] f32
+  int* counters;  // and the arrivals of every (tile, block), zero at the start
+};
+
+// Row bytes of a step from LDS into registers (codes of kq_codes.h).  The long blocks come in two halves, to leave
+// room for the activation fragments; the short ones whole, byte b being dword b / 4 again once the last piece has been
+// moved to where its bytes belong.
+template <int C>
+constexpr int row_parts() { return MidGeom<C>::BYTES >= 160 ? 2 : 1; }
+template <int C, int P>
+struct RowPart {
+  using G = MidGeom<C>;
+  static constexpr int LEN = G::BYTES / row_parts<C>(), BASE = P * LEN, NDW = (LEN + 15) / 16 * 4;
+  RowRegs<NDW> r;
+  template <int OFF>
+  __device__ __forceinline__ uint32_t u32() const { return r.template u32<OFF - BASE>(); }
+  template <int OFF>
+  __device__ __forceinline__ uint32_t u16() const { return r.template u16<OFF - BASE>(); }
+  template <int OFF>
+  __device__ __forceinline__ uint32_t u8() const { return r.template u8<OFF - BASE>(); }
+  __device__ __forceinline__ void load(const uint8_t* b) {
+    if constexpr (row_parts<C>() == 2) {
+      static_assert(row_parts<C>() == 1 || (G::BYTES % 16 == 0 && LEN % 8 == 0), "halves of whole pieces in 8-byte reads");
+#pragma unroll
+      for (int i = 0; i < LEN / 8; i++) {
+        const u32x2 v = *reinterpret_cast<const u32x2*>(b + BASE + 8 * i);
+        r.d[2 * i] = v[0];
+        r.d[2 * i + 1] = v[1];
+      }
+    } else {
+      constexpr int R = G::BYTES % 16;
+      StaticFor<G::PIECES>::run([&](auto pc) {
+        constexpr int p = decltype(pc)::value;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(b + 16 * p);
+        constexpr int sh = p < G::PIECES - 1 || R == 0 ? 0 : 16 - R;
+        const uint32_t e[5] = {v[0], v[1], v[2], v[3], 0u};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int q = sh / 4 + i;
+          r.d[4 * p + i] = q >= 4 ? 0u : sh % 4 == 0 ? e[q] : __builtin_amdgcn_alignbyte(e[q + 1], e[q], sh % 4);
+        }
+      });
+    }
+  }
+};
+
+// B operand of the fp4 codecs by the hardware's fp4 -> f16 conversion: a byte gives the pair of its two codes.  nvfp4:
+// times the 16-weight scale, an f16 number (its bits (x & 0x7f) << 7 read the e4m3 value / 256; 0x7f decodes to 0), so
+// nothing is left to do after the MFMA; mxfp4: the codes doubled, as the block scale expects them.
+template <int C, int J, class R>
+__device__ __forceinline__ f16x8 fp4_frag(const R& row, int kg) {
+  constexpr int off = C == KQ_NVFP4 ? (J / 4) * 36 + 4 + 8 * (J & 3) : (J / 2) * 17 + 1 + 8 * (J & 1);
+  const uint32_t w = pick(kg, row.template u32<off>(), row.template u32<off + 4>());
+  constexpr float cs = C == KQ_NVFP4 ? 1.0f : 2.0f;
+  f16x2 p[4];
+  p[0] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, cs, 0);
+  p[1] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, cs, 1);
+  p[2] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, cs, 2);
+  p[3] = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, cs, 3);
+  if constexpr (C == KQ_NVFP4) {
+    const uint32_t x = row.template u8<(J / 4) * 36 + (J & 3)>();
+    const uint32_t hb = x == 0x7fu ? 0u : (x & 0x7fu) << 7;
+    const f16x2 sp = __builtin_bit_cast(f16x2, hb | (hb << 16)) * f16x2{(_Float16)256.0f, (_Float16)256.0f};
+#pragma unroll
+    for (int e = 0; e < 4; e++) p[e] *= sp;
+  }
+  return f16x8{p[0][0], p[0][1], p[1][0], p[1][1], p[2][0], p[2][1], p[3][0], p[3][1]};
+}
+
+__device__ __forceinline__ void mid_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// acc += (32 weight rows of the step in LDS at b_lane) . (32 activation rows in the fragments a)
+template <int C>
+__device__ __forceinline__ void mid_step(const uint8_t* b_lane, int kg, const f16x8 (&a)[MidGeom<C>::NF], const Tables& tabs,
+                                         const kqfrag::KMasks& masks, int kvalid, f32x16& acc) {
+  if constexpr (k_quant<C>()) {
+    kqfrag::KRow<C> row;
+    row.load(b_lane, kg);
+    f32x16 part = f32x16{0};
+    StaticFor<16>::run([&](auto jc) {
+      constexpr int J = decltype(jc)::value;
+      f16x8 b[2];
+      row.template frag<J>(kg, masks, b);
+      part = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[J], b[0], part, 0, 0, 0);
+      if constexpr (kqfrag::KRow<C>::TERMS == 2) part = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[J], b[1], part, 0, 0, 0);
+    });
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[i] = fmaf(row.d, part[i], acc[i]);
+    if constexpr (kqfrag::KRow<C>::NSUM > 0) {
+      const f16x8 m = row.template min_frag<0>(kg);
+      part = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[16], m, f32x16{0}, 0, 0, 0);
+      if constexpr (kqfrag::KRow<C>::NSUM == 2) part = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[17], m, part, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[i] = fmaf(row.dm, part[i], acc[i]);
+    }
+  } else {
+    using G = CodeGeom<C>;
+    constexpr int MPS = G::SB / 16, PARTS = row_parts<C>(), JP = 16 / PARTS;
+    auto run = [&](auto full_c) {
+      constexpr bool FULL = decltype(full_c)::value;
+      f32x16 part[2];
+      f16x8 mins = {};
+      StaticFor<PARTS>::run([&](auto pc) {
+        constexpr int P = decltype(pc)::value;
+        RowPart<C, P> row;
+        row.load(b_lane);
+        StaticFor<JP>::run([&](auto jc) {
+          constexpr int J = P * JP + decltype(jc)::value;
+          if (FULL || 16 * J < kvalid) {  // uniform
+            if constexpr (C == KQ_NVFP4) {
+              acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[J], fp4_frag<C, J>(row, kg), acc, 0, 0, 0);
+              return;
+            }
+            f16x8 b;
+            if constexpr (C == KQ_MXFP4) b = fp4_frag<C, J>(row, kg);
+            else b = codes<C, J>(row, kg, tabs);
+            constexpr int sbi = J / MPS, slot = sbi & 1;
+            if constexpr (J % MPS == 0)
+              part[slot] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[J], b, f32x16{0}, 0, 0, 0);
+            else
+              part[slot] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[J], b, part[slot], 0, 0, 0);
+            if constexpr (J % MPS == MPS - 1) {
+              float mn;
+              const float sc = block_scale<C, sbi>(row, mn);
+#pragma unroll
+              for (int i = 0; i < 16; i++) acc[i] = fmaf(sc, part[slot][i], acc[i]);
+              if constexpr (G::HAS_MIN) mins[sbi] = (_Float16)mn;  // the f16 it came from
+            }
+          }
+        });
+      });
+      if constexpr (G::HAS_MIN) {  // blocks past the end of K: minimum 0 on sums of zeros
+        part[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[16], mins, f32x16{0}, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[i] = fmaf(32.0f, part[0][i], acc[i]);
+      }
+    };
+    if (kvalid >= CK_STEP)
+      run(std::true_type{});
+    else
+      run(std::false_type{});
+  }
+}
+
+template <int C, int DT>
+__global__ __launch_bounds__(64 * MID_WAVES, 1) void mid_kernel(MidArgs a) {
+  using G = MidGeom<C>;
+  constexpr int SLOT = mid_slot_bytes<C>(), NW = MID_WAVES, NT = 64 * NW;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  uint8_t* ring = smem + mid_table_bytes<C>();
+  int* which = reinterpret_cast<int*>(ring + NW * 2 * SLOT);  // [NW] slot a wave's sums lie in, [NW] = last arrival
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, kg = lane >> 5;
+  const int N = a.N, K = a.K, rpt = a.rpt, mblocks = a.mblocks, G_x = gridDim.x;
+  const int nsteps = (K + CK_STEP - 1) / CK_STEP;
+  const uint32_t row_bytes = (uint32_t)(K / G::WPB) * G::BPB;
+  const uint32_t slot_lds = lds_addr(ring + wave * 2 * SLOT);
+
+  kqfrag::KMasks masks;
+  masks.init<C>();
+  Tables tabs{smem, smem, 2};
+  if constexpr (mid_table_bytes<C>() > 0) {
+    uint8_t* spread = smem + CodeGeom<C>::GROUPED_GRID_BYTES;
+    build_tables<C, NT, true>(smem, spread, a.grids, tid);
+    tabs = Tables{CodeGeom<C>::PAIR_LUT ? smem + 4 * l32 : smem, spread, 7};
+    lds_barrier();
+  }
+
+  // a position of the stream: item (tile, block of activation rows, range of steps) and step of the item's range
+  struct Pos {
+    int id, st, end;
+  };
+  // (tile, block)s run over (group of 8 tiles, block, tile of the group): workgroups go to the 8 XCDs in turn, so the
+  // blocks of a tile meet in one L2
+  auto tile_of = [&](int id, int& tile, int& mb) {
+    const int t = id / a.splits, g = t / (8 * mblocks), r = t - g * 8 * mblocks;
+    mb = r >> 3;
+    tile = 8 * g + (r & 7);
+  };
+  const int ntiles = (N + rpt - 1) / rpt;
+  auto first = [&](int id) {
+    int tile, mb;
+    tile_of(id, tile, mb);
+    const int s0 = (id % a.splits) * a.steps_per_split;
+    const int s1 = s0 + a.steps_per_split < nsteps ? s0 + a.steps_per_split : nsteps;
+    // st >= end: this wave has no step in the item (or the item is a gap) and only joins the barriers
+    return Pos{id, s0 + wave, tile < ntiles ? s1 : 0};
+  };
+  auto advance = [&](Pos p) {
+    p.st += NW;
+    return p.st < p.end ? p : first(p.id + G_x);
+  };
+  uint32_t voff[G::LOADS];
+  StaticFor<G::LOADS>::run([&](auto tc) {
+    constexpr int T = decltype(tc)::value;
+    const int i = lane + 64 * T, r = i / G::LP, p = i - r * G::LP;
+    const int off = 16 * p < G::BYTES - 16 ? 16 * p : G::BYTES - 16;
+    voff[T] = (uint32_t)r * row_bytes + (uint32_t)off;
+  });
+  auto request = [&](Pos p, int slot, f16x8 (&an)[G::NF]) {
+    int tile, mb;
+    tile_of(p.id, tile, mb);
+    if (p.st >= p.end) return;
+    const int row0 = tile * rpt, nrows = N - row0 < rpt ? N - row0 : rpt;
+    const uint8_t* base = a.w + (size_t)row0 * row_bytes + (size_t)p.st * G::BYTES;
+    const uint32_t l0 = slot_lds + slot * SLOT;
+    const bool ragged_end = (K & (CK_STEP - 1)) != 0 && p.st == nsteps - 1 && row0 + nrows == N;
+    if (!ragged_end) {
+      StaticFor<G::LOADS>::run([&](auto tc) {
+        constexpr int T = decltype(tc)::value;
+        if (64 * T + lane < nrows * G::LP) dma16(base, voff[T], l0 + 1024 * T);
+      });
+    } else {
+      // the matrix ends inside this step: nothing past its last byte is read
+      const int valid = (K - CK_STEP * p.st) / G::WPB * G::BPB;  // bytes of the step that exist in a row
+      uint8_t* dst = ring + wave * 2 * SLOT + slot * SLOT;
+      for (int i = lane; i < nrows * G::LP; i += 64) {
+        const int r = i / G::LP, pc = i - r * G::LP;
+        const int off = 16 * pc < G::BYTES - 16 ? 16 * pc : G::BYTES - 16;
+        u32x4 v = {0, 0, 0, 0};
+        for (int t = 0; t < 16; t++)
+          if (off + t < valid) v[t >> 2] |= (uint32_t)base[(size_t)r * row_bytes + off + t] << (8 * (t & 3));
+        *reinterpret_cast<u32x4*>(dst + 16 * i) = v;
+      }
+      mid_wave_sync();
+    }
+    const uint8_t* fr = a.xf + ((size_t)mb * nsteps + p.st) * (G::NF * 1024) + 16 * lane;
+#pragma unroll
+    for (int j = 0; j < G::NF; j++) an[j] = *reinterpret_cast<const f16x8*>(fr + 1024 * j);
+  };
+
+  f32x16 acc = f32x16{0};
+  auto finish_tile = [&](int id, int slot) {
+    // the waves' sums meet in the slots just read (a wave's other slot may be receiving its next step)
+    float* mine = reinterpret_cast<float*>(ring + (wave * 2 + slot) * SLOT);
+#pragma unroll
+    for (int i = 0; i < 16; i++) mine[i * 64 + lane] = acc[i];
+    acc = f32x16{0};
+    if (lane == 0) which[wave] = slot;
+    lds_barrier();
+    int tile, mb;
+    tile_of(id, tile, mb);
+    const int row0 = tile * rpt, nrows = N - row0 < rpt ? N - row0 : rpt;
+    auto store = [&](int e, float v) {
+      const int i = e >> 6, l = e & 63;
+      const int m = 32 * mb + 8 * (i >> 2) + 4 * (l >> 5) + (i & 3), c = l & 31;
+      if (m < a.M && c < nrows && tile < ntiles) {
+        v *= a.rs[m];
+        a.y[(size_t)m * N + row0 + c] = DT == KQ_F16 ? kq::f2f16(v) : kq::f2bf16(v);
+      }
+    };
+    static_assert(1024 % NT == 0, "whole passes over the tile");
+    float v[1024 / NT];
+#pragma unroll
+    for (int k = 0; k < 1024 / NT; k++) {
+      v[k] = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; w++) v[k] += reinterpret_cast<const float*>(ring + (w * 2 + which[w]) * SLOT)[tid + NT * k];
+    }
+    if (a.splits == 1) {
+#pragma unroll
+      for (int k = 0; k < 1024 / NT; k++) store(tid + NT * k, v[k]);
+      lds_barrier();
+      return;
+    }
+    // The ranges of a tile are added by the workgroup that arrives last.  The sums travel in device-scope atomic
+    // stores and loads, which bypass the L2s (one per XCD, not coherent with each other); a wave counts as arrived
+    // once its stores have been acknowledged.  No fence: that would write back a whole L2.
+    float* part = a.part + (size_t)id * 1024;
+#pragma unroll
+    for (int k = 0; k < 1024 / NT; k++)
+      __hip_atomic_store(part + tid + NT * k, v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    vmwait<0>();
+    lds_barrier();
+    if (tid == 0)
+      which[NW] = __hip_atomic_fetch_add(a.counters + id / a.splits, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.splits - 1;
+    lds_barrier();
+    if (which[NW]) {
+      const float* p0 = a.part + (size_t)(id - id % a.splits) * 1024;
+#pragma unroll
+      for (int k = 0; k < 1024 / NT; k++) {
+        float sum = 0.f;
+        for (int r = 0; r < a.splits; r++)
+          sum += __hip_atomic_load(p0 + (size_t)r * 1024 + tid + NT * k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        store(tid + NT * k, sum);
+      }
+    }
+    lds_barrier();
+  };
+
+  f16x8 a0[G::NF], a1[G::NF];
+#pragma unroll
+  for (int j = 0; j < G::NF; j++) a0[j] = a1[j] = f16x8{};
+  Pos cur = first(blockIdx.x);
+  request(cur, 0, a0);
+  // one step: wait for it, ask for the next one, multiply
+  auto body = [&](f16x8 (&ac)[G::NF], f16x8 (&an)[G::NF], int slot) -> bool {
+    vmwait<0>();
+    lgkm_drain();  // the other slot has been read: it may be filled again
+#pragma unroll
+    for (int j = 0; j < G::NF; j++) asm volatile("" : "+v"(ac[j]));
+    const Pos nxt = advance(cur);
+    const bool more = nxt.id < a.items;
+    if (more) request(nxt, slot ^ 1, an);
+    if (cur.st < cur.end)
+      mid_step<C>(ring + (wave * 2 + slot) * SLOT + l32 * G::LROW, kg, ac, tabs, masks, K - CK_STEP * cur.st, acc);
+    if (nxt.id != cur.id) {
+      mid_wave_sync();
+      finish_tile(cur.id, slot);
+    }
+    cur = nxt;
+    return more;
+  };
+  while (true) {
+    if (!body(a0, a1, 0)) break;
+    if (!body(a1, a0, 1)) break;
+  }
+}
+
+int mid_cus() {
+  static std::atomic<int> cus[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cus[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cus[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+size_t mid_align(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// Tiles, ranges and workgroups of a call.  At least one tile per CU: 32-row tiles dealt out in rounds, levelled to the
+// same number of rows.  Fewer: the steps are cut into ranges of two or more per wave, as many as fill the CUs; a K too
+// short for that takes shorter tiles (some lanes then decode for nobody, but more CUs pull).  q4_k, 32 rows, us, prepass
+// included: 4096 rows of K = 14336 on 16-row tiles 23.5, cut in two 20.7; of K = 4096 (one step per wave when cut) 11.2
+// and 11.7.
+struct MidPlan {
+  int rpt, ntiles, splits, steps_per_split, items, grid;
+};
+MidPlan mid_plan(int M, int N, int K) {
+  MidPlan p;
+  const int cus = mid_cus(), mblocks = (M + 31) / 32, nsteps = (K + CK_STEP - 1) / CK_STEP;
+  const int t32 = (N + 31) / 32 * mblocks;
+  p.splits = 1;
+  if (t32 < cus) p.splits = std::max(1, std::min(cus / t32, nsteps / (2 * MID_WAVES)));
+  p.steps_per_split = (nsteps + p.splits - 1) / p.splits;
+  p.splits = (nsteps + p.steps_per_split - 1) / p.steps_per_split;
+  p.rpt = 32;
+  if (p.splits == 1) {
+    const int64_t rounds = (t32 + cus - 1) / cus;
+    const int rpt = (int)((((int64_t)N * mblocks + cus * rounds - 1) / (cus * rounds) + 3) & ~3);
+    p.rpt = rpt < 8 ? 8 : rpt > 32 ? 32 : rpt;
+    // (the last tile and the last group of eight may be partly empty)
+    while (p.rpt < 32 && (int64_t)((N + p.rpt - 1) / p.rpt + 7) / 8 * 8 * mblocks > cus * rounds) p.rpt += 4;
+  }
+  p.ntiles = (N + p.rpt - 1) / p.rpt;
+  p.items = (p.ntiles + 7) / 8 * 8 * mblocks * p.splits;  // gaps in the last group of eight tiles included
+  p.grid = p.items < cus ? p.items : cus;
+  return p;
+}
+
+template <int C, int DT>
+int launch_mid(const void* x, MidArgs a, uint8_t* xf, float* rs, hipStream_t s) {
+  using G = MidGeom<C>;
+  constexpr size_t lds = (size_t)mid_table_bytes<C>() + (size_t)MID_WAVES * 2 * mid_slot_bytes<C>() + 64;
+  static_assert(lds <= 160 * 1024, "the ring does not fit the LDS of a CU");
+  const int nsteps = (a.K + CK_STEP - 1) / CK_STEP;
+  const MidPlan p = mid_plan(a.M, a.N, a.K);
+  a.rpt = p.rpt;
+  a.items = p.items;
+  a.splits = p.splits;
+  a.steps_per_split = p.steps_per_split;
+  const int ncounters = p.splits > 1 ? p.items / p.splits : 0;
+  a.part = reinterpret_cast<float*>(a.counters + mid_align((size_t)ncounters * 4) / 4);
+  hipLaunchKernelGGL((mid_prepass_kernel<DT, G::ORD, G::NSUM>), dim3(a.M), dim3(MP_THREADS), 0, s,
+                     static_cast<const uint16_t*>(x), xf, rs, a.K, nsteps, a.counters, ncounters);
+  KQ_HIP_CHECK(hipGetLastError());
+  auto kern = mid_kernel<C, DT>;
+  KQ_SET_MAX_LDS_ONCE((kern), lds);
+  hipLaunchKernelGGL(kern, dim3(p.grid), dim3(64 * MID_WAVES), lds, s, a);
+  KQ_HIP_CHECK(hipGetLastError());
+  return KQ_OK;
+}
+
+}  // namespace
+
+static int g_mid_tile = 0;  // 32: every call the kernel can run; another forced tile: none
+void kq_mid_force_tile(int rows) { g_mid_tile = rows; }
+
+bool kq_mid_supported(int M, int N, int K, int codec) {
+  if (g_mid_tile != 0 && g_mid_tile != 32) return false;
+  if (codec < 0 || codec >= KQ_NUM_CODECS || M <= 8 || N < 8 || K < CK_STEP || K % kq_geom(codec).wpb) return false;
+  const int64_t row_bytes = (int64_t)(K / kq_geom(codec).wpb) * kq_geom(codec).bpb;
+  if (row_bytes & 1) return false;  // the direct-to-LDS loads take 2-byte aligned addresses
+  if (row_bytes * 32 >= ((int64_t)1 << 31) || (int64_t)N * ((M + 31) / 32) >= ((int64_t)1 << 31)) return false;
+  if (g_mid_tile == 32) return M <= KQ_MID_MAX_ROWS;
+  // Against the tile GEMMs, us at 32 / 64 / 128 rows: q4_k 4096^2 11 / 13 / 18 (64-row kernel 19 / 23 / 25), 28672 x 8192
+  // 55 / 84 / 149 (64 / 70 / 114): from two row blocks on the tile GEMM of the K-quants with exact integers is ahead on
+  // the large matrices, where a weight decoded once per 64 rows counts.  The any-codec kernel the others have there is
+  // behind on every shape: mxfp4 28672 x 8192 56 / 85 / 147 (131 / 164 / 298), q8_0 77 / 113 / 193 (114 / 136 / 229).
+  const bool tile_gemm = codec == KQ_Q4_K || codec == KQ_Q5_K || codec == KQ_Q6_K;
+  if (tile_gemm) return M <= 32 || (M <= 64 && (int64_t)N * K <= (int64_t)64 << 20);
+  return M <= KQ_MID_MAX_ROWS;
+}
+
+size_t kq_mid_workspace_bytes(int M, int N, int K) {
+  const size_t mb = (M + 31) / 32, nsteps = (K + CK_STEP - 1) / CK_STEP;
+  const MidPlan p = mid_plan(M, N, K);
+  const size_t cut = p.splits > 1 ? mid_align((size_t)(p.items / p.splits) * 4) + (size_t)p.items * 4096 : 0;
+  return mid_align(mb * nsteps * 18 * 1024) + mid_align(mb * 32 * 4) + cut;
+}
+
+int kq_launch_mid(const void* x, const uint8_t* w, void* y, int M, int N, int K, int codec, int dtype, void* ws, hipStream_t s) {
+  if (!kq_mid_supported(M, N, K, codec) || (reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(ws) & 15) ||
+      (reinterpret_cast<uintptr_t>(w) & 1) || (K & 7))
+    return KQ_ERR_UNSUPPORTED;
+  const size_t mb = (M + 31) / 32, nsteps = (K + CK_STEP - 1) / CK_STEP;
+  uint8_t* xf = static_cast<uint8_t*>(ws);
+  float* rs = reinterpret_cast<float*>(xf + mid_align(mb * nsteps * 18 * 1024));
+  MidArgs a{};
+  a.xf = xf;
+  a.rs = rs;
+  a.w = w;
+  a.y = static_cast<uint16_t*>(y);
+  a.grids = kq_device_grids();
+  if (!a.grids) return KQ_ERR_HIP;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.mblocks = (int)mb;
+  a.counters = reinterpret_cast<int*>(reinterpret_cast<uint8_t*>(rs) + mid_align(mb * 32 * 4));
+  switch (codec) {
+#define KQ_CASE(c) \
+  case c:          \
+    return dtype == KQ_F16 ? launch_mid<c, KQ_F16>(x, a, xf, rs, s) : launch_mid<c, KQ_BF16>(x, a, xf, rs, s);
+    KQ_CASE(KQ_Q2_K) KQ_CASE(KQ_Q3_K) KQ_CASE(KQ_Q4_K) KQ_CASE(KQ_Q5_K) KQ_CASE(KQ_Q6_K) KQ_CASE(KQ_Q4_0) KQ_CASE(KQ_Q4_1)
+    KQ_CASE(KQ_Q5_0) KQ_CASE(KQ_Q5_1) KQ_CASE(KQ_Q8_0) KQ_CASE(KQ_IQ4_NL) KQ_CASE(KQ_IQ4_XS) KQ_CASE(KQ_IQ3_S)
+    KQ_CASE(KQ_IQ3_XXS) KQ_CASE(KQ_IQ2_XXS) KQ_CASE(KQ_IQ2_XS) KQ_CASE(KQ_IQ2_S) KQ_CASE(KQ_IQ1_S) KQ_CASE(KQ_IQ1_M)
+    KQ_CASE(KQ_MXFP4) KQ_CASE(KQ_NVFP4)
+#undef KQ_CASE
+  }
+  return KQ_ERR_UNSUPPORTED;
+}

@@ -1,0 +1,75 @@
+"""GPU parity of the matmul between the skinny kernels and the tile GEMMs (9 ... 128 activation rows) at the places where
+its tiling can go wrong: one weight row and one step, a ragged last tile, K ending inside a step, several rounds of
+persistent workgroups, steps cut over workgroups (also under graph replay), one to four blocks of activation rows."""
+import pytest
+import torch
+
+import oracle_lib as O
+from gpu_util import dev_to_bits, make_x, rel_l2, wire_to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def kq():
+    import kq as _kq
+    return _kq
+
+
+@pytest.fixture
+def mid(kq):
+    import ctypes
+    f = kq._load().kq_set_gemm_tile_rows
+    f.argtypes = [ctypes.c_int]
+    f(32)
+    yield kq
+    f(0)
+
+
+def all_codecs():
+    from kq.codec_geometry import CODEC_GEOMETRY
+    return sorted(CODEC_GEOMETRY)
+
+
+@pytest.mark.parametrize("codec", all_codecs())
+def test_mid_rows_edges(mid, codec):
+    wpb = mid.CODEC_GEOMETRY[codec][3]
+    # (rows, N, K): the least of everything; ragged tile, two row blocks and a K tail; cut steps; several rounds
+    shapes = [(9, 8, 256), (33, 1003, 2048 + (wpb if wpb < 256 else 256)), (32, 96, 8192), (12, 8205, 512)]
+    for i, (M, N, K) in enumerate(shapes):
+        dtype = "bfloat16" if i % 2 == 0 else "float16"
+        wire = O.synth_wire(codec, N * K // wpb, seed=40 + i).reshape(N, -1)
+        xb, xt = make_x((M, K), dtype, seed=50 + i)
+        got = dev_to_bits(mid.quantized_matmul(xt, wire_to_dev(wire), None, codec))
+        err = rel_l2(got, O.qmm(xb, wire, codec, True, dtype), dtype)
+        assert err <= 1e-3, (codec, M, N, K, err)
+
+
+@pytest.mark.parametrize("M", [31, 64, 65, 128])
+def test_mid_row_blocks(mid, M):
+    N, K = 264, 1024
+    wire = O.synth_wire("q4_k", N * K // 256, seed=3).reshape(N, -1)
+    xb, xt = make_x((M, K), "bfloat16", seed=4)
+    got = dev_to_bits(mid.quantized_matmul(xt, wire_to_dev(wire), None, "q4_k"))
+    assert rel_l2(got, O.qmm(xb, wire, "q4_k", True, "bfloat16"), "bfloat16") <= 1e-3
+
+
+def test_mid_cut_steps_replay(mid):
+    """The arrival counters are set anew by every call: replays of a captured call on changing inputs equal eager calls."""
+    N, K, M = 512, 12288, 17
+    w = wire_to_dev(O.synth_wire("q6_k", N * K // 256, seed=5).reshape(N, -1))
+    xs = [make_x((M, K), "bfloat16", seed=60 + i)[1] for i in range(4)]
+    want = [mid.quantized_matmul(x, w, None, "q6_k") for x in xs]
+    buf = xs[0].clone()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        mid.quantized_matmul(buf, w, None, "q6_k")
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = mid.quantized_matmul(buf, w, None, "q6_k")
+    for r in range(8):
+        buf.copy_(xs[r % 4])
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[r % 4]), r
