@@ -12,6 +12,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "lib", "libkq.so")
+HOST = os.path.join(HERE, "lib", "_kqhost.so")
 BLOB = os.path.join(HERE, "data", "kq_iq_grids.bin")
 
 # (source, extra flags[, object name]).  kq_generic.hip holds the bit-exact decoders: no FMA contraction.
@@ -82,12 +83,35 @@ def _compile(item):
     return out
 
 
+def build_host():
+    """The native call path of the Python ops (kq_host.cpp): host code only, against torch's C++ headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-fPIC", "-shared", "-std=c++17", "-fvisibility=hidden", "-Wall",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-I", os.path.join(ROOT, "include"),
+           "-I", sysconfig.get_paths()["include"]]
+    for p in include_paths():
+        cmd += ["-isystem", p]
+    cmd += [os.path.join(CSRC, "kq_host.cpp"), "-o", HOST, "-L", libs, "-ltorch_python", "-ltorch_cpu", "-lc10", "-ldl"]
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed for kq_host.cpp:\n" + r.stdout)
+    if r.stdout.strip():
+        print(r.stdout)
+
+
 def build_all(verbose=True):
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(os.path.dirname(LIB), exist_ok=True)
     _write_grid_inc()
     with ThreadPoolExecutor(max_workers=6) as ex:
+        host = ex.submit(build_host)
         objs = list(ex.map(_compile, SOURCES))
+        host.result()
     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if r.returncode != 0:

@@ -988,3 +988,131 @@ for _name in ("dequantize", "quantized_matmul", "quantized_matmul_qmv_bias", "ga
               "gather_qmv_bias", "gather_qmv_mix_bias", "moe_router_topk", "quantize"):
     globals()[_name] = _on_stream(globals()[_name])
 del _name
+
+
+# ------------------------------------------------------------------ native call path
+# The ops a model calls per layer and step go through csrc/kq_host.cpp first: it takes the ordinary call (contiguous
+# tensors of the op's own types on the current device, no gradient, no stream argument) from the tensors to the C ABI
+# without the interpreter in between, and answers None for every other one, invalid ones included, which the functions
+# above then convert or refuse as ever.  A q4_k matmul of one row on 4096 x 4096, host us per call: 16.5 through the
+# function above, 6.5 here.
+_HOST_PATH = os.path.join(os.path.dirname(_HERE), "lib", "_kqhost.so")
+
+
+class _Native:
+    """The functions of kq_host.cpp; loaded with libkq at the first call."""
+
+    def __getattr__(self, name):
+        from importlib.machinery import ExtensionFileLoader
+        from importlib.util import module_from_spec, spec_from_file_location
+        if not os.path.exists(_HOST_PATH):
+            raise RuntimeError(f"[kq] {_HOST_PATH} is missing: build it with `python mlx-kquant_amd/build.py`")
+        lib = _load()
+        mod = module_from_spec(spec_from_file_location("_kqhost", _HOST_PATH, loader=ExtensionFileLoader("_kqhost", _HOST_PATH)))
+        mod.init(lib._handle, torch._C._cuda_getCurrentRawStream)
+        for k in ("qmm", "dequantize", "gather_qmm", "moe_glu", "gather_qmv", "moe_glu_shexp", "mix", "router", "quantize"):
+            setattr(self, k, getattr(mod, k))
+        return self.__dict__[name]
+
+
+_native = _Native()
+_SCORINGS = {"softmax": 0, "sqrtsoftplus": 1}
+_checked = {_n: globals()[_n] for _n in ("dequantize", "quantized_matmul", "gather_qmm", "moe_glu_gather_kq", "gather_qmv_kq",
+                                          "moe_glu_gather_shexp_kq", "gather_qmv_mix_kq", "gather_qmv_mix_ns_kq",
+                                          "moe_router_topk", "quantize")}
+_qmm_checked = _checked["quantized_matmul"]
+
+
+def quantized_matmul(x, w, scales, kquant_type, transpose=True, *, stream=None):
+    if stream is None:
+        y = _native.qmm(x, w, kquant_type, transpose)
+        if y is not None:
+            return y
+    return _qmm_checked(x, w, scales, kquant_type, transpose, stream=stream)
+
+
+def dequantize(w, scales, kquant_type, dtype=None, *, stream=None):
+    if stream is None:
+        code = KQ_F16 if dtype is None else _DT.get(dtype)
+        y = _native.dequantize(w, kquant_type, code) if code is not None else None
+        if y is not None:
+            return y
+    return _checked["dequantize"](w, scales, kquant_type, dtype, stream=stream)
+
+
+def gather_qmm(x, w, scales, kquant_type, lhs_indices=None, rhs_indices=None, transpose=True,
+               sorted_indices=False, *, stream=None):
+    if stream is None and lhs_indices is not None and rhs_indices is not None:
+        y = _native.gather_qmm(x, w, kquant_type, lhs_indices, rhs_indices, transpose)
+        if y is not None:
+            return y
+    return _checked["gather_qmm"](x, w, scales, kquant_type, lhs_indices, rhs_indices, transpose, sorted_indices,
+                                  stream=stream)
+
+
+def moe_glu_gather_kq(x, gate_w, up_w, kquant_type, indices, act="silu", limit=0.0, gate_bias=None, up_bias=None,
+                      alpha=0.0, *, stream=None):
+    if stream is None and act in _ACTS:
+        y = _native.moe_glu(x, gate_w, up_w, kquant_type, indices, _ACTS[act], limit, gate_bias, up_bias, alpha)
+        if y is not None:
+            return y
+    return _checked["moe_glu_gather_kq"](x, gate_w, up_w, kquant_type, indices, act, limit, gate_bias, up_bias, alpha,
+                                         stream=stream)
+
+
+def gather_qmv_kq(x, w, kquant_type, indices, bias=None, *, stream=None):
+    if stream is None:
+        y = _native.gather_qmv(x, w, kquant_type, indices, bias)
+        if y is not None:
+            return y
+    return _checked["gather_qmv_kq"](x, w, kquant_type, indices, bias, stream=stream)
+
+
+def moe_glu_gather_shexp_kq(x, gate_w, up_w, shexp_gate_w, shexp_up_w, kquant_type, indices, act="silu",
+                            shexp_kquant_type="", *, stream=None):
+    if stream is None and act in _ACTS:
+        y = _native.moe_glu_shexp(x, gate_w, up_w, shexp_gate_w, shexp_up_w, kquant_type, indices, _ACTS[act],
+                                  shexp_kquant_type or "")
+        if y is not None:
+            return y
+    return _checked["moe_glu_gather_shexp_kq"](x, gate_w, up_w, shexp_gate_w, shexp_up_w, kquant_type, indices, act,
+                                               shexp_kquant_type, stream=stream)
+
+
+def gather_qmv_mix_kq(x, w, shexp_w, kquant_type, indices, scores, shexp_kquant_type="", *, stream=None):
+    if stream is None and shexp_w is not None:
+        y = _native.mix(x, w, shexp_w, kquant_type, shexp_kquant_type or "", indices, scores)
+        if y is not None:
+            return y
+    return _checked["gather_qmv_mix_kq"](x, w, shexp_w, kquant_type, indices, scores, shexp_kquant_type, stream=stream)
+
+
+def gather_qmv_mix_ns_kq(x, w, kquant_type, indices, scores, *, stream=None):
+    if stream is None:
+        y = _native.mix(x, w, None, kquant_type, "", indices, scores)
+        if y is not None:
+            return y
+    return _checked["gather_qmv_mix_ns_kq"](x, w, kquant_type, indices, scores, stream=stream)
+
+
+def moe_router_topk(logits, top_k, norm_topk_prob, shared_gate=True, per_expert_scale=None, bias=None,
+                    scoring="softmax", scale=1.0, *, stream=None):
+    if stream is None and scoring in _SCORINGS:
+        r = _native.router(logits, top_k, norm_topk_prob, shared_gate, per_expert_scale, bias, _SCORINGS[scoring], scale)
+        if r is not None:
+            return r
+    return _checked["moe_router_topk"](logits, top_k, norm_topk_prob, shared_gate, per_expert_scale, bias, scoring, scale,
+                                       stream=stream)
+
+
+def quantize(w, kquant_type, imatrix=None, *, stream=None):
+    if stream is None:
+        wire = _native.quantize(w, kquant_type, imatrix)
+        if wire is not None:
+            return wire, torch.zeros(1, dtype=torch.uint8, device=w.device)
+    return _checked["quantize"](w, kquant_type, imatrix, stream=stream)
+
+
+for _n, _f in _checked.items():
+    globals()[_n].__doc__ = _f.__doc__
+del _n, _f

@@ -118,7 +118,8 @@ class KQuantLinear(_KQuantBase):
         # decode (one row) with a real bias on q8_0: the add is fused into the matvec (reference :122-140)
         if self.bias is not None and self.kquant_type == "q8_0" and x.numel() // x.shape[-1] == 1:
             return kq.quantized_matmul_qmv_bias(x, self.weight, self.scales, self.bias, self.kquant_type)
-        y = kq.quantized_matmul(x, self.weight, self.scales, self.kquant_type, transpose=True)
+        b = self._buffers  # (attribute lookups of buffers go through Module.__getattr__)
+        y = kq.quantized_matmul(x, b["weight"], b["scales"], self.kquant_type)
         if self.bias is not None:
             y = y + self.bias
         return y
@@ -185,11 +186,12 @@ class KQuantMultiLinear(_KQuantBase):
         if cached is not None and cached[0] == (B, Hx, x.device):
             lhs, rhs = cached[1], cached[2]
         else:
-            rhs = torch.arange(nh, dtype=torch.int64, device=x.device).reshape(1, nh).expand(B, nh)
+            # int32 and packed: what the op reads, so that it converts nothing per call
+            rhs = torch.arange(nh, dtype=torch.int32, device=x.device).repeat(B, 1)
             if Hx == nh:
-                lhs = torch.arange(B * nh, dtype=torch.int64, device=x.device).reshape(B, nh)
+                lhs = torch.arange(B * nh, dtype=torch.int32, device=x.device).reshape(B, nh)
             elif Hx == 1:
-                lhs = torch.arange(B, dtype=torch.int64, device=x.device).reshape(B, 1).expand(B, nh)
+                lhs = torch.arange(B, dtype=torch.int32, device=x.device).reshape(B, 1).repeat(1, nh)
             else:
                 raise ValueError(f"KQuantMultiLinear: head axis {Hx} is neither 1 nor num_heads={nh} "
                                  f"(x.shape={tuple(x.shape)})")
