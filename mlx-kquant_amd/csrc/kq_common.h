@@ -138,7 +138,8 @@ int kq_launch_gather_tuned(const void* x, const uint8_t* w, const uint8_t* w2, c
                            int dtype, int E, KqOutMap om, hipStream_t s);
 // Every codec, 9 ... KQ_MID_MAX_ROWS activation rows: waves stream the weights, one launch behind a prepass that puts the
 // activations into ws (kq_mid_workspace_bytes) in matrix-operand order (kq_mid.hip).
-#define KQ_MID_MAX_ROWS 128
+#define KQ_MID_MAX_ROWS 512
+bool kq_tall_fills(int M, int N, int codec);  // the rule between it and the tall-tile GEMMs
 bool kq_mid_supported(int M, int N, int K, int codec);
 size_t kq_mid_workspace_bytes(int M, int N, int K);
 void kq_mid_force_tile(int rows);

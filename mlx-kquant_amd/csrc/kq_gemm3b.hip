@@ -414,8 +414,8 @@ int launch_b3_call(const void* x, const uint8_t* w, void* y, int M, int N, int K
 
 }  // namespace
 
-// Taken for calls of 128 rows or more whose half-height tiles fill three quarters of the CUs; smaller calls stay on
-// the any-codec kernel (small workgroups, K cut over the grid).
+// Taken for calls of 128 rows or more whose half-height tiles fill enough of the CUs (kq_tall_fills); smaller calls stay
+// on the streamed kernel or, beyond its rows, the any-codec kernel.
 bool kq_gemm3b_supported(int M, int N, int K, int codec) {
   if (codec != KQ_Q8_0 && codec != KQ_Q4_0 && codec != KQ_IQ4_NL && codec != KQ_Q4_1 && codec != KQ_Q5_0 && codec != KQ_Q5_1)
     return false;
@@ -423,7 +423,7 @@ bool kq_gemm3b_supported(int M, int N, int K, int codec) {
   const int64_t row_bytes = (int64_t)(K >> 5) * 34;  // the largest block of the six
   if (256 * row_bytes >= ((int64_t)1 << 32) || (int64_t)M * K * 2 >= ((int64_t)1 << 32)) return false;
   if (g_b3_force > 0) return true;  // a forced tile height takes every shape (tests reach the kernel on small matrices)
-  return 4 * (int64_t)((M + 127) / 128) * ((N + 255) / 256) >= 3 * (int64_t)b3_num_cus();
+  return kq_tall_fills(M, N, codec);
 }
 
 size_t kq_gemm3b_workspace_bytes(int M, int K) { return (size_t)M * K * 2 + (size_t)M * 4 + 256; }

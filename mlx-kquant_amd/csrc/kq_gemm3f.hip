@@ -379,15 +379,15 @@ int launch_f3_call(const void* x, const uint8_t* w, void* y, int M, int N, int K
 
 }  // namespace
 
-// Taken for calls of 128 rows or more whose half-height tiles fill three quarters of the CUs; smaller calls stay on
-// the any-codec kernel.
+// Taken for calls of 128 rows or more whose half-height tiles fill enough of the CUs (kq_tall_fills); smaller calls stay
+// on the streamed kernel or, beyond its rows, the any-codec kernel.
 bool kq_gemm3f_supported(int M, int N, int K, int codec) {
   if (codec != KQ_MXFP4 && codec != KQ_NVFP4) return false;
   if (M < 128 || N <= 0 || K < 64 || (K & 63)) return false;
   const int64_t row_bytes = (int64_t)(K >> 6) * (codec == KQ_MXFP4 ? 34 : 36);
   if (256 * row_bytes >= ((int64_t)1 << 32) || (int64_t)M * K * 2 >= ((int64_t)1 << 32)) return false;
   if (g_f3_force > 0) return true;  // a forced tile height takes every shape (tests reach the kernel on small matrices)
-  return 4 * (int64_t)((M + 127) / 128) * ((N + 255) / 256) >= 3 * (int64_t)f3_num_cus();
+  return kq_tall_fills(M, N, codec);
 }
 
 size_t kq_gemm3f_workspace_bytes(int M, int K) { return (size_t)M * K * 2 + (size_t)M * 4 + 256; }

@@ -428,14 +428,14 @@ bool i3_codec(int codec) {
 
 }  // namespace
 
-// Taken for calls of 128 rows or more whose half-height tiles fill three quarters of the CUs; smaller calls stay on
-// the any-codec kernel.
+// Taken for calls of 128 rows or more whose half-height tiles fill enough of the CUs (kq_tall_fills); smaller calls stay
+// on the streamed kernel or, beyond its rows, the any-codec kernel.
 bool kq_gemm3i_supported(int M, int N, int K, int codec) {
   if (!i3_codec(codec)) return false;
   if (M < 128 || N <= 0 || K < 256 || (K & 255)) return false;
   if ((int64_t)256 * (K >> 8) * 110 >= ((int64_t)1 << 32) || (int64_t)M * K * 2 >= ((int64_t)1 << 32)) return false;
   if (g_i3_force > 0) return true;  // a forced tile height takes every shape (tests reach the kernel on small matrices)
-  return 4 * (int64_t)((M + 127) / 128) * ((N + 255) / 256) >= 3 * (int64_t)i3_num_cus();
+  return kq_tall_fills(M, N, codec);
 }
 
 size_t kq_gemm3i_workspace_bytes(int M, int K) { return (size_t)M * K * 2 + (size_t)M * 4 + 256; }

@@ -1,5 +1,5 @@
-// Matmul of 9 ... a few dozen activation rows, every codec: y[M,N] = x[M,K] . W^T between the streamed skinny kernel
-// (M <= 8) and the tile GEMMs.
+// Matmul of 9 ... 512 activation rows, every codec: y[M,N] = x[M,K] . W^T between the streamed skinny kernel (M <= 8)
+// and the tile GEMMs.
 //
 // What bounds it: the weight bytes (HBM).  A call of 32 rows does 64 operations per weight, a tenth of what the matrix
 // cores could do in the time the weights take to arrive, so the kernel is built like the skinny ones: every wave streams
@@ -599,9 +599,29 @@ bool kq_mid_supported(int M, int N, int K, int codec) {
   // 55 / 84 / 149 (64 / 70 / 114): from two row blocks on the tile GEMM of the K-quants with exact integers is ahead on
   // the large matrices, where a weight decoded once per 64 rows counts.  The any-codec kernel the others have there is
   // behind on every shape: mxfp4 28672 x 8192 56 / 85 / 147 (131 / 164 / 298), q8_0 77 / 113 / 193 (114 / 136 / 229).
+  // Narrow matrices leave that GEMM with too few tiles up to 192 rows (q4_k / q6_k, 192 rows, us: 1024 x 4096 14 / 17
+  // against 22 / 24, 4096 x 4096 26 / 34 against 31 / 39, 4096 x 14336 61 / 86 against 69 / 99; 14336 x 4096 63 / 91
+  // against 56 / 84).
   const bool tile_gemm = codec == KQ_Q4_K || codec == KQ_Q5_K || codec == KQ_Q6_K;
-  if (tile_gemm) return M <= 32 || (M <= 64 && (int64_t)N * K <= (int64_t)64 << 20);
-  return M <= KQ_MID_MAX_ROWS;
+  if (tile_gemm) return M <= 32 || (M <= 64 && (int64_t)N * K <= (int64_t)64 << 20) || (M <= 192 && N <= 4096);
+  if (M <= 128) return true;
+  // 129 ... 512 rows: until the codec's tall tiles fill enough of the chip (one workgroup per CU and no K split there, so
+  // an unfilled round costs a whole one).  us here / on tall tiles / on the any-codec kernel, which had these calls:
+  // mxfp4 4096 x 14336 256 rows 76 / 235 / 147, 512 rows 161 / 236 / 266, 14336 x 4096 333 rows 111 / 84 / 282; iq3_s
+  // 14336 x 4096 192 rows 89 / 87 / 154; q8_0 14336 x 4096 256 rows 101 / 97 / 130, 333 rows 137 / 103 / 210.
+  return M <= KQ_MID_MAX_ROWS && !kq_tall_fills(M, N, codec);
+}
+
+// Whether the tall-tile GEMM of a codec (128 x 256 tiles, a workgroup per CU) has the tiles to beat the streamed kernel:
+// three fifths of a round for two or three terms per weight, seven sixteenths for one term; a whole round for the 128-row
+// kernel of q2_k / q3_k / iq4_xs.  Above the rows of the streamed kernel the alternative is the any-codec kernel, and a
+// quarter of a round is enough (4096 x 4096, 768 rows, us: mxfp4 84 against 152, q8_0 101 against 120).
+bool kq_tall_fills(int M, int N, int codec) {
+  const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256), cus = mid_cus();
+  if (codec == KQ_Q2_K || codec == KQ_Q3_K || codec == KQ_IQ4_XS) return tiles >= 256;
+  if (M > KQ_MID_MAX_ROWS) return 4 * tiles >= cus;
+  const bool two = codec == KQ_Q8_0 || codec == KQ_Q4_0 || codec == KQ_IQ4_NL || codec == KQ_Q4_1 || codec == KQ_Q5_0 || codec == KQ_Q5_1;
+  return two ? 5 * tiles >= 3 * cus : 16 * tiles >= 7 * cus;
 }
 
 size_t kq_mid_workspace_bytes(int M, int N, int K) {

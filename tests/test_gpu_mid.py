@@ -54,6 +54,18 @@ def test_mid_row_blocks(mid, M):
     assert rel_l2(got, O.qmm(xb, wire, "q4_k", True, "bfloat16"), "bfloat16") <= 1e-3
 
 
+@pytest.mark.parametrize("codec,M", [("iq4_xs", 129), ("q2_k", 333), ("q8_0", 333), ("mxfp4", 512), ("iq3_s", 511),
+                                     ("q6_k", 192), ("q4_k", 129)])
+def test_mid_many_row_blocks_as_routed(kq, codec, M):
+    """Five to sixteen blocks of activation rows on a narrow matrix, by the dispatch's own rule: a ragged tile, cut steps."""
+    N, K = 136, 8192
+    wpb = kq.CODEC_GEOMETRY[codec][3]
+    wire = O.synth_wire(codec, N * K // wpb, seed=6).reshape(N, -1)
+    xb, xt = make_x((M, K), "bfloat16", seed=7)
+    got = dev_to_bits(kq.quantized_matmul(xt, wire_to_dev(wire), None, codec))
+    assert rel_l2(got, O.qmm(xb, wire, codec, True, "bfloat16"), "bfloat16") <= 1e-3
+
+
 def test_mid_cut_steps_replay(mid):
     """The arrival counters are set anew by every call: replays of a captured call on changing inputs equal eager calls."""
     N, K, M = 512, 12288, 17
