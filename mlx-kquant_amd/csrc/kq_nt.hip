@@ -19,7 +19,9 @@
 // the tile's columns, contiguous per row; for the 256-weight codecs the whole superblock, which two column tiles
 // share) into its own LDS area with dword loads issued one step ahead, and the decoders read the bytes from there:
 // decoding straight from global memory costs about 130 byte-wide loads a step.  Calls of 96 rows and more run
-// gemm_nt_wide_kernel below, which decodes a step once for 128 activation rows.
+// gemm_nt_wide_kernel below, which decodes a step once for 128 activation rows, calls of 512 and more
+// gemm_nt_tall_kernel (256 rows).
+#include <algorithm>
 #include <type_traits>
 
 #include "kq_decode.h"
@@ -55,6 +57,7 @@ struct NtArgs {
   // ([ksplit, M, N]) and are added by nt_reduce_kernel
   int ksplit, steps_per_split;
   float* part;
+  bool tall;  // 256-row tiles
 };
 
 __device__ __forceinline__ uint32_t pack_hi(float a, float b) {
@@ -284,7 +287,7 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
 // as packed bf16 pairs where the MFMA operands of all four waves lie (LDS, [k group h][t][c] x 16 bytes, hi and lo
 // planes), and after one barrier every wave reads its 16 operands back.  Staging and operand buffers are double:
 // one barrier per step.
-template <int C, int DT, int MRW>
+template <int C, int DT, int MRW, bool VEC>
 __global__ __launch_bounds__(NT_THREADS, 2) void gemm_nt_wide_kernel(NtArgs a, const uint8_t* __restrict__ grids) {
   using G = NtGeom<C>;
   constexpr int BPB = G::BPB, GPB = G::GPB, PDW = G::PDW, STRIDE = G::STRIDE;
@@ -332,19 +335,17 @@ __global__ __launch_bounds__(NT_THREADS, 2) void gemm_nt_wide_kernel(NtArgs a, c
       const int row = idx / PDW, boff = 4 * (idx - row * PDW);
       const int eoff = boff < piece_here - 4 ? boff : piece_here - 4;
       const int k = NT_KSTEP * st + row < a.K ? NT_KSTEP * st + row : klast;
-      const uint32_t v = *reinterpret_cast<const u32_a1*>(wt + (size_t)k * row_bytes + eoff);
-      wreg[j] = v >> (8 * ((boff - eoff) & 3));
+      wreg[j] = *reinterpret_cast<const u32_a1*>(wt + (size_t)k * row_bytes + eoff);
     }
     const int k0 = NT_KSTEP * st + 8 * h;
 #pragma unroll
     for (int q = 0; q < MRW; q++) {
-#pragma unroll
-      for (int j = 0; j < 4; j++) xreg[q][j] = 0u;
-      if (a.x_vec) {
+      if constexpr (VEC) {
         const uint4 v = *reinterpret_cast<const uint4*>(xr[q] + (k0 < a.K ? k0 : 0));
-        const bool in = k0 < a.K;
-        xreg[q][0] = in ? v.x : 0u, xreg[q][1] = in ? v.y : 0u, xreg[q][2] = in ? v.z : 0u, xreg[q][3] = in ? v.w : 0u;
+        xreg[q][0] = v.x, xreg[q][1] = v.y, xreg[q][2] = v.z, xreg[q][3] = v.w;
       } else {
+#pragma unroll
+        for (int j = 0; j < 4; j++) xreg[q][j] = 0u;
 #pragma unroll
         for (int i = 0; i < 8; i++)
           if (k0 + i < a.K) xreg[q][i >> 1] |= (uint32_t)xr[q][k0 + i] << (16 * (i & 1));
@@ -355,7 +356,8 @@ __global__ __launch_bounds__(NT_THREADS, 2) void gemm_nt_wide_kernel(NtArgs a, c
 #pragma unroll
     for (int j = 0; j < NDWW; j++) {
       const int idx = tid + NT_THREADS * j;
-      if (idx < NT_KSTEP * PDW) *reinterpret_cast<uint32_t*>(stage + 4 * idx) = wreg[j];
+      const int boff = 4 * (idx % PDW), eoff = boff < piece_here - 4 ? boff : piece_here - 4;
+      if (idx < NT_KSTEP * PDW) *reinterpret_cast<uint32_t*>(stage + 4 * idx) = wreg[j] >> (8 * ((boff - eoff) & 3));
     }
   };
 
@@ -373,6 +375,7 @@ __global__ __launch_bounds__(NT_THREADS, 2) void gemm_nt_wide_kernel(NtArgs a, c
     bf16x8 ah[MRW], al[MRW];
 #pragma unroll
     for (int q = 0; q < MRW; q++) {
+      if (VEC && NT_KSTEP * st + NT_KSTEP > a.K && NT_KSTEP * st + 8 * h >= a.K) xreg[q][0] = xreg[q][1] = xreg[q][2] = xreg[q][3] = 0u;
       if constexpr (DT == KQ_BF16) {
         ah[q] = __builtin_bit_cast(bf16x8, make_uint4(xreg[q][0], xreg[q][1], xreg[q][2], xreg[q][3]));
       } else {
@@ -388,7 +391,7 @@ __global__ __launch_bounds__(NT_THREADS, 2) void gemm_nt_wide_kernel(NtArgs a, c
       }
     }
     if (st == st_begin) __syncthreads();  // the first staging buffer is complete (later ones: the barrier below)
-    if (st + 1 < nsteps) fetch(st + 1);
+    fetch(st + 1 < nsteps ? st + 1 : st);
     {  // decode this lane's two rows and put them where the operands lie
       float w0[8], w1[8];
       kq::decode8<C>(stage + blk_off, g, grids, w0);
@@ -455,6 +458,203 @@ __global__ __launch_bounds__(NT_THREADS, 2) void gemm_nt_wide_kernel(NtArgs a, c
   }
 }
 
+// Many activation rows: 256 rows x 128 columns per workgroup of eight waves, 64 rows of K a step.  The 8192 weights of a
+// step are decoded once for all 256 rows: wave w decodes rows 8w ... 8w + 7 of the step's 64 (lane (c, h): rows 8w + 2h,
+// + 1 of column group c) into operand order as above.  A wave multiplies 64 rows with half of the columns (t = 4 wc ...
+// 4 wc + 3), so an operand read feeds eight MFMAs and is made by four waves instead of by all.  Operands of step s + 1
+// are decoded in the interval that multiplies step s, the two waves of a SIMD in opposite order, so that one decodes
+// while the other multiplies; wire bytes are two steps ahead, activations one, one barrier per step.  82 - 93 KB of LDS:
+// one workgroup per CU.
+// Bound by the vector ALU (decode and bf16 split) and the matrix cores together.  4096 x 4096, us, against
+// gemm_nt_wide_kernel (and that kernel before its loads were left unconverted until their use): q4_k 1024 rows 108 against
+// 150 (219), 2048 rows 180 against 188 (226); q8_0 109 against 204 (205), 181 against 223.  128-row tiles of the same form:
+// 124 and 246 (q4_k), so a row group more per operand read is what it lives on.
+constexpr int TALL_WAVES = 8, TALL_THREADS = 64 * TALL_WAVES, TALL_K = 64, TALL_RG = 4;
+
+template <int C, int DT>
+__global__ __launch_bounds__(TALL_THREADS, 2) void gemm_nt_tall_kernel(NtArgs a, const uint8_t* __restrict__ grids) {
+  using G = NtGeom<C>;
+  constexpr int BPB = G::BPB, GPB = G::GPB, PDW = G::PDW, STRIDE = G::STRIDE, RG = TALL_RG;
+  constexpr int STG = TALL_K * STRIDE;                                      // one staging buffer: the step's row pieces
+  constexpr int NDWW = (TALL_K * PDW + TALL_THREADS - 1) / TALL_THREADS;    // dwords a thread copies per step
+  constexpr int PLANE = (TALL_K / 8) * 8 * 16 * 16;                         // one operand plane
+  constexpr int OPB = 2 * PLANE;                                            // hi + lo
+  __shared__ __attribute__((aligned(16))) uint8_t lds[2 * STG + 2 * OPB];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wr = wave & 3, wc = wave >> 2;
+  const int c = lane & 15, h = lane >> 4;  // h: k group as operand reader, row pair as decoder
+  const int item = a.ksplit > 1 ? 0 : blockIdx.z, split = a.ksplit > 1 ? blockIdx.z : 0;
+  const uint32_t e = a.rhs ? a.rhs[item] : 0u;
+  if (e >= (uint32_t)a.E) return;  // the whole workgroup leaves: the entry's output rows stay untouched
+  const int tile = blockIdx.x;
+  const int ngroups = a.N / 8;
+  const int gi = tile * 16 + c;
+  const bool col_ok = gi < ngroups;
+  const size_t row_bytes = (size_t)(a.N / G::WPB) * BPB;
+  const int pi = G::SUPER ? tile >> 1 : tile;
+  const int gp = (col_ok ? gi : ngroups - 1) - pi * (G::PCOLS / 8);
+  const uint8_t* wt = a.w + (size_t)e * (size_t)a.w_expert_stride + (size_t)pi * G::PIECE;
+  const int cols_here = a.N - G::PCOLS * pi < G::PCOLS ? a.N - G::PCOLS * pi : G::PCOLS;
+  const int piece_here = cols_here / G::WPB * BPB;
+  const int blk_off = (gp / GPB) * BPB + (8 * wave + 2 * h) * STRIDE;  // this lane's first row inside a staging buffer
+  const int g = gp % GPB, klast = a.K - 1;
+  const int m0 = blockIdx.y * (64 * RG) + 16 * RG * wr;
+  const uint16_t* xr[RG];
+#pragma unroll
+  for (int q = 0; q < RG; q++) {
+    const int mrow = m0 + 16 * q + c < a.M ? m0 + 16 * q + c : a.M - 1;
+    xr[q] = static_cast<const uint16_t*>(a.x) + (a.lhs ? (size_t)a.lhs[item] * (size_t)a.x_batch_stride : 0) +
+            (size_t)mrow * a.K;
+  }
+  f32x4 acc[RG][4];
+#pragma unroll
+  for (int q = 0; q < RG; q++)
+#pragma unroll
+    for (int t = 0; t < 4; t++) acc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  uint32_t wreg[NDWW];
+  auto fetch_w = [&](int st) {  // as in gemm_nt_mfma_kernel, the step's pieces spread over the whole workgroup
+#pragma unroll
+    for (int j = 0; j < NDWW; j++) {
+      const int idx = tid + TALL_THREADS * j < TALL_K * PDW ? tid + TALL_THREADS * j : TALL_K * PDW - 1;
+      const int row = idx / PDW, boff = 4 * (idx - row * PDW);
+      const int eoff = boff < piece_here - 4 ? boff : piece_here - 4;
+      const int k = TALL_K * st + row < a.K ? TALL_K * st + row : klast;
+      wreg[j] = *reinterpret_cast<const u32_a1*>(wt + (size_t)k * row_bytes + eoff);
+    }
+  };
+  auto park = [&](uint8_t* stage) {
+#pragma unroll
+    for (int j = 0; j < NDWW; j++) {
+      const int idx = tid + TALL_THREADS * j;
+      const int boff = 4 * (idx % PDW), eoff = boff < piece_here - 4 ? boff : piece_here - 4;
+      if (idx < TALL_K * PDW) *reinterpret_cast<uint32_t*>(stage + 4 * idx) = wreg[j] >> (8 * ((boff - eoff) & 3));
+    }
+  };
+  auto fetch_x = [&](int st, uint4 (&xv)[RG][2]) {
+#pragma unroll
+    for (int q = 0; q < RG; q++)
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        const int k0 = TALL_K * st + 32 * s + 8 * h;
+        // K is a multiple of 8: a group of 8 lies inside the row or past it (masked by multiply)
+        xv[q][s] = *reinterpret_cast<const uint4*>(xr[q] + (k0 < a.K ? k0 : 0));
+      }
+  };
+  auto decode = [&](const uint8_t* stage, uint8_t* opnd) {
+    float w0[8], w1[8];
+    kq::decode8<C>(stage + blk_off, g, grids, w0);
+    kq::decode8<C>(stage + blk_off + STRIDE, g, grids, w1);
+    uint8_t* dst = opnd + ((wave * 8) * 16 + c) * 16 + 4 * h;
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+      *reinterpret_cast<uint32_t*>(dst + t * 256) = pack_hi(w0[t], w1[t]);
+      *reinterpret_cast<uint32_t*>(dst + t * 256 + PLANE) = pack_rne(w0[t] - trunc_bf16(w0[t]), w1[t] - trunc_bf16(w1[t]));
+    }
+  };
+  auto multiply = [&](int st, const uint8_t* opnd, const uint4 (&xv)[RG][2]) {
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      if (s && TALL_K * st + 32 >= a.K) break;  // rows past K are multiplied (by zero) up to the next multiple of 32 only
+      bf16x8 ah[RG], al[RG];
+#pragma unroll
+      for (int q = 0; q < RG; q++) {
+        uint32_t v[4] = {xv[q][s].x, xv[q][s].y, xv[q][s].z, xv[q][s].w};
+        if (TALL_K * st + TALL_K > a.K && TALL_K * st + 32 * s + 8 * h >= a.K) v[0] = v[1] = v[2] = v[3] = 0u;
+        if constexpr (DT == KQ_BF16) {
+          ah[q] = __builtin_bit_cast(bf16x8, make_uint4(v[0], v[1], v[2], v[3]));
+        } else {
+          uint32_t hi[4], lo[4];
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const float f0 = kq::h2f((uint16_t)(v[j] & 0xffffu)), f1 = kq::h2f((uint16_t)(v[j] >> 16));
+            hi[j] = pack_hi(f0, f1);
+            lo[j] = pack_hi(f0 - trunc_bf16(f0), f1 - trunc_bf16(f1));
+          }
+          ah[q] = __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+          al[q] = __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+        }
+      }
+      const uint8_t* src = opnd + (((4 * s + h) * 8 + 4 * wc) * 16 + c) * 16;
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        const bf16x8 wh = *reinterpret_cast<const bf16x8*>(src + t * 256);
+        const bf16x8 wl = *reinterpret_cast<const bf16x8*>(src + t * 256 + PLANE);
+#pragma unroll
+        for (int q = 0; q < RG; q++) acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[q], wh, acc[q][t], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < RG; q++) acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[q], wl, acc[q][t], 0, 0, 0);
+        if constexpr (DT == KQ_F16) {
+#pragma unroll
+          for (int q = 0; q < RG; q++) acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[q], wh, acc[q][t], 0, 0, 0);
+        }
+      }
+    }
+  };
+
+  const int steps_all = (a.K + TALL_K - 1) / TALL_K;
+  const int st_begin = split * a.steps_per_split;
+  const int nsteps = st_begin + a.steps_per_split < steps_all ? st_begin + a.steps_per_split : steps_all;
+  uint8_t* const ops = lds + 2 * STG;
+  uint4 xnext[RG][2];
+  if (st_begin < nsteps) {
+    fetch_w(st_begin);
+    fetch_x(st_begin, xnext);
+    park(lds);
+    if (st_begin + 1 < nsteps) fetch_w(st_begin + 1);
+    __syncthreads();
+    decode(lds, ops);
+    if (st_begin + 1 < nsteps) park(lds + STG);
+    __syncthreads();
+  }
+  for (int st = st_begin; st < nsteps; st++) {
+    const int b = (st - st_begin) & 1;
+    uint4 xv[RG][2];
+#pragma unroll
+    for (int q = 0; q < RG; q++) xv[q][0] = xnext[q][0], xv[q][1] = xnext[q][1];
+    // (no branch around the loads: past the range they repeat its last step)
+    fetch_w(st + 2 < nsteps ? st + 2 : nsteps - 1);
+    fetch_x(st + 1 < nsteps ? st + 1 : nsteps - 1, xnext);
+    // read here: staging and operands of step st + 1 (st).  Written here: operands of st + 1, staging of st + 2, whose
+    // buffers were last read before the previous barrier
+    if (wc == 0) {
+      multiply(st, ops + b * OPB, xv);
+      if (st + 1 < nsteps) decode(lds + (b ^ 1) * STG, ops + (b ^ 1) * OPB);
+    } else {
+      if (st + 1 < nsteps) decode(lds + (b ^ 1) * STG, ops + (b ^ 1) * OPB);
+      multiply(st, ops + b * OPB, xv);
+    }
+    if (st + 2 < nsteps) park(lds + b * STG);
+    __syncthreads();
+  }
+
+  if (!col_ok) return;
+  const size_t col = 8 * (size_t)gi + 4 * wc;
+#pragma unroll
+  for (int q = 0; q < RG; q++) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int m = m0 + 16 * q + 4 * h + r;
+      if (m < a.M) {
+        if (a.ksplit > 1) {
+          *reinterpret_cast<float4*>(a.part + ((size_t)split * a.M + m) * a.N + col) =
+              make_float4(acc[q][0][r], acc[q][1][r], acc[q][2][r], acc[q][3][r]);
+        } else {
+          uint32_t o[2];
+#pragma unroll
+          for (int j = 0; j < 2; j++) {
+            const float v0 = acc[q][2 * j][r], v1 = acc[q][2 * j + 1][r];
+            const uint16_t lo = DT == KQ_F16 ? kq::f2f16(v0) : kq::f2bf16(v0);
+            const uint16_t hi = DT == KQ_F16 ? kq::f2f16(v1) : kq::f2bf16(v1);
+            o[j] = (uint32_t)lo | ((uint32_t)hi << 16);
+          }
+          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.y) + ((size_t)item * a.M + m) * a.N + col) = make_uint2(o[0], o[1]);
+        }
+      }
+    }
+  }
+}
+
 // y[i] = sum over the K ranges of part[s][i], 8 outputs per thread, ranges added in order
 template <int DT>
 __global__ __launch_bounds__(256) void nt_reduce_kernel(const float* __restrict__ part, void* __restrict__ y,
@@ -477,12 +677,25 @@ __global__ __launch_bounds__(256) void nt_reduce_kernel(const float* __restrict_
   reinterpret_cast<uint4*>(y)[i] = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// K ranges of a dense call: enough workgroups for two per CU, at least eight steps each
+// Calls of the 256-row kernel: 512 rows and more of aligned activations, K long enough for its pipeline.  (q4_k 4096 x 4096
+// 512 rows, us: 66 here in two ranges' worth of partial sums, 64 on the 128-row tiles; 8192 x 8192 512 rows 192 against 200,
+// q8_0 192 against 227; below, its last row tile is mostly padding.)
+bool nt_tall(int M, int K) { return M >= 512 && K >= 512 && !(K & 7); }
+
+// K ranges of a dense call.  256-row tiles: one workgroup per CU.  Otherwise enough workgroups for two per CU (8192 x 8192,
+// 500 rows, 256 tiles in two ranges: q8_0 227 us, uncut 410), at least eight steps each.
 int nt_ksplit(int M, int N, int K) {
+  const int cols = (N + NT_COLS - 1) / NT_COLS;
+  if (nt_tall(M, K)) {
+    const int64_t tiles = (int64_t)cols * ((M + 64 * TALL_RG - 1) / (64 * TALL_RG));
+    const int steps = (K + TALL_K - 1) / TALL_K;
+    const int64_t s = std::min<int64_t>(256 / tiles, steps / 4);
+    return s < 2 ? 1 : (int)s;
+  }
   const int rows = M <= 16 ? 16 : M < NT_SHARED_ROWS ? 32 : 128;  // activation rows per workgroup
-  const int64_t tiles = (int64_t)((N + NT_COLS - 1) / NT_COLS) * ((M + rows - 1) / rows);
+  const int64_t tiles = (int64_t)cols * ((M + rows - 1) / rows);
   const int steps = (K + NT_KSTEP - 1) / NT_KSTEP;
-  if (tiles >= 256 || steps < 16) return 1;
+  if (tiles >= (rows == 128 ? 512 : 256) || steps < 16) return 1;
   int s = (int)((512 + tiles - 1) / tiles);
   if (s > steps / 8) s = steps / 8;
   if (s > 32) s = 32;
@@ -491,31 +704,42 @@ int nt_ksplit(int M, int N, int K) {
 
 template <int C>
 struct NtRun {
+  template <int DT>
+  static void reduce(const NtArgs& a, hipStream_t s) {
+    if (a.ksplit <= 1) return;
+    const size_t groups = (size_t)a.M * a.N / 8;
+    hipLaunchKernelGGL((nt_reduce_kernel<DT>), dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s, a.part, a.y, groups,
+                       a.ksplit);
+  }
   template <int DT, int MR>
   static void go(const NtArgs& a, int B, const uint8_t* grids, hipStream_t s) {
     dim3 grid((a.N + NT_COLS - 1) / NT_COLS, (a.M + 16 * MR - 1) / (16 * MR), a.ksplit > 1 ? a.ksplit : B);
     hipLaunchKernelGGL((gemm_nt_mfma_kernel<C, DT, MR>), grid, dim3(NT_THREADS), 0, s, a, grids);
-    if (a.ksplit > 1) {
-      const size_t groups = (size_t)a.M * a.N / 8;
-      hipLaunchKernelGGL((nt_reduce_kernel<DT>), dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s, a.part, a.y,
-                         groups, a.ksplit);
-    }
+    reduce<DT>(a, s);
+  }
+  template <int DT, bool VEC>
+  static void go_shared(const NtArgs& a, int B, const uint8_t* grids, hipStream_t s) {
+    // (256-row tiles on four waves, MRW = 4, measured slower: 316 against 223 us at 2048 rows of 4096 x 4096 q4_k; their
+    // 212 - 250 registers leave two workgroups per CU where the 128-row form runs three)
+    dim3 grid((a.N + NT_COLS - 1) / NT_COLS, (a.M + 127) / 128, a.ksplit > 1 ? a.ksplit : B);
+    hipLaunchKernelGGL((gemm_nt_wide_kernel<C, DT, 2, VEC>), grid, dim3(NT_THREADS), 0, s, a, grids);
+    reduce<DT>(a, s);
   }
   template <int DT>
-  static void go_shared(const NtArgs& a, int B, const uint8_t* grids, hipStream_t s) {
-    // (256-row tiles, MRW = 4, measured slower: 316 against 223 us at 2048 rows of 4096 x 4096 q4_k; their 212 - 250
-    // registers leave two workgroups per CU where the 128-row form runs three)
-    dim3 grid((a.N + NT_COLS - 1) / NT_COLS, (a.M + 127) / 128, a.ksplit > 1 ? a.ksplit : B);
-    hipLaunchKernelGGL((gemm_nt_wide_kernel<C, DT, 2>), grid, dim3(NT_THREADS), 0, s, a, grids);
-    if (a.ksplit > 1) {
-      const size_t groups = (size_t)a.M * a.N / 8;
-      hipLaunchKernelGGL((nt_reduce_kernel<DT>), dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, s, a.part, a.y,
-                         groups, a.ksplit);
-    }
+  static void go_tall(const NtArgs& a, int B, const uint8_t* grids, hipStream_t s) {
+    dim3 grid((a.N + NT_COLS - 1) / NT_COLS, (a.M + 64 * TALL_RG - 1) / (64 * TALL_RG), a.ksplit > 1 ? a.ksplit : B);
+    hipLaunchKernelGGL((gemm_nt_tall_kernel<C, DT>), grid, dim3(TALL_THREADS), 0, s, a, grids);
+    reduce<DT>(a, s);
+  }
+  template <int DT>
+  static void many_rows(const NtArgs& a, int B, const uint8_t* grids, hipStream_t s) {
+    if (a.tall) go_tall<DT>(a, B, grids, s);
+    else if (a.x_vec) go_shared<DT, true>(a, B, grids, s);
+    else go_shared<DT, false>(a, B, grids, s);
   }
   static int run(const NtArgs& a, int B, int dt, const uint8_t* grids, hipStream_t s) {
     if (a.M >= NT_SHARED_ROWS) {
-      dt == KQ_F16 ? go_shared<KQ_F16>(a, B, grids, s) : go_shared<KQ_BF16>(a, B, grids, s);
+      dt == KQ_F16 ? many_rows<KQ_F16>(a, B, grids, s) : many_rows<KQ_BF16>(a, B, grids, s);
     } else if (a.M <= 16) {
       dt == KQ_F16 ? go<KQ_F16, 1>(a, B, grids, s) : go<KQ_BF16, 1>(a, B, grids, s);
     } else if (nt_wide(C) && a.M > 32) {
@@ -563,12 +787,14 @@ int kq_launch_nt_mfma(const void* x, const uint8_t* w, const uint32_t* lhs, cons
   if (reinterpret_cast<uintptr_t>(out) & 15) return KQ_ERR_UNSUPPORTED;
   const uint8_t* grids = kq_device_grids();
   if (!grids) return KQ_ERR_HIP;
-  NtArgs a{x, w, out, lhs, rhs, M, N, K, E, x_batch_stride, w_expert_stride, 0, 1, (K + NT_KSTEP - 1) / NT_KSTEP, nullptr};
+  NtArgs a{x, w, out, lhs, rhs, M, N, K, E, x_batch_stride, w_expert_stride, 0, 1, 0, nullptr, false};
   a.x_vec = !(K & 7) && !(reinterpret_cast<uintptr_t>(x) & 15) && !(x_batch_stride & 7);
+  a.tall = a.x_vec && nt_tall(M, K);
+  const int kstep = a.tall ? TALL_K : NT_KSTEP, steps = (K + kstep - 1) / kstep;
+  a.steps_per_split = steps;
   if (!rhs && B == 1 && ws && !(reinterpret_cast<uintptr_t>(ws) & 15)) {
     const int sp = nt_ksplit(M, N, K);
     if (sp > 1 && ws_bytes >= (size_t)sp * M * N * 4) {
-      const int steps = (K + NT_KSTEP - 1) / NT_KSTEP;
       a.steps_per_split = (steps + sp - 1) / sp;
       a.ksplit = (steps + a.steps_per_split - 1) / a.steps_per_split;
       a.part = static_cast<float*>(ws);

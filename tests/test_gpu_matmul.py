@@ -257,6 +257,23 @@ def test_qmm_no_transpose_many_rows(kq, codec, M, K, N, dtype):
     assert rel_l2(dev_to_bits(got), want, dtype) <= TOL, (codec, M, K, N, dtype)
 
 
+@pytest.mark.parametrize("M,K,N,dtype", [
+    (512, 512, 256, "bfloat16"),    # the least the 256-row tiles take, K cut
+    (600, 1056, 768, "float16"),    # ragged row tile, a last step of half its rows, an odd number of column tiles
+    (513, 1064, 256, "bfloat16"),   # one row in the last tile, a last step that ends inside a group of 32
+    (512, 1001, 256, "bfloat16"),   # rows of x that cannot be read 16 bytes at a time: the 128-row tiles
+])
+@pytest.mark.parametrize("codec", ["q4_k", "q8_0", "iq2_xxs", "mxfp4"])
+def test_qmm_no_transpose_256_row_tiles(kq, codec, M, K, N, dtype):
+    if O.geometry(codec)[0] == 32:
+        N += 96  # columns that do not fill the last tile
+    wire = _wire(codec, K, N, seed=92)
+    xb, xt = make_x((M, K), dtype, seed=93)
+    got = kq.quantized_matmul(xt, wire_to_dev(wire), None, codec, transpose=False)
+    want = O.qmm(xb, wire, codec, False, dtype)
+    assert rel_l2(dev_to_bits(got), want, dtype) <= TOL, (codec, M, K, N, dtype)
+
+
 def test_qmm_dtype_rules_and_shapes(kq):
     N, K = 64, 256
     wire = _wire("q4_k", N, K, seed=34)
