@@ -1,8 +1,8 @@
 // Grouped MoE GEMM: the fused gate/up GLU op and the gathered down projection for many
 // (token, expert) pairs.  Pairs are counting-sorted by expert on the device and cut into segments
-// of at most 32 pairs of one expert; a workgroup multiplies one segment (the 32 activation rows of
-// v_mfma_f32_32x32x16_f16) by a 128-row slab of that expert's weights, so an expert's wire bytes are
-// streamed from HBM once per 32 pairs instead of once per pair.
+// of at most 32 or 64 pairs of one expert (moe_seg_rows); a workgroup multiplies one segment (one or two
+// times the 32 activation rows of v_mfma_f32_32x32x16_f16) by a 128-row slab of that expert's weights, so an
+// expert's wire bytes are streamed once per segment instead of once per pair.
 //
 // Workgroup = 4 waves.  Plain op: each wave owns 32 of the slab's 128 weight rows.  GLU: the slab
 // is 64 gate rows + the same 64 up rows (waves 0/2 gate, 1/3 up); the up waves hand their
@@ -10,6 +10,8 @@
 // rounding.  K advances one 256-wide superblock per step; wire bytes and the gathered activation
 // rows (converted to f16 by the activation prepass) are fetched one step ahead with coalesced
 // 16-byte loads and parked in LDS.
+#include <algorithm>
+
 #include "kq_epilogue.h"
 #include "kq_mma.h"
 #include "kq_moe_sort.h"
@@ -52,12 +54,12 @@ __global__ __launch_bounds__(PP_THREADS) void moe_prologue_kernel(const uint16_t
                                                                   _Float16* __restrict__ xhl, float* __restrict__ rs,
                                                                   int rows, int K, const uint32_t* __restrict__ idx, int P,
                                                                   int E, int* __restrict__ order,
-                                                                  Segment* __restrict__ segs, int* __restrict__ nseg_out) {
+                                                                  Segment* __restrict__ segs, int* __restrict__ nseg_out, int seg_rows) {
   __shared__ int cnt[SORT_MAX_E];
   __shared__ int scan_p[PP_THREADS], scan_s[PP_THREADS];
   __shared__ float red[PP_THREADS / 64];
   if (blockIdx.x == 0)  // the sort is the longest workgroup of the launch (a chain of barriers): it goes first
-    moe_sort_body<PP_THREADS>(idx, P, E, order, segs, nseg_out, cnt, scan_p, scan_s);
+    moe_sort_body<PP_THREADS>(idx, P, E, order, segs, nseg_out, cnt, scan_p, scan_s, seg_rows);
   else
     prepass_row<DT>(x, xh, xhl, rs, rows, K, blockIdx.x - 1, threadIdx.x, red);
 }
@@ -89,19 +91,29 @@ __global__ __launch_bounds__(256) void pad_idx_kernel(const uint32_t* __restrict
 // out[t][n] = T(sum_s scores[t][s] * yf[t][s][n]), f32, slots in order.  idx [T][routed]: the expert ids of the
 // first `routed` slots; a slot whose id is >= E was skipped by the matmul kernels (its row of yf holds nothing)
 // and adds nothing.
-template <int DT>
+// VEC outputs per thread (4 where N and the alignment allow 16-byte reads: 1000 tokens of 2048, 8 slots, 30 -> 12 us).
+template <int DT, int VEC>
 __global__ __launch_bounds__(256) void mix_slots_kernel(const float* __restrict__ yf, const float* __restrict__ scores,
                                                         const uint32_t* __restrict__ idx, int routed, int E,
                                                         uint16_t* __restrict__ out, int T, int S, int N) {
+  typedef float fv __attribute__((ext_vector_type(VEC)));
+  const int per_row = N / VEC;
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (int64_t)T * N) return;
-  const int t = (int)(i / N), n = (int)(i - (int64_t)t * N);
-  float v = 0.f;
+  if (i >= (int64_t)T * per_row) return;
+  const int t = (int)(i / per_row), n = VEC * (int)(i - (int64_t)t * per_row);
+  fv v = fv(0.f);
   for (int s = 0; s < S; s++) {
     if (s < routed && idx[(size_t)t * routed + s] >= (uint32_t)E) continue;
-    v = fmaf(scores[t * S + s], yf[((size_t)t * S + s) * N + n], v);
+    const fv y = *reinterpret_cast<const fv*>(yf + ((size_t)t * S + s) * N + n);
+    const float sc = scores[t * S + s];
+#pragma unroll
+    for (int e = 0; e < VEC; e++) v[e] = fmaf(sc, y[e], v[e]);
   }
-  out[i] = DT == KQ_F16 ? kq::f2f16(v) : kq::f2bf16(v);
+  typedef uint16_t hv __attribute__((ext_vector_type(VEC)));
+  hv o;
+#pragma unroll
+  for (int e = 0; e < VEC; e++) o[e] = DT == KQ_F16 ? kq::f2f16(v[e]) : kq::f2bf16(v[e]);
+  *reinterpret_cast<hv*>(out + (size_t)t * N + n) = o;
 }
 
 // ------------------------------------------------------------------ expert tile map (sorted prefill GEMM)
@@ -238,19 +250,22 @@ struct MoeArgs {
   KqOutMap om;
 };
 
-template <int C, int DT, bool GLU>
-__global__ __launch_bounds__(MOE_THREADS, 3) void moe_grouped_kernel(MoeArgs a) {
+// MT = 1: segments of up to 32 pairs; MT = 2: up to 64, whose decoded weights feed two MFMAs each (a segment of 32 or fewer
+// still multiplies one block of rows only).  Two workgroups per CU instead of three or four.
+template <int C, int DT, bool GLU, int MT>
+__global__ __launch_bounds__(MOE_THREADS, MT == 1 ? 3 : 2) void moe_grouped_kernel(MoeArgs a) {
   using G = Wire<C>;
+  constexpr int SEG = 32 * MT;
   constexpr int WPT = (SLAB * G::PP + MOE_THREADS - 1) / MOE_THREADS;  // wire pieces per thread per step
-  constexpr int APT = SEG_M * 32 / MOE_THREADS;                         // activation pieces per thread per step (4)
+  constexpr int APT = SEG * 32 / MOE_THREADS;                         // activation pieces per thread per step (4)
   constexpr int NCOLS = GLU ? SLAB / 2 : SLAB;                          // output columns per workgroup
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   // two stages of: activations [32][A_STRIDE] | wire [128][LBPB] | X halves [32][32] | side-channel d [128]
-  constexpr int B_OFF = SEG_M * A_STRIDE, H_OFF = B_OFF + SLAB * G::LBPB, D_OFF = H_OFF + SEG_M * 32;
+  constexpr int B_OFF = SEG * A_STRIDE, H_OFF = B_OFF + SLAB * G::LBPB, D_OFF = H_OFF + SEG * 32;
   constexpr int STAGE = D_OFF + SLAB * 2;
   static_assert(STAGE % 16 == 0, "stages keep 16-byte alignment");
   int* pair_lds = reinterpret_cast<int*>(smem + MOE_STAGES * STAGE);  // [32] output row of each segment slot, -1 = none
-  float* rs_lds = reinterpret_cast<float*>(pair_lds + SEG_M);         // [32]
+  float* rs_lds = reinterpret_cast<float*>(pair_lds + SEG);         // [32]
 
   // Workgroups go to the 8 XCDs round-robin in launch order.  Launch position L = 8 j + c runs slab j % tiles of
   // segment 8 (j / tiles) + c: all slabs of a segment sit on one XCD, back to back, so the segment's activation
@@ -282,7 +297,7 @@ __global__ __launch_bounds__(MOE_THREADS, 3) void moe_grouped_kernel(MoeArgs a) 
     }
   };
 
-  if (tid < SEG_M) {
+  if (tid < SEG) {
     const int pr = tid < seg.count ? a.order[seg.start + tid] : -1;
     pair_lds[tid] = pr;
     rs_lds[tid] = pr >= 0 ? a.rs[pr / a.x_div] : 0.f;
@@ -300,7 +315,7 @@ __global__ __launch_bounds__(MOE_THREADS, 3) void moe_grouped_kernel(MoeArgs a) 
   });
   size_t h_goff;
   {
-    const int slot = (tid & 63) >> 1;
+    const int slot = (tid & (2 * SEG - 1)) >> 1;
     const int pr = a.order[seg.start + (slot < seg.count ? slot : 0)];
     h_goff = (size_t)(pr / a.x_div) * nsb * 16 + 8 * (tid & 1);
   }
@@ -357,18 +372,25 @@ __global__ __launch_bounds__(MOE_THREADS, 3) void moe_grouped_kernel(MoeArgs a) 
       if (w_loff[T] != 0xffffffffu) *reinterpret_cast<u32x4*>(stage + B_OFF + w_loff[T]) = wreg[T];
     });
     if constexpr (G::MINS) {
-      if (tid < 64) *reinterpret_cast<u32x4*>(stage + H_OFF + 16 * tid) = hreg;
+      if (tid < 2 * SEG) *reinterpret_cast<u32x4*>(stage + H_OFF + 16 * tid) = hreg;
     }
     if constexpr (G::SIDE_D) {
       if (tid < SLAB) reinterpret_cast<uint16_t*>(stage + D_OFF)[tid] = dreg;
     }
   };
 
-  f32x16 acc[1] = {f32x16{0}};
+  f32x16 acc[MT];
+#pragma unroll
+  for (int t = 0; t < MT; t++) acc[t] = f32x16{0};
   auto multiply = [&](const uint8_t* stage) {
     const uint16_t d_side = G::SIDE_D ? reinterpret_cast<const uint16_t*>(stage + D_OFF)[wave * 32 + l32] : (uint16_t)0;
-    superblock_mma<C, 1>(stage + B_OFF + (wave * 32 + l32) * G::LBPB, d_side, kg, stage + l32 * A_STRIDE + 32 * kg, 0,
-                        stage + H_OFF + l32 * 32 + 16 * kg, 0, acc);
+    const uint8_t* b_lane = stage + B_OFF + (wave * 32 + l32) * G::LBPB;
+    const uint8_t* a_lane = stage + l32 * A_STRIDE + 32 * kg;
+    const uint8_t* h_lane = stage + H_OFF + l32 * 32 + 16 * kg;
+    if (MT == 1 || seg.count > 32)  // uniform over the workgroup
+      superblock_mma<C, MT>(b_lane, d_side, kg, a_lane, 32 * A_STRIDE, h_lane, 32 * 32, acc);
+    else
+      superblock_mma<C, 1>(b_lane, d_side, kg, a_lane, 0, h_lane, 0, acc);
   };
 
   issue(0);
@@ -400,40 +422,60 @@ __global__ __launch_bounds__(MOE_THREADS, 3) void moe_grouped_kernel(MoeArgs a) 
     if constexpr (MOE_STAGES == 1) lds_barrier();  // the step buffers are free: reuse them for the up accumulators
     // The gate wave (even) and the up wave (odd) of a column block swap half of their accumulators and finish eight
     // outputs each: the gate wave registers 0 .. 7, the up wave 8 .. 15.
-    float* ex = reinterpret_cast<float*>(smem);  // [2 column blocks][16][64]
+    float* ex = reinterpret_cast<float*>(smem);  // [MT][2 column blocks][16][64]
     const int nb = wave >> 1;
     const bool upw = (wave & 1) != 0;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int give = upw ? i : 8 + i;  // the register the partner finishes
-      ex[(nb * 16 + give) * 64 + lane] = upw ? acc[0][i] : acc[0][8 + i];
-    }
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const int give = upw ? i : 8 + i;  // the register the partner finishes
+        ex[((2 * t + nb) * 16 + give) * 64 + lane] = upw ? acc[t][i] : acc[t][8 + i];
+      }
     lds_barrier();
     const int col = nb * 32 + l32;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int i = upw ? 8 + j : j;
-      const int slot = 8 * (i >> 2) + 4 * kg + (i & 3);
-      const int pr = pair_lds[slot];
-      if (pr >= 0 && col < ncols) {
-        const float r = rs_lds[slot];
-        const float mine = (upw ? acc[0][8 + j] : acc[0][j]) * r, other = ex[(nb * 16 + i) * 64 + lane] * r;
-        const float v = kq::glu_epilogue_fast(a.act, upw ? other : mine, upw ? mine : other, a.limit, 1.0f);
-        kq::store_result<DT>(a.y, a.om, (size_t)kq::out_row(a.om, pr) * N + n0 + col, v);
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const int i = upw ? 8 + j : j;
+        const int slot = 32 * t + 8 * (i >> 2) + 4 * kg + (i & 3);
+        const int pr = pair_lds[slot];
+        if (pr >= 0 && col < ncols) {
+          const float r = rs_lds[slot];
+          const float mine = (upw ? acc[t][8 + j] : acc[t][j]) * r, other = ex[((2 * t + nb) * 16 + i) * 64 + lane] * r;
+          const float v = kq::glu_epilogue_fast(a.act, upw ? other : mine, upw ? mine : other, a.limit, 1.0f);
+          kq::store_result<DT>(a.y, a.om, (size_t)kq::out_row(a.om, pr) * N + n0 + col, v);
+        }
       }
-    }
   } else {
     const int col = wave * 32 + l32;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      const int slot = 8 * (i >> 2) + 4 * kg + (i & 3);
-      const int pr = pair_lds[slot];
-      if (pr >= 0 && col < ncols) {
-        const float v = acc[0][i] * rs_lds[slot];
-        kq::store_result<DT>(a.y, a.om, (size_t)kq::out_row(a.om, pr) * N + n0 + col, v);
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        const int slot = 32 * t + 8 * (i >> 2) + 4 * kg + (i & 3);
+        const int pr = pair_lds[slot];
+        if (pr >= 0 && col < ncols) {
+          const float v = acc[t][i] * rs_lds[slot];
+          kq::store_result<DT>(a.y, a.om, (size_t)kq::out_row(a.om, pr) * N + n0 + col, v);
+        }
       }
-    }
   }
+}
+
+// Pairs per segment of a call.  64 halve the decode of an expert's weights but leave two workgroups per CU: taken from 32
+// pairs per expert on average where the CUs stay filled (router + GLU + down + mix, us, down on 32 / 64: q4_k 128 experts
+// of 2048 <-> 768 top 8, 700 tokens 250 / 229, 1000 tokens 320 / 292, 384 tokens, 24 pairs per expert, 165 / 169; 8 experts
+// of 2048 <-> 4096 top 2, 400 tokens 147 / 134, 200 tokens, 128 workgroups, 90 / 100).  The fused op gains less, and
+// nothing where the average is about the segment itself (half of the experts then leave a short second one): 37 pairs per
+// expert 91 / 87, 44 250 / 239, 62 320 / 326, 100 147 / 138.
+int moe_seg_rows(int P, int E, int N, bool glu) {
+  const int ncols = glu ? SLAB / 2 : SLAB;
+  const int64_t wgs = (int64_t)std::max(E, P / 64) * ((N + ncols - 1) / ncols);
+  if (wgs < 256 || P < 32 * (int64_t)E) return 32;
+  if (glu && (P < 36 * (int64_t)E || (P > 56 * (int64_t)E && P < 96 * (int64_t)E))) return 32;
+  return 64;
 }
 
 struct MoeWorkspace {
@@ -469,19 +511,26 @@ MoeWorkspace carve(void* ws, int rows, int P, int E, int K) {
   return m;
 }
 
-template <int C, int DT, bool GLU>
-int launch_grouped(const MoeArgs& a, int P, int E, hipStream_t s) {
+template <int C, int DT, bool GLU, int MT>
+int launch_grouped_mt(const MoeArgs& a, int P, int E, hipStream_t s) {
   using G = Wire<C>;
+  constexpr int SEG = 32 * MT;
   constexpr int NCOLS = GLU ? SLAB / 2 : SLAB;
   const int ntiles = (a.N + NCOLS - 1) / NCOLS;
-  int maxseg = E + P / SEG_M;  // sum over experts of ceil(c_e / 32) <= E + P / 32
+  int maxseg = E + P / SEG;  // sum over experts of ceil(c_e / SEG) <= E + P / SEG
   if (maxseg > P) maxseg = P;
   maxseg = (maxseg + 7) & ~7;  // the kernel's launch-position map needs a multiple of 8
-  const size_t lds = (size_t)MOE_STAGES * (SEG_M * A_STRIDE + SLAB * G::LBPB + SEG_M * 32 + SLAB * 2) + SEG_M * 8;
-  auto kern = moe_grouped_kernel<C, DT, GLU>;
+  const size_t lds = (size_t)MOE_STAGES * (SEG * A_STRIDE + SLAB * G::LBPB + SEG * 32 + SLAB * 2) + SEG * 8;
+  auto kern = moe_grouped_kernel<C, DT, GLU, MT>;
+  KQ_SET_MAX_LDS_ONCE((kern), lds);
   hipLaunchKernelGGL(kern, dim3(ntiles, maxseg), dim3(MOE_THREADS), lds, s, a);
   KQ_HIP_CHECK(hipGetLastError());
   return KQ_OK;
+}
+
+template <int C, int DT, bool GLU>
+int launch_grouped(const MoeArgs& a, int P, int E, hipStream_t s) {
+  return moe_seg_rows(P, E, a.N, GLU) == 64 ? launch_grouped_mt<C, DT, GLU, 2>(a, P, E, s) : launch_grouped_mt<C, DT, GLU, 1>(a, P, E, s);
 }
 
 template <bool GLU>
@@ -559,13 +608,11 @@ int kq_launch_pad_idx(const uint32_t* idx, uint32_t* idx2, int T, int S, hipStre
 int kq_launch_mix_slots(const float* yf, const float* scores, const uint32_t* idx, int routed, int E, void* out, int T,
                         int S, int N, int dtype, hipStream_t s) {
   if (T <= 0 || N <= 0) return KQ_OK;
-  const unsigned blocks = (unsigned)(((int64_t)T * N + 255) / 256);
-  if (dtype == KQ_F16)
-    hipLaunchKernelGGL(mix_slots_kernel<KQ_F16>, dim3(blocks), dim3(256), 0, s, yf, scores, idx, routed, E,
-                       static_cast<uint16_t*>(out), T, S, N);
-  else
-    hipLaunchKernelGGL(mix_slots_kernel<KQ_BF16>, dim3(blocks), dim3(256), 0, s, yf, scores, idx, routed, E,
-                       static_cast<uint16_t*>(out), T, S, N);
+  const bool wide = !(N & 3) && !(reinterpret_cast<uintptr_t>(yf) & 15) && !(reinterpret_cast<uintptr_t>(out) & 7);
+  const unsigned blocks = (unsigned)(((int64_t)T * (wide ? N / 4 : N) + 255) / 256);
+  auto kern = dtype == KQ_F16 ? (wide ? mix_slots_kernel<KQ_F16, 4> : mix_slots_kernel<KQ_F16, 1>)
+                              : (wide ? mix_slots_kernel<KQ_BF16, 4> : mix_slots_kernel<KQ_BF16, 1>);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, s, yf, scores, idx, routed, E, static_cast<uint16_t*>(out), T, S, N);
   KQ_HIP_CHECK(hipGetLastError());
   return KQ_OK;
 }
@@ -591,10 +638,10 @@ int kq_launch_moe_grouped(const void* x, const uint8_t* w, const uint8_t* w2, co
   const MoeWorkspace m = carve(ws, rows, P, E, K);
   if (dtype == KQ_F16)
     hipLaunchKernelGGL(moe_prologue_kernel<KQ_F16>, dim3(rows + 1), dim3(PP_THREADS), 0, s, static_cast<const uint16_t*>(x),
-                       m.xh, m.xhl, m.rs, rows, K, idx, P, E, m.order, m.segs, m.nseg);
+                       m.xh, m.xhl, m.rs, rows, K, idx, P, E, m.order, m.segs, m.nseg, moe_seg_rows(P, E, N, glu));
   else
     hipLaunchKernelGGL(moe_prologue_kernel<KQ_BF16>, dim3(rows + 1), dim3(PP_THREADS), 0, s, static_cast<const uint16_t*>(x),
-                       m.xh, m.xhl, m.rs, rows, K, idx, P, E, m.order, m.segs, m.nseg);
+                       m.xh, m.xhl, m.rs, rows, K, idx, P, E, m.order, m.segs, m.nseg, moe_seg_rows(P, E, N, glu));
   KQ_HIP_CHECK(hipGetLastError());
   MoeArgs a{};
   a.xh = m.xh;

@@ -6,7 +6,7 @@
 
 namespace kqsort {
 
-constexpr int SEG_M = 32;  // pairs per segment at most
+constexpr int SEG_M = 32;  // pairs per segment at most, unless the caller says otherwise
 constexpr int SORT_MAX_E = 4096;
 
 struct Segment {
@@ -14,7 +14,7 @@ struct Segment {
 };
 
 // ------------------------------------------------------------------ pair sort (one workgroup)
-// order[] = pair ids grouped by expert; segs[] = (expert, first position in order, pairs <= 32).
+// order[] = pair ids grouped by expert; segs[] = (expert, first position in order, pairs <= seg_rows).
 // Pairs whose expert id is out of range are left out (their output rows are not written).
 // One pass over the indices: a pair's rank inside its expert is what the histogram's atomic add returns, so the
 // scatter needs no second count (the order inside an expert is then arbitrary, which no consumer depends on: every
@@ -23,7 +23,7 @@ struct Segment {
 template <int THREADS>
 __device__ __forceinline__ void moe_sort_body(const uint32_t* __restrict__ idx, int P, int E, int* __restrict__ order,
                                               Segment* __restrict__ segs, int* __restrict__ nseg_out, int* cnt,
-                                              int* scan_p, int* scan_s) {
+                                              int* scan_p, int* scan_s, int seg_rows = SEG_M) {
   constexpr int PPT = 8, NW = THREADS / 64;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const bool small = P <= THREADS * PPT;
@@ -40,9 +40,16 @@ __device__ __forceinline__ void moe_sort_body(const uint32_t* __restrict__ idx, 
 #pragma unroll
     for (int i = 0; i < PPT; i++) rk[i] = ev[i] < (uint32_t)E ? atomicAdd(&cnt[ev[i]], 1) : -1;
   } else {
-    for (int p = tid; p < P; p += THREADS) {
-      const uint32_t e = idx[p];
-      if (e < (uint32_t)E) atomicAdd(&cnt[e], 1);
+    for (int p0 = tid; p0 < P; p0 += THREADS * PPT) {
+      // PPT loads in flight: one at a time costs its latency per pair (prologue of 8000 pairs 24 -> 12 us)
+#pragma unroll
+      for (int i = 0; i < PPT; i++) {
+        const int p = p0 + THREADS * i;
+        ev[i] = p < P ? idx[p] : 0xffffffffu;
+      }
+#pragma unroll
+      for (int i = 0; i < PPT; i++)
+        if (ev[i] < (uint32_t)E) atomicAdd(&cnt[ev[i]], 1);
     }
   }
   __syncthreads();
@@ -53,7 +60,7 @@ __device__ __forceinline__ void moe_sort_body(const uint32_t* __restrict__ idx, 
     const int e = tid * ch + i;
     if (e < E) {
       lp += cnt[e];
-      ls += (cnt[e] + SEG_M - 1) / SEG_M;
+      ls += (cnt[e] + seg_rows - 1) / seg_rows;
     }
   }
   int ip = lp, is = ls;  // inclusive scan inside the wave
@@ -88,8 +95,8 @@ __device__ __forceinline__ void moe_sort_body(const uint32_t* __restrict__ idx, 
     const int e = tid * ch + i;
     if (e < E) {
       const int c = cnt[e];
-      for (int k = 0, sg = bs; k < c; k += SEG_M, sg++) segs[sg] = Segment{e, bp + k, c - k < SEG_M ? c - k : SEG_M, 0};
-      bs += (c + SEG_M - 1) / SEG_M;
+      for (int k = 0, sg = bs; k < c; k += seg_rows, sg++) segs[sg] = Segment{e, bp + k, c - k < seg_rows ? c - k : seg_rows, 0};
+      bs += (c + seg_rows - 1) / seg_rows;
       cnt[e] = bp;  // first position of the expert's pairs (small) / running cursor
       bp += c;
     }
@@ -100,9 +107,17 @@ __device__ __forceinline__ void moe_sort_body(const uint32_t* __restrict__ idx, 
     for (int i = 0; i < PPT; i++)
       if (rk[i] >= 0) order[cnt[ev[i]] + rk[i]] = tid + THREADS * i;
   } else {
-    for (int p = tid; p < P; p += THREADS) {
-      const uint32_t e = idx[p];
-      if (e < (uint32_t)E) order[atomicAdd(&cnt[e], 1)] = p;
+    for (int p0 = tid; p0 < P; p0 += THREADS * PPT) {
+#pragma unroll
+      for (int i = 0; i < PPT; i++) {
+        const int p = p0 + THREADS * i;
+        ev[i] = p < P ? idx[p] : 0xffffffffu;
+      }
+#pragma unroll
+      for (int i = 0; i < PPT; i++) rk[i] = ev[i] < (uint32_t)E ? atomicAdd(&cnt[ev[i]], 1) : -1;
+#pragma unroll
+      for (int i = 0; i < PPT; i++)
+        if (rk[i] >= 0) order[rk[i]] = p0 + THREADS * i;
     }
   }
 }

@@ -97,6 +97,28 @@ def test_gather_qmv_mix_ns(kq, codec, T, S):
         assert bool(((a - b).abs() <= bound).all()), (codec, T, float((a - b).abs().max()))
 
 
+@pytest.mark.parametrize("codec", ["q4_k", "q5_k", "q6_k"])
+@pytest.mark.parametrize("T,S,E,N", [(90, 2, 3, 11008),   # 60 pairs per expert: segments of 33 to 64 pairs, one of a few
+                                     (64, 2, 2, 16384),   # exactly one full segment each; the fused op too
+                                     (310, 7, 9, 136)])   # more pairs than the sort keeps in registers
+def test_grouped_ops_on_64_pair_segments(kq, codec, T, S, E, N):
+    K = 256
+    w, w2 = _stack(codec, E, N, K, 71), _stack(codec, E, N, K, 72)
+    rng = np.random.default_rng(73)
+    idx = rng.permutation(np.arange(T * S) % E).reshape(T, S)
+    idx[0, 0] = (idx[0, 0] + 1) % E
+    scores = rng.uniform(0.05, 1.0, (T, S)).astype(np.float32)
+    xb, xt = make_x((T, S, K), "bfloat16", seed=74, scale=0.05)
+    got = kq.gather_qmv_mix_ns_kq(xt, wire_to_dev(w), codec, _idx_dev(idx), torch.from_numpy(scores).cuda())
+    want = O.gather_qmv_mix(xb, w, None, codec, None, idx, scores, "bfloat16")
+    assert rel_l2(dev_to_bits(got), want, "bfloat16") <= TOL, (codec, T, S)
+    xb, xt = make_x((T, K), "bfloat16", seed=75, scale=0.05)
+    for n in (T, T // 2):
+        got = kq.moe_glu_gather_kq(xt[:n], wire_to_dev(w), wire_to_dev(w2), codec, _idx_dev(idx[:n]))
+        want = O.moe_glu_gather(xb[:n], w, w2, codec, idx[:n], "silu", dtype="bfloat16")
+        assert rel_l2(dev_to_bits(got), want, "bfloat16") <= TOL, (codec, n, S)
+
+
 @pytest.mark.parametrize("T", [1, 3, 20])
 @pytest.mark.parametrize("shared", [False, True])
 def test_gather_qmv_mix_skips_expert_ids_outside_the_stack(kq, shared, T):
