@@ -132,6 +132,24 @@ def test_gather_qmm_no_transpose_many_rows_per_entry(kq, codec):
     assert rel_l2(dev_to_bits(out[keep]), want, "bfloat16") <= TOL
 
 
+@pytest.mark.parametrize("codec,dtype", [("q4_k", "bfloat16"), ("q8_0", "float16"), ("iq3_s", "bfloat16")])
+@pytest.mark.parametrize("M,B", [(1, 70), (3, 64), (8, 13), (1, 600)])
+def test_gather_qmm_no_transpose_entries_of_one_expert_share_tiles(kq, codec, dtype, M, B):
+    """transpose=False with more than twice as many entries as experts: experts named once, more often than a tile holds,
+    and not at all, repeated lhs rows, an expert id outside the stack."""
+    E, K, N = 5, 72, 256 if codec != "q8_0" else 160
+    wire = _stack(codec, E, K, N, seed=246)
+    xb, xt = make_x((B, M, K), dtype, seed=247)
+    rng = np.random.default_rng(248)
+    lhs, rhs = rng.integers(0, B, B), rng.choice(3, B)
+    rhs[B // 2], rhs[1] = 4, 9
+    got = kq.gather_qmm(xt, wire_to_dev(wire), None, codec, lhs_indices=_idx_dev(lhs), rhs_indices=_idx_dev(rhs),
+                        transpose=False)
+    keep = [i for i in range(B) if i != 1]
+    want = O.gather_qmm(xb, wire, codec, lhs[keep], rhs[keep], False, dtype)
+    assert rel_l2(dev_to_bits(got[keep]), want, dtype) <= TOL
+
+
 def test_gather_qmm_reference_moe_fixture_and_strided_experts(kq):
     wire = np.load(os.path.join(GOLD, "q4_k_moe.npz"))["wire"]  # [4, 128, 288]
     E, N, K, B = 4, 128, 512, 64
