@@ -88,32 +88,32 @@ __global__ __launch_bounds__(MP_THREADS) void mid_prepass_kernel(const uint16_t*
     const int g = tid + MP_THREADS * r;
     keep[r] = g < ngroups ? fetch(g) : u32x4{0, 0, 0, 0};
   }
-  float inv = 1.f, scale = 1.f;
-  if constexpr (DT == KQ_BF16) {
-    float amax = 0.f;
-    auto take = [&](u32x4 v) {
+  // The row's power of two puts its largest magnitude into [2^14, 2^15), f16 rows too where that scales up (exact): the
+  // hi / lo sums below need room under them.  Left as they came, f16 rows of 6e-5 had their sums rounded to 2^-24, 0.18 % of
+  // a q4_1 result.
+  float inv = 1.f, scale = 1.f, amax = 0.f;
+  auto lo_f = [](uint32_t v) { return DT == KQ_BF16 ? __builtin_bit_cast(float, v << 16) : kq::h2f((uint16_t)(v & 0xffffu)); };
+  auto hi_f = [](uint32_t v) { return DT == KQ_BF16 ? __builtin_bit_cast(float, v & 0xffff0000u) : kq::h2f((uint16_t)(v >> 16)); };
+  auto take = [&](u32x4 v) {
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] << 16)));
-        amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] & 0xffff0000u)));
-      }
-    };
+    for (int e = 0; e < 4; e++) amax = fmaxf(amax, fmaxf(fabsf(lo_f(v[e])), fabsf(hi_f(v[e]))));
+  };
 #pragma unroll
-    for (int r = 0; r < MP_REGS; r++) take(keep[r]);
-    for (int g = tid + MP_THREADS * MP_REGS; g < ngroups; g += MP_THREADS) take(fetch(g));
+  for (int r = 0; r < MP_REGS; r++) take(keep[r]);
+  for (int g = tid + MP_THREADS * MP_REGS; g < ngroups; g += MP_THREADS) take(fetch(g));
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
-    if ((tid & 63) == 0) red[tid >> 6] = amax;
-    __syncthreads();
+  for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+  if ((tid & 63) == 0) red[tid >> 6] = amax;
+  __syncthreads();
 #pragma unroll
-    for (int w = 0; w < MP_THREADS / 64; w++) amax = fmaxf(amax, red[w]);
-    const uint32_t eb = (__builtin_bit_cast(uint32_t, amax) >> 23) & 0xff;
-    if (eb != 0 && eb != 0xff) {
-      int e = (int)eb - 127 - 14;  // the largest magnitude lands in [2^14, 2^15)
-      if (e < -100) e = -100;
-      scale = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
-      inv = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23);
-    }
+  for (int w = 0; w < MP_THREADS / 64; w++) amax = fmaxf(amax, red[w]);
+  const uint32_t eb = (__builtin_bit_cast(uint32_t, amax) >> 23) & 0xff;
+  if (eb != 0 && eb != 0xff) {
+    int e = (int)eb - 127 - 14;
+    if (e < -100) e = -100;
+    if (DT == KQ_F16 && e > 0) e = 0;
+    scale = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
+    inv = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23);
   }
   if (tid == 0) rs[m] = scale;
   uint8_t* base = xf + (size_t)(m >> 5) * nsteps * NF * 1024 + 16 * (m & 31);
@@ -121,13 +121,8 @@ __global__ __launch_bounds__(MP_THREADS) void mid_prepass_kernel(const uint16_t*
     _Float16 h[8];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      if constexpr (DT == KQ_BF16) {
-        h[2 * e] = (_Float16)(__builtin_bit_cast(float, v[e] << 16) * inv);
-        h[2 * e + 1] = (_Float16)(__builtin_bit_cast(float, v[e] & 0xffff0000u) * inv);
-      } else {
-        h[2 * e] = __builtin_bit_cast(_Float16, (uint16_t)(v[e] & 0xffff));
-        h[2 * e + 1] = __builtin_bit_cast(_Float16, (uint16_t)(v[e] >> 16));
-      }
+      h[2 * e] = (_Float16)(lo_f(v[e]) * inv);
+      h[2 * e + 1] = (_Float16)(hi_f(v[e]) * inv);
     }
     const int st = g >> 5, pc = g & 31;
     uint8_t* step = base + (size_t)st * NF * 1024;

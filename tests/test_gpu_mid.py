@@ -85,3 +85,24 @@ def test_mid_cut_steps_replay(mid):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want[r % 4]), r
+
+
+@pytest.mark.parametrize("codec", ["q4_1", "q5_1", "q2_k"])
+def test_mid_small_f16_rows_keep_their_sums(mid, codec):
+    """f16 activations of about 2^-14 under weights with a large block minimum: the sums that multiply the minimum are two
+    f16 terms and need the row's power of two.  One rounding of the result to f16 is at most 2^-11 of it; unscaled sums
+    (granularity 2^-24) put q4_1 1.8e-3 and q5_1 0.9e-3 off here."""
+    import numpy as np
+    M, N, K = 16, 64, 1024
+    wpb = mid.CODEC_GEOMETRY[codec][3]
+    blocks = O.synth_wire(codec, N * K // wpb, seed=8).reshape(N * K // wpb, -1)
+    # codes and minima that nearly cancel
+    d, m = (np.array([v], np.float16).view(np.uint8) for v in {"q4_1": (16, -128), "q5_1": (16, -256), "q2_k": (64, 96)}[codec])
+    if codec == "q2_k":  # d and dmin end the block; 4-bit scales and minima of their own
+        blocks[:, -4:-2], blocks[:, -2:] = d, m
+    else:
+        blocks[:, 0:2], blocks[:, 2:4] = d, m
+    wire = blocks.reshape(N, -1)
+    xb, xt = make_x((M, K), "float16", seed=9, scale=2.0**-14)
+    got = dev_to_bits(mid.quantized_matmul(xt, wire_to_dev(wire), None, codec))
+    assert rel_l2(got, O.qmm(xb, wire, codec, True, "float16"), "float16") <= 2.0**-11
