@@ -58,6 +58,24 @@ def test_sqrtsoftplus_bias_ties(kq, dtype, e, r, spread):
            scale=1.5)
 
 
+@pytest.mark.parametrize("e,r", [(1, 1), (2, 2), (63, 16), (127, 8), (128, 8), (129, 8), (255, 3), (256, 16), (257, 16), (1000, 7)])
+def test_ties_and_masked_experts_at_the_lane_split_edges(kq, e, r):
+    """Few distinct logits (ties across lanes and inside one), experts masked with -inf: exactly the oracle's picks."""
+    rng = np.random.default_rng(e)
+    logits = rng.integers(-2, 3, (11, e)).astype(np.float32)
+    if e > 2:
+        logits[3, rng.integers(0, e, e // 3)] = -np.inf
+        logits[4] = 1.0
+        logits[4, : e - 1] = -np.inf  # fewer live experts than picks
+    want_i, want_s = O.router_topk(O.f32_to_bits(logits, "float32"), "float32", r, True, False, None, None, 0, 1.0)
+    got_i, got_s = kq.moe_router_topk(torch.from_numpy(logits).cuda(), r, True, shared_gate=False)
+    live = [t for t in range(11) if t != 4]
+    assert np.array_equal(got_i.cpu().numpy().view(np.uint32)[live], want_i[live])
+    assert np.allclose(got_s.cpu().numpy()[live], want_s[live], rtol=1e-5, atol=1e-6)
+    first = got_i.cpu().numpy()[4, 0], want_i[4, 0]
+    assert first[0] == first[1] and got_i.max() < e
+
+
 def test_feeds_the_fused_moe_ops(kq):
     """indices / scores come out in the form the fused MoE ops take."""
     from gpu_util import make_x, wire_to_dev
