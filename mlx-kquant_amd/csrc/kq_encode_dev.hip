@@ -20,6 +20,11 @@ namespace {
 __device__ __forceinline__ float clamp_level(float v, float lo, float hi) {  // clampi(rne(v), lo, hi), kept as a float
   return __builtin_amdgcn_fmed3f(__builtin_rintf(v), lo, hi);
 }
+// The same where the levels go below zero and v may be a NaN: the integer conversion made that level 0, the median of three
+// makes it the lower bound.  (With lo = 0 both are 0.)
+__device__ __forceinline__ float clamp_level_signed(float v, float lo, float hi) {
+  return v == v ? clamp_level(v, lo, hi) : 0.f;
+}
 
 // four weights at element i (a multiple of four) of w, widened exactly
 __device__ __forceinline__ float4 load4(const void* w, int dtype, int64_t i) {
@@ -70,7 +75,8 @@ __global__ __launch_bounds__(LEG_THREADS) void encode_legacy_kernel(const void* 
   const int64_t blk = min(blk0 + b, nblocks - 1);  // lanes past the end redo the last block; their bytes are not stored
   const float4 v4 = load4_any(w, dtype, blk * 32 + 4 * t, aligned);
   const float v[4] = {v4.x, v4.y, v4.z, v4.w};
-  float amax = 0.f, lo = v[0], hi = v[0];
+  // the block's first weight starts the minimum and the maximum (a NaN there stays); a later NaN is passed over
+  float amax = 0.f, lo = t == 0 ? v[0] : INFINITY, hi = t == 0 ? v[0] : -INFINITY;
   for (int i = 0; i < 4; i++) {
     amax = std::max(amax, std::fabs(v[i]));
     lo = std::min(lo, v[i]);
@@ -203,8 +209,10 @@ __device__ __forceinline__ float fit_scale_min(const float (&x)[N], const float 
   return flat ? 0.f : scale;
 }
 
-// kqenc::fit_signed16 (the acceptance test compares against a rounded running best, so the candidates stay in order)
-template <int NMAX>
+// kqenc::fit_signed16 (the acceptance test compares against a rounded running best, so the candidates stay in order).
+// FINITE: no weight of the wave is infinite or a NaN, so no level is a NaN either (the factors are finite: peaks below 1e-30
+// return 0 whatever the scan did).
+template <int NMAX, bool FINITE>
 __device__ __forceinline__ float fit_signed16(const float (&x)[16], const float (&wt)[16]) {
   float peak = 0.f, apeak = 0.f;
 #pragma unroll
@@ -222,7 +230,8 @@ __device__ __forceinline__ float fit_signed16(const float (&x)[16], const float 
     slx = sl2 = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; i++) {
-      const float l = clamp_level(inv * x[i], -float(NMAX), float(NMAX - 1));
+      const float l = FINITE ? clamp_level(inv * x[i], -float(NMAX), float(NMAX - 1))
+                             : clamp_level_signed(inv * x[i], -float(NMAX), float(NMAX - 1));
       slx += wx[i] * l;
       sl2 += wt[i] * l * l;
     }
@@ -410,7 +419,10 @@ __global__ __launch_bounds__(64) void encode_k_kernel(const void* __restrict__ w
         s_lv[sb][N * j + i] = ds == 0.f ? 0 : (uint8_t)(int)clamp_level((x[i] + dm) / ds, 0.f, float(KGeom<C>::NMAX));
   } else {
     constexpr int NMAX = C == KQ_Q6_K ? 32 : 4;
-    s_sc[sb][j] = fit_signed16<NMAX>(x, wt);
+    bool finite = true;
+#pragma unroll
+    for (int i = 0; i < N; i++) finite &= std::fabs(x[i]) < INFINITY;
+    s_sc[sb][j] = __builtin_amdgcn_ballot_w64(!finite) == 0 ? fit_signed16<NMAX, true>(x, wt) : fit_signed16<NMAX, false>(x, wt);
     __syncthreads();
     float peak = 0.f, apeak = 0.f;
     for (int i = 0; i < 16; i++) {
@@ -441,7 +453,7 @@ __global__ __launch_bounds__(64) void encode_k_kernel(const void* __restrict__ w
 #pragma unroll
     for (int i = 0; i < N; i++)
       s_lv[sb][N * j + i] =
-          de == 0.f ? NMAX : (uint8_t)((int)clamp_level(x[i] / de, -float(NMAX), float(NMAX - 1)) + NMAX);
+          de == 0.f ? NMAX : (uint8_t)((int)clamp_level_signed(x[i] / de, -float(NMAX), float(NMAX - 1)) + NMAX);
   }
   __syncthreads();
 

@@ -149,3 +149,18 @@ def test_device_encoder_both_lane_splits_and_ragged_ends(kq, codec, dtype):
             wd = flat[off:off + rows * K].copy_(w.reshape(-1)).reshape(rows, K)
             dev = kq.quantize(wd, codec, None if im is None else im.cuda())[0]
             assert torch.equal(dev.cpu(), host), (codec, rows, K, off)
+
+
+@pytest.mark.parametrize("codec", DEV_CODECS)
+def test_device_encoder_nonfinite_weights_keep_their_bytes(kq, codec):
+    """NaN, infinite and f16-overflowing weights: the bytes that the sequential block encoders write when compiled for the
+    device, where a NaN level converts to 0 (tests/golden/encode_nonfinite.npz, made by them on gfx950; the host build
+    converts a NaN to the lowest int, so kq_quantize is no reference here).  Rows: a NaN as each lane's first weight of the
+    legacy blocks, infinities, whole NaN blocks, scales past the f16 range."""
+    gold = np.load(os.path.join(GOLD, "encode_nonfinite.npz"))
+    w, im = torch.from_numpy(gold["w"]).cuda(), torch.from_numpy(gold["imatrix"]).cuda()
+    for key, imat in ((codec, None), (codec + "_im", im)):
+        if key in gold:
+            got = kq.quantize(w, codec, imat)[0].cpu().numpy()
+            bad = np.argwhere((got != gold[key]).any(axis=1)).ravel().tolist()
+            assert not bad, (key, bad)
