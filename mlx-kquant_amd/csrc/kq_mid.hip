@@ -14,12 +14,16 @@
 //     fragment is one coalesced 16-byte load per lane straight into registers (L2 serves every tile after the first).
 //     Loads of a wave return in order, so fragments and wire bytes of the next step are requested together and waited
 //     for together.
+//   * bf16 activations become f16 under their row's power of two: exact down to 2^-31 of the row's largest value.  A row of
+//     wider range (a value as large as a mask's beside ordinary ones) is flagged by the prepass, and its block of 32 rows
+//     takes the activations as they are (wide_step).
 //   * 33 rows and more run as blocks of 32 rows: the blocks of a tile are neighbours in launch order on one XCD, so that
 //     the second one finds the wire bytes in its L2.
 // Measured: see the routing in kq_mid_supported.
 #include <algorithm>
 
 #include "kq_codes.h"
+#include "kq_decode.h"
 #include "kq_dma.h"
 #include "kq_kfrag.h"
 
@@ -27,6 +31,7 @@ namespace {
 
 using namespace kqcodes;
 using namespace kqdma;
+using kqmma::RowRange;
 using kqmma::u32x4;
 
 template <int C>
@@ -66,6 +71,7 @@ constexpr int mid_table_bytes() {
 // x[j], x[j + 16] interleaved over every 32 (ORD 3: x[j], x[j + 8] over every 16).  NSUM 1: fragment 16 = sums of the eight 32-wide blocks, kg 0 the f16 part hi,
 // kg 1 the remainder lo, X = 32 (hi + lo); NSUM 2: fragments 16 / 17 = hi / lo of the sixteen 16-wide sums, X = 16 (hi + lo).
 // Rows past M are not written: what they hold reaches output rows that are not stored.
+// rs[m] is negative for a wide row (RowRange).
 constexpr int MP_THREADS = 512, MP_REGS = 4;
 
 template <int DT, int ORD, int NSUM>
@@ -74,6 +80,7 @@ __global__ __launch_bounds__(MP_THREADS) void mid_prepass_kernel(const uint16_t*
                                                                  int* __restrict__ counters, int ncounters) {
   constexpr int NF = 16 + NSUM;
   __shared__ float red[MP_THREADS / 64];
+  __shared__ uint32_t range_lds[MP_THREADS / 64 + 2];
   const int m = blockIdx.x, tid = threadIdx.x;
   // arrival counters of the main kernel's cut tiles
   for (int i = m * MP_THREADS + tid; i < ncounters; i += gridDim.x * MP_THREADS) counters[i] = 0;
@@ -115,12 +122,13 @@ __global__ __launch_bounds__(MP_THREADS) void mid_prepass_kernel(const uint16_t*
     scale = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
     inv = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23);
   }
-  if (tid == 0) rs[m] = scale;
+  RowRange range;
   uint8_t* base = xf + (size_t)(m >> 5) * nsteps * NF * 1024 + 16 * (m & 31);
   auto convert = [&](int g, u32x4 v) {  // whole octets of lanes stay together
     _Float16 h[8];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
+      if constexpr (DT == KQ_BF16) range.take(v[e]);
       h[2 * e] = (_Float16)(lo_f(v[e]) * inv);
       h[2 * e + 1] = (_Float16)(hi_f(v[e]) * inv);
     }
@@ -171,12 +179,16 @@ __global__ __launch_bounds__(MP_THREADS) void mid_prepass_kernel(const uint16_t*
     if (g < ngroups) convert(g, keep[r]);
   }
   for (int g = tid + MP_THREADS * MP_REGS; g < ngroups; g += MP_THREADS) convert(g, fetch(g));
+  bool wide = false;
+  if constexpr (DT == KQ_BF16) wide = range.wide<MP_THREADS / 64>(scale, eb == 0xff, xi, K, tid, range_lds);
+  if (tid == 0) rs[m] = wide ? -scale : scale;
 }
 
 // ------------------------------------------------------------------ main kernel
 constexpr int MID_WAVES = 8;
 
 struct MidArgs {
+  const uint16_t* x;
   const uint8_t* xf;
   const float* rs;
   const uint8_t* w;
@@ -335,6 +347,36 @@ __device__ __forceinline__ void mid_step(const uint8_t* b_lane, int kg, const f1
   }
 }
 
+// The step of a block that holds a row of wide range: bf16 activations as they are, weights by the reference-order decoder
+// from global memory in two bf16 terms (16 significant bits), the numerics of the any-codec kernel.  Rare, so small code
+// rather than speed: q8_0 4096 x 4096, 32 rows, 32 us (ordinary rows 13, the any-codec kernel 18).
+template <int C>
+__device__ __forceinline__ void wide_step(const MidArgs& a, int row0, int nrows, int mb, int st, int l32, int kg,
+                                          uint32_t row_bytes, f32x16& acc) {
+  using G = MidGeom<C>;
+  typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+  const int m = 32 * mb + l32 < a.M ? 32 * mb + l32 : a.M - 1, n = row0 + (l32 < nrows ? l32 : nrows - 1);
+  const uint16_t* x = a.x + (size_t)m * a.K;
+  const uint8_t* w = a.w + (size_t)n * row_bytes;
+  const int end = CK_STEP * (st + 1) < a.K ? CK_STEP * (st + 1) : a.K;
+#pragma unroll 1
+  for (int k0 = CK_STEP * st; k0 < end; k0 += 16) {  // K is a multiple of 32
+    const int k = k0 + 8 * kg;
+    float f[8];
+    kq::decode8<C>(w + (size_t)(k / G::WPB) * G::BPB, k % G::WPB / 8, a.grids, f);
+    bf16x8 hi, lo;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const uint32_t top = __builtin_bit_cast(uint32_t, f[e]) & 0xffff0000u;
+      hi[e] = __builtin_bit_cast(__bf16, (uint16_t)(top >> 16));
+      lo[e] = (__bf16)(f[e] - __builtin_bit_cast(float, top));
+    }
+    const bf16x8 xv = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(x + k));
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv, hi, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv, lo, acc, 0, 0, 0);
+  }
+}
+
 template <int C, int DT>
 __global__ __launch_bounds__(64 * MID_WAVES, 1) void mid_kernel(MidArgs a) {
   using G = MidGeom<C>;
@@ -391,9 +433,12 @@ __global__ __launch_bounds__(64 * MID_WAVES, 1) void mid_kernel(MidArgs a) {
     const int off = 16 * p < G::BYTES - 16 ? 16 * p : G::BYTES - 16;
     voff[T] = (uint32_t)r * row_bytes + (uint32_t)off;
   });
-  auto request = [&](Pos p, int slot, f16x8 (&an)[G::NF]) {
+  // rs of a block's rows, one per lane
+  auto row_scale = [&](int mb) { return a.rs[32 * mb + l32 < a.M ? 32 * mb + l32 : a.M - 1]; };
+  auto request = [&](Pos p, int slot, f16x8 (&an)[G::NF], float& rsn) {
     int tile, mb;
     tile_of(p.id, tile, mb);
+    if constexpr (DT == KQ_BF16) rsn = row_scale(mb);
     if (p.st >= p.end) return;
     const int row0 = tile * rpt, nrows = N - row0 < rpt ? N - row0 : rpt;
     const uint8_t* base = a.w + (size_t)row0 * row_bytes + (size_t)p.st * G::BYTES;
@@ -424,7 +469,7 @@ __global__ __launch_bounds__(64 * MID_WAVES, 1) void mid_kernel(MidArgs a) {
   };
 
   f32x16 acc = f32x16{0};
-  auto finish_tile = [&](int id, int slot) {
+  auto finish_tile = [&](int id, int slot, bool wide) {
     // the waves' sums meet in the slots just read (a wave's other slot may be receiving its next step)
     float* mine = reinterpret_cast<float*>(ring + (wave * 2 + slot) * SLOT);
 #pragma unroll
@@ -439,7 +484,7 @@ __global__ __launch_bounds__(64 * MID_WAVES, 1) void mid_kernel(MidArgs a) {
       const int i = e >> 6, l = e & 63;
       const int m = 32 * mb + 8 * (i >> 2) + 4 * (l >> 5) + (i & 3), c = l & 31;
       if (m < a.M && c < nrows && tile < ntiles) {
-        v *= a.rs[m];
+        if (!wide) v *= a.rs[m];
         a.y[(size_t)m * N + row0 + c] = DT == KQ_F16 ? kq::f2f16(v) : kq::f2bf16(v);
       }
     };
@@ -485,29 +530,38 @@ __global__ __launch_bounds__(64 * MID_WAVES, 1) void mid_kernel(MidArgs a) {
   f16x8 a0[G::NF], a1[G::NF];
 #pragma unroll
   for (int j = 0; j < G::NF; j++) a0[j] = a1[j] = f16x8{};
+  float rs0 = 0.f, rs1 = 0.f;
   Pos cur = first(blockIdx.x);
-  request(cur, 0, a0);
+  request(cur, 0, a0, rs0);
   // one step: wait for it, ask for the next one, multiply
-  auto body = [&](f16x8 (&ac)[G::NF], f16x8 (&an)[G::NF], int slot) -> bool {
+  auto body = [&](f16x8 (&ac)[G::NF], f16x8 (&an)[G::NF], float& rsc, float& rsn, int slot) -> bool {
     vmwait<0>();
     lgkm_drain();  // the other slot has been read: it may be filled again
 #pragma unroll
     for (int j = 0; j < G::NF; j++) asm volatile("" : "+v"(ac[j]));
     const Pos nxt = advance(cur);
     const bool more = nxt.id < a.items;
-    if (more) request(nxt, slot ^ 1, an);
-    if (cur.st < cur.end)
+    bool wide = false;
+    if constexpr (DT == KQ_BF16) wide = __builtin_amdgcn_ballot_w64(rsc < 0.f) != 0;
+    if (__builtin_expect(wide && cur.st < cur.end, 0)) {  // before the request: its registers are free here
+      int tile, mb;
+      tile_of(cur.id, tile, mb);
+      const int row0 = tile * rpt;
+      wide_step<C>(a, row0, N - row0 < rpt ? N - row0 : rpt, mb, cur.st, l32, kg, row_bytes, acc);
+    }
+    if (more) request(nxt, slot ^ 1, an, rsn);
+    if (__builtin_expect(cur.st < cur.end && !wide, 1))
       mid_step<C>(ring + (wave * 2 + slot) * SLOT + l32 * G::LROW, kg, ac, tabs, masks, K - CK_STEP * cur.st, acc);
     if (nxt.id != cur.id) {
       mid_wave_sync();
-      finish_tile(cur.id, slot);
+      finish_tile(cur.id, slot, wide);
     }
     cur = nxt;
     return more;
   };
   while (true) {
-    if (!body(a0, a1, 0)) break;
-    if (!body(a1, a0, 1)) break;
+    if (!body(a0, a1, rs0, rs1, 0)) break;
+    if (!body(a1, a0, rs1, rs0, 1)) break;
   }
 }
 
@@ -634,6 +688,7 @@ int kq_launch_mid(const void* x, const uint8_t* w, void* y, int M, int N, int K,
   uint8_t* xf = static_cast<uint8_t*>(ws);
   float* rs = reinterpret_cast<float*>(xf + mid_align(mb * nsteps * 18 * 1024));
   MidArgs a{};
+  a.x = static_cast<const uint16_t*>(x);
   a.xf = xf;
   a.rs = rs;
   a.w = w;

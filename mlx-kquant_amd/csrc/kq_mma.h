@@ -60,6 +60,45 @@ __device__ __forceinline__ uint32_t opaque_sgpr(uint32_t v) {
   return v;
 }
 
+// ------------------------------------------------------------------ bf16 rows beyond the range of f16
+// A bf16 row in f16 under its power of two (largest magnitude in [2^14, 2^15)) is exact down to 2^-31 of that magnitude;
+// smaller values lose bits, and from 2^-39 on they are 0.  Where the large values meet zero weights (a mask's value beside
+// ordinary ones) the small ones are the result.  A row is wide if more than one in 4096 of its nonzero values lost bits (a
+// row of fewer nonzero values: any), or if it holds an infinity.
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+struct RowRange {
+  u16x2 low = {0xffff, 0xffff};  // smallest nonzero magnitudes (15-bit patterns) less one
+  __device__ __forceinline__ void take(uint32_t pair) {
+    low = __builtin_elementwise_min(low, (u16x2)(__builtin_bit_cast(u16x2, pair & 0x7fff7fffu) - (uint16_t)1));
+  }
+  // over a workgroup of NW waves, all of it calling; row: its K values, lds: NW + 2 words
+  template <int NW>
+  __device__ __forceinline__ bool wide(float scale, bool infinite, const uint16_t* row, int K, int tid, uint32_t* lds) const {
+    // magnitudes from 1 to cut - 1 lose bits: below 2^-17 in the row's unit
+    const uint32_t cut = ((__builtin_bit_cast(uint32_t, scale) >> 23) - 17) << 7;
+    const uint64_t any = __builtin_amdgcn_ballot_w64((low[0] < low[1] ? low[0] : low[1]) < cut - 1);
+    if ((tid & 63) == 0) lds[tid >> 6] = any != 0;
+    if (tid < 2) lds[NW + tid] = 0;
+    __syncthreads();
+    uint32_t some = 0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) some |= lds[w];
+    if (__builtin_expect(some != 0, 0)) {  // uniform: count
+      uint32_t lost = 0, nonzero = 0;
+      for (int i = tid; i < K; i += 64 * NW) {
+        const uint32_t mag = row[i] & 0x7fffu;
+        lost += mag - 1 < cut - 1;
+        nonzero += mag != 0;
+      }
+      atomicAdd(&lds[NW], lost);
+      atomicAdd(&lds[NW + 1], nonzero);
+      __syncthreads();
+      infinite |= lds[NW] > lds[NW + 1] >> 12;
+    }
+    return infinite;
+  }
+};
+
 // ------------------------------------------------------------------ activation prepass (one row, 256 threads)
 // Outputs for row m (rows >= M are written as zeros):
 //   xh   f16 [Mpad][K]            x * 2^-e[m], k permuted inside 8-groups to k0 k2 k1 k3 k4 k6 k5 k7

@@ -106,3 +106,38 @@ def test_mid_small_f16_rows_keep_their_sums(mid, codec):
     xb, xt = make_x((M, K), "float16", seed=9, scale=2.0**-14)
     got = dev_to_bits(mid.quantized_matmul(xt, wire_to_dev(wire), None, codec))
     assert rel_l2(got, O.qmm(xb, wire, codec, True, "float16"), "float16") <= 2.0**-11
+
+
+def wide_rows_case(codec, M, K, N, seed):
+    """Weights whose first block is zero in every row, and bf16 activations with rows of a range beyond f16's: a mask's value
+    over the zero block beside ordinary ones, one large value beside tiny ones, half of the row large."""
+    wpb = O.geometry(codec)[0]
+    wire = O.synth_wire(codec, N * K // wpb, seed=seed).reshape(N, K // wpb, -1)
+    wire[:, 0] = 0
+    x = torch.randn((M, K), generator=torch.Generator().manual_seed(seed + 1))
+    x[3 % M, 1] = -3.0e38
+    x[M - 1, :wpb] = 1e30
+    x[M - 1, wpb:] *= 1e-12
+    x[M // 2, wpb - 1] = 7e9
+    x[M // 2, wpb:] *= 1e-3
+    xt = x.to(torch.bfloat16)
+    return wire.reshape(N, -1), xt.view(torch.int16).numpy().view("uint16"), xt.cuda()
+
+
+def row_errors(got, want):
+    """Largest relative 2-norm error of a row, bf16 bit patterns."""
+    import numpy as np
+    f = [(b.astype(np.uint32) << 16).view(np.float32).astype(np.float64) for b in (got, want)]
+    return np.max(np.linalg.norm(f[0] - f[1], axis=1) / np.linalg.norm(f[1], axis=1))
+
+
+@pytest.mark.parametrize("codec", all_codecs())
+def test_mid_rows_of_wide_range(mid, codec):
+    """Both blocks of rows, K with a tail where the codec has one, steps cut over workgroups: every row on its own within two
+    roundings to bf16 (2^-9 each, the reference's and the kernel's)."""
+    wpb = mid.CODEC_GEOMETRY[codec][3]
+    for M, N, K in ((9, 40, 512), (40, 72, 1024 + wpb), (33, 64, 8192)):
+        wire, xb, xt = wide_rows_case(codec, M, K, N, seed=70 + M)
+        got = dev_to_bits(mid.quantized_matmul(xt, wire_to_dev(wire), None, codec))
+        err = row_errors(got, O.qmm(xb, wire, codec, True, "bfloat16"))
+        assert err <= 2.0**-8, (codec, M, N, K, err)
