@@ -114,12 +114,15 @@ struct AnyArgs {
   KqOutMap om;          // grouped: where pair results go
   float* partial;       // dense split-K: f32 partial sums [ksplit][M][N] (null: round and store y)
   int steps_per_split;  // dense: K steps per blockIdx.y
+  KqRedo redo;          // MODE 3: the flags (see kq_common.h)
 };
 
-// MODE 0 = dense, 1 = grouped, 2 = grouped GLU (slab = 64 gate + 64 up rows; waves 0/2 gate, 1/3 up)
+// MODE 0 = dense, 1 = grouped, 2 = grouped GLU (slab = 64 gate + 64 up rows; waves 0/2 gate, 1/3 up), 3 = dense, only the
+// rows and columns that a tall-tile GEMM flagged
 template <int C, int DT, int MT, int MODE>
 __global__ __launch_bounds__(AM_THREADS, 1) void any_mma_kernel(AnyArgs a) {
   using G = StepGeom<C>;
+  constexpr bool DENSE = MODE == 0 || MODE == 3;
   constexpr int NA = DT == KQ_F16 ? 2 : 1;         // bf16 planes of the activation tile
   constexpr int TM = 32 * MT;
   constexpr int APT = TM * 32 / AM_THREADS;        // 16-byte activation pieces per thread per step
@@ -137,7 +140,7 @@ __global__ __launch_bounds__(AM_THREADS, 1) void any_mma_kernel(AnyArgs a) {
 
   Segment seg{0, 0, 0, 0};
   int m0 = 0, n0;
-  if constexpr (MODE == 0) {
+  if constexpr (DENSE) {
     const int mt = blockIdx.x % a.mtiles, nt = blockIdx.x / a.mtiles;  // consecutive workgroups share the weight rows
     m0 = mt * TM;
     n0 = nt * NCOLS;
@@ -145,6 +148,16 @@ __global__ __launch_bounds__(AM_THREADS, 1) void any_mma_kernel(AnyArgs a) {
     if ((int)blockIdx.y >= *a.nseg) return;  // uniform: the grid is sized for the worst case
     seg = a.segs[blockIdx.y];
     n0 = blockIdx.x * NCOLS;
+  }
+  if constexpr (MODE == 3) {  // uniform: a tile without a flag leaves
+    __shared__ int hit[AM_THREADS / 64];
+    bool flag = false;
+    if (tid < TM) flag = m0 + tid < a.M && a.redo.rows[m0 + tid];
+    if (tid < AM_BN / 32) flag |= n0 + 32 * tid < N && a.redo.cols[n0 / 32 + tid];
+    const bool any = __builtin_amdgcn_ballot_w64(flag) != 0;
+    if (lane == 0) hit[wave] = any;
+    __syncthreads();
+    if (!(hit[0] | hit[1] | hit[2] | hit[3])) return;
   }
   const int ncols = N - n0 < NCOLS ? N - n0 : NCOLS;
   const uint8_t* wbase = a.w + (size_t)seg.expert * (size_t)a.w_expert_stride;
@@ -163,7 +176,7 @@ __global__ __launch_bounds__(AM_THREADS, 1) void any_mma_kernel(AnyArgs a) {
     }
   };
 
-  if constexpr (MODE != 0) {
+  if constexpr (!DENSE) {
     if (tid < 32) pair_lds[tid] = tid < seg.count ? a.order[seg.start + tid] : -1;
   }
 
@@ -174,7 +187,7 @@ __global__ __launch_bounds__(AM_THREADS, 1) void any_mma_kernel(AnyArgs a) {
   for (int t = 0; t < APT; t++) {
     const int slot = a_slot + 8 * t;
     size_t row;
-    if constexpr (MODE == 0) {
+    if constexpr (DENSE) {
       row = (size_t)(m0 + slot < a.M ? m0 + slot : a.M - 1);
     } else {
       row = (size_t)(a.order[seg.start + (slot < seg.count ? slot : 0)] / a.x_div);
@@ -200,7 +213,7 @@ __global__ __launch_bounds__(AM_THREADS, 1) void any_mma_kernel(AnyArgs a) {
   // dense tiles past M are zero-filled without a load (a skinny call has 32 - M such rows)
   bool a_live[APT];
 #pragma unroll
-  for (int t = 0; t < APT; t++) a_live[t] = MODE != 0 || m0 + a_slot + 8 * t < a.M;
+  for (int t = 0; t < APT; t++) a_live[t] = !DENSE || m0 + a_slot + 8 * t < a.M;
 
   u32x4 areg[APT], wreg[G::WPT];
   auto issue = [&](int st) {
@@ -270,7 +283,7 @@ __global__ __launch_bounds__(AM_THREADS, 1) void any_mma_kernel(AnyArgs a) {
 
   // dense split-K: blockIdx.y owns K steps [st0, st1)
   int st0 = 0, st1 = nsteps;
-  if constexpr (MODE == 0) {
+  if constexpr (DENSE) {
     st0 = (int)blockIdx.y * a.steps_per_split;
     st1 = st0 + a.steps_per_split < nsteps ? st0 + a.steps_per_split : nsteps;
   }
@@ -315,7 +328,7 @@ __global__ __launch_bounds__(AM_THREADS, 1) void any_mma_kernel(AnyArgs a) {
   // ---- epilogue
   uint16_t* y = static_cast<uint16_t*>(a.y);
   auto store = [&](size_t off, float v) { y[off] = DT == KQ_F16 ? kq::f2f16(v) : kq::f2bf16(v); };
-  if constexpr (MODE == 0) {
+  if constexpr (DENSE) {
     const int n = n0 + wave * 32 + l32;
     float* part = a.partial ? a.partial + (size_t)blockIdx.y * a.M * N : nullptr;
 #pragma unroll
@@ -323,7 +336,7 @@ __global__ __launch_bounds__(AM_THREADS, 1) void any_mma_kernel(AnyArgs a) {
 #pragma unroll
       for (int i = 0; i < 16; i++) {
         const int m = m0 + t * 32 + 8 * (i >> 2) + 4 * kg + (i & 3);
-        if (m < a.M && n < N) {
+        if (m < a.M && n < N && (MODE != 3 || a.redo.rows[m] || a.redo.cols[n >> 5])) {
           if (part)
             part[(size_t)m * N + n] = acc[t][i];
           else
@@ -398,6 +411,16 @@ constexpr int SEG_M = 32;
 template <int C>
 struct AnyRun {
   static int run(const AnyArgs& a, int mode, int dt, int P, int E, hipStream_t s) {
+    if (mode == 3) {
+      if constexpr (C <= KQ_Q6_K || C == KQ_IQ4_XS) return KQ_ERR_UNSUPPORTED;  // (these have no tall-tile GEMM that flags)
+      else {
+        AnyArgs b = a;
+        const int tm = dt == KQ_F16 ? 64 : 128;
+        b.mtiles = (a.M + tm - 1) / tm;
+        const dim3 grid(b.mtiles * ((a.N + AM_BN - 1) / AM_BN), 1);
+        return dt == KQ_F16 ? launch_any<C, KQ_F16, 2, 3>(b, grid, s) : launch_any<C, KQ_BF16, 4, 3>(b, grid, s);
+      }
+    }
     if (mode == 0) {
       // one to four 32-row activation groups per workgroup; K split over blockIdx.y when the caller brought a
       // workspace (a.partial) and the plan asked for it
@@ -502,6 +525,24 @@ int kq_launch_anymma_dense(const void* x, const uint8_t* w, void* y, int M, int 
     a.steps_per_split = any_steps_per_split(M, N, K, dtype);
   }
   return dispatch_any(codec, a, 0, dtype, 0, 1, s);
+}
+
+// The rows and columns of y that a tall-tile GEMM has flagged, over what it wrote.
+int kq_launch_anymma_redo(const void* x, const uint8_t* w, void* y, int M, int N, int K, int codec, int dtype, KqRedo redo,
+                          hipStream_t s) {
+  AnyArgs a{};
+  a.x = x;
+  a.w = w;
+  a.y = y;
+  a.grids = kq_device_grids();
+  if (!a.grids) return KQ_ERR_HIP;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.x_div = 1;
+  a.steps_per_split = (K + AM_STEP - 1) / AM_STEP;
+  a.redo = redo;
+  return dispatch_any(codec, a, 3, dtype, 0, 1, s);
 }
 
 // Workspace of the batched MoE path: sorted pair list, segment table, segment count.

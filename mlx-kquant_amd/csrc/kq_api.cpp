@@ -129,9 +129,9 @@ size_t kq_qmm_workspace_size(int M, int N, int K, int transpose, int codec, int 
   size_t any = (M > 8 && kq_anymma_supported(M, N, K, codec)) ? kq_anymma_dense_workspace_bytes(M, N, K, dtype) : 0;
   if (mid > any) any = mid;
   if (kq_gemm2_low_supported(M, N, K, codec) && kq_gemm2_low_workspace_bytes(M, K) > any) any = kq_gemm2_low_workspace_bytes(M, K);
-  if (kq_gemm3b_supported(M, N, K, codec) && kq_gemm3b_workspace_bytes(M, K) > any) any = kq_gemm3b_workspace_bytes(M, K);
-  if (kq_gemm3f_supported(M, N, K, codec) && kq_gemm3f_workspace_bytes(M, K) > any) any = kq_gemm3f_workspace_bytes(M, K);
-  if (kq_gemm3i_supported(M, N, K, codec) && kq_gemm3i_workspace_bytes(M, K) > any) any = kq_gemm3i_workspace_bytes(M, K);
+  if (kq_gemm3b_supported(M, N, K, codec) && kq_gemm3b_workspace_bytes(M, N, K) > any) any = kq_gemm3b_workspace_bytes(M, N, K);
+  if (kq_gemm3f_supported(M, N, K, codec) && kq_gemm3f_workspace_bytes(M, N, K) > any) any = kq_gemm3f_workspace_bytes(M, N, K);
+  if (kq_gemm3i_supported(M, N, K, codec) && kq_gemm3i_workspace_bytes(M, N, K) > any) any = kq_gemm3i_workspace_bytes(M, N, K);
   return tuned > any ? tuned : any;
 }
 
@@ -172,15 +172,15 @@ int kq_qmm(const void* x_dev, const void* w_dev, void* y_dev, int M, int N, int 
     const int rcl = kq_launch_gemm2_low(x_dev, static_cast<const uint8_t*>(w_dev), y_dev, M, N, K, codec, dtype, workspace_dev, s);
     if (rcl != KQ_ERR_UNSUPPORTED) return rcl;
   }
-  if (kq_gemm3b_supported(M, N, K, codec) && workspace_dev && workspace_bytes >= kq_gemm3b_workspace_bytes(M, K)) {
+  if (kq_gemm3b_supported(M, N, K, codec) && workspace_dev && workspace_bytes >= kq_gemm3b_workspace_bytes(M, N, K)) {
     const int rcb = kq_launch_gemm3b(x_dev, static_cast<const uint8_t*>(w_dev), y_dev, M, N, K, codec, dtype, workspace_dev, s);
     if (rcb != KQ_ERR_UNSUPPORTED) return rcb;
   }
-  if (kq_gemm3f_supported(M, N, K, codec) && workspace_dev && workspace_bytes >= kq_gemm3f_workspace_bytes(M, K)) {
+  if (kq_gemm3f_supported(M, N, K, codec) && workspace_dev && workspace_bytes >= kq_gemm3f_workspace_bytes(M, N, K)) {
     const int rcf = kq_launch_gemm3f(x_dev, static_cast<const uint8_t*>(w_dev), y_dev, M, N, K, codec, dtype, workspace_dev, s);
     if (rcf != KQ_ERR_UNSUPPORTED) return rcf;
   }
-  if (kq_gemm3i_supported(M, N, K, codec) && workspace_dev && workspace_bytes >= kq_gemm3i_workspace_bytes(M, K)) {
+  if (kq_gemm3i_supported(M, N, K, codec) && workspace_dev && workspace_bytes >= kq_gemm3i_workspace_bytes(M, N, K)) {
     const int rci = kq_launch_gemm3i(x_dev, static_cast<const uint8_t*>(w_dev), y_dev, M, N, K, codec, dtype, workspace_dev, s);
     if (rci != KQ_ERR_UNSUPPORTED) return rci;
   }

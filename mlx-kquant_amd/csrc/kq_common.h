@@ -140,6 +140,19 @@ int kq_launch_gather_tuned(const void* x, const uint8_t* w, const uint8_t* w2, c
 // activations into ws (kq_mid_workspace_bytes) in matrix-operand order (kq_mid.hip).
 #define KQ_MID_MAX_ROWS 512
 bool kq_tall_fills(int M, int N, int codec);  // the rule between it and the tall-tile GEMMs
+// What a tall-tile GEMM of kq_gemm3b / 3f / 3i.hip could not hold in f16: activation rows (wide bf16 rows, RowRange of
+// kq_mma.h) and groups of 32 weight rows (results that are not finite, fp4 blocks too far apart), 1 = to be done again by
+// kq_launch_anymma_redo.  Null: nobody asks.
+struct KqRedo {
+  int* rows;  // [M]
+  int* cols;  // [(N + 31) / 32]
+};
+inline size_t kq_redo_bytes(int M, int N) { return ((size_t)M + (size_t)((N + 31) / 32)) * 4; }
+// Where the flags of a call lie in its workspace, behind the f16 activations and the row scales.  Calls that fill less than
+// three quarters of the chip only: the others have always been as the tall tiles give them, and pay for no second launch.
+KqRedo kq_tall_redo(void* ws, int M, int N, int K);
+int kq_launch_anymma_redo(const void* x, const uint8_t* w, void* y, int M, int N, int K, int codec, int dtype, KqRedo redo,
+                          hipStream_t s);
 bool kq_mid_supported(int M, int N, int K, int codec);
 size_t kq_mid_workspace_bytes(int M, int N, int K);
 void kq_mid_force_tile(int rows);
@@ -163,14 +176,14 @@ int kq_launch_gemm3(const void* xh, const void* xhl, const float* rs, const uint
 // 256-row / 128-row wave tiles for the 32-weight-block codecs with an f16 scale (q8_0, q4_0): every weight as two
 // exact f16 terms (kq_gemm3b.hip).  Runs its own activation prepass into ws (kq_gemm3b_workspace_bytes).
 bool kq_gemm3b_supported(int M, int N, int K, int codec);
-size_t kq_gemm3b_workspace_bytes(int M, int K);
+size_t kq_gemm3b_workspace_bytes(int M, int N, int K);
 void kq_gemm3b_force_tile(int rows);
 int kq_launch_gemm3b(const void* x, const uint8_t* w, void* y, int M, int N, int K, int codec, int dtype, void* ws,
                      hipStream_t s);
 // The same tiles for the fp4 codecs (mxfp4, nvfp4): one exact f16 term per weight, converted from the wire nibbles by
 // the hardware's fp4 -> f16 instruction (kq_gemm3f.hip).  Runs its own activation prepass into ws.
 bool kq_gemm3f_supported(int M, int N, int K, int codec);
-size_t kq_gemm3f_workspace_bytes(int M, int K);
+size_t kq_gemm3f_workspace_bytes(int M, int N, int K);
 void kq_gemm3f_force_tile(int rows);
 int kq_launch_gemm3f(const void* x, const uint8_t* w, void* y, int M, int N, int K, int codec, int dtype, void* ws,
                      hipStream_t s);
@@ -178,7 +191,7 @@ int kq_launch_gemm3f(const void* x, const uint8_t* w, void* y, int M, int N, int
 // weight (the reference-order decoder with d = 1), d in the unit of the running sums (kq_gemm3i.hip).  Runs its own
 // activation prepass into ws.
 bool kq_gemm3i_supported(int M, int N, int K, int codec);
-size_t kq_gemm3i_workspace_bytes(int M, int K);
+size_t kq_gemm3i_workspace_bytes(int M, int N, int K);
 void kq_gemm3i_force_tile(int rows);
 int kq_launch_gemm3i(const void* x, const uint8_t* w, void* y, int M, int N, int K, int codec, int dtype, void* ws,
                      hipStream_t s);

@@ -51,18 +51,25 @@ constexpr int f3_lds_bytes() {
 // a = 32 (G / 2) + 8 (G % 2) + 4 kg, D = 16 (mxfp4).
 template <int C, int DT>
 __global__ __launch_bounds__(256) void f3_prepass_kernel(const uint16_t* __restrict__ x, _Float16* __restrict__ xh,
-                                                         float* __restrict__ rs, int K) {
+                                                         float* __restrict__ rs, int K,
+                                                         KqRedo redo, int ncols) {
   __shared__ float red[4];
+  __shared__ uint32_t range_lds[6];
   const int m = blockIdx.x, tid = threadIdx.x, ngroups = K >> 3;
   const uint16_t* xi = x + (size_t)m * K;
   _Float16* xo = xh + (size_t)m * K;
   float inv = 1.f, scale = 1.f;
+  bool infinite = false;
+  RowRange range;
+  if (redo.cols)
+    for (int i = m * 256 + tid; i < ncols; i += gridDim.x * 256) redo.cols[i] = 0;
   if constexpr (DT == KQ_BF16) {
     float amax = 0.f;
     for (int g = tid; g < ngroups; g += 256) {
       const u32x4 v = *reinterpret_cast<const u32x4*>(xi + 8 * g);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
+        range.take(v[e]);
         amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] << 16)));
         amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] & 0xffff0000u)));
       }
@@ -73,6 +80,7 @@ __global__ __launch_bounds__(256) void f3_prepass_kernel(const uint16_t* __restr
     __syncthreads();
     amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     const uint32_t eb = (__builtin_bit_cast(uint32_t, amax) >> 23) & 0xff;
+    infinite = eb == 0xff;
     if (eb != 0 && eb != 0xff) {
       int e = (int)eb - 127 - 14;
       if (e < -100) e = -100;
@@ -81,6 +89,11 @@ __global__ __launch_bounds__(256) void f3_prepass_kernel(const uint16_t* __restr
     }
   }
   if (tid == 0) rs[m] = scale;
+  if (redo.rows) {
+    bool wide = false;
+    if constexpr (DT == KQ_BF16) wide = range.wide<4>(scale, infinite, xi, K, tid, range_lds);
+    if (tid == 0) redo.rows[m] = wide;
+  }
   for (int op = tid; op < ngroups; op += 256) {
     const int step = op >> 3, pi = op & 7;
     const int G = 2 * (pi >> 2) + (pi & 1), kg = (pi >> 1) & 1;
@@ -108,7 +121,7 @@ __global__ __launch_bounds__(64 * F3_WAVES, 1) void fp4_gemm3_kernel(const _Floa
                                                                     const float* __restrict__ rs,
                                                                     const uint8_t* __restrict__ w,
                                                                     uint16_t* __restrict__ y, int M, int N, int K,
-                                                                    int mtiles, int nt0) {
+                                                                    int mtiles, int nt0, int* redo_cols) {
   using G_ = F3Geom<C>;
   constexpr bool MX = C == KQ_MXFP4;
   constexpr int TM = 32 * MT, A_STAGE = TM * F3_KS * 2, AQ = MT / 2;
@@ -182,6 +195,7 @@ __global__ __launch_bounds__(64 * F3_WAVES, 1) void fp4_gemm3_kernel(const _Floa
   // mxfp4: the running sums of this column are in units of 2^uoff; B = code x 2^(E - uoff - 127) with the exponent
   // field E - uoff kept inside [104, 140]
   int uoff = 0, uoff_n = 0, pending = 0;
+  bool far = false;  // a block with nonzero codes lay below the window: its weights lost bits
   auto load_regs = [&](int slot, bool first) -> Regs {
     const uint8_t* rb = slot0 + slot * F3_SLOT + l32 * 48;
     Regs rg;
@@ -217,6 +231,8 @@ __global__ __launch_bounds__(64 * F3_WAVES, 1) void fp4_gemm3_kernel(const _Floa
       pending = uoff_n - target;  // the sums change unit by 2^pending when this step is entered
       uoff_n = target;
       const int f0 = e0 - target, f1 = e1 - target;  // a block below the window becomes zeros (field <= 0: 2^-127)
+      if (lo - target < 104)
+        far |= (f0 < 104 && ((rg.q[0] | rg.q[1]) & 0x77777777u)) || (f1 < 104 && ((rg.q[2] | rg.q[3]) & 0x77777777u));
       rg.s[0] = (uint32_t)(f0 > 0 ? f0 : 0) << 23;
       rg.s[1] = (uint32_t)(f1 > 0 ? f1 : 0) << 23;
     } else {
@@ -309,6 +325,7 @@ __global__ __launch_bounds__(64 * F3_WAVES, 1) void fp4_gemm3_kernel(const _Floa
 
   // ---- epilogue: back to plain units, undo the per-row activation scale, round once, store
   const int n = n0 + wave * 32 + l32;
+  bool redo = MX && far;
 #pragma unroll
   for (int t = 0; t < MT; t++) {
 #pragma unroll
@@ -317,15 +334,17 @@ __global__ __launch_bounds__(64 * F3_WAVES, 1) void fp4_gemm3_kernel(const _Floa
       if (m < M && n < N) {
         float v = acc[t][i] * rs[m];
         if constexpr (MX) v = __builtin_ldexpf(v, uoff);
+        redo |= !(fabsf(v) < INFINITY);
         y[(size_t)m * N + n] = DT == KQ_F16 ? kq::f2f16(v) : kq::f2bf16(v);
       }
     }
   }
+  if (redo_cols && redo && n < N) redo_cols[n >> 5] = 1;
 }
 
 template <int C, int DT, int MT>
 int launch_f3(const _Float16* xh, const float* rs, const uint8_t* w, void* y, int M, int N, int K, int nt0, int ntiles,
-              hipStream_t s) {
+              int* redo_cols, hipStream_t s) {
   if (ntiles <= 0) return KQ_OK;
   const int mtiles = (M + 32 * MT - 1) / (32 * MT);
   constexpr int lds = f3_lds_bytes<MT>();
@@ -333,16 +352,16 @@ int launch_f3(const _Float16* xh, const float* rs, const uint8_t* w, void* y, in
   auto kern = fp4_gemm3_kernel<C, DT, MT>;
   KQ_SET_MAX_LDS_ONCE((kern), lds);
   hipLaunchKernelGGL(kern, dim3(mtiles * ntiles), dim3(64 * F3_WAVES), lds, s, xh, rs, w, static_cast<uint16_t*>(y), M, N, K,
-                     mtiles, nt0);
+                     mtiles, nt0, redo_cols);
   KQ_HIP_CHECK(hipGetLastError());
   return KQ_OK;
 }
 
 template <int C, int DT>
 int launch_f3_tiles(const _Float16* xh, const float* rs, const uint8_t* w, void* y, int M, int N, int K, int nt0,
-                    int ntiles, int tile_rows, hipStream_t s) {
-  return tile_rows == 128 ? launch_f3<C, DT, 4>(xh, rs, w, y, M, N, K, nt0, ntiles, s)
-                          : launch_f3<C, DT, 8>(xh, rs, w, y, M, N, K, nt0, ntiles, s);
+                    int ntiles, int tile_rows, int* redo_cols, hipStream_t s) {
+  return tile_rows == 128 ? launch_f3<C, DT, 4>(xh, rs, w, y, M, N, K, nt0, ntiles, redo_cols, s)
+                          : launch_f3<C, DT, 8>(xh, rs, w, y, M, N, K, nt0, ntiles, redo_cols, s);
 }
 
 int f3_num_cus() {
@@ -355,14 +374,15 @@ int f3_num_cus() {
 static int g_f3_force = 0;  // kq_set_gemm_tile_rows: 1024 / 1025 force one tile height for every column tile, 64 switches the kernel off
 
 template <int C, int DT>
-int launch_f3_call(const void* x, const uint8_t* w, void* y, int M, int N, int K, void* ws, int force, hipStream_t s) {
+int launch_f3_call(const void* x, const uint8_t* w, void* y, int M, int N, int K, void* ws, int force, KqRedo redo, hipStream_t s) {
   _Float16* xh = static_cast<_Float16*>(ws);
   float* rs = reinterpret_cast<float*>(xh + (size_t)M * K);
-  hipLaunchKernelGGL((f3_prepass_kernel<C, DT>), dim3(M), dim3(256), 0, s, static_cast<const uint16_t*>(x), xh, rs, K);
+  hipLaunchKernelGGL((f3_prepass_kernel<C, DT>), dim3(M), dim3(256), 0, s, static_cast<const uint16_t*>(x), xh, rs, K,
+                     redo, (N + 31) / 32);
   KQ_HIP_CHECK(hipGetLastError());
   // tile heights by whole rounds of one workgroup per CU, as for the other tall-tile kernels
   const int nt256 = (N + 255) / 256, mt256 = (M + 255) / 256, mt128 = (M + 127) / 128;
-  if (force) return launch_f3_tiles<C, DT>(xh, rs, w, y, M, N, K, 0, nt256, force, s);
+  if (force) return launch_f3_tiles<C, DT>(xh, rs, w, y, M, N, K, 0, nt256, force, redo.cols, s);
   const int64_t cus = f3_num_cus();
   auto rounds = [&](int64_t wgs) { return (wgs + cus - 1) / cus; };
   const int64_t c128 = rounds((int64_t)mt128 * nt256) * 119;
@@ -371,10 +391,10 @@ int launch_f3_call(const void* x, const uint8_t* w, void* y, int M, int N, int K
   const int rest = nt256 - tall;
   const int64_t rest256 = rounds((int64_t)mt256 * rest) * 200, rest128 = rounds((int64_t)mt128 * rest) * 119;
   const int64_t c256 = full * 200 + (rest128 < rest256 ? rest128 : rest256);
-  if (c128 < c256) return launch_f3_tiles<C, DT>(xh, rs, w, y, M, N, K, 0, nt256, 128, s);
-  const int rc = launch_f3_tiles<C, DT>(xh, rs, w, y, M, N, K, 0, tall, 256, s);
+  if (c128 < c256) return launch_f3_tiles<C, DT>(xh, rs, w, y, M, N, K, 0, nt256, 128, redo.cols, s);
+  const int rc = launch_f3_tiles<C, DT>(xh, rs, w, y, M, N, K, 0, tall, 256, redo.cols, s);
   if (rc != KQ_OK) return rc;
-  return launch_f3_tiles<C, DT>(xh, rs, w, y, M, N, K, tall, rest, rest128 < rest256 ? 128 : 256, s);
+  return launch_f3_tiles<C, DT>(xh, rs, w, y, M, N, K, tall, rest, rest128 < rest256 ? 128 : 256, redo.cols, s);
 }
 
 }  // namespace
@@ -390,7 +410,7 @@ bool kq_gemm3f_supported(int M, int N, int K, int codec) {
   return kq_tall_fills(M, N, codec);
 }
 
-size_t kq_gemm3f_workspace_bytes(int M, int K) { return (size_t)M * K * 2 + (size_t)M * 4 + 256; }
+size_t kq_gemm3f_workspace_bytes(int M, int N, int K) { return (size_t)M * K * 2 + (size_t)M * 4 + 256 + kq_redo_bytes(M, N); }
 
 void kq_gemm3f_force_tile(int rows) { g_f3_force = rows == 1024 ? 256 : rows == 1025 ? 128 : rows == 64 ? -1 : 0; }
 
@@ -400,9 +420,14 @@ int kq_launch_gemm3f(const void* x, const uint8_t* w, void* y, int M, int N, int
   if ((reinterpret_cast<uintptr_t>(w) & 1) || (reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(ws) & 15))
     return KQ_ERR_UNSUPPORTED;
   const int force = g_f3_force;
-  if (codec == KQ_MXFP4)
-    return dtype == KQ_F16 ? launch_f3_call<KQ_MXFP4, KQ_F16>(x, w, y, M, N, K, ws, force, s)
-                           : launch_f3_call<KQ_MXFP4, KQ_BF16>(x, w, y, M, N, K, ws, force, s);
-  return dtype == KQ_F16 ? launch_f3_call<KQ_NVFP4, KQ_F16>(x, w, y, M, N, K, ws, force, s)
-                         : launch_f3_call<KQ_NVFP4, KQ_BF16>(x, w, y, M, N, K, ws, force, s);
+  const KqRedo redo = kq_tall_redo(ws, M, N, K);
+  auto run = [&]() -> int {
+    if (codec == KQ_MXFP4)
+      return dtype == KQ_F16 ? launch_f3_call<KQ_MXFP4, KQ_F16>(x, w, y, M, N, K, ws, force, redo, s)
+                             : launch_f3_call<KQ_MXFP4, KQ_BF16>(x, w, y, M, N, K, ws, force, redo, s);
+    return dtype == KQ_F16 ? launch_f3_call<KQ_NVFP4, KQ_F16>(x, w, y, M, N, K, ws, force, redo, s)
+                           : launch_f3_call<KQ_NVFP4, KQ_BF16>(x, w, y, M, N, K, ws, force, redo, s);
+  };
+  const int rc = run();
+  return rc != KQ_OK || !redo.rows ? rc : kq_launch_anymma_redo(x, w, y, M, N, K, codec, dtype, redo, s);
 }

@@ -76,18 +76,25 @@ constexpr int i3_lds_bytes() {
 // magnitude lands in [2^14, 2^15); f16 rows pass through).
 template <int DT>
 __global__ __launch_bounds__(256) void i3_prepass_kernel(const uint16_t* __restrict__ x, _Float16* __restrict__ xh,
-                                                         float* __restrict__ rs, int K) {
+                                                         float* __restrict__ rs, int K,
+                                                         KqRedo redo, int ncols) {
   __shared__ float red[4];
+  __shared__ uint32_t range_lds[6];
   const int m = blockIdx.x, tid = threadIdx.x, ngroups = K >> 3;
   const uint16_t* xi = x + (size_t)m * K;
   _Float16* xo = xh + (size_t)m * K;
   float inv = 1.f, scale = 1.f;
+  bool infinite = false;
+  RowRange range;
+  if (redo.cols)
+    for (int i = m * 256 + tid; i < ncols; i += gridDim.x * 256) redo.cols[i] = 0;
   if constexpr (DT == KQ_BF16) {
     float amax = 0.f;
     for (int g = tid; g < ngroups; g += 256) {
       const u32x4 v = *reinterpret_cast<const u32x4*>(xi + 8 * g);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
+        range.take(v[e]);
         amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] << 16)));
         amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] & 0xffff0000u)));
       }
@@ -98,6 +105,7 @@ __global__ __launch_bounds__(256) void i3_prepass_kernel(const uint16_t* __restr
     __syncthreads();
     amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     const uint32_t eb = (__builtin_bit_cast(uint32_t, amax) >> 23) & 0xff;
+    infinite = eb == 0xff;
     if (eb != 0 && eb != 0xff) {
       int e = (int)eb - 127 - 14;
       if (e < -100) e = -100;
@@ -106,6 +114,11 @@ __global__ __launch_bounds__(256) void i3_prepass_kernel(const uint16_t* __restr
     }
   }
   if (tid == 0) rs[m] = scale;
+  if (redo.rows) {
+    bool wide = false;
+    if constexpr (DT == KQ_BF16) wide = range.wide<4>(scale, infinite, xi, K, tid, range_lds);
+    if (tid == 0) redo.rows[m] = wide;
+  }
   for (int g = tid; g < ngroups; g += 256) {
     const u32x4 v = *reinterpret_cast<const u32x4*>(xi + 8 * g);
     if constexpr (DT == KQ_BF16) {
@@ -128,7 +141,7 @@ __global__ __launch_bounds__(64 * I3_WAVES, 1) void iq_gemm3_kernel(const _Float
                                                                    const uint8_t* __restrict__ w,
                                                                    const uint8_t* __restrict__ grids,
                                                                    uint16_t* __restrict__ y, int M, int N, int K,
-                                                                   int mtiles, int nt0) {
+                                                                   int mtiles, int nt0, int* redo_cols) {
   using G = I3Geom<C>;
   constexpr int BPB = G::BPB, DPR = i3_dpr<C>(), DPL = i3_dpl<C>(), STAGE = i3_stage<C>();
   constexpr int NEL = 32 * DPL, NI = (NEL + 63) / 64;  // dwords of a stage, load instructions for them
@@ -355,6 +368,7 @@ __global__ __launch_bounds__(64 * I3_WAVES, 1) void iq_gemm3_kernel(const _Float
 
   // ---- epilogue: back to plain units, undo the per-row activation scale, round once, store
   const int n = n0 + wave * 32 + l32;
+  bool redo = false;
 #pragma unroll
   for (int t = 0; t < MT; t++) {
 #pragma unroll
@@ -362,15 +376,17 @@ __global__ __launch_bounds__(64 * I3_WAVES, 1) void iq_gemm3_kernel(const _Float
       const int m = m0 + t * 32 + 8 * (i >> 2) + 4 * kg + (i & 3);
       if (m < M && n < N) {
         const float v = acc[t][i] * r * rs[m];
+        redo |= !(fabsf(v) < INFINITY);
         y[(size_t)m * N + n] = DT == KQ_F16 ? kq::f2f16(v) : kq::f2bf16(v);
       }
     }
   }
+  if (redo_cols && redo && n < N) redo_cols[n >> 5] = 1;
 }
 
 template <int C, int DT, int MT>
 int launch_i3(const _Float16* xh, const float* rs, const uint8_t* w, const uint8_t* grids, void* y, int M, int N, int K,
-              int nt0, int ntiles, hipStream_t s) {
+              int nt0, int ntiles, int* redo_cols, hipStream_t s) {
   if (ntiles <= 0) return KQ_OK;
   const int mtiles = (M + 32 * MT - 1) / (32 * MT);
   constexpr int lds = i3_lds_bytes<C, MT>();
@@ -378,7 +394,7 @@ int launch_i3(const _Float16* xh, const float* rs, const uint8_t* w, const uint8
   auto kern = iq_gemm3_kernel<C, DT, MT>;
   KQ_SET_MAX_LDS_ONCE((kern), lds);
   hipLaunchKernelGGL(kern, dim3(mtiles * ntiles), dim3(64 * I3_WAVES), lds, s, xh, rs, w, grids, static_cast<uint16_t*>(y), M,
-                     N, K, mtiles, nt0);
+                     N, K, mtiles, nt0, redo_cols);
   KQ_HIP_CHECK(hipGetLastError());
   return KQ_OK;
 }
@@ -393,16 +409,17 @@ int i3_num_cus() {
 static int g_i3_force = 0;  // kq_set_gemm_tile_rows: 1024 / 1025 force one tile height for every column tile, 64 switches the kernel off
 
 template <int C, int DT>
-int launch_i3_call(const void* x, const uint8_t* w, void* y, int M, int N, int K, void* ws, int force, hipStream_t s) {
+int launch_i3_call(const void* x, const uint8_t* w, void* y, int M, int N, int K, void* ws, int force, KqRedo redo, hipStream_t s) {
   const uint8_t* grids = kq_device_grids();
   if (!grids) return KQ_ERR_HIP;
   _Float16* xh = static_cast<_Float16*>(ws);
   float* rs = reinterpret_cast<float*>(xh + (size_t)M * K);
-  hipLaunchKernelGGL((i3_prepass_kernel<DT>), dim3(M), dim3(256), 0, s, static_cast<const uint16_t*>(x), xh, rs, K);
+  hipLaunchKernelGGL((i3_prepass_kernel<DT>), dim3(M), dim3(256), 0, s, static_cast<const uint16_t*>(x), xh, rs, K,
+                     redo, (N + 31) / 32);
   KQ_HIP_CHECK(hipGetLastError());
   auto tiles = [&](int nt0, int ntiles, int rows) {
-    return rows == 128 ? launch_i3<C, DT, 4>(xh, rs, w, grids, y, M, N, K, nt0, ntiles, s)
-                       : launch_i3<C, DT, 8>(xh, rs, w, grids, y, M, N, K, nt0, ntiles, s);
+    return rows == 128 ? launch_i3<C, DT, 4>(xh, rs, w, grids, y, M, N, K, nt0, ntiles, redo.cols, s)
+                       : launch_i3<C, DT, 8>(xh, rs, w, grids, y, M, N, K, nt0, ntiles, redo.cols, s);
   };
   // tile heights by whole rounds of one workgroup per CU, as for the other tall-tile kernels
   const int nt256 = (N + 255) / 256, mt256 = (M + 255) / 256, mt128 = (M + 127) / 128;
@@ -438,7 +455,7 @@ bool kq_gemm3i_supported(int M, int N, int K, int codec) {
   return kq_tall_fills(M, N, codec);
 }
 
-size_t kq_gemm3i_workspace_bytes(int M, int K) { return (size_t)M * K * 2 + (size_t)M * 4 + 256; }
+size_t kq_gemm3i_workspace_bytes(int M, int N, int K) { return (size_t)M * K * 2 + (size_t)M * 4 + 256 + kq_redo_bytes(M, N); }
 
 void kq_gemm3i_force_tile(int rows) { g_i3_force = rows == 1024 ? 256 : rows == 1025 ? 128 : rows == 64 ? -1 : 0; }
 
@@ -448,17 +465,22 @@ int kq_launch_gemm3i(const void* x, const uint8_t* w, void* y, int M, int N, int
   if ((reinterpret_cast<uintptr_t>(w) & 1) || (reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(ws) & 15))
     return KQ_ERR_UNSUPPORTED;
   const int force = g_i3_force;
-#define KQ_I3_CASE(CODEC)                                                                                   \
-  if (codec == CODEC)                                                                                        \
-    return dtype == KQ_F16 ? launch_i3_call<CODEC, KQ_F16>(x, w, y, M, N, K, ws, force, s)                   \
-                           : launch_i3_call<CODEC, KQ_BF16>(x, w, y, M, N, K, ws, force, s);
-  KQ_I3_CASE(KQ_IQ2_XXS)
-  KQ_I3_CASE(KQ_IQ2_XS)
-  KQ_I3_CASE(KQ_IQ2_S)
-  KQ_I3_CASE(KQ_IQ3_XXS)
-  KQ_I3_CASE(KQ_IQ3_S)
-  KQ_I3_CASE(KQ_IQ1_S)
-  KQ_I3_CASE(KQ_IQ1_M)
-#undef KQ_I3_CASE
-  return KQ_ERR_UNSUPPORTED;
+  const KqRedo redo = kq_tall_redo(ws, M, N, K);
+  auto run = [&]() -> int {
+  #define KQ_I3_CASE(CODEC)                                                                                   \
+    if (codec == CODEC)                                                                                        \
+      return dtype == KQ_F16 ? launch_i3_call<CODEC, KQ_F16>(x, w, y, M, N, K, ws, force, redo, s)                   \
+                             : launch_i3_call<CODEC, KQ_BF16>(x, w, y, M, N, K, ws, force, redo, s);
+    KQ_I3_CASE(KQ_IQ2_XXS)
+    KQ_I3_CASE(KQ_IQ2_XS)
+    KQ_I3_CASE(KQ_IQ2_S)
+    KQ_I3_CASE(KQ_IQ3_XXS)
+    KQ_I3_CASE(KQ_IQ3_S)
+    KQ_I3_CASE(KQ_IQ1_S)
+    KQ_I3_CASE(KQ_IQ1_M)
+  #undef KQ_I3_CASE
+    return KQ_ERR_UNSUPPORTED;
+  };
+  const int rc = run();
+  return rc != KQ_OK || !redo.rows ? rc : kq_launch_anymma_redo(x, w, y, M, N, K, codec, dtype, redo, s);
 }

@@ -673,6 +673,12 @@ bool kq_tall_fills(int M, int N, int codec) {
   return two ? 5 * tiles >= 3 * cus : 16 * tiles >= 7 * cus;
 }
 
+KqRedo kq_tall_redo(void* ws, int M, int N, int K) {
+  if (4 * (int64_t)((M + 127) / 128) * ((N + 255) / 256) >= 3 * (int64_t)mid_cus()) return KqRedo{nullptr, nullptr};
+  int* rows = reinterpret_cast<int*>(static_cast<uint8_t*>(ws) + (size_t)M * K * 2 + (size_t)M * 4);
+  return KqRedo{rows, rows + M};
+}
+
 size_t kq_mid_workspace_bytes(int M, int N, int K) {
   const size_t mb = (M + 31) / 32, nsteps = (K + CK_STEP - 1) / CK_STEP;
   const MidPlan p = mid_plan(M, N, K);

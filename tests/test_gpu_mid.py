@@ -141,3 +141,62 @@ def test_mid_rows_of_wide_range(mid, codec):
         got = dev_to_bits(mid.quantized_matmul(xt, wire_to_dev(wire), None, codec))
         err = row_errors(got, O.qmm(xb, wire, codec, True, "bfloat16"))
         assert err <= 2.0**-8, (codec, M, N, K, err)
+
+
+TALL = ["q8_0", "q4_0", "iq4_nl", "q5_0", "q4_1", "q5_1", "mxfp4", "nvfp4", "iq2_xxs", "iq2_xs", "iq2_s", "iq3_xxs", "iq3_s",
+        "iq1_s", "iq1_m"]
+
+
+@pytest.fixture(params=[1024, 1025])
+def tall(request):
+    import ctypes
+    import kq
+    f = kq._load().kq_set_gemm_tile_rows
+    f.argtypes = [ctypes.c_int]
+    f(request.param)
+    yield kq
+    f(0)
+
+
+@pytest.mark.parametrize("codec", TALL)
+def test_tall_tiles_rows_of_wide_range(tall, codec):
+    """Tall-tile calls that fill less than three quarters of the chip: rows beyond f16's range are done again."""
+    M, N, K = 160, 264, 1024
+    wire, xb, xt = wide_rows_case(codec, M, K, N, seed=90)
+    got = dev_to_bits(tall.quantized_matmul(xt, wire_to_dev(wire), None, codec))
+    err = row_errors(got, O.qmm(xb, wire, codec, True, "bfloat16"))
+    assert err <= 2.0**-8, (codec, err)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("codec,scale", [("q8_0", 600), ("iq4_nl", 600), ("q4_0", 9000), ("q5_0", 5000), ("q4_1", 5000),
+                                         ("q5_1", 3000)])
+def test_tall_tiles_weights_beyond_f16(tall, codec, scale, dtype):
+    """Block scales whose products with the codes pass 65504, in two weight rows: those columns are done again."""
+    import numpy as np
+    M, N, K = 130, 264, 512
+    wire = O.synth_wire(codec, N * K // 32, seed=95).reshape(N, K // 32, -1)
+    wire[[37, 263], :, 0:2] = np.array([scale], np.float16).view(np.uint8)
+    wire = wire.reshape(N, -1)
+    xb, xt = make_x((M, K), dtype, seed=96, scale=2.0**-6)
+    got, want = dev_to_bits(tall.quantized_matmul(xt, wire_to_dev(wire), None, codec)), O.qmm(xb, wire, codec, True, dtype)
+    for cols in ([37, 263], [i for i in range(N) if i not in (37, 263)]):
+        assert rel_l2(got[:, cols], want[:, cols], dtype) <= 1e-3, (codec, cols[:2])
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+def test_tall_tiles_fp4_blocks_far_apart(tall, dtype):
+    """mxfp4 blocks of one 64-weight step whose exponents differ by 40, under activations that are zero over the large one; a
+    weight row with empty blocks of the smallest exponent beside it."""
+    M, N, K = 130, 264, 512
+    wire = O.synth_wire("mxfp4", N * K // 32, seed=97).reshape(N, K // 32, 17)
+    wire[5, 0::2, 0], wire[5, 1::2, 0] = 150, 110
+    wire[6, 0::2] = 0
+    xb, xt = make_x((M, K), dtype, seed=98)
+    xt = xt.clone()
+    xt.view(M, K // 32, 32)[:, 0::2] = 0
+    xb = dev_to_bits(xt)
+    wire = wire.reshape(N, -1)
+    got, want = dev_to_bits(tall.quantized_matmul(xt, wire_to_dev(wire), None, "mxfp4")), O.qmm(xb, wire, "mxfp4", True, dtype)
+    for cols in ([5], [6], [i for i in range(N) if i not in (5, 6)]):
+        assert rel_l2(got[:, cols], want[:, cols], dtype) <= 1e-3, cols[:2]
