@@ -118,8 +118,7 @@ class KQuantLinear(_KQuantBase):
         # decode (one row) with a real bias on q8_0: the add is fused into the matvec (reference :122-140)
         if self.bias is not None and self.kquant_type == "q8_0" and x.numel() // x.shape[-1] == 1:
             return kq.quantized_matmul_qmv_bias(x, self.weight, self.scales, self.bias, self.kquant_type)
-        b = self._buffers  # (attribute lookups of buffers go through Module.__getattr__)
-        y = kq.quantized_matmul(x, b["weight"], b["scales"], self.kquant_type)
+        y = kq.quantized_matmul(x, self.weight, self.scales, self.kquant_type)
         if self.bias is not None:
             y = y + self.bias
         return y

@@ -78,3 +78,34 @@ def test_gather_qmm_seg_rejects_bad_inputs():
         kq.expert_tile_map(torch.zeros((0,), dtype=torch.int32), 4)
     with pytest.raises(RuntimeError):  # valid arguments, but no device: there is no CPU path
         kq.gather_qmm_seg(x_ok, w, s, "iq2_xxs", good, cnt)
+
+
+def test_linear_reads_its_weight_as_an_attribute(monkeypatch):
+    """A weight held as a frozen parameter, given by a property of a subclass or by a parametrization reaches the op."""
+    import kq
+    import kq.nn as knn
+    seen = []
+    monkeypatch.setattr(kq, "quantized_matmul", lambda x, w, scales, codec, *a, **k: seen.append((w, scales)) or x)
+    x, w = torch.zeros(2, 256), torch.arange(8 * 144).to(torch.uint8).reshape(8, 144)
+
+    lin = knn.KQuantLinear(256, 8, False, "q4_k")
+    del lin.weight
+    lin.weight = torch.nn.Parameter(w, requires_grad=False)
+    lin(x)
+
+    class Moved(knn.KQuantLinear):
+        weight = property(lambda self: w)
+
+        def _wire_buffers(self, shape, device=None):
+            self.register_buffer("scales", torch.zeros(1, dtype=torch.uint8))
+
+    Moved(256, 8, False, "q4_k")(x)
+
+    class Flip(torch.nn.Module):
+        def forward(self, t):
+            return 255 - t
+
+    lin = knn.KQuantLinear(256, 8, False, "q4_k").load_wire(w)
+    torch.nn.utils.parametrize.register_parametrization(lin, "weight", Flip())
+    lin(x)
+    assert torch.equal(seen[0][0], w) and seen[1][0] is w and torch.equal(seen[2][0], 255 - w)
