@@ -5,8 +5,10 @@ import os
 import re
 import subprocess
 import sys
+import warnings
 
 import pytest
+import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB = os.path.join(ROOT, "mlx-kquant_amd", "lib", "libkq.so")
@@ -74,3 +76,21 @@ def test_python_front_end_refuses_cpu_tensors():
         kq.quantized_matmul(torch.zeros((1, 256), dtype=torch.float16), w, None, "q4_k")
     with pytest.raises(ValueError):
         kq.quantized_matmul(torch.zeros((1, 128), dtype=torch.float16), w, None, "q4_k")
+
+
+@pytest.mark.parametrize("content", [None, b"not a shared library"])
+def test_ops_do_without_the_native_call_path(monkeypatch, tmp_path, content):
+    """_kqhost.so missing or unloadable: one warning, every native function declines, and an op's own checks answer."""
+    import kq
+
+    path = tmp_path / "_kqhost.so"
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(kq, "_HOST_PATH", str(path))
+    monkeypatch.setattr(kq, "_native", kq._Native())
+    with pytest.warns(RuntimeWarning, match="native call path"):
+        with pytest.raises(ValueError, match="uint8"):
+            kq.quantized_matmul(torch.zeros(1, 256), torch.zeros(8, 144), None, "q4_k")
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert all(getattr(kq._native, k)() is None for k in kq._NATIVE_OPS)
