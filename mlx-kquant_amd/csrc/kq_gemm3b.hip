@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256) void b3_prepass_kernel(const uint16_t* __restr
       const u32x4 v = *reinterpret_cast<const u32x4*>(xi + 8 * g);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        range.take(v[e]);
+        if (redo.rows) range.take(v[e]);
         amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] << 16)));
         amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] & 0xffff0000u)));
       }
@@ -354,9 +354,17 @@ __global__ __launch_bounds__(64 * B3_WAVES, 1) void block32_gemm3_kernel(const _
     cur = nxt;
   }
 
+  if (redo_cols) {  // sums that are not finite make a NaN of their products with 0
+    float z = 0.f;
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) z = fmaf(acc[t][i], 0.f, z);
+    const int n = n0 + wave * 32 + l32;
+    if (z != 0.f && n < N) redo_cols[n >> 5] = 1;
+  }
   // ---- epilogue: undo the per-row activation scale, round once, store
   const int n = n0 + wave * 32 + l32;
-  bool redo = false;
 #pragma unroll
   for (int t = 0; t < MT; t++) {
 #pragma unroll
@@ -364,12 +372,10 @@ __global__ __launch_bounds__(64 * B3_WAVES, 1) void block32_gemm3_kernel(const _
       const int m = m0 + t * 32 + 8 * (i >> 2) + 4 * kg + (i & 3);
       if (m < M && n < N) {
         const float v = acc[t][i] * rs[m];
-        redo |= !(fabsf(v) < INFINITY);
         y[(size_t)m * N + n] = DT == KQ_F16 ? kq::f2f16(v) : kq::f2bf16(v);
       }
     }
   }
-  if (redo_cols && redo && n < N) redo_cols[n >> 5] = 1;
 }
 
 template <int C, int DT, int MT>

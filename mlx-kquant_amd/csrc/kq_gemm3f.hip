@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256) void f3_prepass_kernel(const uint16_t* __restr
       const u32x4 v = *reinterpret_cast<const u32x4*>(xi + 8 * g);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        range.take(v[e]);
+        if (redo.rows) range.take(v[e]);
         amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] << 16)));
         amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] & 0xffff0000u)));
       }
@@ -219,20 +219,22 @@ __global__ __launch_bounds__(64 * F3_WAVES, 1) void fp4_gemm3_kernel(const _Floa
       // would overflow, and the blocks that asked for it are far below one ulp of the sums anyway: the column keeps
       // its unit and those blocks go in as what is left of them in the window (f32 accumulation of the decoded
       // weights loses them the same way).  Rare: the sums are read only when some column wants to move down.
-      if (!first && __builtin_amdgcn_ballot_w64(target < uoff_n) != 0) {
-        float amax = 0.f;
+      if (first || __builtin_amdgcn_ballot_w64(target != uoff_n) != 0) {
+        if (!first && __builtin_amdgcn_ballot_w64(target < uoff_n) != 0) {
+          float amax = 0.f;
 #pragma unroll
-        for (int t = 0; t < MT; t++)
+          for (int t = 0; t < MT; t++)
 #pragma unroll
-          for (int i = 0; i < 16; i++) amax = fmaxf(amax, fabsf(acc[t][i]));
-        const int ex = (int)((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xffu);  // biased exponent of the largest sum
-        if (target < uoff_n && ex + (uoff_n - target) > 127 + 90) target = uoff_n;
+            for (int i = 0; i < 16; i++) amax = fmaxf(amax, fabsf(acc[t][i]));
+          const int ex = (int)((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xffu);  // biased exponent of the largest sum
+          if (target < uoff_n && ex + (uoff_n - target) > 127 + 90) target = uoff_n;
+        }
+        // (a block below the window asks for a move, so none is missed here)
+        far |= (e0 - target < 104 && ((rg.q[0] | rg.q[1]) & 0x77777777u)) || (e1 - target < 104 && ((rg.q[2] | rg.q[3]) & 0x77777777u));
       }
       pending = uoff_n - target;  // the sums change unit by 2^pending when this step is entered
       uoff_n = target;
       const int f0 = e0 - target, f1 = e1 - target;  // a block below the window becomes zeros (field <= 0: 2^-127)
-      if (lo - target < 104)
-        far |= (f0 < 104 && ((rg.q[0] | rg.q[1]) & 0x77777777u)) || (f1 < 104 && ((rg.q[2] | rg.q[3]) & 0x77777777u));
       rg.s[0] = (uint32_t)(f0 > 0 ? f0 : 0) << 23;
       rg.s[1] = (uint32_t)(f1 > 0 ? f1 : 0) << 23;
     } else {
@@ -323,9 +325,17 @@ __global__ __launch_bounds__(64 * F3_WAVES, 1) void fp4_gemm3_kernel(const _Floa
     }
   }
 
+  if (redo_cols) {  // sums that are not finite make a NaN of their products with 0
+    float z = MX && far ? NAN : 0.f;
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) z = fmaf(acc[t][i], 0.f, z);
+    const int n = n0 + wave * 32 + l32;
+    if (z != 0.f && n < N) redo_cols[n >> 5] = 1;
+  }
   // ---- epilogue: back to plain units, undo the per-row activation scale, round once, store
   const int n = n0 + wave * 32 + l32;
-  bool redo = MX && far;
 #pragma unroll
   for (int t = 0; t < MT; t++) {
 #pragma unroll
@@ -334,12 +344,10 @@ __global__ __launch_bounds__(64 * F3_WAVES, 1) void fp4_gemm3_kernel(const _Floa
       if (m < M && n < N) {
         float v = acc[t][i] * rs[m];
         if constexpr (MX) v = __builtin_ldexpf(v, uoff);
-        redo |= !(fabsf(v) < INFINITY);
         y[(size_t)m * N + n] = DT == KQ_F16 ? kq::f2f16(v) : kq::f2bf16(v);
       }
     }
   }
-  if (redo_cols && redo && n < N) redo_cols[n >> 5] = 1;
 }
 
 template <int C, int DT, int MT>

@@ -63,8 +63,9 @@ __device__ __forceinline__ uint32_t opaque_sgpr(uint32_t v) {
 // ------------------------------------------------------------------ bf16 rows beyond the range of f16
 // A bf16 row in f16 under its power of two (largest magnitude in [2^14, 2^15)) is exact down to 2^-31 of that magnitude;
 // smaller values lose bits, and from 2^-39 on they are 0.  Where the large values meet zero weights (a mask's value beside
-// ordinary ones) the small ones are the result.  A row is wide if more than one in 4096 of its nonzero values lost bits (a
-// row of fewer nonzero values: any), or if it holds an infinity.
+// ordinary ones) the small ones are the result.  A row is wide if more than one in 4096 of its nonzero values (any in a row of
+// fewer than 1024) lost bits, or if it holds an infinity: normally distributed rows lose one in 10^9, and one such value
+// among a thousand that are kept is no reason for the longer way.
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 struct RowRange {
   u16x2 low = {0xffff, 0xffff};  // smallest nonzero magnitudes (15-bit patterns) less one
@@ -93,7 +94,7 @@ struct RowRange {
       atomicAdd(&lds[NW], lost);
       atomicAdd(&lds[NW + 1], nonzero);
       __syncthreads();
-      infinite |= lds[NW] > lds[NW + 1] >> 12;
+      infinite |= lds[NW] > (lds[NW + 1] + 3072) >> 12;
     }
     return infinite;
   }
