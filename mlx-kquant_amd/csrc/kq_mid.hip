@@ -658,16 +658,16 @@ bool kq_mid_supported(int M, int N, int K, int codec) {
   // an unfilled round costs a whole one).  us here / on tall tiles / on the any-codec kernel, which had these calls:
   // mxfp4 4096 x 14336 256 rows 76 / 235 / 147, 512 rows 161 / 236 / 266, 14336 x 4096 333 rows 111 / 84 / 282; iq3_s
   // 14336 x 4096 192 rows 89 / 87 / 154; q8_0 14336 x 4096 256 rows 101 / 97 / 130, 333 rows 137 / 103 / 210.
-  return M <= KQ_MID_MAX_ROWS && !kq_tall_fills(M, N, codec);
+  // The kernel that would take the call is asked itself: it has conditions on K and M of its own.
+  return M <= KQ_MID_MAX_ROWS && !kq_gemm2_low_supported(M, N, K, codec) && !kq_gemm3b_supported(M, N, K, codec) &&
+         !kq_gemm3f_supported(M, N, K, codec) && !kq_gemm3i_supported(M, N, K, codec);
 }
 
 // Whether the tall-tile GEMM of a codec (128 x 256 tiles, a workgroup per CU) has the tiles to beat the streamed kernel:
-// three fifths of a round for two or three terms per weight, seven sixteenths for one term; a whole round for the 128-row
-// kernel of q2_k / q3_k / iq4_xs.  Above the rows of the streamed kernel the alternative is the any-codec kernel, and a
+// three fifths of a round for two or three terms per weight, seven sixteenths for one term.  Above the rows of the streamed kernel the alternative is the any-codec kernel, and a
 // quarter of a round is enough (4096 x 4096, 768 rows, us: mxfp4 84 against 152, q8_0 101 against 120).
 bool kq_tall_fills(int M, int N, int codec) {
   const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256), cus = mid_cus();
-  if (codec == KQ_Q2_K || codec == KQ_Q3_K || codec == KQ_IQ4_XS) return tiles >= 256;
   if (M > KQ_MID_MAX_ROWS) return 4 * tiles >= cus;
   const bool two = codec == KQ_Q8_0 || codec == KQ_Q4_0 || codec == KQ_IQ4_NL || codec == KQ_Q4_1 || codec == KQ_Q5_0 || codec == KQ_Q5_1;
   return two ? 5 * tiles >= 3 * cus : 16 * tiles >= 7 * cus;

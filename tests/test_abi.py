@@ -94,3 +94,20 @@ def test_ops_do_without_the_native_call_path(monkeypatch, tmp_path, content):
     with warnings.catch_warnings():
         warnings.simplefilter("error")
         assert all(getattr(kq._native, k)() is None for k in kq._NATIVE_OPS)
+
+
+def _workspace(lib, codec, M, N, K):
+    lib.kq_qmm_workspace_size.restype = C.c_size_t
+    return lib.kq_qmm_workspace_size(M, N, K, 1, lib.kq_codec_id(codec.encode()), 2)
+
+
+def _streamed(lib, codec, M, N, K):
+    """Whether a dense call is given the streamed kernel's workspace: 18 KiB per 32 rows and 256 weights of K."""
+    return _workspace(lib, codec, M, N, K) >= -(-M // 32) * -(-K // 256) * 18 * 1024
+
+
+@pytest.mark.parametrize("codec,M,N,K", [("iq4_xs", 140, 33024, 4096), ("q2_k", 255, 128256, 4096), ("q3_k", 129, 32768, 4096),
+                                         ("q8_0", 333, 28672, 4128), ("q4_1", 512, 28672, 4128), ("iq4_nl", 160, 28672, 4128)])
+def test_streamed_kernel_takes_what_the_tall_tiles_cannot(lib, codec, M, N, K):
+    """Calls wide enough for tall tiles, with fewer rows or another K than the codec's tall-tile GEMM accepts."""
+    assert _streamed(lib, codec, M, N, K)

@@ -200,3 +200,12 @@ def test_tall_tiles_fp4_blocks_far_apart(tall, dtype):
     got, want = dev_to_bits(tall.quantized_matmul(xt, wire_to_dev(wire), None, "mxfp4")), O.qmm(xb, wire, "mxfp4", True, dtype)
     for cols in ([5], [6], [i for i in range(N) if i not in (5, 6)]):
         assert rel_l2(got[:, cols], want[:, cols], dtype) <= 1e-3, cols[:2]
+
+
+@pytest.mark.parametrize("codec,M,N,K", [("iq4_xs", 140, 32776, 256), ("q3_k", 129, 32768, 256), ("q8_0", 333, 13320, 288)])
+def test_streamed_where_the_tall_tiles_cannot(kq, codec, M, N, K):
+    """As routed: as many tiles as the tall-tile GEMMs want, but fewer rows or another K than theirs accept."""
+    wire = O.synth_wire(codec, N * K // kq.CODEC_GEOMETRY[codec][3], seed=11).reshape(N, -1)
+    xb, xt = make_x((M, K), "bfloat16", seed=12)
+    got = dev_to_bits(kq.quantized_matmul(xt, wire_to_dev(wire), None, codec))
+    assert rel_l2(got, O.qmm(xb, wire, codec, True, "bfloat16"), "bfloat16") <= 1e-3
