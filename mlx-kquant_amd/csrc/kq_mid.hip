@@ -637,6 +637,11 @@ int launch_mid(const void* x, MidArgs a, uint8_t* xf, float* rs, hipStream_t s) 
 static int g_mid_tile = 0;  // 32: every call the kernel can run; another forced tile: none
 void kq_mid_force_tile(int rows) { g_mid_tile = rows; }
 
+// Codecs that the any-codec kernel decodes fast: one table entry of eight weights per index.
+static bool short_any_decode(int codec) {
+  return codec == KQ_IQ1_S || codec == KQ_IQ1_M || codec == KQ_IQ2_XXS || codec == KQ_IQ2_XS;
+}
+
 bool kq_mid_supported(int M, int N, int K, int codec) {
   if (g_mid_tile != 0 && g_mid_tile != 32) return false;
   if (codec < 0 || codec >= KQ_NUM_CODECS || M <= 8 || N < 8 || K < CK_STEP || K % kq_geom(codec).wpb) return false;
@@ -663,14 +668,22 @@ bool kq_mid_supported(int M, int N, int K, int codec) {
          !kq_gemm3f_supported(M, N, K, codec) && !kq_gemm3i_supported(M, N, K, codec);
 }
 
-// Whether the tall-tile GEMM of a codec (128 x 256 tiles, a workgroup per CU) has the tiles to beat the streamed kernel:
-// three fifths of a round for two or three terms per weight, seven sixteenths for one term.  Above the rows of the streamed kernel the alternative is the any-codec kernel, and a
-// quarter of a round is enough (4096 x 4096, 768 rows, us: mxfp4 84 against 152, q8_0 101 against 120).
+// Whether the tall-tile GEMM of a codec (kq_gemm3b / 3f / 3i.hip: 128 x 256 tiles, a workgroup per CU) has the tiles to beat
+// the streamed kernel: three fifths of a round for two or three terms per weight, seven sixteenths for one term.
+// Above the rows of the streamed kernel the alternative is the any-codec kernel.  Tall tiles against it, by tiles of 256 CUs
+// (640 ... 1400 rows of 1024 ... 8192 weight rows; an unfilled round costs a whole one): mxfp4 48 tiles 1.00, 60 0.88, nvfp4
+// 40 0.81; q8_0 / q5_0 60 1.25, 64 1.29, 72 0.91, 80 0.95 ... 1.01, q4_0 / iq4_nl 64 1.13 ... 1.19, 72 0.80; iq2_s / iq3_s /
+// iq3_xxs 64 1.02 ... 1.12, 72 0.84 ... 0.92; iq1_s / iq1_m / iq2_xs / iq2_xxs, whose any-codec decode is short, 64 1.31 ... 1.36,
+// 72 1.02 ... 1.08, 80 0.88 ... 0.96; q4_1 / q5_1 with their third term 96 0.91 ... 1.10, 128 1.06 ... 1.19, 132 0.90, 140 0.63.
 bool kq_tall_fills(int M, int N, int codec) {
   const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256), cus = mid_cus();
-  if (M > KQ_MID_MAX_ROWS) return 4 * tiles >= cus;
-  const bool two = codec == KQ_Q8_0 || codec == KQ_Q4_0 || codec == KQ_IQ4_NL || codec == KQ_Q4_1 || codec == KQ_Q5_0 || codec == KQ_Q5_1;
-  return two ? 5 * tiles >= 3 * cus : 16 * tiles >= 7 * cus;
+  const bool three = codec == KQ_Q4_1 || codec == KQ_Q5_1;
+  if (M > KQ_MID_MAX_ROWS) {
+    const bool fp4 = codec == KQ_MXFP4 || codec == KQ_NVFP4;
+    return three ? 2 * tiles > cus : 32 * tiles >= (fp4 ? 8 : short_any_decode(codec) ? 10 : 9) * cus;
+  }
+  const bool two = codec == KQ_Q8_0 || codec == KQ_Q4_0 || codec == KQ_IQ4_NL || codec == KQ_Q5_0;
+  return two || three ? 5 * tiles >= 3 * cus : 16 * tiles >= 7 * cus;
 }
 
 KqRedo kq_tall_redo(void* ws, int M, int N, int K) {

@@ -111,3 +111,12 @@ def _streamed(lib, codec, M, N, K):
 def test_streamed_kernel_takes_what_the_tall_tiles_cannot(lib, codec, M, N, K):
     """Calls wide enough for tall tiles, with fewer rows or another K than the codec's tall-tile GEMM accepts."""
     assert _streamed(lib, codec, M, N, K)
+
+
+@pytest.mark.parametrize("codec,M,N", [("q8_0", 1024, 2048), ("q4_0", 1024, 2048), ("iq3_s", 1024, 2048), ("iq2_xxs", 768, 2880),
+                                       ("q4_1", 1024, 4096), ("q5_1", 640, 4096)])
+def test_any_codec_kernel_keeps_calls_of_few_tall_tiles(lib, codec, M, N):
+    """Beyond the streamed kernel's rows, K long enough for the f16 activations of the tall tiles to be the larger workspace:
+    the any-codec kernel's is a multiple of the output (partial sums)."""
+    assert _workspace(lib, codec, M, N, 65536) % (4 * M * N) == 0
+    assert _workspace(lib, codec, M, 3 * N, 65536) > 2 * M * 65536
