@@ -658,6 +658,21 @@ bool kq_mid_supported(int M, int N, int K, int codec) {
   // against 56 / 84).
   const bool tile_gemm = codec == KQ_Q4_K || codec == KQ_Q5_K || codec == KQ_Q6_K;
   if (tile_gemm) return M <= 32 || (M <= 64 && (int64_t)N * K <= (int64_t)64 << 20) || (M <= 192 && N <= 4096);
+  // Against the any-codec kernel's 128-row tiles with its short decode for these codecs: a weight decoded once per 128 rows
+  // instead of once per 32 wins where its last tile is (nearly) full and it has the tiles to cut K into whole rounds.  Here /
+  // there: iq2_xs 128 rows 8192 x 8192 68 / 61, 14336 x 4096 64 / 60, 256 rows 4096 x 14336 114 / 96, 8192 x 4096 76 / 62, 400 rows
+  // 4096 x 4096 70 / 59, 512 80 / 62; but 160 rows 8192 x 8192 82 / 98 and 1024 x 4096, 256 rows, 16 / 22.  The others at 512 rows of 4096 x 4096:
+  // iq1_m 74 / 63, iq1_s 66 / 60, iq2_xxs 71 / 65, but 2880 x 2816 (92 tiles, no whole rounds) 0.92 ... 0.85 of it, as at 256 rows of
+  // 4096 x 4096.
+  if (short_any_decode(codec)) {
+    const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
+    const int blocks = (M + 31) / 32, full = (M + 127) / 128 * 4;
+    if (4 * tiles >= mid_cus()) {
+      const bool whole = 2 * mid_cus() % tiles == 0;
+      if (codec == KQ_IQ2_XS && M > 96 && (8 * blocks >= 7 * full || (whole && 5 * blocks >= 4 * full))) return false;
+      if (M > 384 && blocks == full && whole) return false;
+    }
+  }
   if (M <= 128) return true;
   // 129 ... 512 rows: until the codec's tall tiles fill enough of the chip (one workgroup per CU and no K split there, so
   // an unfilled round costs a whole one).  us here / on tall tiles / on the any-codec kernel, which had these calls:

@@ -120,3 +120,13 @@ def test_any_codec_kernel_keeps_calls_of_few_tall_tiles(lib, codec, M, N):
     the any-codec kernel's is a multiple of the output (partial sums)."""
     assert _workspace(lib, codec, M, N, 65536) % (4 * M * N) == 0
     assert _workspace(lib, codec, M, 3 * N, 65536) > 2 * M * 65536
+
+
+@pytest.mark.parametrize("codec,M,N,streamed", [("iq2_xs", 256, 4096, False),
+                                                ("iq2_xs", 160, 8192, True), ("iq2_xs", 256, 1024, True),
+                                                ("iq1_m", 512, 4096, False), ("iq1_s", 512, 2880, True), ("iq2_s", 512, 4096, True)])
+def test_any_codec_kernel_keeps_full_tiles_of_short_decode(lib, codec, M, N, streamed):
+    if streamed:
+        assert _streamed(lib, codec, M, N, 65536)
+    else:
+        assert _workspace(lib, codec, M, N, 65536) % (4 * M * N) == 0
