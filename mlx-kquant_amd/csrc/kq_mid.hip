@@ -443,23 +443,20 @@ __global__ __launch_bounds__(64 * MID_WAVES, 1) void mid_kernel(MidArgs a) {
     const int row0 = tile * rpt, nrows = N - row0 < rpt ? N - row0 : rpt;
     const uint8_t* base = a.w + (size_t)row0 * row_bytes + (size_t)p.st * G::BYTES;
     const uint32_t l0 = slot_lds + slot * SLOT;
+    // The row that ends the matrix inside this step: nothing past its last byte is read (the rows before it read on into the
+    // next one, as everywhere), and what would lie there is not used.  Its last, partial piece is the 16 bytes up to the end,
+    // shifted.
     const bool ragged_end = (K & (CK_STEP - 1)) != 0 && p.st == nsteps - 1 && row0 + nrows == N;
-    if (!ragged_end) {
-      StaticFor<G::LOADS>::run([&](auto tc) {
-        constexpr int T = decltype(tc)::value;
-        if (64 * T + lane < nrows * G::LP) dma16(base, voff[T], l0 + 1024 * T);
-      });
-    } else {
-      // the matrix ends inside this step: nothing past its last byte is read
-      const int valid = (K - CK_STEP * p.st) / G::WPB * G::BPB;  // bytes of the step that exist in a row
-      uint8_t* dst = ring + wave * 2 * SLOT + slot * SLOT;
-      for (int i = lane; i < nrows * G::LP; i += 64) {
-        const int r = i / G::LP, pc = i - r * G::LP;
-        const int off = 16 * pc < G::BYTES - 16 ? 16 * pc : G::BYTES - 16;
-        u32x4 v = {0, 0, 0, 0};
-        for (int t = 0; t < 16; t++)
-          if (off + t < valid) v[t >> 2] |= (uint32_t)base[(size_t)r * row_bytes + off + t] << (8 * (t & 3));
-        *reinterpret_cast<u32x4*>(dst + 16 * i) = v;
+    const int valid = ragged_end ? (K - CK_STEP * p.st) / G::WPB * G::BPB : 0;  // bytes of the step in that row, 17 or more
+    const int npieces = ragged_end ? (nrows - 1) * G::LP + valid / 16 : nrows * G::LP;
+    StaticFor<G::LOADS>::run([&](auto tc) {
+      constexpr int T = decltype(tc)::value;
+      if (64 * T + lane < npieces) dma16(base, voff[T], l0 + 1024 * T);
+    });
+    if (__builtin_expect(valid % 16, 0)) {
+      if (lane == 0) {
+        const u32x4 end = *reinterpret_cast<const u32x4_a1*>(base + (size_t)(nrows - 1) * row_bytes + valid - 16);
+        *reinterpret_cast<u32x4*>(ring + wave * 2 * SLOT + slot * SLOT + 16 * npieces) = shr_bytes(end, 16 - valid % 16);
       }
       mid_wave_sync();
     }
