@@ -121,7 +121,7 @@ int kq_dequantize(const void* w_dev, void* out_dev, uint64_t num_weights, int co
 size_t kq_qmm_workspace_size(int M, int N, int K, int transpose, int codec, int dtype) {
   (void)dtype;
   if (!codec_ok(codec)) return 0;
-  if (!transpose) return kq_nt_workspace_bytes(M, N, K);  // optional: partial sums of a K range cut over the grid
+  if (!transpose) return kq_nt_workspace_bytes(M, N, K, codec);  // optional: partial sums of a K range cut over the grid
   const size_t mid = kq_mid_supported(M, N, K, codec) ? kq_mid_workspace_bytes(M, N, K) : 0;
   if (kq_gemm_supported(M, N, K, codec)) return std::max(mid, kq_gemm_workspace_bytes(M, N, K));
   // split-K partial sums (optional) of whichever skinny kernel takes the call

@@ -713,16 +713,11 @@ __global__ __launch_bounds__(256) void nt_reduce_kernel(const float* __restrict_
   reinterpret_cast<uint4*>(y)[i] = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// Calls of the 256-row kernel: 512 rows and more of aligned activations, K long enough for its pipeline.  (q4_k 4096 x 4096
-// 512 rows, us: 66 here in two ranges' worth of partial sums, 64 on the 128-row tiles; 8192 x 8192 512 rows 192 against 200,
-// q8_0 192 against 227; below, its last row tile is mostly padding.)
-bool nt_tall(int M, int K) { return M >= 512 && K >= 512 && !(K & 7); }
-
 // K ranges of a dense call.  256-row tiles: one workgroup per CU.  Otherwise enough workgroups for two per CU (8192 x 8192,
 // 500 rows, 256 tiles in two ranges: q8_0 227 us, uncut 410), at least eight steps each.
-int nt_ksplit(int M, int N, int K) {
+int nt_ranges(int M, int N, int K, bool tall) {
   const int cols = (N + NT_COLS - 1) / NT_COLS;
-  if (nt_tall(M, K)) {
+  if (tall) {
     const int64_t tiles = (int64_t)cols * ((M + 64 * TALL_RG - 1) / (64 * TALL_RG));
     const int steps = (K + TALL_K - 1) / TALL_K;
     const int64_t s = std::min<int64_t>(256 / tiles, steps / 4);
@@ -736,6 +731,31 @@ int nt_ksplit(int M, int N, int K) {
   if (s > steps / 8) s = steps / 8;
   if (s > 32) s = 32;
   return s < 2 ? 1 : s;
+}
+
+// Calls of the 256-row kernel: 512 rows and more of aligned activations, K long enough for its pipeline, and not more than
+// 5 % (10 %) over the 128-row kernel by the work of their busiest CU, in 64-row steps of K.  256-row tiles run one per CU, so an
+// unfilled round costs a whole one, and two steps more to fill the pipeline; of the 128-row tiles two run per CU, each half a
+// step per 32 rows, and a last round evens out but for a quarter.  Measured / by this, 256-row over 128-row kernel, q4_k:
+// 600 rows 4096 x 4096 (reduction x outputs) 1.27 / 1.41, 4096 x 14336 1.39 / 1.51, 1024 rows 4096 x 4096 1.01 / 1.05, 2048 x 6144
+// 1.14 / 1.21, 1400 rows 4096 x 4096 1.26 / 1.25, 8192 x 8192 1.42 / 1.25, 1800 rows 4096 x 4096 0.91 / 0.96, 2048 rows 4096 x 14336
+// 1.20 / 1.17.  q6_k, q8_0, q5_0, iq4_xs and mxfp4 lie a tenth below that.  Never for the codebook codecs, whose table reads
+// from eight waves decoding together make the 256-row kernel 1.3 - 1.5 times the other (1.1 where it is best).
+// cut: K may be cut over the grid; entries: 1 for a dense call.
+constexpr bool nt_codebook(int codec) {
+  return codec == KQ_IQ1_S || codec == KQ_IQ1_M || codec == KQ_IQ2_XXS || codec == KQ_IQ2_XS || codec == KQ_IQ2_S ||
+         codec == KQ_IQ3_XXS || codec == KQ_IQ3_S;
+}
+bool nt_tall(int codec, int M, int N, int K, bool cut, int entries) {
+  if (M < 512 || K < 512 || (K & 7) || nt_codebook(codec)) return false;
+  const int64_t cols = (int64_t)((N + NT_COLS - 1) / NT_COLS) * entries;
+  const int st = cut ? nt_ranges(M, N, K, true) : 1, sw = cut ? nt_ranges(M, N, K, false) : 1;
+  const int64_t tall_wgs = cols * ((M + 64 * TALL_RG - 1) / (64 * TALL_RG)) * st;
+  const double rounds = (double)(cols * ((M + 127) / 128) * sw) / 512, steps = (double)K / TALL_K;
+  const double tall = (double)((tall_wgs + 255) / 256) * (steps / st + 2);
+  const double wide = (rounds <= 1 ? 1 : rounds + 0.25) * (steps / sw + 0.5);
+  const bool light = codec == KQ_Q6_K || codec == KQ_Q8_0 || codec == KQ_Q5_0 || codec == KQ_IQ4_XS || codec == KQ_MXFP4;
+  return tall <= (light ? 1.10 : 1.05) * wide;
 }
 
 // Entries of one expert share tiles: two or more fit a tile, an expert comes twice on average, and the list is short enough
@@ -773,8 +793,9 @@ struct NtRun {
   }
   template <int DT>
   static void many_rows(const NtArgs& a, int B, const uint8_t* grids, hipStream_t s) {
-    if (a.tall) go_tall<DT>(a, B, grids, s);
-    else if (a.x_vec) go_shared<DT, true>(a, B, grids, s);
+    if constexpr (!nt_codebook(C))
+      if (a.tall) return go_tall<DT>(a, B, grids, s);
+    if (a.x_vec) go_shared<DT, true>(a, B, grids, s);
     else go_shared<DT, false>(a, B, grids, s);
   }
   static int run(const NtArgs& a, int B, int dt, const uint8_t* grids, hipStream_t s) {
@@ -812,9 +833,9 @@ int nt_dispatch(int codec, const A&... a) {
 }  // namespace
 
 // f32 partial sums of a dense call whose K range is cut (0: the call runs uncut)
-size_t kq_nt_workspace_bytes(int M, int N, int K) {
+size_t kq_nt_workspace_bytes(int M, int N, int K, int codec) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  const int s = nt_ksplit(M, N, K);
+  const int s = nt_ranges(M, N, K, nt_tall(codec, M, N, K, true, 1));
   return s > 1 ? (size_t)s * M * N * 4 : 0;
 }
 
@@ -831,16 +852,23 @@ int kq_launch_nt_mfma(const void* x, const uint8_t* w, const uint32_t* lhs, cons
   if (!grids) return KQ_ERR_HIP;
   NtArgs a{x, w, out, lhs, rhs, M, N, K, E, x_batch_stride, w_expert_stride, 0, 1, 0, nullptr, false};
   a.x_vec = !(K & 7) && !(reinterpret_cast<uintptr_t>(x) & 15) && !(x_batch_stride & 7);
-  a.tall = a.x_vec && nt_tall(M, K);
+  // K is cut into the ranges that kq_nt_workspace_bytes was asked for, into what fits where unaligned activations turn the call
+  // to the 128-row kernel, or not at all
+  bool cut = !rhs && B == 1 && ws && !(reinterpret_cast<uintptr_t>(ws) & 15);
+  a.tall = a.x_vec && nt_tall(codec, M, N, K, cut, B);
+  int sp = cut ? nt_ranges(M, N, K, a.tall) : 1;
+  const size_t fit = ws_bytes / ((size_t)M * N * 4);
+  if ((size_t)sp > fit && sp > 1) {
+    cut = fit >= 2 && !a.tall && !a.x_vec;
+    sp = cut ? (int)fit : 1;
+    a.tall = !cut && a.x_vec && nt_tall(codec, M, N, K, false, B);
+  }
   const int kstep = a.tall ? TALL_K : NT_KSTEP, steps = (K + kstep - 1) / kstep;
   a.steps_per_split = steps;
-  if (!rhs && B == 1 && ws && !(reinterpret_cast<uintptr_t>(ws) & 15)) {
-    const int sp = nt_ksplit(M, N, K);
-    if (sp > 1 && ws_bytes >= (size_t)sp * M * N * 4) {
-      a.steps_per_split = (steps + sp - 1) / sp;
-      a.ksplit = (steps + a.steps_per_split - 1) / a.steps_per_split;
-      a.part = static_cast<float*>(ws);
-    }
+  if (cut && sp > 1) {
+    a.steps_per_split = (steps + sp - 1) / sp;
+    a.ksplit = (steps + a.steps_per_split - 1) / a.steps_per_split;
+    a.part = static_cast<float*>(ws);
   }
   return nt_dispatch<NtRun>(codec, a, B, dtype, grids, s);
 }

@@ -130,3 +130,16 @@ def test_any_codec_kernel_keeps_full_tiles_of_short_decode(lib, codec, M, N, str
         assert _streamed(lib, codec, M, N, 65536)
     else:
         assert _workspace(lib, codec, M, N, 65536) % (4 * M * N) == 0
+
+
+@pytest.mark.parametrize("codec,M,N,K,ranges", [
+    ("q8_0", 600, 4096, 4096, 4),      # three row tiles of 256: 192 workgroups in two ranges, against 640 of 128 rows in four
+    ("q6_k", 640, 4096, 14336, 4),
+    ("q8_0", 1024, 4096, 4096, 2),     # (either kernel)
+    ("q4_k", 512, 768, 16384, 21),     # 256-row tiles: 12 in 21 ranges
+    ("iq2_xs", 512, 768, 16384, 22),   # 128-row tiles for the codebook codecs: 24 in 22
+])
+def test_transposed_product_takes_256_row_tiles_where_they_fill(lib, codec, M, N, K, ranges):
+    """The route of y = x W as its workspace shows it: f32 partial sums of so many K ranges."""
+    lib.kq_qmm_workspace_size.restype = C.c_size_t
+    assert lib.kq_qmm_workspace_size(M, N, K, 0, lib.kq_codec_id(codec.encode()), 2) == ranges * M * N * 4
