@@ -130,6 +130,10 @@ void kq_set_gemm_tile_rows(int rows);
  * 5 = same as 0.  Process-wide, not thread-safe. */
 void kq_set_skinny_variant(int variant);
 
+/* Query without a counterpart in the reference: pairs per segment (32 or 64) that the grouped K-quant MoE kernel cuts a
+ * call of T tokens with R experts each into, 0 if it does not take the call.  glu: the fused gate / up op. */
+int kq_moe_segment_rows(int T, int R, int E, int N, int K, int glu, int codec);
+
 /* out[b] = x[lhs[b]] . W[rhs[b]]^T for b < B; x batches are [M,K] matrices
  * `x_batch_stride` elements apart, experts are [N, bytes_per_row] wire matrices
  * `w_expert_stride_bytes` apart (64-bit, so strided / >2 GiB stacks work); out is

@@ -11,6 +11,7 @@
 // rows (converted to f16 by the activation prepass) are fetched one step ahead with coalesced
 // 16-byte loads and parked in LDS.
 #include <algorithm>
+#include <cmath>
 
 #include "kq_epilogue.h"
 #include "kq_mma.h"
@@ -245,6 +246,7 @@ struct MoeArgs {
   const Segment* segs;
   const int* nseg;
   int N, K, x_div, act;
+  int seg_rows;         // pairs per segment at most: 32 or 64
   int64_t w_expert_stride;
   float limit;
   KqOutMap om;
@@ -257,15 +259,15 @@ __global__ __launch_bounds__(MOE_THREADS, MT == 1 ? 3 : 2) void moe_grouped_kern
   using G = Wire<C>;
   constexpr int SEG = 32 * MT;
   constexpr int WPT = (SLAB * G::PP + MOE_THREADS - 1) / MOE_THREADS;  // wire pieces per thread per step
-  constexpr int APT = SEG * 32 / MOE_THREADS;                         // activation pieces per thread per step (4)
+  constexpr int APT = SEG * 32 / MOE_THREADS;                          // activation pieces per thread per step
   constexpr int NCOLS = GLU ? SLAB / 2 : SLAB;                          // output columns per workgroup
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  // two stages of: activations [32][A_STRIDE] | wire [128][LBPB] | X halves [32][32] | side-channel d [128]
+  // MOE_STAGES of: activations [SEG][A_STRIDE] | wire [128][LBPB] | X halves [SEG][32] | side-channel d [128]
   constexpr int B_OFF = SEG * A_STRIDE, H_OFF = B_OFF + SLAB * G::LBPB, D_OFF = H_OFF + SEG * 32;
   constexpr int STAGE = D_OFF + SLAB * 2;
   static_assert(STAGE % 16 == 0, "stages keep 16-byte alignment");
-  int* pair_lds = reinterpret_cast<int*>(smem + MOE_STAGES * STAGE);  // [32] output row of each segment slot, -1 = none
-  float* rs_lds = reinterpret_cast<float*>(pair_lds + SEG);         // [32]
+  int* pair_lds = reinterpret_cast<int*>(smem + MOE_STAGES * STAGE);  // [SEG] output row of each segment slot, -1 = none
+  float* rs_lds = reinterpret_cast<float*>(pair_lds + SEG);           // [SEG]
 
   // Workgroups go to the 8 XCDs round-robin in launch order.  Launch position L = 8 j + c runs slab j % tiles of
   // segment 8 (j / tiles) + c: all slabs of a segment sit on one XCD, back to back, so the segment's activation
@@ -464,18 +466,41 @@ __global__ __launch_bounds__(MOE_THREADS, MT == 1 ? 3 : 2) void moe_grouped_kern
   }
 }
 
-// Pairs per segment of a call.  64 halve the decode of an expert's weights but leave two workgroups per CU: taken from 32
-// pairs per expert on average where the CUs stay filled (router + GLU + down + mix, us, down on 32 / 64: q4_k 128 experts
-// of 2048 <-> 768 top 8, 700 tokens 250 / 229, 1000 tokens 320 / 292, 384 tokens, 24 pairs per expert, 165 / 169; 8 experts
-// of 2048 <-> 4096 top 2, 400 tokens 147 / 134, 200 tokens, 128 workgroups, 90 / 100).  The fused op gains less, and
-// nothing where the average is about the segment itself (half of the experts then leave a short second one): 37 pairs per
-// expert 91 / 87, 44 250 / 239, 62 320 / 326, 100 147 / 138.
-int moe_seg_rows(int P, int E, int N, bool glu) {
-  const int ncols = glu ? SLAB / 2 : SLAB;
-  const int64_t wgs = (int64_t)std::max(E, P / 64) * ((N + ncols - 1) / ncols);
-  if (wgs < 256 || P < 32 * (int64_t)E) return 32;
-  if (glu && (P < 36 * (int64_t)E || (P > 56 * (int64_t)E && P < 96 * (int64_t)E))) return 32;
-  return 64;
+// Segments of `seg` pairs that an expert makes on average when every token picks R of E experts evenly, `mean` pairs for each:
+// the sum over k of the chance of more than k seg pairs (normal approximation of the binomial count).
+double moe_mean_segments(double mean, int R, int E, int seg) {
+  const double sd = std::sqrt(mean * (1.0 - (double)std::min(R, E) / E)) + 1e-9, top = mean + 6 * sd;
+  int k = (int)std::max(0.0, (mean - 6 * sd) / seg);
+  double n = k;
+  for (; k * seg < top + 1; k++) n += 0.5 * std::erfc((k * seg + 0.5 - mean) / (sd * 1.4142135623730951));
+  return n;
+}
+// Rounds of workgroups, ntiles to a segment, over the chip's slots: the second one costs nearly a whole one however short
+// (if there is one: less than a segment beyond the first is the chance of one), later ones even out.
+double moe_rounds(double wgs, int slots, int ntiles) {
+  const double x = wgs / slots, c = std::ceil(x);
+  return x <= 1 ? 1 : x + (c == 2 ? 0.75 : 0.25) * (c - x) * std::min(1.0, (wgs - (c - 1) * slots) / ntiles);
+}
+
+// Pairs per segment of a call.  64 halve the decode of an expert's weights but leave two workgroups per CU where 32 leave
+// three.  Plain op: from 32 pairs per expert where the CUs stay filled (down product with the mix, us on 32 / 64: q4_k 128
+// experts of 2048 <-> 768 top 8, 700 tokens 250 / 229, 1000 tokens 320 / 292, 384 tokens, 24 pairs per expert, 165 / 169; 8 experts
+// of 2048 <-> 4096 top 2, 400 tokens 147 / 134, 200 tokens, 128 workgroups, 90 / 100).
+// The fused op gains less, and how much depends on the segments that the routing leaves (62 pairs per expert make 1.4 of 64 or
+// 2.4 of 32; 44 make 1.0 or 2.0): it takes 64 where their rounds, times what a workgroup of the 64-pair form takes longer per
+// round (the lighter the decode and the shorter K the more), come out below those of 32.  Measured on 64 over 32, q4_k: 128
+// experts of 2048 -> 768, 34 pairs per expert 1.01, 44 0.91, 76 1.06, 112 0.92; 32 of 1024 -> 2048 44 0.99, 70 1.25, 200 1.03; 8 of
+// 2048 -> 4096 44 0.90, 64 1.17, 100 0.94; q5_k / q6_k 128 of 2048 -> 768 28 1.08 / 1.11, 44 0.87 / 0.85, 70 0.97 / 0.92.  Over 606 calls on
+// eight stacks that the constants were not taken from, the choice is 1.4 % behind the better form (always 32: 10 %).
+int moe_seg_rows(int P, int R, int E, int N, int K, bool glu, int codec) {
+  const int ncols = glu ? SLAB / 2 : SLAB, ntiles = (N + ncols - 1) / ncols;
+  if ((int64_t)std::max(E, P / 64) * ntiles < 256 || P < (glu ? 28 : 32) * (int64_t)E) return 32;
+  const double mean = (double)P / E;
+  if (!glu || mean > 1024) return 64;
+  const double wgs64 = moe_mean_segments(mean, R, E, 64) * E * ntiles, wgs32 = moe_mean_segments(mean, R, E, 32) * E * ntiles;
+  if (wgs32 < 1.2 * wgs64) return 32;  // hardly an expert with a second segment to save
+  const double per_round = (codec == KQ_Q4_K ? 1.01 : codec == KQ_Q5_K ? 0.91 : 0.90) * std::sqrt(1 + 512.0 / K);
+  return per_round * moe_rounds(wgs64, 2 * 256, ntiles) <= 0.98 * moe_rounds(wgs32, 3 * 256, ntiles) ? 64 : 32;
 }
 
 struct MoeWorkspace {
@@ -530,7 +555,7 @@ int launch_grouped_mt(const MoeArgs& a, int P, int E, hipStream_t s) {
 
 template <int C, int DT, bool GLU>
 int launch_grouped(const MoeArgs& a, int P, int E, hipStream_t s) {
-  return moe_seg_rows(P, E, a.N, GLU) == 64 ? launch_grouped_mt<C, DT, GLU, 2>(a, P, E, s) : launch_grouped_mt<C, DT, GLU, 1>(a, P, E, s);
+  return a.seg_rows == 64 ? launch_grouped_mt<C, DT, GLU, 2>(a, P, E, s) : launch_grouped_mt<C, DT, GLU, 1>(a, P, E, s);
 }
 
 template <bool GLU>
@@ -622,6 +647,10 @@ bool kq_moe_grouped_supported(int P, int E, int N, int K, int codec) {
          (K & 255) == 0 && N > 0 && (int64_t)E + P / SEG_M < 65535;
 }
 
+extern "C" int kq_moe_segment_rows(int T, int R, int E, int N, int K, int glu, int codec) {
+  return kq_moe_grouped_supported(T * R, E, N, K, codec) ? moe_seg_rows(T * R, R, E, N, K, glu != 0, codec) : 0;
+}
+
 // rows = activation rows the prepass converts: T for the GLU op (x is [T,K]), T*R for the down op.
 size_t kq_moe_grouped_workspace_bytes(int rows, int P, int E, int K) { return carve(nullptr, rows, P, E, K).bytes; }
 
@@ -636,12 +665,13 @@ int kq_launch_moe_grouped(const void* x, const uint8_t* w, const uint8_t* w2, co
       (reinterpret_cast<uintptr_t>(ws) & 255))
     return KQ_ERR_UNSUPPORTED;
   const MoeWorkspace m = carve(ws, rows, P, E, K);
+  const int seg_rows = moe_seg_rows(P, P / std::max(rows, 1), E, N, K, glu, codec);
   if (dtype == KQ_F16)
     hipLaunchKernelGGL(moe_prologue_kernel<KQ_F16>, dim3(rows + 1), dim3(PP_THREADS), 0, s, static_cast<const uint16_t*>(x),
-                       m.xh, m.xhl, m.rs, rows, K, idx, P, E, m.order, m.segs, m.nseg, moe_seg_rows(P, E, N, glu));
+                       m.xh, m.xhl, m.rs, rows, K, idx, P, E, m.order, m.segs, m.nseg, seg_rows);
   else
     hipLaunchKernelGGL(moe_prologue_kernel<KQ_BF16>, dim3(rows + 1), dim3(PP_THREADS), 0, s, static_cast<const uint16_t*>(x),
-                       m.xh, m.xhl, m.rs, rows, K, idx, P, E, m.order, m.segs, m.nseg, moe_seg_rows(P, E, N, glu));
+                       m.xh, m.xhl, m.rs, rows, K, idx, P, E, m.order, m.segs, m.nseg, seg_rows);
   KQ_HIP_CHECK(hipGetLastError());
   MoeArgs a{};
   a.xh = m.xh;
@@ -653,6 +683,7 @@ int kq_launch_moe_grouped(const void* x, const uint8_t* w, const uint8_t* w2, co
   a.order = m.order;
   a.segs = m.segs;
   a.nseg = m.nseg;
+  a.seg_rows = seg_rows;
   a.N = N;
   a.K = K;
   a.x_div = x_div < 1 ? 1 : x_div;

@@ -143,3 +143,17 @@ def test_transposed_product_takes_256_row_tiles_where_they_fill(lib, codec, M, N
     """The route of y = x W as its workspace shows it: f32 partial sums of so many K ranges."""
     lib.kq_qmm_workspace_size.restype = C.c_size_t
     assert lib.kq_qmm_workspace_size(M, N, K, 0, lib.kq_codec_id(codec.encode()), 2) == ranges * M * N * 4
+
+
+def test_fused_moe_segments_follow_the_routing(lib):
+    """64-pair segments of the fused op by the segments that an even routing leaves: at 44 pairs per expert one instead of two,
+    at 64 and 76 about half of the experts a short second one, at 112 again two instead of four; heavier decodes sooner."""
+    def rows(codec, ppe, R=8, E=128, N=768, K=2048):
+        return lib.kq_moe_segment_rows(ppe * E // R, R, E, N, K, 1, lib.kq_codec_id(codec.encode()))
+
+    assert [rows("q4_k", p) for p in (24, 30, 44, 76, 112, 200)] == [32, 32, 64, 32, 64, 64]
+    assert [rows("q6_k", p) for p in (24, 30, 44, 62, 92, 200)] == [32, 32, 64, 64, 64, 64]
+    assert [rows("q4_k", p, R=8, E=8, N=4096) for p in (64, 92, 128)] == [64, 32, 64]  # every expert has every token
+    assert rows("q4_k", 44, E=32, N=2048, K=512) == 32  # short K
+    assert rows("q5_k", 44, R=2, E=2) == 32             # too few workgroups
+    assert lib.kq_moe_segment_rows(125, 8, 8, 768, 2048, 1, lib.kq_codec_id(b"q8_0")) == 0

@@ -97,13 +97,19 @@ def test_gather_qmv_mix_ns(kq, codec, T, S):
         assert bool(((a - b).abs() <= bound).all()), (codec, T, float((a - b).abs().max()))
 
 
+def _segment_rows(kq, codec, T, R, E, N, K, glu):
+    lib = kq._load()
+    return lib.kq_moe_segment_rows(T, R, E, N, K, int(glu), lib.kq_codec_id(codec.encode()))
+
+
 @pytest.mark.parametrize("codec", ["q4_k", "q5_k", "q6_k"])
 @pytest.mark.parametrize("T,S,E,N", [(90, 2, 3, 11008),   # 60 pairs per expert: segments of 33 to 64 pairs, one of a few
-                                     (64, 2, 2, 16384),   # exactly one full segment each; the fused op too
-                                     (310, 7, 9, 136)])   # more pairs than the sort keeps in registers
-def test_grouped_ops_on_64_pair_segments(kq, codec, T, S, E, N):
+                                     (64, 2, 2, 16384),   # exactly one full segment each
+                                     (310, 7, 9, 1104)])  # more pairs than the sort keeps in registers
+def test_down_product_on_64_pair_segments(kq, codec, T, S, E, N):
     K = 256
-    w, w2 = _stack(codec, E, N, K, 71), _stack(codec, E, N, K, 72)
+    assert _segment_rows(kq, codec, T, S, E, N, K, False) == 64
+    w = _stack(codec, E, N, K, 71)
     rng = np.random.default_rng(73)
     idx = rng.permutation(np.arange(T * S) % E).reshape(T, S)
     idx[0, 0] = (idx[0, 0] + 1) % E
@@ -112,11 +118,23 @@ def test_grouped_ops_on_64_pair_segments(kq, codec, T, S, E, N):
     got = kq.gather_qmv_mix_ns_kq(xt, wire_to_dev(w), codec, _idx_dev(idx), torch.from_numpy(scores).cuda())
     want = O.gather_qmv_mix(xb, w, None, codec, None, idx, scores, "bfloat16")
     assert rel_l2(dev_to_bits(got), want, "bfloat16") <= TOL, (codec, T, S)
-    xb, xt = make_x((T, K), "bfloat16", seed=75, scale=0.05)
-    for n in (T, T // 2):
-        got = kq.moe_glu_gather_kq(xt[:n], wire_to_dev(w), wire_to_dev(w2), codec, _idx_dev(idx[:n]))
-        want = O.moe_glu_gather(xb[:n], w, w2, codec, idx[:n], "silu", dtype="bfloat16")
-        assert rel_l2(dev_to_bits(got), want, "bfloat16") <= TOL, (codec, n, S)
+
+
+@pytest.mark.parametrize("codec,act,dtype", [("q4_k", "silu", "bfloat16"), ("q4_k", "gelu", "float16"),
+                                             ("q5_k", "silu", "float16"), ("q6_k", "gelu", "bfloat16")])
+@pytest.mark.parametrize("N", [4096, 4088])
+def test_fused_op_on_64_pair_segments(kq, codec, act, dtype, N):
+    """44 pairs per expert on average: one expert with 100 (a full segment and one of 36), one with 64, one with none, the
+    others below and above 32."""
+    T, R, E, K = 44, 8, 8, 256
+    assert _segment_rows(kq, codec, T, R, E, N, K, True) == 64
+    counts = [100, 64, 0, 63, 65, 33, 26, 1]
+    idx = np.random.default_rng(76).permutation(np.repeat(np.arange(E), counts)).reshape(T, R)
+    w, w2 = _stack(codec, E, N, K, 77), _stack(codec, E, N, K, 78)
+    xb, xt = make_x((T, K), dtype, seed=79, scale=0.05)
+    got = kq.moe_glu_gather_kq(xt, wire_to_dev(w), wire_to_dev(w2), codec, _idx_dev(idx), act)
+    want = O.moe_glu_gather(xb, w, w2, codec, idx, act, dtype=dtype)
+    assert rel_l2(dev_to_bits(got), want, dtype) <= TOL, (codec, act, dtype)
 
 
 @pytest.mark.parametrize("T", [1, 3, 20])
