@@ -21,31 +21,58 @@ def wire(codec, rows, K, seed):
     return wire_to_dev(O.synth_wire(codec, rows * K // O.geometry(codec)[0], seed).reshape(rows, -1))
 
 
-def test_native_ops_give_the_checked_functions_bits(kq):
+class Spy:
+    """The native functions, keeping what each call was answered with."""
+
+    def __init__(self, native):
+        self.native, self.answers = native, []
+
+    def __getattr__(self, name):
+        f = getattr(self.native, name)
+
+        def call(*args):
+            self.answers.append((name, f(*args)))
+            return self.answers[-1][1]
+
+        return call
+
+
+def test_native_ops_take_ordinary_calls_with_the_checked_functions_bits(kq, monkeypatch):
     E, N, K, T, R = 4, 64, 512, 3, 2
     x = make_x((T, K), "bfloat16", 1)[1]
     g, u, d = (wire(c, E * n, k, s).reshape(E, n, -1) for c, n, k, s in (("q4_k", N, K, 2), ("q4_k", N, K, 3), ("q6_k", K, 256, 4)))
-    xs = make_x((T, R, 256), "bfloat16", 5)[1]
+    mg, mu = (wire("mxfp4", E * N, K, s).reshape(E, N, -1) for s in (7, 8))
+    gb, ub = torch.randn(E, N, device="cuda"), torch.randn(E, N, device="cuda")
+    xs, xn = make_x((T, R, 256), "bfloat16", 5)[1], make_x((T, R, K), "float16", 9)[1]
     idx = torch.tensor([[0, 3], [1, 2], [2, 0]], dtype=torch.int32, device="cuda")
     sc = torch.rand(T, R, device="cuda")
+    im = torch.rand(512, device="cuda") + 0.1
     lhs, rhs = (torch.tensor(v, dtype=torch.int32, device="cuda") for v in ([2, 0, 1], [3, 1, 1]))
     calls = {
-        "quantized_matmul": [(x, g[0], None, "q4_k"), (dy := make_x((5, N), "float16", 6)[1], g[1], None, "q4_k", False)],
-        "dequantize": [(g, None, "q4_k"), (d, None, "q6_k", torch.float32)],
-        "gather_qmm": [(x[:, None], g, None, "q4_k", lhs, rhs)],
-        "moe_glu_gather_kq": [(x, g, u, "q4_k", idx, "gelu")],
-        "gather_qmv_kq": [(xs, d, "q6_k", idx)],
+        "quantized_matmul": [(x, g[0], None, "q4_k"), (make_x((5, N), "float16", 6)[1], g[1], None, "q4_k", False)],
+        "dequantize": [(g, None, "q4_k"), (d, None, "q6_k", torch.float32), (g, None, "q4_k", torch.bfloat16)],
+        "gather_qmm": [(x[:, None], g, None, "q4_k", lhs, rhs), (x[:, None, :64].contiguous(), g, None, "q4_k", lhs, rhs, False)],
+        "moe_glu_gather_kq": [(x, g, u, "q4_k", idx, "gelu"), (x, g, u, "q4_k", idx, "silu_limit", 7.0),
+                              (x, mg, mu, "mxfp4", idx, "swiglu_clamp", 7.0, gb, ub, 1.702)],
+        "gather_qmv_kq": [(xs, d, "q6_k", idx), (xn, mg, "mxfp4", idx, gb)],
         "moe_glu_gather_shexp_kq": [(x, g, u, g[1], u[2], "q4_k", idx)],
         "gather_qmv_mix_ns_kq": [(xs, d, "q6_k", idx, sc)],
         "gather_qmv_mix_kq": [(xs, d, d[1], "q6_k", idx[:, :1].contiguous(), sc)],
-        "moe_router_topk": [(torch.randn(T, E + 1, device="cuda"), 2, True)],
-        "quantize": [(torch.randn(3, 512, device="cuda"), "q5_k")],
+        "moe_router_topk": [(torch.randn(T, E + 1, device="cuda"), 2, True),
+                            (torch.randn(T, E, device="cuda"), 2, True, False, sc.new_ones(E), sc.new_zeros(E), "sqrtsoftplus", 2.5)],
+        "quantize": [(torch.randn(3, 512, device="cuda"), "q5_k"), (torch.randn(3, 512, device="cuda").half(), "q2_k", im)],
     }
+    spy = Spy(kq._native)
+    monkeypatch.setattr(kq, "_native", spy)
     for name, variants in calls.items():
         for args in variants:
+            spy.answers.clear()
             got, want = getattr(kq, name)(*args), kq._checked[name](*args)
-            for a, b in zip(*((v if isinstance(v, tuple) else (v,)) for v in (got, want))):
-                assert a.dtype == b.dtype and torch.equal(a, b), name
+            assert len(spy.answers) == 1 and spy.answers[0][1] is not None, name
+            got, want = ((v if isinstance(v, tuple) else (v,)) for v in (got, want))
+            assert len(got) == len(want), name
+            for a, b in zip(got, want):
+                assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), name
 
 
 def test_declined_calls_convert_or_raise(kq):
