@@ -1,4 +1,4 @@
-"""GPU parity of the matmul between the skinny kernels and the tile GEMMs (9 ... 128 activation rows) at the places where
+"""GPU parity of the matmul between the skinny kernels and the tile GEMMs (9 ... 512 activation rows) at the places where
 its tiling can go wrong: one weight row and one step, a ragged last tile, K ending inside a step, several rounds of
 persistent workgroups, steps cut over workgroups (also under graph replay), one to four blocks of activation rows."""
 import pytest
@@ -209,3 +209,29 @@ def test_streamed_where_the_tall_tiles_cannot(kq, codec, M, N, K):
     xb, xt = make_x((M, K), "bfloat16", seed=12)
     got = dev_to_bits(kq.quantized_matmul(xt, wire_to_dev(wire), None, codec))
     assert rel_l2(got, O.qmm(xb, wire, codec, True, "bfloat16"), "bfloat16") <= 1e-3
+
+
+@pytest.mark.parametrize("codec,M,tile", [("q8_0", 40, 32), ("mxfp4", 160, 1025), ("iq3_s", 160, 1024)])
+def test_wide_rows_under_replay(kq, codec, M, tile):
+    """The flags belong to the call's own rows: replays on ordinary and wide rows in turn equal eager calls."""
+    import ctypes
+    f = kq._load().kq_set_gemm_tile_rows
+    f.argtypes = [ctypes.c_int]
+    f(tile)
+    try:
+        wire, _, wide = wide_rows_case(codec, M, 1024, 264, seed=13)
+        w = wire_to_dev(wire)
+        xs = [make_x((M, 1024), "bfloat16", seed=14)[1], wide, make_x((M, 1024), "bfloat16", seed=15)[1], wide.flip(0).contiguous()]
+        want = [kq.quantized_matmul(x, w, None, codec) for x in xs]
+        buf = xs[0].clone()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            out = kq.quantized_matmul(buf, w, None, codec)
+        for r in range(8):
+            buf.copy_(xs[r % 4])
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want[r % 4]), r
+    finally:
+        f(0)
