@@ -91,8 +91,9 @@ int kq_qmm(const void* x_dev, const void* w_dev, void* y_dev, int M, int N, int 
  * q6_k keeps its converted activations there: about 2.2 * M * K bytes) is rejected with KQ_ERR_WORKSPACE; the
  * optional part of kq_qmm_workspace_size (partial sums of a K range cut over the grid) is used when it fits
  * and left out otherwise.  All calls on one GPU share that GPU's buffer: calls that overlap in time on the same
- * GPU (different streams or threads) race; the buffer keeps the last call's contents, and the kernels write
- * every element they later read, so nothing needs clearing between calls.  The first call of a shape on a
+ * GPU (different streams or threads) race; the buffer keeps the last call's contents, and no result
+ * depends on them (padding rows that a call leaves unwritten may be read, into sums that are not stored), so nothing needs
+ * clearing between calls.  The first call of a shape on a
  * device looks the buffer's address up and sets kernel attributes: make one eager call of each shape before
  * capturing it into a HIP graph.
  * No counterpart in the reference. */
@@ -113,7 +114,7 @@ int kq_qmv_bias(const void* x_dev, const void* w_dev, const void* bias_dev, void
  * 1024 = 256 x 256 on eight waves with 256-row wave tiles on one accumulator set (q4_k / q5_k / q6_k) for every
  * column tile, 1025 = the 128 x 256 form of that kernel (q6_k only; other codecs fall back to automatic); for
  * q8_0 / q4_0 / q4_1 / q5_0 / q5_1 / iq4_nl / mxfp4 / nvfp4 and the codebook codecs (iq1 / iq2 / iq3), 1024 / 1025 force the 256- / 128-row form of their tall-tile kernels on any
- * shape of 128 rows or more and 64 keeps them on the any-codec kernel; 32 = the streamed kernel of 9 ... 128 activation
+ * shape of 128 rows or more and 64 keeps them on the any-codec kernel; 32 = the streamed kernel of 9 ... 512 activation
  * rows wherever it can run (every other forced shape switches it off);
  * anything else restores the automatic choice (q4_k / q5_k / q6_k with 256 rows or more: the 256 x 256 kernel on the
  * column tiles that fill whole rounds of one workgroup per CU, a 128 x 256 kernel on the rest; q6_k matrices of
