@@ -1,6 +1,7 @@
 // C ABI of libkq (declared in include/kq.h): argument validation, error reporting, the device copy of the
 // IQ codebooks and routing to the HIP launchers.  Compiled by hipcc as HIP (the codebooks are a __device__ array).
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -81,6 +82,18 @@ const uint8_t* kq_device_grids(void) {
     g_grids[dev] = static_cast<const uint8_t*>(p);
   }
   return g_grids[dev];
+}
+
+int kq_num_cus() {
+  static std::atomic<int> cus[kMaxDevices] = {};  // looked up once per device
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 256;
+  int n = cus[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cus[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
 }
 
 extern "C" {

@@ -136,6 +136,7 @@ int kq_launch_gather_tuned(const void* x, const uint8_t* w, const uint8_t* w2, c
                            const uint32_t* rhs, void* out, int B, int M, int N, int K, int x_div,
                            int64_t x_batch_stride, int64_t w_expert_stride, int glu, int act, float limit, int codec,
                            int dtype, int E, KqOutMap om, hipStream_t s);
+int kq_num_cus();  // CUs of the current device (256 if it cannot be asked)
 // Every codec, 9 ... KQ_MID_MAX_ROWS activation rows: waves stream the weights, one launch behind a prepass that puts the
 // activations into ws (kq_mid_workspace_bytes) in matrix-operand order (kq_mid.hip).
 #define KQ_MID_MAX_ROWS 512

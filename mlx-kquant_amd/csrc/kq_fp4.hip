@@ -26,7 +26,6 @@
 // two m-tiles on the same weight registers).  fp4_glu_tiles_kernel: the waves split the column tiles, a wave reads
 // four consecutive steps of its gate and up tile per load group, one group ahead, and the activation terms of a step
 // are loaded by one wave and shared through LDS (the fused op on one m-tile).
-#include <atomic>
 #include <type_traits>
 
 #include "kq_common.h"
@@ -613,18 +612,6 @@ __global__ __launch_bounds__(64 * NW, 2) void fp4_glu_tiles_kernel(F4Args a) {
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
-int f4_num_cus() {
-  // compute units of the current device, looked up once per device
-  static std::atomic<int> cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cus[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
 int f4_steps(int K) { return ((K >> 5) + 3) / 4; }
 
 }  // namespace
@@ -718,7 +705,7 @@ int kq_launch_fp4_moe(const void* x, const uint8_t* w, const uint8_t* w2, const 
   if (KQ_F4_TILES && glu && !two) {  // the fused op on one m-tile per pass: the waves split the column tiles
     // few pairs: 32-column workgroups of two waves where 64-column groups would leave most CUs one workgroup or none
     // (32 experts of 2880 x 2880: 8 pairs 25.5 -> 23.1 us; 12 pairs 27.6 -> 29.1 and 16 pairs 33.9 -> 36.2 the other way)
-    const bool narrow = (int64_t)4 * P * ((N + 63) / 64) < (int64_t)7 * f4_num_cus();
+    const bool narrow = (int64_t)4 * P * ((N + 63) / 64) < (int64_t)7 * kq_num_cus();
     if (dtype == KQ_F16) { if (narrow) KQ_F4_LAUNCH_TILES(KQ_F16, 2); else KQ_F4_LAUNCH_TILES(KQ_F16, 4); }
     else { if (narrow) KQ_F4_LAUNCH_TILES(KQ_BF16, 2); else KQ_F4_LAUNCH_TILES(KQ_BF16, 4); }
   } else if (glu) {

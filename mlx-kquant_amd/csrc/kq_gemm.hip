@@ -244,19 +244,6 @@ int launch_gemm_mt(const _Float16* xh, const _Float16* xhl, const float* rs, con
 }
 
 
-int gemm_num_cus() {
-  // compute units of the current device, looked up once per device
-  static std::atomic<int> cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cus[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
 template <int C, int DT>
 int launch_gemm(const void* x, const uint8_t* w, void* y, int M, int N, int K, void* ws, size_t ws_bytes, hipStream_t s) {
   const int mpad = ((M + BM - 1) / BM) * BM, nsb = K >> 8;
@@ -285,7 +272,7 @@ int launch_gemm(const void* x, const uint8_t* w, void* y, int M, int N, int K, v
     const int nt256 = (N + 255) / 256;
     if (tile == 1024 && kq_gemm3_supported(M, mpad, N, K, C)) return kq_launch_gemm3(xh, xhl, rs, w, y, M, mpad, N, K, C, DT, 0, nt256, s);
     if (tile == 0 && M >= 256 && kq_gemm3_supported(M, mpad, N, K, C)) {
-      const int mt256 = (M + 255) / 256, cus = gemm_num_cus();
+      const int mt256 = (M + 255) / 256, cus = kq_num_cus();
       const int64_t tiles = (int64_t)mt256 * nt256;
       int tall = (int)((tiles / cus) * cus / mt256);  // column tiles in whole rounds
       if (tall == 0 && 4 * tiles >= 3 * (int64_t)cus) tall = nt256;
@@ -308,7 +295,7 @@ int launch_gemm(const void* x, const uint8_t* w, void* y, int M, int N, int K, v
     // 96 + 16 column tiles = 3 rounds + 1 round of half-height tiles).  `1024` forces the 256-row form for every
     // column tile, `1025` the 128-row form.
     const int nt256 = (N + 255) / 256, mt256 = (M + 255) / 256, mt128 = (M + 127) / 128;
-    const int64_t cus = gemm_num_cus();
+    const int64_t cus = kq_num_cus();
     if ((tile == 1024 || tile == 1025) && kq_gemm3_supported(M, mpad, N, K, C))
       return kq_launch_gemm3(xh, xhl, rs, w, y, M, mpad, N, K, C, DT, 0, nt256, s, tile == 1025 ? 128 : 256);
     if (tile == 0 && M >= 128 && kq_gemm3_supported(M, mpad, N, K, C)) {

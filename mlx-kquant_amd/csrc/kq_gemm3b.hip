@@ -400,13 +400,6 @@ int launch_b3_tiles(const _Float16* xh, const float* rs, const uint8_t* w, void*
                           : launch_b3<C, DT, 8>(xh, rs, w, y, M, N, K, nt0, ntiles, redo_cols, s);
 }
 
-int b3_num_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-  return n;
-}
-
 static int g_b3_force = 0;  // kq_set_gemm_tile_rows: 1024 / 1025 force one tile height for every column tile, 64 switches the kernel off
 
 template <int C, int DT>
@@ -421,7 +414,7 @@ int launch_b3_call(const void* x, const uint8_t* w, void* y, int M, int N, int K
   // tiles that fill whole rounds at 256 rows and the rest at whichever height is cheaper.
   const int nt256 = (N + 255) / 256, mt256 = (M + 255) / 256, mt128 = (M + 127) / 128;
   if (force) return launch_b3_tiles<C, DT>(xh, rs, w, y, M, N, K, 0, nt256, force, redo.cols, s);
-  const int64_t cus = b3_num_cus();
+  const int64_t cus = kq_num_cus();
   auto rounds = [&](int64_t wgs) { return (wgs + cus - 1) / cus; };
   const int64_t c128 = rounds((int64_t)mt128 * nt256) * 119;
   const int64_t full = (int64_t)mt256 * nt256 / cus;

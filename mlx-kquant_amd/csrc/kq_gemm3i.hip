@@ -405,13 +405,6 @@ int launch_i3(const _Float16* xh, const float* rs, const uint8_t* w, const uint8
   return KQ_OK;
 }
 
-int i3_num_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-  return n;
-}
-
 static int g_i3_force = 0;  // kq_set_gemm_tile_rows: 1024 / 1025 force one tile height for every column tile, 64 switches the kernel off
 
 template <int C, int DT>
@@ -430,7 +423,7 @@ int launch_i3_call(const void* x, const uint8_t* w, void* y, int M, int N, int K
   // tile heights by whole rounds of one workgroup per CU, as for the other tall-tile kernels
   const int nt256 = (N + 255) / 256, mt256 = (M + 255) / 256, mt128 = (M + 127) / 128;
   if (force) return tiles(0, nt256, force);
-  const int64_t cus = i3_num_cus();
+  const int64_t cus = kq_num_cus();
   auto rounds = [&](int64_t wgs) { return (wgs + cus - 1) / cus; };
   const int64_t c128 = rounds((int64_t)mt128 * nt256) * 119;
   const int64_t full = (int64_t)mt256 * nt256 / cus;

@@ -562,18 +562,6 @@ __global__ __launch_bounds__(64 * MID_WAVES, 1) void mid_kernel(MidArgs a) {
   }
 }
 
-int mid_cus() {
-  static std::atomic<int> cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cus[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
 size_t mid_align(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // Tiles, ranges and workgroups of a call.  At least one tile per CU: 32-row tiles dealt out in rounds, levelled to the
@@ -586,7 +574,7 @@ struct MidPlan {
 };
 MidPlan mid_plan(int M, int N, int K) {
   MidPlan p;
-  const int cus = mid_cus(), mblocks = (M + 31) / 32, nsteps = (K + CK_STEP - 1) / CK_STEP;
+  const int cus = kq_num_cus(), mblocks = (M + 31) / 32, nsteps = (K + CK_STEP - 1) / CK_STEP;
   const int t32 = (N + 31) / 32 * mblocks;
   p.splits = 1;
   if (t32 < cus) p.splits = std::max(1, std::min(cus / t32, nsteps / (2 * MID_WAVES)));
@@ -650,22 +638,23 @@ bool kq_mid_supported(int M, int N, int K, int codec) {
   // 55 / 84 / 149 (64 / 70 / 114): from two row blocks on the tile GEMM of the K-quants with exact integers is ahead on
   // the large matrices, where a weight decoded once per 64 rows counts.  The any-codec kernel the others have there is
   // behind on every shape: mxfp4 28672 x 8192 56 / 85 / 147 (131 / 164 / 298), q8_0 77 / 113 / 193 (114 / 136 / 229).
-  // Narrow matrices leave that GEMM with too few tiles up to 192 rows (q4_k / q6_k, 192 rows, us: 1024 x 4096 14 / 17
-  // against 22 / 24, 4096 x 4096 26 / 34 against 31 / 39, 4096 x 14336 61 / 86 against 69 / 99; 14336 x 4096 63 / 91
-  // against 56 / 84).
+  // Matrices of up to 4096 rows leave that GEMM with too few tiles up to 192 activation rows.  Here over there, 128 and 192
+  // rows, q4_k: K = 4096, 1024 rows 0.68, 0.66, 2048 rows 0.62, 0.82, 4096 rows 0.74, 0.79, K = 14336, 4096 rows 0.97, 0.93; q6_k 0.73,
+  // 0.71, 0.69, 0.91, 0.89, 0.87, 1.03, 0.94.  Past that a line in rows no longer tells: K = 4096, 6144 rows 0.81, 0.85, 8192 0.92,
+  // 0.97, 11008 0.96, 0.95, 14336 1.05, 1.10, 5120 x 13824 1.08, 1.08, 8192 x 8192 1.01, 0.97; those calls stay there.
   const bool tile_gemm = codec == KQ_Q4_K || codec == KQ_Q5_K || codec == KQ_Q6_K;
   if (tile_gemm) return M <= 32 || (M <= 64 && (int64_t)N * K <= (int64_t)64 << 20) || (M <= 192 && N <= 4096);
   // Against the any-codec kernel's 128-row tiles with its short decode for these codecs: a weight decoded once per 128 rows
   // instead of once per 32 wins where its last tile is (nearly) full and it has the tiles to cut K into whole rounds.  Here /
-  // there: iq2_xs 128 rows 8192 x 8192 68 / 61, 14336 x 4096 64 / 60, 256 rows 4096 x 14336 114 / 96, 8192 x 4096 76 / 62, 400 rows
-  // 4096 x 4096 70 / 59, 512 80 / 62; but 160 rows 8192 x 8192 82 / 98 and 1024 x 4096, 256 rows, 16 / 22.  The others at 512 rows of 4096 x 4096:
-  // iq1_m 74 / 63, iq1_s 66 / 60, iq2_xxs 71 / 65, but 2880 x 2816 (92 tiles, no whole rounds) 0.92 ... 0.85 of it, as at 256 rows of
-  // 4096 x 4096.
+  // there, us: iq2_xs 128 rows 8192 x 8192 68 / 61, 14336 x 4096 64 / 60, 256 rows 4096 x 14336 114 / 96, 8192 x 4096 76 / 62, 400 rows
+  // 4096 x 4096 70 / 59, 512 80 / 62; but 160 rows 8192 x 8192 82 / 98 and 1024 x 4096, 256 rows, 16 / 22.  The others at 512 rows
+  // of 4096 x 4096: iq1_m 74 / 63, iq1_s 66 / 60, iq2_xxs 71 / 65, but of 2880 x 2816 (92 tiles, no whole rounds) 0.92 ... 0.85 of
+  // it, as at 256 rows of 4096 x 4096.
   if (short_any_decode(codec)) {
     const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
     const int blocks = (M + 31) / 32, full = (M + 127) / 128 * 4;
-    if (4 * tiles >= mid_cus()) {
-      const bool whole = 2 * mid_cus() % tiles == 0;
+    if (4 * tiles >= kq_num_cus()) {
+      const bool whole = 2 * kq_num_cus() % tiles == 0;
       if (codec == KQ_IQ2_XS && M > 96 && (8 * blocks >= 7 * full || (whole && 5 * blocks >= 4 * full))) return false;
       if (M > 384 && blocks == full && whole) return false;
     }
@@ -688,7 +677,7 @@ bool kq_mid_supported(int M, int N, int K, int codec) {
 // iq3_xxs 64 1.02 ... 1.12, 72 0.84 ... 0.92; iq1_s / iq1_m / iq2_xs / iq2_xxs, whose any-codec decode is short, 64 1.31 ... 1.36,
 // 72 1.02 ... 1.08, 80 0.88 ... 0.96; q4_1 / q5_1 with their third term 96 0.91 ... 1.10, 128 1.06 ... 1.19, 132 0.90, 140 0.63.
 bool kq_tall_fills(int M, int N, int codec) {
-  const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256), cus = mid_cus();
+  const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256), cus = kq_num_cus();
   const bool three = codec == KQ_Q4_1 || codec == KQ_Q5_1;
   if (M > KQ_MID_MAX_ROWS) {
     const bool fp4 = codec == KQ_MXFP4 || codec == KQ_NVFP4;
@@ -699,7 +688,7 @@ bool kq_tall_fills(int M, int N, int codec) {
 }
 
 KqRedo kq_tall_redo(void* ws, int M, int N, int K) {
-  if (4 * (int64_t)((M + 127) / 128) * ((N + 255) / 256) >= 3 * (int64_t)mid_cus()) return KqRedo{nullptr, nullptr};
+  if (4 * (int64_t)((M + 127) / 128) * ((N + 255) / 256) >= 3 * (int64_t)kq_num_cus()) return KqRedo{nullptr, nullptr};
   int* rows = reinterpret_cast<int*>(static_cast<uint8_t*>(ws) + (size_t)M * K * 2 + (size_t)M * 4);
   return KqRedo{rows, rows + M};
 }

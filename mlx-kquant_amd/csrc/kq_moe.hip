@@ -490,8 +490,8 @@ double moe_rounds(double wgs, int slots, int ntiles) {
 // 2.4 of 32; 44 make 1.0 or 2.0): it takes 64 where their rounds, times what a workgroup of the 64-pair form takes longer per
 // round (the lighter the decode and the shorter K the more), come out below those of 32.  Measured on 64 over 32, q4_k: 128
 // experts of 2048 -> 768, 34 pairs per expert 1.01, 44 0.91, 76 1.06, 112 0.92; 32 of 1024 -> 2048 44 0.99, 70 1.25, 200 1.03; 8 of
-// 2048 -> 4096 44 0.90, 64 1.17, 100 0.94; q5_k / q6_k 128 of 2048 -> 768 28 1.08 / 1.11, 44 0.87 / 0.85, 70 0.97 / 0.92.  Over 606 calls on
-// eight stacks that the constants were not taken from, the choice is 1.4 % behind the better form (always 32: 10 %).
+// 2048 -> 4096 44 0.90, 64 1.17, 100 0.94; q5_k / q6_k 128 of 2048 -> 768 28 1.08 / 1.11, 44 0.87 / 0.85, 70 0.97 / 0.92.  Over 606
+// calls on eight stacks that the constants were not taken from, the choice is 1.4 % behind the better form (always 32: 10 %).
 int moe_seg_rows(int P, int R, int E, int N, int K, bool glu, int codec) {
   const int ncols = glu ? SLAB / 2 : SLAB, ntiles = (N + ncols - 1) / ncols;
   if ((int64_t)std::max(E, P / 64) * ntiles < 256 || P < (glu ? 28 : 32) * (int64_t)E) return 32;

@@ -1476,19 +1476,6 @@ __global__ __launch_bounds__(256) void st_splitk_reduce_kernel(const float* __re
   y[i] = DT == KQ_F16 ? kq::f2f16(v) : kq::f2bf16(v);
 }
 
-int st_num_cus() {
-  // compute units of the current device, looked up once per device
-  static std::atomic<int> cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int n = cus[dev].load(std::memory_order_relaxed);
-  if (n == 0) {
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cus[dev].store(n, std::memory_order_relaxed);
-  }
-  return n;
-}
-
 // K split: a workgroup takes at most 16 superblocks (32 where the kernel with eight units per wave applies: codecs
 // with four A register pairs per unit, up to four rows); with fewer row tiles than g_st_fill_pct per 100 CUs the
 // range is cut further so that about two workgroups per CU exist.
@@ -1562,7 +1549,7 @@ int st_launch_one(StArgs a, int splits, hipStream_t s) {
   constexpr int WGS = lds <= 80 * 1024 && NW == 4 ? 2 : 1;
   auto kern = stream_gemv_kernel<C, DT, MB, D, WGS, XU, NW>;
   KQ_SET_MAX_LDS_ONCE((kern), lds);
-  int gx = WGS * st_num_cus() / splits;
+  int gx = WGS * kq_num_cus() / splits;
   if (gx < 1) gx = 1;
   // rows per tile: when the 32-row tiles do not fill a whole number of rounds of the resident workgroups, the
   // busiest CU decides the time (448 tiles on 512 slots: two tiles on 192 CUs, one on 64).  Spreading the rows
@@ -1663,14 +1650,14 @@ bool kq_stream_supported(int M, int N, int K, int codec, const void* x, const vo
 
 size_t kq_stream_workspace_bytes(int M, int N, int K, int codec) {
   if (!st_codec_ok(codec) || M < 1 || M > 8 || !st_k_ok(K, codec)) return 0;
-  const StSplit p = st_split_plan(M, N, 256 * st_k_units(K), codec, st_num_cus());
+  const StSplit p = st_split_plan(M, N, 256 * st_k_units(K), codec, kq_num_cus());
   return p.ksplit > 1 ? (size_t)p.ksplit * M * N * sizeof(float) : 0;
 }
 
 int kq_launch_qmm_stream(const void* x, const uint8_t* w, void* y, int M, int N, int K, int codec, int dtype, void* ws,
                          size_t ws_bytes, hipStream_t s, const void* bias) {
   if (!kq_stream_supported(M, N, K, codec, x, w)) return KQ_ERR_UNSUPPORTED;
-  const StSplit p = st_split_plan(M, N, 256 * st_k_units(K), codec, st_num_cus());
+  const StSplit p = st_split_plan(M, N, 256 * st_k_units(K), codec, kq_num_cus());
   if (bias && p.ksplit > 1) return KQ_ERR_UNSUPPORTED;  // the bias joins the sum in the unsplit epilogue only
   // three or more rows of a table-decoded 4-bit codec whose K range has to be cut (few row tiles): the code-level
   // kernel needs no reduction launch and is ahead (mxfp4 3072 -> 2880: 4 rows 7.8 us against 10.4 here, 8 rows 9.1
