@@ -593,8 +593,8 @@ int launch_gemm2_low(const void* x, const uint8_t* w, void* y, int M, int N, int
 
 }  // namespace
 
-// q2_k / q3_k on the 128 x 256 tile kernel: M >= 256 and enough tiles to fill the chip; the any-codec kernel keeps
-// the smaller shapes.
+// q2_k / q3_k / iq4_xs on the 128 x 256 tile kernel: M >= 256 and enough tiles to fill the chip; smaller calls stay on the
+// streamed kernel or, beyond its rows, the any-codec kernel.
 bool kq_gemm2_low_supported(int M, int N, int K, int codec) {
   return (codec == KQ_Q2_K || codec == KQ_Q3_K || codec == KQ_IQ4_XS) && M >= 256 && K >= 256 && (K & 255) == 0 && N > 0 &&
          (int64_t)((M + 127) / 128) * ((N + 255) / 256) >= 256 && (int64_t)N * (K >> 8) * 136 < ((int64_t)1 << 32) &&

@@ -19,8 +19,8 @@
 // the tile's columns, contiguous per row; for the 256-weight codecs the whole superblock, which two column tiles
 // share) into its own LDS area with dword loads issued one step ahead, and the decoders read the bytes from there:
 // decoding straight from global memory costs about 130 byte-wide loads a step.  Calls of 96 rows and more run
-// gemm_nt_wide_kernel below, which decodes a step once for 128 activation rows, calls of 512 and more
-// gemm_nt_tall_kernel (256 rows).
+// gemm_nt_wide_kernel below, which decodes a step once for 128 activation rows, or from 512 rows on, where its tiles fill the
+// chip (nt_tall), gemm_nt_tall_kernel (256 rows).
 #include <algorithm>
 #include <type_traits>
 
