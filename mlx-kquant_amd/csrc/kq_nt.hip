@@ -427,7 +427,10 @@ __global__ __launch_bounds__(NT_THREADS, 2) void gemm_nt_wide_kernel(NtArgs a, c
       }
     }
     if (st == st_begin) __syncthreads();  // the first staging buffer is complete (later ones: the barrier below)
-    fetch(st + 1 < nsteps ? st + 1 : st);
+    // Under a branch, unlike the 256-row kernel's: as one block of code with the decode (the last step fetched again) the codecs of
+    // short decode lost a tenth.  us, one block / branch (reduction x outputs): q8_0 600 rows 4096 x 14336 277 / 246, 128 rows 14336 x 4096 67 / 56, q6_k 2048
+    // rows 4096 x 4096 252 / 222, q4_0 96 ... 511 rows 0.94 of it, q4_k level
+    if (st + 1 < nsteps) fetch(st + 1);
     {  // decode this lane's two rows and put them where the operands lie
       float w0[8], w1[8];
       kq::decode8<C>(stage + blk_off, g, grids, w0);
