@@ -428,8 +428,8 @@ __global__ __launch_bounds__(NT_THREADS, 2) void gemm_nt_wide_kernel(NtArgs a, c
     }
     if (st == st_begin) __syncthreads();  // the first staging buffer is complete (later ones: the barrier below)
     // Under a branch, unlike the 256-row kernel's: as one block of code with the decode (the last step fetched again) the codecs of
-    // short decode lost a tenth.  us, one block / branch (reduction x outputs): q8_0 600 rows 4096 x 14336 277 / 246, 128 rows 14336 x 4096 67 / 56, q6_k 2048
-    // rows 4096 x 4096 252 / 222, q4_0 96 ... 511 rows 0.94 of it, q4_k level
+    // short decode lost a tenth.  us, one block / branch: q8_0 600 rows 4096 x 14336 (reduction x outputs) 277 / 246, 128 rows
+    // 14336 x 4096 67 / 56, q6_k 2048 rows 4096 x 4096 252 / 222, q4_0 96 ... 511 rows 0.94 of it, q4_k level
     if (st + 1 < nsteps) fetch(st + 1);
     {  // decode this lane's two rows and put them where the operands lie
       float w0[8], w1[8];
@@ -737,13 +737,14 @@ int nt_ranges(int M, int N, int K, bool tall) {
 }
 
 // Calls of the 256-row kernel: 512 rows and more of aligned activations, K long enough for its pipeline, and not more than
-// 5 % (10 %) over the 128-row kernel by the work of their busiest CU, in 64-row steps of K.  256-row tiles run one per CU, so an
+// 5 % over the 128-row kernel by the work of their busiest CU, in 64-row steps of K.  256-row tiles run one per CU, so an
 // unfilled round costs a whole one, and two steps more to fill the pipeline; of the 128-row tiles two run per CU, each half a
 // step per 32 rows, and a last round evens out but for a quarter.  Measured / by this, 256-row over 128-row kernel, q4_k:
-// 600 rows 4096 x 4096 (reduction x outputs) 1.27 / 1.41, 4096 x 14336 1.39 / 1.51, 1024 rows 4096 x 4096 1.01 / 1.05, 2048 x 6144
-// 1.14 / 1.21, 1400 rows 4096 x 4096 1.26 / 1.25, 8192 x 8192 1.42 / 1.25, 1800 rows 4096 x 4096 0.91 / 0.96, 2048 rows 4096 x 14336
-// 1.20 / 1.17.  q6_k, q8_0, q5_0, iq4_xs and mxfp4 lie a tenth below that.  Never for the codebook codecs, whose table reads
-// from eight waves decoding together make the 256-row kernel 1.3 - 1.5 times the other (1.1 where it is best).
+// 600 rows 4096 x 4096 (reduction x outputs) 1.28 / 1.37, 4096 x 14336 1.38 / 1.52, 1024 rows 4096 x 4096 1.03 / 1.05, 2048 x 6144
+// 1.15 / 1.18, 1400 rows 4096 x 4096 1.27 / 1.25, 8192 x 8192 1.39 / 1.25, 1800 rows 4096 x 4096 0.93 / 0.96, 2048 rows 4096 x 14336
+// 1.19 / 1.09.  The others lie within 5 % of that (q5_0 a tenth below) but for q2_k and q4_1 a twentieth above it, which therefore
+// take 95 %.  Over 70 calls per codec the choice is 0.2 ... 1.0 % behind the better kernel.  Never for the codebook codecs, whose table
+// reads from eight waves decoding together make the 256-row kernel 1.3 - 1.5 times the other (1.1 where it is best).
 // cut: K may be cut over the grid; entries: 1 for a dense call.
 constexpr bool nt_codebook(int codec) {
   return codec == KQ_IQ1_S || codec == KQ_IQ1_M || codec == KQ_IQ2_XXS || codec == KQ_IQ2_XS || codec == KQ_IQ2_S ||
@@ -757,8 +758,7 @@ bool nt_tall(int codec, int M, int N, int K, bool cut, int entries) {
   const double rounds = (double)(cols * ((M + 127) / 128) * sw) / 512, steps = (double)K / TALL_K;
   const double tall = (double)((tall_wgs + 255) / 256) * (steps / st + 2);
   const double wide = (rounds <= 1 ? 1 : rounds + 0.25) * (steps / sw + 0.5);
-  const bool light = codec == KQ_Q6_K || codec == KQ_Q8_0 || codec == KQ_Q5_0 || codec == KQ_IQ4_XS || codec == KQ_MXFP4;
-  return tall <= (light ? 1.10 : 1.05) * wide;
+  return tall <= (codec == KQ_Q2_K || codec == KQ_Q4_1 ? 0.95 : 1.05) * wide;
 }
 
 // Entries of one expert share tiles: two or more fit a tile, an expert comes twice on average, and the list is short enough

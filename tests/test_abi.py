@@ -137,6 +137,7 @@ def test_any_codec_kernel_keeps_full_tiles_of_short_decode(lib, codec, M, N, str
     ("q6_k", 640, 4096, 14336, 4),
     ("q8_0", 1024, 4096, 4096, 2),     # (either kernel)
     ("q4_k", 512, 768, 16384, 21),     # 256-row tiles: 12 in 21 ranges
+    ("q8_0", 1800, 1024, 1536, 5),     # 128-row tiles: 120 in five, against 64 of 256 rows in four
     ("iq2_xs", 512, 768, 16384, 22),   # 128-row tiles for the codebook codecs: 24 in 22
 ])
 def test_transposed_product_takes_256_row_tiles_where_they_fill(lib, codec, M, N, K, ranges):
