@@ -36,6 +36,7 @@ SOURCES = [
     ("kq_tile.hip", ["-Wno-inline-asm", "-DKQ_TILE_NB=2"], "kq_tile_2"),
     ("kq_tile.hip", ["-Wno-inline-asm", "-DKQ_TILE_NB=3"], "kq_tile_3"),
     ("kq_tile.hip", ["-Wno-inline-asm", "-DKQ_TILE_NB=4"], "kq_tile_4"),
+    ("kq_mix.hip", ["-Wno-inline-asm", "-ffp-contract=off"]),
     ("kq_moe.hip", []),
     ("kq_moe_tile.hip", ["-Wno-inline-asm"]),
     ("kq_anymma.hip", ["-ffp-contract=off"]),

@@ -751,18 +751,16 @@ int kq_moe_glu_gather_shexp(const void* x_dev, const void* gate_w_dev, const voi
                              0.f, 0.f, shexp_codec, dtype, sub, sub_bytes, KqOutMap{1, R + 1, R, 0}, stream);
 }
 
-// Decode-sized calls.  One launch on the streamed kernel with the mix folded in (kq_launch_mix_stream) where a token's slots
-// are short enough for it.  Else, one token: f32 slot rows of the streamed gathered kernel and a mix launch where that kernel has
-// the codec; what is left, and up to three tokens with a shared expert (whose other form takes six launches), runs as a
-// workgroup per output element (kq_launch_gather_mix_generic).  Larger calls: the gathered kernels and the mix launch.
-static bool mix_streamed(int T, int S, int N, int K, int codec, int shexp_codec) {
-  return T <= 16 && (shexp_codec < 0 || shexp_codec == codec) && kq_mix_stream_fits(T, S, N, K, codec);
-}
+// Decode-sized calls run as one kernel.  One token, or up to three with a shared expert (whose other form takes six launches):
+// f32 sums of the decoded weights, kq_launch_mix where a token's slots are short enough for it.  More tokens, up to 16: the
+// streamed kernel with the mix folded in, within the same bound.  Else, one token: f32 slot rows of the streamed gathered kernel and
+// a mix launch where that kernel has the codec; what is left of up to three tokens: a workgroup per output element
+// (kq_launch_gather_mix_generic).  Larger calls: the gathered kernels and the mix launch.
+static bool mix_f32(int T, int S, bool shared) { return S <= 32 && T <= (shared ? 3 : 1); }
 static bool mix_single_launch(int T, int S, int N, int K, int codec, int shexp_codec) {
   const bool shared = shexp_codec >= 0;
-  if (S > 32 || T > (shared ? 3 : 1)) return false;
-  if (shared || mix_streamed(T, S, N, K, codec, shexp_codec)) return true;
-  return !kq_gather_stream_takes(nullptr, nullptr, nullptr, S, N, K, false, 0, 0, false, codec);
+  if (!mix_f32(T, S, shared)) return false;
+  return shared || kq_mix_fits(S, N, K, codec) || !kq_gather_stream_takes(nullptr, nullptr, nullptr, S, N, K, false, 0, 0, false, codec);
 }
 
 size_t kq_gather_qmv_mix_workspace_size(int T, int S, int E, int N, int K, int codec, int shexp_codec, int dtype) {
@@ -796,9 +794,15 @@ static int gather_qmv_mix_impl(const char* op, const void* x_dev, const void* w_
   if (!x_dev || !w_dev || !idx_dev || !scores_dev || !out_dev) return kq_set_error(KQ_ERR_INVALID, "%s: null buffer", op);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int64_t expert_stride = (int64_t)N * (K / kCodecs[codec].weights_per_block) * kCodecs[codec].bytes_per_block;
-  if (mix_streamed(T, S, N, K, codec, shared ? shexp_codec : -1)) {
-    rc = kq_launch_mix_stream(x_dev, static_cast<const uint8_t*>(w_dev), static_cast<const uint8_t*>(shexp_w_dev), idx_dev,
-                              scores_dev, bias_dev, out_dev, T, S, E, N, K, expert_stride, codec, dtype, s);
+  if (!shared || shexp_codec == codec) {
+    if (mix_f32(T, S, shared))
+      rc = kq_launch_mix(x_dev, static_cast<const uint8_t*>(w_dev), static_cast<const uint8_t*>(shexp_w_dev), idx_dev, scores_dev,
+                         bias_dev, out_dev, T, S, E, N, K, expert_stride, codec, dtype, s);
+    else if (T <= 16)
+      rc = kq_launch_mix_stream(x_dev, static_cast<const uint8_t*>(w_dev), static_cast<const uint8_t*>(shexp_w_dev), idx_dev,
+                                scores_dev, bias_dev, out_dev, T, S, E, N, K, expert_stride, codec, dtype, s);
+    else
+      rc = KQ_ERR_UNSUPPORTED;
     if (rc != KQ_ERR_UNSUPPORTED) return rc;
   }
   if (mix_single_launch(T, S, N, K, codec, shared ? shexp_codec : -1)) {

@@ -141,8 +141,13 @@ int kq_launch_gather_stream(const void* x, const uint8_t* w, const uint8_t* w2, 
 bool kq_gather_stream_takes(const void* x, const void* w, const void* w2, int entries, int N, int K, bool strided_x,
                             int64_t x_row_stride, int64_t w_expert_stride, bool second_bias_without_glu, int codec);
 int kq_gather_stream_max_entries();
-// The down projection of MoE decode with the routing mix on the streamed kernel: out[t] = sum over the slots of scores x
-// (row t S + s of x . matrix), the last slot on shexp_w if there is one (its codec is the experts').
+// The down projection of MoE decode with the routing mix in one launch: out[t] = sum over the slots of scores x (row t S + s of
+// x . matrix), the last slot on shexp_w if there is one (its codec is the experts').  kq_launch_mix: the f32 sums of
+// kq_launch_gather_mix_generic (kq_mix.hip); kq_launch_mix_stream: the streamed kernel's (activations as scaled f16).
+bool kq_mix_fits(int S, int N, int K, int codec);
+int kq_launch_mix(const void* x, const uint8_t* w, const uint8_t* shexp_w, const uint32_t* idx, const float* scores,
+                  const float* bias, void* out, int T, int S, int E, int N, int K, int64_t w_expert_stride, int codec,
+                  int dtype, hipStream_t s);
 bool kq_mix_stream_fits(int T, int S, int N, int K, int codec);
 int kq_launch_mix_stream(const void* x, const uint8_t* w, const uint8_t* shexp_w, const uint32_t* idx, const float* scores,
                          const float* bias, void* out, int T, int S, int E, int N, int K, int64_t w_expert_stride, int codec,

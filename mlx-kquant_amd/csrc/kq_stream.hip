@@ -279,11 +279,15 @@ struct StArgs {
   const float* bias2;  // the same for the up sums of the fused form
   int64_t w_expert_stride;
   KqOutMap om;
-  // mixed calls (down projection of MoE decode): token t = blockIdx.x / tiles_per_entry sums scores[t][s] * (row t S + s of x).
-  // (matrix rhs[t * routed + s]) over its S = x_div slots; slots from `routed` on take the shared expert's matrix w2
+};
+// mixed calls (down projection of MoE decode): token t = blockIdx.x / tiles_per_entry sums scores[t][s] * (row t S + s of x).
+// (matrix rhs[t * routed + s]) over its S = x_div slots; slots from `routed` on take the shared expert's matrix w2.
+struct StMixArgs : StArgs {
   const float* scores;
   int routed;
 };
+template <int GM>
+using StArgsOf = std::conditional_t<GM == 3, StMixArgs, StArgs>;
 
 // ------------------------------------------------------------------ q4_k / q5_k unit
 // Lane (row, kg) owns sub-blocks 4 kg .. 4 kg + 3.  LDS row: d, dmin, scales[12] | (q5_k: qh[32]) | qs[128].
@@ -917,10 +921,12 @@ constexpr int st_xch() { return MB > 4 ? 2 : MB; }  // activation rows staged at
 // superblock is two units (the gate rows, then the same rows of the up matrix) with an accumulator each, and the
 // tile's result is act(gate) * up.
 template <int C, int DT, int MB, int D, int WGS, int XU, int NW, int GM = 0>
-__global__ __launch_bounds__(64 * NW, WGS) void stream_gemv_kernel(StArgs a) {
+__global__ __launch_bounds__(64 * NW, WGS) void stream_gemv_kernel(StArgsOf<GM> a) {
   static_assert(GM == 0 || MB == 1, "gathered entries carry one activation row");
   // GM = 3 (mixed): the slots of a token are one long row, S nsb units of it, each with a matrix of its own: a workgroup does
-  // all slots of its weight rows and no f32 slot results pass through memory.
+  // all slots of its weight rows and no f32 slot results pass through memory.  What only this form needs is kept out of the
+  // other forms' expressions and arguments: written into them (a branch around `base`, a field more) it changed the dense
+  // kernels' code, and the seven projections of a block took 1.4 % longer at one row.
   constexpr int ST_XU = XU, ST_WAVES = NW;
   constexpr int UPS = GM == 2 ? 2 : 1;  // units per superblock
   using G = StGeom<C>;
@@ -944,6 +950,7 @@ __global__ __launch_bounds__(64 * NW, WGS) void stream_gemv_kernel(StArgs a) {
   const uint32_t tail_bytes = (uint32_t)tail_blocks * (G::BPB / 8);  // and their bytes
   // gathered: this workgroup's entry and its tile inside the entry's matrix (the tile loop below runs once)
   const int slots = GM == 3 ? a.x_div : 1;
+  (void)slots;
   const int g_entry = GM ? __builtin_amdgcn_readfirstlane((int)blockIdx.x / a.tiles_per_entry) : 0;
   const int g_tile = GM ? (int)blockIdx.x - g_entry * a.tiles_per_entry : 0;
   const uint8_t* wmat = a.w;
@@ -973,8 +980,8 @@ __global__ __launch_bounds__(64 * NW, WGS) void stream_gemv_kernel(StArgs a) {
 
   // this workgroup's K range and this wave's units: superblocks sb_begin + wave + 4 u
   const int sb_begin = a.ksplit > 1 ? (int)blockIdx.z * a.sb_per_split : 0;
-  int sb_end = a.ksplit > 1 ? sb_begin + a.sb_per_split : slots * nsb;
-  sb_end = sb_end < slots * nsb ? sb_end : slots * nsb;
+  int sb_end = a.ksplit > 1 ? sb_begin + a.sb_per_split : (GM == 3 ? slots * nsb : nsb);
+  sb_end = sb_end < (GM == 3 ? slots * nsb : nsb) ? sb_end : (GM == 3 ? slots * nsb : nsb);
   const int sbn = sb_end - sb_begin;
   const int nu = UPS * (sbn > wave ? (sbn - wave + ST_WAVES - 1) / ST_WAVES : 0);  // wave-uniform, 0..XU
 
@@ -1048,15 +1055,13 @@ __global__ __launch_bounds__(64 * NW, WGS) void stream_gemv_kernel(StArgs a) {
       SFor<U::FULL + 1>::run([&](auto t) { constexpr int T = decltype(t)::value; goff[T] = piece_off(lane + 64 * T, row0); });
       goff_row0 = row0;
     }
-    const uint8_t* base;
+    const uint8_t* base = ((GM == 2 && (iu & 1)) ? wmat2 : wmat) + (size_t)row0 * row_bytes +
+                          (size_t)(sb_begin + wave + ST_WAVES * (iu / UPS)) * G::BPB;
     if constexpr (GM == 3) {
       const uint32_t e = (uint32_t)__builtin_amdgcn_readlane((int)u_expert, iu);
       const int g = wave + ST_WAVES * iu, slot = __builtin_amdgcn_readfirstlane(g / nsb);
       base = (e == ~0u ? a.w2 : a.w + (e == ~1u ? 0 : (int64_t)e * a.w_expert_stride)) + (size_t)row0 * row_bytes +
              (size_t)(g - slot * nsb) * G::BPB;
-    } else {
-      base = ((GM == 2 && (iu & 1)) ? wmat2 : wmat) + (size_t)row0 * row_bytes +
-             (size_t)(sb_begin + wave + ST_WAVES * (iu / UPS)) * G::BPB;
     }
     const uint32_t l0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(wb_lds + islot * U::SLOT));
     bool tail_unit = false;
@@ -1389,7 +1394,10 @@ __global__ __launch_bounds__(64 * NW, WGS) void stream_gemv_kernel(StArgs a) {
     const int nrows = N - row0 < rpt ? N - row0 : rpt;
     const int crow = n < nrows ? n : nrows - 1;
     if constexpr (GM == 3) {
-      if (__builtin_expect(wide, 0)) {  // f32 on the reference-order weights, the numerics of gather_mix_generic_kernel
+      // f32 on the reference-order weights, the numerics of gather_mix_generic_kernel.  Rare (normally distributed activations
+      // hold one such value in 10^9), so small code rather than speed: of 4 tokens, q6_k, top-8 of 2048 x 768, one such value
+      // in one token 24 us, in every slot of every token 46 (ordinary ones 10).
+      if (__builtin_expect(wide, 0)) {
         vmwait<0>();
 #pragma unroll 1
         for (int u = 0; u < nu; u++) {
@@ -1412,7 +1420,7 @@ __global__ __launch_bounds__(64 * NW, WGS) void stream_gemv_kernel(StArgs a) {
     }
     SFor<ST_XU>::run([&](auto uu) {
       constexpr int u = decltype(uu)::value;
-      if (u < nu && !wide) {
+      if (u < nu && !(GM == 3 && wide)) {
         // loads issued after this unit's: inflight - 1 units
         const int younger = inflight - 1;
         if (younger >= 3) vmwait<3 * U::UPI>();
@@ -1422,10 +1430,13 @@ __global__ __launch_bounds__(64 * NW, WGS) void stream_gemv_kernel(StArgs a) {
         const uint8_t* slot = wb + cslot * U::SLOT;
         const uint8_t* bl = slot + crow * G::LBPB;
         constexpr int us = u / UPS;  // the wave's superblock this unit belongs to
-        float unit_sum[R];
+        float* acc = (GM == 2 && (u & 1)) ? acc_b : acc_a;
+        float unit_sum[GM == 3 ? R : 1];
+        if constexpr (GM == 3) {
 #pragma unroll
-        for (int r = 0; r < R; r++) unit_sum[r] = 0.f;
-        float* acc = GM == 3 ? unit_sum : (GM == 2 && (u & 1)) ? acc_b : acc_a;
+          for (int r = 0; r < R; r++) unit_sum[r] = 0.f;
+          acc = unit_sum;
+        }
         const int nvalid = sb_begin + wave + ST_WAVES * us == tail_sb ? tail_blocks : 8;
         (void)nvalid;
         if constexpr (TAIL) {
@@ -1707,7 +1718,7 @@ int st_launch_gather_nw(const StArgs& a, int entries, bool glu, hipStream_t s) {
 
 // Mixed calls: eight waves, one round of a workgroup per CU (tiles of 8 to 32 rows; the loads of a unit cover 32 either way).
 template <int C, int DT>
-int st_launch_mix(StArgs a, int T, hipStream_t s) {
+int st_launch_mix(StMixArgs a, int T, hipStream_t s) {
   constexpr int D = 2, XU = 4, NW = 8;
   constexpr size_t lds = st_lds_bytes<C, 1, D, XU, NW, 3>();
   static_assert(lds <= 160 * 1024, "workgroup does not fit the LDS of a CU");
@@ -1883,10 +1894,10 @@ int kq_launch_gather_stream(const void* x, const uint8_t* w, const uint8_t* w2, 
 }
 
 // Down projection of MoE decode with the routing mix in one launch: at most 32 units (256 weights of a slot) a token, tiles of up
-// to 32 weight rows of all tokens in one round of the CUs, or two where a token has the units to pay for it.  us, top-8 on 128
-// experts of 2048 x 768 (before: one token a workgroup per output element on the vector ALU, more the gathered kernels and a
-// launch for the mix): q6_k 1 / 2 / 4 / 8 tokens 9.6 / 9.6 / 10.7 / 19.2 (12.7 / 14.3 / 21.7 / 35), q4_k 6.8 / 7.1 / 7.3 / 12.8
-// (14.6 / 11.7 / 15.6 / 26.6), q8_0 8.5 / 8.8 (9.4 / 14.2); 2 slots, two rounds (6 tokens, 6 units each) would be 11.8 against 10.5.
+// to 32 weight rows of all tokens in one round of the CUs, or two where a token has the units to pay for it.  For the calls whose
+// sums are those of the units anyway (the gathered kernel and a launch for the mix had them; kq_launch_mix has what is summed in
+// f32).  us, top-8 on 128 experts of 2048 x 768, 2 / 4 / 8 tokens (before): q6_k 8.9 / 10.0 / 18.1 (14.3 / 21.7 / 35), q4_k 8.1 / 8.5 /
+// 12.2 (11.7 / 15.6 / 26.6); 2 slots, two rounds (6 tokens, 6 units each) would be 11.8 against 10.5.
 bool kq_mix_stream_fits(int T, int S, int N, int K, int codec) {
   const int64_t tiles = (int64_t)T * ((N + ST_ROWS - 1) / ST_ROWS), cus = kq_num_cus();
   if (T > 1 && tiles > cus && (tiles > 2 * cus || S * (K >> 8) < 12)) return false;
@@ -1901,7 +1912,7 @@ int kq_launch_mix_stream(const void* x, const uint8_t* w, const uint8_t* shexp_w
       (shexp_w && !kq_gather_stream_takes(x, shexp_w, nullptr, 1, N, K, false, 0, 0, false, codec)) ||
       (int64_t)T * ((N + 7) / 8) > 65535 * 16)
     return KQ_ERR_UNSUPPORTED;
-  StArgs a{};
+  StMixArgs a{};
   a.x = x;
   a.w = w;
   a.w2 = shexp_w;

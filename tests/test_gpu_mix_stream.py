@@ -1,6 +1,6 @@
-"""GPU parity of the one-launch down projection with the routing mix (streamed kernel) where its tiling can go wrong: one slot of
-one unit, 32 units, a ragged last tile, tiles of 8 / 12 / 32 rows, two rounds of workgroups, the shared slot, ids outside the stack,
-biases, activations of wide range."""
+"""GPU parity of the one-launch down projection with the routing mix where its tiling can go wrong: one slot of one unit, 32 units,
+several rounds of workgroups, the shared slot, ids outside the stack, activations of wide range; and its sums against
+those of the kernel without tiles, bit for bit."""
 import numpy as np
 import pytest
 import torch
@@ -31,8 +31,9 @@ def run(xt, w, sw, codec, idx, scores):
 
 @pytest.mark.parametrize("codec", STREAMED)
 def test_mix_stream_edges(codec):
-    # (tokens, slots, N, K): the least; 32 units on a ragged 12-row tile; two rounds of 32-row tiles
-    for i, (T, S, N, K) in enumerate([(1, 1, 8, 256), (2, 8, 1064, 1024), (9, 3, 1496, 1024)]):
+    # (tokens, slots, N, K): the least, of the kernel for one token and of the streamed one; 32 units on a ragged 12-row tile; two
+    # rounds of 32-row tiles
+    for i, (T, S, N, K) in enumerate([(1, 1, 8, 256), (2, 8, 1064, 1024), (9, 3, 1496, 1024), (2, 1, 8, 256)]):
         dtype = ("bfloat16", "float16")[i % 2]
         w, _, idx, scores = case(codec, T, S, 4, N, K, 310 + i)
         xb, xt = make_x((T, S, K), dtype, seed=320 + i, scale=0.05)
@@ -41,7 +42,7 @@ def test_mix_stream_edges(codec):
 
 
 @pytest.mark.parametrize("codec", ["q6_k", "iq3_s", "q8_0"])
-@pytest.mark.parametrize("T", [1, 3])
+@pytest.mark.parametrize("T", [1, 3, 5])
 def test_mix_stream_shared_slot_and_ids_outside(codec, T):
     """An id outside the stack adds nothing, whatever expert 0 (which its loads read) holds; the shared slot stays."""
     S, E, N, K = 5, 3, 264, 768
@@ -75,12 +76,13 @@ def test_mix_stream_rows_of_wide_range(codec):
 
 
 def test_mix_stream_tokens_are_independent_and_replay():
-    """A token's result does not depend on how many share the launch (tile heights differ); replays follow the inputs."""
+    """A token's result does not depend on how many share the launch (tile heights differ; one token alone has the f32 sums of a
+    kernel of its own); replays follow the inputs."""
     S, E, N, K = 8, 6, 2048, 768
     w, _, idx, scores = case("q4_k", 8, S, E, N, K, 350)
     _, xt = make_x((8, S, K), "bfloat16", seed=351, scale=0.05)
     wd, sc, ix = wire_to_dev(w), torch.from_numpy(scores).cuda(), _idx_dev(idx).to(torch.int32)
-    want = torch.cat([kq.gather_qmv_mix_ns_kq(xt[t:t + 1], wd, "q4_k", ix[t:t + 1], sc[t:t + 1]) for t in range(8)])
+    want = torch.cat([kq.gather_qmv_mix_ns_kq(xt[t:t + 2], wd, "q4_k", ix[t:t + 2], sc[t:t + 2]) for t in range(0, 8, 2)])
     assert torch.equal(kq.gather_qmv_mix_ns_kq(xt, wd, "q4_k", ix, sc), want)
     buf = xt[:1].clone()
     torch.cuda.synchronize()
@@ -92,3 +94,52 @@ def test_mix_stream_tokens_are_independent_and_replay():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, kq.gather_qmv_mix_ns_kq(buf, wd, "q4_k", ix[:1], sc[:1]))
+
+
+def c_call(xt, w, sw, codec, idx, scores):
+    """The C entry point without a workspace."""
+    lib, (T, S, K), (E, N) = kq._load(), xt.shape, w.shape[:2]
+    out = torch.full((T, N), float("nan"), dtype=xt.dtype, device="cuda")
+    c = lib.kq_codec_id(codec.encode())
+    rc = lib.kq_gather_qmv_mix(xt.data_ptr(), w.data_ptr(), None if sw is None else sw.data_ptr(), idx.data_ptr(), scores.data_ptr(),
+                               out.data_ptr(), T, S, E, N, K, c, -1 if sw is None else c, 1 if xt.dtype == torch.float16 else 2, None, 0,
+                               torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.kq_last_error()
+    return out
+
+
+def unaligned(t):
+    """A copy that starts at an odd multiple of two bytes: the call runs a workgroup per output element."""
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")
+    buf[1:].copy_(t.reshape(-1))
+    return buf[1:].view(t.shape)
+
+
+# (tokens, slots, N, K, shared slot): the least; 32 units; three long slots; the shared slot; 32 slots; a slot of 32 units
+@pytest.mark.parametrize("codec", STREAMED)
+@pytest.mark.parametrize("T,S,N,K,shared", [(1, 1, 8, 256, False), (1, 8, 1064, 1024, False), (1, 3, 264, 2560, False),
+                                            (3, 5, 264, 768, True), (1, 32, 40, 256, False), (1, 1, 24, 8192, False)])
+def test_sums_are_those_of_the_kernel_without_tiles(codec, T, S, N, K, shared):
+    """f32 products of the activations as they are, in one order: activations with a mean, whose sums cancel where weights are
+    multiplied with an offset."""
+    w, sw, idx, scores = case(codec, T, S, 3, N, K, 360 + S, shared)
+    idx[0, 0] = 2  # the stack's last matrix
+    dtype = ("bfloat16", "float16")[S % 2]
+    x = (torch.randn((T, S, K), generator=torch.Generator().manual_seed(361)) * 0.1 + 1.0).to(getattr(torch, dtype)).cuda()
+    args = (wire_to_dev(w), None if sw is None else wire_to_dev(sw), codec, _idx_dev(idx).to(torch.int32), torch.from_numpy(scores).cuda())
+    got, want = c_call(x, *args), c_call(unaligned(x), *args)
+    assert torch.isfinite(want).all()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (codec, float((got != want).float().mean()))
+
+
+@pytest.mark.parametrize("codec", ["q4_k", "q6_k", "q8_0"])
+def test_infinite_activation(codec):
+    """An infinity times a weight is an infinity of the weight's sign, as in the kernel without tiles."""
+    T, S, E, N, K = 1, 4, 3, 72, 512
+    w, _, idx, scores = case(codec, T, S, E, N, K, 370)
+    x = (torch.randn((T, S, K), generator=torch.Generator().manual_seed(371)) * 0.1).to(torch.float16).cuda()
+    x[0, 1, 77] = float("inf")
+    args = (wire_to_dev(w), None, codec, _idx_dev(idx).to(torch.int32), torch.from_numpy(scores).cuda())
+    got, want = c_call(x, *args), c_call(unaligned(x), *args)
+    assert torch.isinf(want).any()
+    assert torch.equal(got.nan_to_num(7.0, 9.0, -9.0), want.nan_to_num(7.0, 9.0, -9.0))
