@@ -751,21 +751,15 @@ int kq_moe_glu_gather_shexp(const void* x_dev, const void* gate_w_dev, const voi
                              0.f, 0.f, shexp_codec, dtype, sub, sub_bytes, KqOutMap{1, R + 1, R, 0}, stream);
 }
 
-// Decode-sized calls run as one kernel.  One token, or up to three with a shared expert (whose other form takes six launches):
-// f32 sums of the decoded weights, kq_launch_mix where a token's slots are short enough for it.  More tokens, up to 16: the
-// streamed kernel with the mix folded in, within the same bound.  Else, one token: f32 slot rows of the streamed gathered kernel and
-// a mix launch where that kernel has the codec; what is left of up to three tokens: a workgroup per output element
-// (kq_launch_gather_mix_generic).  Larger calls: the gathered kernels and the mix launch.
+// Decode-sized calls run as one kernel.  One token, or up to three with a shared expert (whose other form takes six launches): f32
+// sums of the decoded weights without a workspace, kq_launch_mix where it takes the call, else a workgroup per output element
+// (kq_launch_gather_mix_generic).  More tokens, up to 16: the streamed kernel with the mix folded in where a token's slots are short
+// enough for it.  Larger calls: the gathered kernels into f32 slot rows and a launch for the mix.
 static bool mix_f32(int T, int S, bool shared) { return S <= 32 && T <= (shared ? 3 : 1); }
-static bool mix_single_launch(int T, int S, int N, int K, int codec, int shexp_codec) {
-  const bool shared = shexp_codec >= 0;
-  if (!mix_f32(T, S, shared)) return false;
-  return shared || kq_mix_fits(S, N, K, codec) || !kq_gather_stream_takes(nullptr, nullptr, nullptr, S, N, K, false, 0, 0, false, codec);
-}
 
 size_t kq_gather_qmv_mix_workspace_size(int T, int S, int E, int N, int K, int codec, int shexp_codec, int dtype) {
   if (T <= 0 || S <= 0) return 0;
-  if (mix_single_launch(T, S, N, K, codec, shexp_codec)) return 0;
+  if (mix_f32(T, S, shexp_codec >= 0)) return 0;
   size_t fixed = align256((size_t)T * S * N * 4);  // f32 slot results
   size_t sub = kq_moe_workspace_size(T, S, E, N, K, 0, codec, dtype);
   if (shexp_codec >= 0) {
@@ -805,7 +799,7 @@ static int gather_qmv_mix_impl(const char* op, const void* x_dev, const void* w_
       rc = KQ_ERR_UNSUPPORTED;
     if (rc != KQ_ERR_UNSUPPORTED) return rc;
   }
-  if (mix_single_launch(T, S, N, K, codec, shared ? shexp_codec : -1)) {
+  if (mix_f32(T, S, shared)) {
     rc = kq_launch_gather_mix_generic(x_dev, static_cast<const uint8_t*>(w_dev), static_cast<const uint8_t*>(shexp_w_dev),
                                       idx_dev, scores_dev, bias_dev, out_dev, T, S, E, N, K, expert_stride, codec,
                                       shared ? shexp_codec : codec, dtype, s);

@@ -7,13 +7,16 @@
 // What bounds it: at one token latency (expert id -> address -> weights -> results), then the vector ALU (decode, product and sum of
 // a weight in f32).  That kernel reads a weight's bytes one by one in the order of their use, a workgroup per output element.  Here:
 //   * Workgroup = 8 waves, 8 weight rows: wave = virtual wave x half of the rows, so that a fetched activation serves four rows.
-//   * All that a wave will read (its slots' activations and, per slot, four rows, which lie one behind another) is requested at once
-//     with direct-to-LDS loads; at most 32 units (256 weights of a slot) a token, 50 - 104 KB of LDS.
+//   * What a wave will read (its slots' activations and, per slot, four rows, which lie one behind another) is requested at once
+//     with direct-to-LDS loads, as many slots as fit (mix_depth); a slot that has been read makes room for the next.
 //   * Weights are decoded from words in LDS instead of bytes from memory.
 //   * A row's last 32 groups of 8, where K is an odd multiple of 256, would idle half of the lanes: they take two rows at once.
 // us, top-8 on 128 experts of 2048 x 768, one token (without tiles): q6_k 7.6 (12.7), q4_k 7.7 (14.6), q8_0 7.6 (9.4); of q6_k's 9.6 before,
-// 8-byte reads of half-word alignment were 1.1 and the idle lanes 0.6.  32 experts of 4096 x 2048, top-4, q6_k, a workgroup per CU and
-// two rounds of them, 15.4 (20.5).  From two tokens on kq_mix_stream's matrix instructions are ahead, 4096 x 2048 10.2 at one token.
+// 8-byte reads of half-word alignment were 1.1 and the idle lanes 0.6.  Longer slots, 64 experts: top-8 of 4096 x 1536 q6_k 15.4 (28.4),
+// q4_k 15.8 (35.3); top-4 of 4096 x 2816 mxfp4 16.7 (26.8); top-2 of 4096 x 4096 q6_k 23.0 (26.3).  The streamed kernel's matrix
+// instructions would take 10 us for the 33 M weights of 4096 x 2048 top-4 (here q6_k 15.7), in less precise sums.
+#include <algorithm>
+
 #include "kq_decode.h"
 #include "kq_dma.h"
 #include "kq_epilogue.h"
@@ -23,7 +26,7 @@ namespace {
 using namespace kqdma;
 
 constexpr int MX_CLASSES = 4, MX_HALVES = 2, MX_WAVES = MX_CLASSES * MX_HALVES, MX_R = 4, MX_ROWS = MX_R * MX_HALVES;
-constexpr int MX_UNITS = 32;  // units of 256 weights a token: S K / 256
+constexpr int MX_LDS = 160 * 1024 - (int)sizeof(float) * MX_CLASSES * MX_ROWS;
 
 struct MixArgs {
   const uint16_t* x;       // [T][S][K]
@@ -35,6 +38,7 @@ struct MixArgs {
   void* out;               // [T][N]
   const uint8_t* grids;
   int S, routed, E, N, K, tiles;
+  int depth;               // regions of a wave: slots under way at once
   int64_t w_expert_stride;
 };
 
@@ -44,7 +48,7 @@ constexpr int mix_grid_bytes() { return C == KQ_IQ3_S || C == KQ_IQ2_XXS ? 2048 
 template <int C>
 constexpr int mix_grid_at() { return C == KQ_IQ3_S ? KQ_GRID_IQ3S : KQ_GRID_IQ2XXS; }
 
-// LDS of a wave and slot: the slot's activations, four rows of weights, what 16-byte alignment adds and what words8 reads past them
+// A region, LDS of a wave and slot: the slot's activations, four rows of weights, what 16-byte alignment adds and what words8 reads past them
 __host__ __device__ constexpr int mix_region(int K, int row_bytes) { return 2 * K + ((MX_R * row_bytes + 15) & ~15) + 32; }
 
 // 8 bytes of a codec's block.  Blocks of no whole number of words: from the three words that hold them (an 8-byte LDS read of
@@ -257,13 +261,16 @@ __global__ __launch_bounds__(64 * MX_WAVES, 4) void mix_kernel(MixArgs a) {
       for (int o = 0; o < mix_grid_bytes<C>(); o += 1024)
         dma16(a.grids + mix_grid_at<C>() + o, 16 * lane, lds0 + wave * mix_grid_bytes<C>() + o);
     }
-    auto region_of = [&](int u) { return first + (uint32_t)((cls + MX_CLASSES * u) * MX_HALVES + half) * region; };
-    for (int u = 0; u < nsl; u++) {
+    const int classes = S < MX_CLASSES ? S : MX_CLASSES, depth = a.depth;
+    auto region_of = [&](int u) { return first + (uint32_t)((half * classes + cls) * depth + (u < depth ? u : u % depth)) * region; };
+    auto request_x = [&](int u) {
       const uint32_t to = lds0 + region_of(u);
       const uint8_t* xs = uniform(a.x + ((size_t)t * S + cls + MX_CLASSES * u) * K);
       for (int o = 0; o < K / 8; o += 64)
         if (o + lane < K / 8) dma16(xs, 16 * (o + lane), to + 16 * o);
-    }
+    };
+    const int ahead = nsl < depth ? nsl : depth;
+    for (int u = 0; u < ahead; u++) request_x(u);
     // The rows of a slot are one run of bytes.  Fetched in 16-byte pieces: from the aligned address in front of it, where the matrix
     // has bytes in front and behind; the matrix's first rows from their start, its last up to their end.
     const uint32_t run = MX_R * row_bytes;
@@ -272,22 +279,22 @@ __global__ __launch_bounds__(64 * MX_WAVES, 4) void mix_kernel(MixArgs a) {
       lead = row0 == 0 ? 0 : row0 + MX_R < N ? (uint32_t)reinterpret_cast<uintptr_t>(p) & 15 : (0u - run) & 15;
       return p - lead;
     };
-    for (int u = 0; u < nsl; u++) {
+    auto request_w = [&](int u) {
       const uint32_t to = lds0 + region_of(u);
       uint32_t lead;
       const uint8_t* p = uniform(run_of(expert(u), lead));
       const int pieces = (int)((lead + run + 15) / 16);
       for (int o = 0; o < pieces; o += 64)
         if (o + lane < pieces) dma16(p, 16 * (o + lane), to + 2 * K + 16 * o);
-    }
+    };
+    for (int u = 0; u < ahead; u++) request_w(u);
     const int slot_loads = (int)((run + 1023) / 1024);  // of a slot, or one more
 
     float tot[MX_R] = {};
-    const int ngroups = K / 8, whole = ngroups & ~63, g = lane % GPB;  // ngroups: a multiple of 32
+    const int ngroups = K / 8, whole = ngroups & ~63, g = lane % GPB;
     for (int u = 0; u < nsl; u++) {
-      wait_younger((nsl - 1 - u) * slot_loads);
+      wait_younger(((u + depth < nsl ? u + depth : nsl) - 1 - u) * slot_loads);
       const uint32_t e = expert(u);
-      if (e == ~1u) continue;
       uint32_t lead;
       run_of(e, lead);
       const uint8_t* xs = smem + region_of(u);
@@ -318,8 +325,8 @@ __global__ __launch_bounds__(64 * MX_WAVES, 4) void mix_kernel(MixArgs a) {
       };
       const uint8_t* at = ws + (lane / GPB) * BPB;
       for (int gi = lane; gi < whole; gi += 64, at += 64 / GPB * BPB) add(at, row_bytes, gi, v);
-      if (whole < ngroups) {
-        // the 32 groups left over, lanes 0 .. 31: the upper half of the lanes takes them for every other row
+      if (ngroups - whole == 32) {
+        // the groups left over, of lanes 0 .. 31: the upper half of the lanes takes them for every other row
         const int l32 = lane & 31;
         const uint8_t* tail = ws + (lane >> 5) * row_bytes + (whole / GPB + l32 / GPB) * BPB;
         float lo[MX_R / 2], hi[MX_R / 2];  // rows 2 p and 2 p + 1: their lanes 0 .. 31, 32 .. 63
@@ -328,9 +335,18 @@ __global__ __launch_bounds__(64 * MX_WAVES, 4) void mix_kernel(MixArgs a) {
         add(tail, 2 * row_bytes, whole + l32, lo);
 #pragma unroll
         for (int p = 0; p < MX_R / 2; p++) swap_halves(lo[p], hi[p], v[2 * p], v[2 * p + 1]);
+      } else if (whole + lane < ngroups) {
+        add(at, row_bytes, whole + lane, v);
       }
+      if (e != ~1u) {
 #pragma unroll
-      for (int r = 0; r < MX_R; r++) tot[r] = fmaf(score_of(u), v[r], tot[r]);
+        for (int r = 0; r < MX_R; r++) tot[r] = fmaf(score_of(u), v[r], tot[r]);
+      }
+      if (u + depth < nsl) {
+        lgkm_drain();  // the region has been read
+        request_x(u + depth);
+        request_w(u + depth);
+      }
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1)
@@ -357,14 +373,23 @@ __global__ __launch_bounds__(64 * MX_WAVES, 4) void mix_kernel(MixArgs a) {
   }
 }
 
+// Regions per wave: all of its slots under way at once where they fit, fewer where that lets a second workgroup onto the CU that
+// waits for one (64 experts of 4096 x 1024, top-8, 512 workgroups, us with all under way / with one: q8_0 14.0 / 9.9, q6_k 15.1 / 11.8);
+// 0: not even one fits.
+int mix_depth(int T, int S, int N, int K, int row_bytes, int grid_bytes) {
+  const int waves = MX_HALVES * std::min(S, MX_CLASSES), slots = (S + MX_CLASSES - 1) / MX_CLASSES, each = waves * mix_region(K, row_bytes);
+  const int fit = (MX_LDS - MX_WAVES * grid_bytes) / each, shared = (MX_LDS / 2 - MX_WAVES * grid_bytes) / each;
+  const bool crowded = (int64_t)T * (N / MX_ROWS) > kq_num_cus();
+  return std::min(slots, crowded && shared >= 1 ? shared : fit);
+}
+
 template <int C, int DT>
-int launch(const MixArgs& a, int T, hipStream_t s) {
-  constexpr int MAX_LDS = 160 * 1024 - (int)sizeof(float) * MX_CLASSES * MX_ROWS;
+int launch(MixArgs a, int T, hipStream_t s) {
   const int row_bytes = a.K / kq_geom(C).wpb * kq_geom(C).bpb;
-  const size_t lds = MX_WAVES * mix_grid_bytes<C>() + (size_t)a.S * MX_HALVES * mix_region(a.K, row_bytes);
-  if (lds > MAX_LDS) return KQ_ERR_UNSUPPORTED;
+  a.depth = mix_depth(T, a.S, a.N, a.K, row_bytes, mix_grid_bytes<C>());
+  const size_t lds = MX_WAVES * mix_grid_bytes<C>() + (size_t)MX_HALVES * std::min(a.S, MX_CLASSES) * a.depth * mix_region(a.K, row_bytes);
   auto kern = mix_kernel<C, DT>;
-  KQ_SET_MAX_LDS_ONCE((kern), MAX_LDS);
+  KQ_SET_MAX_LDS_ONCE((kern), MX_LDS);
   hipLaunchKernelGGL(kern, dim3((unsigned)(T * a.tiles)), dim3(64 * MX_WAVES), lds, s, a);
   KQ_HIP_CHECK(hipGetLastError());
   return KQ_OK;
@@ -373,14 +398,19 @@ int launch(const MixArgs& a, int T, hipStream_t s) {
 }  // namespace
 
 bool kq_mix_fits(int S, int N, int K, int codec) {
+  int grid_bytes = 0;
   switch (codec) {
-    case KQ_Q2_K: case KQ_Q3_K: case KQ_Q4_K: case KQ_Q5_K: case KQ_Q6_K: case KQ_IQ4_XS: case KQ_IQ3_S: case KQ_IQ2_XXS:
-    case KQ_Q8_0: case KQ_IQ4_NL: case KQ_Q4_0: case KQ_MXFP4: case KQ_NVFP4:
+    case KQ_IQ3_S: grid_bytes = mix_grid_bytes<KQ_IQ3_S>(); break;
+    case KQ_IQ2_XXS: grid_bytes = mix_grid_bytes<KQ_IQ2_XXS>(); break;
+    case KQ_Q2_K: case KQ_Q3_K: case KQ_Q4_K: case KQ_Q5_K: case KQ_Q6_K: case KQ_IQ4_XS: case KQ_Q8_0: case KQ_IQ4_NL: case KQ_Q4_0:
+    case KQ_MXFP4: case KQ_NVFP4:
       break;
     default:
       return false;
   }
-  return N % MX_ROWS == 0 && K >= 256 && (K & 255) == 0 && S >= 1 && (int64_t)S * (K >> 8) <= MX_UNITS;
+  const KqGeom geom = kq_geom(codec);
+  if (S < 1 || S > 32 || N < MX_ROWS || N % MX_ROWS || K < geom.wpb || K % geom.wpb || K > MX_LDS / 2) return false;
+  return mix_depth(1, S, N, K, K / geom.wpb * geom.bpb, grid_bytes) >= 1;
 }
 
 int kq_launch_mix(const void* x, const uint8_t* w, const uint8_t* shexp_w, const uint32_t* idx, const float* scores, const float* bias,

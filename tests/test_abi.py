@@ -158,3 +158,17 @@ def test_fused_moe_segments_follow_the_routing(lib):
     assert rows("q4_k", 44, E=32, N=2048, K=512) == 32  # short K
     assert rows("q5_k", 44, R=2, E=2) == 32             # too few workgroups
     assert lib.kq_moe_segment_rows(125, 8, 8, 768, 2048, 1, lib.kq_codec_id(b"q8_0")) == 0
+
+
+@pytest.mark.parametrize("codec,S,N,K", [("q6_k", 8, 2048, 768), ("q4_k", 8, 2048, 1536), ("q4_k", 2, 4096, 14336), ("mxfp4", 4, 2880, 2880),
+                                         ("q8_0", 32, 2048, 2048), ("iq1_s", 8, 2048, 2048)])
+def test_mix_of_one_token_needs_no_workspace(lib, codec, S, N, K):
+    """One token without a shared expert, up to 32 slots of any length; up to three with one; more of either need it."""
+    f = lib.kq_gather_qmv_mix_workspace_size
+    f.restype = C.c_size_t
+    c = lib.kq_codec_id(codec.encode())
+    assert f(1, S, 64, N, K, c, -1, 2) == 0
+    assert f(3, S, 64, N, K, c, c, 2) == 0
+    assert f(2, S, 64, N, K, c, -1, 2) > 0
+    assert f(4, S, 64, N, K, c, c, 2) > 0
+    assert f(1, 33, 64, N, K, c, -1, 2) > 0

@@ -132,6 +132,36 @@ def test_sums_are_those_of_the_kernel_without_tiles(codec, T, S, N, K, shared):
     assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (codec, float((got != want).float().mean()))
 
 
+@pytest.mark.parametrize("codec,S,N,K", [(c, 8, 40, 2048) for c in STREAMED] + [
+    ("q4_k", 2, 16, 4096), ("q8_0", 5, 24, 3584), ("q6_k", 13, 8, 2304),  # as many slots under way as the LDS holds, and one
+    ("mxfp4", 4, 48, 2880), ("q8_0", 4, 16, 2880), ("iq4_nl", 9, 24, 736), ("q4_0", 3, 8, 32), ("nvfp4", 3, 16, 1728),
+    ("q4_k", 3, 16, 8192), ("q5_1", 3, 16, 736)])  # (the kernel without tiles)
+def test_one_token_needs_no_workspace(codec, S, N, K):
+    """Any row length, by the C entry point with a null workspace."""
+    w, _, idx, scores = case(codec, 1, S, 3, N, K, 380)
+    idx[0, -1] = 2
+    xb, xt = make_x((1, S, K), "bfloat16", seed=381, scale=0.05)
+    args = (wire_to_dev(w), None, codec, _idx_dev(idx).to(torch.int32), torch.from_numpy(scores).cuda())
+    got = c_call(xt, *args)
+    assert rel_l2(dev_to_bits(got), O.gather_qmv_mix(xb, w, None, codec, None, idx, scores, "bfloat16"), "bfloat16") <= TOL
+    assert torch.equal(got.view(torch.int16), c_call(unaligned(xt), *args).view(torch.int16))
+
+
+@pytest.mark.parametrize("codec", STREAMED)
+def test_one_token_of_long_slots_and_wide_range(codec):
+    """A large value over a zero weight beside tiny ones that are the result, 64 units a token: within the roundings to bf16."""
+    S, E, N, K = 8, 3, 40, 2048
+    wpb, bpb = O.geometry(codec)
+    w, _, idx, scores = case(codec, 1, S, E, N, K, 390)
+    w.reshape(E, N, K // wpb, bpb)[:, :, 0] = 0
+    x = torch.randn((1, S, K), generator=torch.Generator().manual_seed(391)) * 1e-12
+    x[0, :, 0] = 1e30
+    xt = x.to(torch.bfloat16)
+    got = dev_to_bits(run(xt.cuda(), w, None, codec, idx, scores))
+    want = O.gather_qmv_mix(xt.view(torch.int16).numpy().view("uint16"), w, None, codec, None, idx, scores, "bfloat16")
+    assert row_errors(got, want) <= 2.0**-8, codec
+
+
 @pytest.mark.parametrize("codec", ["q4_k", "q6_k", "q8_0"])
 def test_infinite_activation(codec):
     """An infinity times a weight is an infinity of the weight's sign, as in the kernel without tiles."""
