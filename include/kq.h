@@ -131,10 +131,8 @@ void kq_set_gemm_tile_rows(int rows);
  * 5 = same as 0.  Process-wide, not thread-safe. */
 void kq_set_skinny_variant(int variant);
 
-/* Query without a counterpart in the reference: 32 or 64, the better number of pairs per segment for a kernel that
- * multiplies one or two blocks of 32 pairs per decoded weight, for a K-quant MoE call of T tokens with R experts each; 0 if
- * the grouped kernels do not take the call.  glu: the fused gate / up op.  The calls themselves run in segments of 32 pairs
- * or, from about two dozen pairs per expert on, of up to 96. */
+/* Query without a counterpart in the reference: pairs per segment at most, 32 or 96, with which the expert-grouped K-quant
+ * kernels run a call of T tokens with R experts each; 0 if they do not take it.  glu: the fused gate / up op. */
 int kq_moe_segment_rows(int T, int R, int E, int N, int K, int glu, int codec);
 
 /* out[b] = x[lhs[b]] . W[rhs[b]]^T for b < B; x batches are [M,K] matrices

@@ -12,7 +12,6 @@
 // rows (converted to f16 by the activation prepass) are fetched one step ahead with coalesced
 // 16-byte loads and parked in LDS.
 #include <algorithm>
-#include <cmath>
 
 #include "kq_epilogue.h"
 #include "kq_mma.h"
@@ -439,22 +438,6 @@ __global__ __launch_bounds__(MOE_THREADS, 3) void moe_grouped_kernel(MoeArgs a) 
   }
 }
 
-// Segments of `seg` pairs that an expert makes on average when every token picks R of E experts evenly, `mean` pairs for each:
-// the sum over k of the chance of more than k seg pairs (normal approximation of the binomial count).
-double moe_mean_segments(double mean, int R, int E, int seg) {
-  const double sd = std::sqrt(mean * (1.0 - (double)std::min(R, E) / E)) + 1e-9, top = mean + 6 * sd;
-  int k = (int)std::max(0.0, (mean - 6 * sd) / seg);
-  double n = k;
-  for (; k * seg < top + 1; k++) n += 0.5 * std::erfc((k * seg + 0.5 - mean) / (sd * 1.4142135623730951));
-  return n;
-}
-// Rounds of workgroups, ntiles to a segment, over the chip's slots: the second one costs nearly a whole one however short
-// (if there is one: less than a segment beyond the first is the chance of one), later ones even out.
-double moe_rounds(double wgs, int slots, int ntiles) {
-  const double x = wgs / slots, c = std::ceil(x);
-  return x <= 1 ? 1 : x + (c == 2 ? 0.75 : 0.25) * (c - x) * std::min(1.0, (wgs - (c - 1) * slots) / ntiles);
-}
-
 // Whether a call runs in segments of up to 96 pairs: from 22 pairs per expert (fused) or 28 (plain) on, the plain one only if its
 // workgroups fill the chip or there are 48 pairs.  us on 32- and 64-pair segments, single stage in LDS / on those of 96: 128 experts of 2048 <-> 768
 // top 8, fused q4_k 16 pairs per expert 69.1 / 69.8, 24 77.0 / 73.9, 62 144 / 107, q6_k 62 210 / 154; plain q4_k 24 46.7 / 49.9, 32
@@ -463,19 +446,6 @@ double moe_rounds(double wgs, int slots, int ntiles) {
 bool moe_tile_takes(int P, int E, int N, bool glu) {
   if (glu) return P >= 22 * (int64_t)E;
   return P >= 28 * (int64_t)E && ((int64_t)std::max(E, P / KQ_MOE_TILE_SEG) * ((N + SLAB - 1) / SLAB) >= 256 || P >= 48 * (int64_t)E);
-}
-
-// What kq_moe_segment_rows answers: the better one of 32 and 64 pairs per segment, by the segments that an even routing leaves
-// (62 pairs per expert make 1.4 of 64 or 2.4 of 32; 44 make 1.0 or 2.0), the workgroups' rounds and the weight of the decode.
-int moe_seg_rows(int P, int R, int E, int N, int K, bool glu, int codec) {
-  const int ncols = glu ? SLAB / 2 : SLAB, ntiles = (N + ncols - 1) / ncols;
-  if ((int64_t)std::max(E, P / 64) * ntiles < 256 || P < (glu ? 28 : 32) * (int64_t)E) return 32;
-  const double mean = (double)P / E;
-  if (!glu || mean > 1024) return 64;
-  const double wgs64 = moe_mean_segments(mean, R, E, 64) * E * ntiles, wgs32 = moe_mean_segments(mean, R, E, 32) * E * ntiles;
-  if (wgs32 < 1.2 * wgs64) return 32;  // hardly an expert with a second segment to save
-  const double per_round = (codec == KQ_Q4_K ? 1.01 : codec == KQ_Q5_K ? 0.91 : 0.90) * std::sqrt(1 + 512.0 / K);
-  return per_round * moe_rounds(wgs64, 2 * 256, ntiles) <= 0.98 * moe_rounds(wgs32, 3 * 256, ntiles) ? 64 : 32;
 }
 
 struct MoeWorkspace {
@@ -617,7 +587,8 @@ bool kq_moe_grouped_supported(int P, int E, int N, int K, int codec) {
 }
 
 extern "C" int kq_moe_segment_rows(int T, int R, int E, int N, int K, int glu, int codec) {
-  return kq_moe_grouped_supported(T * R, E, N, K, codec) ? moe_seg_rows(T * R, R, E, N, K, glu != 0, codec) : 0;
+  if (!kq_moe_grouped_supported(T * R, E, N, K, codec)) return 0;
+  return moe_tile_takes(T * R, E, N, glu != 0) ? KQ_MOE_TILE_SEG : SEG_M;
 }
 
 // rows = activation rows the prepass converts: T for the GLU op (x is [T,K]), T*R for the down op.

@@ -146,18 +146,17 @@ def test_transposed_product_takes_256_row_tiles_where_they_fill(lib, codec, M, N
     assert lib.kq_qmm_workspace_size(M, N, K, 0, lib.kq_codec_id(codec.encode()), 2) == ranges * M * N * 4
 
 
-def test_fused_moe_segments_follow_the_routing(lib):
-    """64-pair segments of the fused op by the segments that an even routing leaves: at 44 pairs per expert one instead of two,
-    at 64 and 76 about half of the experts a short second one, at 112 again two instead of four; heavier decodes sooner."""
-    def rows(codec, ppe, R=8, E=128, N=768, K=2048):
-        return lib.kq_moe_segment_rows(ppe * E // R, R, E, N, K, 1, lib.kq_codec_id(codec.encode()))
+def moe_segments(lib, codec, ppe, glu, E=128, N=768, K=2048, R=8):
+    return lib.kq_moe_segment_rows(ppe * E // R, R, E, N, K, glu, lib.kq_codec_id(codec.encode()))
 
-    assert [rows("q4_k", p) for p in (24, 30, 44, 76, 112, 200)] == [32, 32, 64, 32, 64, 64]
-    assert [rows("q6_k", p) for p in (24, 30, 44, 62, 92, 200)] == [32, 32, 64, 64, 64, 64]
-    assert [rows("q4_k", p, R=8, E=8, N=4096) for p in (64, 92, 128)] == [64, 32, 64]  # every expert has every token
-    assert rows("q4_k", 44, E=32, N=2048, K=512) == 32  # short K
-    assert rows("q5_k", 44, R=2, E=2) == 32             # too few workgroups
-    assert lib.kq_moe_segment_rows(125, 8, 8, 768, 2048, 1, lib.kq_codec_id(b"q8_0")) == 0
+
+@pytest.mark.parametrize("codec", ["q4_k", "q5_k", "q6_k"])
+def test_moe_segments_by_pairs_per_expert(lib, codec):
+    """In which segments the launcher runs a call: 32 pairs or up to 96, on both sides of its lines."""
+    assert [moe_segments(lib, codec, p, 1) for p in (4, 21, 22, 62, 250)] == [32, 32, 96, 96, 96]
+    assert [moe_segments(lib, codec, p, 0, N=2048, K=768) for p in (4, 27, 28, 62, 250)] == [32, 32, 96, 96, 96]
+    assert moe_segments(lib, "q8_0", 62, 1) == 0  # not theirs
+    assert moe_segments(lib, codec, 1, 1, E=16) == 0  # too few pairs for the grouped kernels
 
 
 @pytest.mark.parametrize("codec,S,N,K", [("q6_k", 8, 2048, 768), ("q4_k", 8, 2048, 1536), ("q4_k", 2, 4096, 14336), ("mxfp4", 4, 2880, 2880),

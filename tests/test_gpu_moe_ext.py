@@ -103,12 +103,12 @@ def _segment_rows(kq, codec, T, R, E, N, K, glu):
 
 
 @pytest.mark.parametrize("codec", ["q4_k", "q5_k", "q6_k"])
-@pytest.mark.parametrize("T,S,E,N", [(90, 2, 3, 11008),   # 60 pairs per expert: segments of 33 to 64 pairs, one of a few
-                                     (64, 2, 2, 16384),   # exactly one full segment each
+@pytest.mark.parametrize("T,S,E,N", [(90, 2, 3, 11008),   # 60 pairs per expert: segments of two blocks of 32
+                                     (96, 2, 2, 16384),   # exactly one full segment each
                                      (310, 7, 9, 1104)])  # more pairs than the sort keeps in registers
-def test_down_product_on_64_pair_segments(kq, codec, T, S, E, N):
+def test_down_product_on_96_pair_segments(kq, codec, T, S, E, N):
     K = 256
-    assert _segment_rows(kq, codec, T, S, E, N, K, False) == 64
+    assert _segment_rows(kq, codec, T, S, E, N, K, False) == 96
     w = _stack(codec, E, N, K, 71)
     rng = np.random.default_rng(73)
     idx = rng.permutation(np.arange(T * S) % E).reshape(T, S)
@@ -123,11 +123,11 @@ def test_down_product_on_64_pair_segments(kq, codec, T, S, E, N):
 @pytest.mark.parametrize("codec,act,dtype", [("q4_k", "silu", "bfloat16"), ("q4_k", "gelu", "float16"),
                                              ("q5_k", "silu", "float16"), ("q6_k", "gelu", "bfloat16")])
 @pytest.mark.parametrize("N", [4096, 4088])
-def test_fused_op_on_64_pair_segments(kq, codec, act, dtype, N):
-    """44 pairs per expert on average: one expert with 100 (a full segment and one of 36), one with 64, one with none, the
+def test_fused_op_on_96_pair_segments(kq, codec, act, dtype, N):
+    """44 pairs per expert on average: one expert with 100 (segments of 64 and 36), one with 64, one with none, the
     others below and above 32."""
     T, R, E, K = 44, 8, 8, 256
-    assert _segment_rows(kq, codec, T, R, E, N, K, True) == 64
+    assert _segment_rows(kq, codec, T, R, E, N, K, True) == 96
     counts = [100, 64, 0, 63, 65, 33, 26, 1]
     idx = np.random.default_rng(76).permutation(np.repeat(np.arange(E), counts)).reshape(T, R)
     w, w2 = _stack(codec, E, N, K, 77), _stack(codec, E, N, K, 78)
