@@ -12,6 +12,7 @@
 // rows (converted to f16 by the activation prepass) are fetched one step ahead with coalesced
 // 16-byte loads and parked in LDS.
 #include <algorithm>
+#include <cmath>
 
 #include "kq_epilogue.h"
 #include "kq_mma.h"
@@ -438,14 +439,34 @@ __global__ __launch_bounds__(MOE_THREADS, 3) void moe_grouped_kernel(MoeArgs a) 
   }
 }
 
-// Whether a call runs in segments of up to 96 pairs: from 22 pairs per expert (fused) or 28 (plain) on, the plain one only if its
-// workgroups fill the chip or there are 48 pairs.  us on 32- and 64-pair segments, single stage in LDS / on those of 96: 128 experts of 2048 <-> 768
-// top 8, fused q4_k 16 pairs per expert 69.1 / 69.8, 24 77.0 / 73.9, 62 144 / 107, q6_k 62 210 / 154; plain q4_k 24 46.7 / 49.9, 32
-// 60.2 / 57.2, 62 93.6 / 80.6, q6_k 24 70.7 / 66.7, 62 126 / 100; 8 of 2048 <-> 4096 top 2, plain, 128 workgroups, 32 29.5 / 32.7,
-// 64 41.8 / 40.5, 250 85.7 / 69.3, fused 250 149 / 103; 64 of 1024 <-> 2048 top 6, fused 24 54.5 / 55.7, 94 143 / 105.
-bool moe_tile_takes(int P, int E, int N, bool glu) {
-  if (glu) return P >= 22 * (int64_t)E;
-  return P >= 28 * (int64_t)E && ((int64_t)std::max(E, P / KQ_MOE_TILE_SEG) * ((N + SLAB - 1) / SLAB) >= 256 || P >= 48 * (int64_t)E);
+// Segments of `seg` pairs that an expert makes on average when every token picks R of E experts evenly, `mean` pairs for each:
+// the sum over k of the chance of more than k seg pairs (normal approximation of the binomial count).
+double moe_mean_segments(double mean, int R, int E, int seg) {
+  const double sd = std::sqrt(mean * (1.0 - (double)std::min(R, E) / E)) + 1e-9, top = mean + 6 * sd;
+  int k = (int)std::max(0.0, (mean - 6 * sd) / seg);
+  double n = k;
+  for (; k * (double)seg < top + 1; k++) n += 0.5 * std::erfc((k * (double)seg + 0.5 - mean) / (sd * 1.4142135623730951));
+  return n;
+}
+
+// Whether a call runs in segments of up to 96 pairs.  Only from 22 pairs per expert (fused) or 28 (plain) on: us on 32- or 64-pair segments,
+// single stage in LDS / on those of 96: 128 experts of 2048 <-> 768 top 8, fused q4_k 16 pairs per expert 69.1 / 69.8, 24 77.0 / 73.9, 62
+// 144 / 107, q6_k 62 210 / 154; plain q4_k 24 46.7 / 49.9, 32 60.2 / 57.2, 62 93.6 / 80.6, q6_k 24 70.7 / 66.7, 62 126 / 100.
+// And not where the 32-pair segments, dealt to the eight XCDs in turn, leave the CUs of the busiest one a workgroup each at most: nothing is
+// then saved by fewer and longer ones.  Fused, 8 experts of 2048 -> 512, q4_k 32 / 64 / 96 / 128 pairs per expert (12 ... 40 of 32 CUs'
+// worth) 1.08 / 1.24 / 1.25 / 0.96 of the time on 32-pair segments, 4096 -> 512 1.09 / 1.28 / 1.30 / 0.98, 2048 -> 768 1.09 / 0.96 / 0.98 / 0.96; 8 of 2048 <-
+// 1536, plain, 64 pairs, q4_k 1.03, q6_k 0.92, 8 of 1024 <- 1536 1.30, 1.29.  The plain q4_k op, whose decode is the lightest, asks for half
+// as many again or for 96-pair segments that fill the chip (16 of 1024 <- 1536, 64 pairs: 1.04; 16 of 2048 <- 1536, 32: 0.87).  Over
+// 432 fused and 540 plain calls of 4 ... 32 experts the choice is 0.2 and 0.4 % behind the better form (without the second condition
+// 1.8 and 5 %).
+bool moe_tile_takes(int P, int R, int E, int N, bool glu, int codec) {
+  if (P < (glu ? 22 : 28) * (int64_t)E) return false;
+  const int ncols = glu ? SLAB / 2 : SLAB, ntiles = (N + ncols - 1) / ncols, cus = kq_num_cus() / 8;
+  // workgroups of the busiest XCD (half a segment beyond whole rounds of eight is taken as chance)
+  auto busiest = [&](int seg) { return std::ceil((E * moe_mean_segments((double)P / E, R, E, seg) - 0.5) / 8) * ntiles; };
+  const double wgs = busiest(SEG_M);
+  if (wgs <= cus) return false;
+  return glu || codec != KQ_Q4_K || wgs > 1.5 * cus || busiest(KQ_MOE_TILE_SEG) >= cus;
 }
 
 struct MoeWorkspace {
@@ -588,7 +609,7 @@ bool kq_moe_grouped_supported(int P, int E, int N, int K, int codec) {
 
 extern "C" int kq_moe_segment_rows(int T, int R, int E, int N, int K, int glu, int codec) {
   if (!kq_moe_grouped_supported(T * R, E, N, K, codec)) return 0;
-  return moe_tile_takes(T * R, E, N, glu != 0) ? KQ_MOE_TILE_SEG : SEG_M;
+  return moe_tile_takes(T * R, glu ? R : 1, E, N, glu != 0, codec) ? KQ_MOE_TILE_SEG : SEG_M;
 }
 
 // rows = activation rows the prepass converts: T for the GLU op (x is [T,K]), T*R for the down op.
@@ -605,7 +626,7 @@ int kq_launch_moe_grouped(const void* x, const uint8_t* w, const uint8_t* w2, co
       (reinterpret_cast<uintptr_t>(ws) & 255))
     return KQ_ERR_UNSUPPORTED;
   const MoeWorkspace m = carve(ws, rows, P, E, K);
-  const bool tile = moe_tile_takes(P, E, N, glu != 0);
+  const bool tile = moe_tile_takes(P, P / std::max(rows, 1), E, N, glu != 0, codec);
   const int seg_rows = tile ? KQ_MOE_TILE_SEG : SEG_M;
   if (dtype == KQ_F16)
     hipLaunchKernelGGL(moe_prologue_kernel<KQ_F16>, dim3(rows + 1), dim3(PP_THREADS), 0, s, static_cast<const uint16_t*>(x),

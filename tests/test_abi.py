@@ -155,6 +155,12 @@ def test_moe_segments_by_pairs_per_expert(lib, codec):
     """In which segments the launcher runs a call: 32 pairs or up to 96, on both sides of its lines."""
     assert [moe_segments(lib, codec, p, 1) for p in (4, 21, 22, 62, 250)] == [32, 32, 96, 96, 96]
     assert [moe_segments(lib, codec, p, 0, N=2048, K=768) for p in (4, 27, 28, 62, 250)] == [32, 32, 96, 96, 96]
+    # nothing to save where the 32-pair segments are a workgroup per CU: 8 experts of 2048 -> 512, 1536 and back
+    assert [moe_segments(lib, codec, p, 1, E=8, N=512, R=2) for p in (32, 64, 96, 140)] == [32, 32, 32, 96]
+    assert [moe_segments(lib, codec, p, 1, E=8, N=1536, R=2) for p in (32, 64)] == [96, 96]
+    assert [moe_segments(lib, codec, p, 0, E=8, N=1024, K=512, R=2) for p in (32, 64, 96)] == [32, 32, 32]
+    assert [moe_segments(lib, codec, p, 0, E=8, N=2048, K=1536, R=2) for p in (40, 64, 96, 128)] == [32, 32 if codec == "q4_k" else 96, 96, 96]
+    assert [moe_segments(lib, codec, p, 0, E=16, N=2048, K=1536, R=2) for p in (32, 64)] == [96, 96]
     assert moe_segments(lib, "q8_0", 62, 1) == 0  # not theirs
     assert moe_segments(lib, codec, 1, 1, E=16) == 0  # too few pairs for the grouped kernels
 

@@ -15,15 +15,22 @@ pytestmark = pytest.mark.gpu
 COUNTS = [96, 97, 64, 65, 32, 33, 1, 0, 200, 95, 193, 84]
 
 
+def takes(codec, idx, E, N, K, glu):
+    """The call runs on this kernel."""
+    lib = kq._load()
+    return lib.kq_moe_segment_rows(idx.shape[0], idx.shape[1], E, N, K, glu, lib.kq_codec_id(codec.encode())) == 96
+
+
 def routing(counts, R, seed):
     idx = np.random.default_rng(seed).permutation(np.repeat(np.arange(len(counts)), counts))
     return idx[:len(idx) // R * R].reshape(-1, R)
 
 
 @pytest.mark.parametrize("codec", ["q4_k", "q5_k", "q6_k"])
-@pytest.mark.parametrize("N,K,act,dtype", [(72, 256, "silu", "bfloat16"), (200, 512, "gelu", "float16"), (64, 1280, "silu", "float16")])
+@pytest.mark.parametrize("N,K,act,dtype", [(456, 256, "silu", "bfloat16"), (584, 512, "gelu", "float16"), (448, 1280, "silu", "float16")])
 def test_fused(codec, N, K, act, dtype):
     E, idx = len(COUNTS), routing(COUNTS, 4, 1)
+    assert takes(codec, idx, E, N, K, 1)
     w, w2 = _stack(codec, E, N, K, 2), _stack(codec, E, N, K, 3)
     xb, xt = make_x((idx.shape[0], K), dtype, seed=4, scale=0.05)
     got = kq.moe_glu_gather_kq(xt, wire_to_dev(w), wire_to_dev(w2), codec, _idx_dev(idx), act)
@@ -31,9 +38,10 @@ def test_fused(codec, N, K, act, dtype):
 
 
 @pytest.mark.parametrize("codec", ["q4_k", "q5_k", "q6_k"])
-@pytest.mark.parametrize("N,K,dtype", [(136, 256, "bfloat16"), (128, 768, "float16"), (248, 1280, "bfloat16")])
+@pytest.mark.parametrize("N,K,dtype", [(1288, 256, "bfloat16"), (1280, 768, "float16"), (1400, 1280, "bfloat16")])
 def test_plain(codec, N, K, dtype):
     E, idx = len(COUNTS), routing(COUNTS, 1, 5)
+    assert takes(codec, idx, E, N, K, 0)
     w = _stack(codec, E, N, K, 6)
     xb, xt = make_x((idx.shape[0], 1, K), dtype, seed=7, scale=0.05)
     got = kq.gather_qmv_kq(xt, wire_to_dev(w), codec, _idx_dev(idx))
@@ -43,8 +51,9 @@ def test_plain(codec, N, K, dtype):
 
 def test_mix_and_ids_outside():
     """The down projection's f32 slot rows; a slot whose id is outside the stack adds nothing."""
-    codec, E, N, K, S = "q6_k", 4, 136, 512, 4
+    codec, E, N, K, S = "q6_k", 4, 2056, 512, 4
     idx = routing([120, 96, 33, 151], S, 8)
+    assert takes(codec, idx, E, N, K, 0)
     w = _stack(codec, E, N, K, 9)
     scores = np.random.default_rng(10).uniform(0.05, 1.0, idx.shape).astype(np.float32)
     bad, zeroed = idx.copy(), scores.copy()
