@@ -61,3 +61,27 @@ def test_mix_and_ids_outside():
     xb, xt = make_x((idx.shape[0], S, K), "bfloat16", seed=11, scale=0.05)
     got = kq.gather_qmv_mix_ns_kq(xt, wire_to_dev(w), codec, _idx_dev(bad), torch.from_numpy(scores).cuda())
     assert rel_l2(dev_to_bits(got), O.gather_qmv_mix(xb, w, None, codec, None, idx, zeroed, "bfloat16"), "bfloat16") <= TOL
+
+
+@pytest.mark.parametrize("codec", ["q4_k", "q6_k"])
+@pytest.mark.parametrize("N,offset", [(1291, 0), (1409, 0), (1288, 1)])  # rows of no whole 16-byte pieces; an output off 16 bytes
+def test_results_stored_one_by_one(codec, N, offset):
+    """gather_qmm takes any N and any output address: every element of every row, and nothing behind the last one."""
+    E, K, idx = len(COUNTS), 256, routing(COUNTS, 1, 12)
+    assert takes(codec, idx, E, N, K, 0)
+    P = idx.shape[0]
+    w = _stack(codec, E, N, K, 13)
+    xb, xt = make_x((P, 1, K), "bfloat16", seed=14, scale=0.05)
+    wd, lhs, rhs = wire_to_dev(w), torch.arange(P, dtype=torch.int32, device="cuda"), _idx_dev(idx[:, 0]).to(torch.int32)
+    buf = torch.full((P * N + 64,), 7.0, dtype=torch.bfloat16, device="cuda")
+    lib, c = kq._load(), kq._load().kq_codec_id(codec.encode())
+    need = lib.kq_gather_qmm_workspace_size(P, 1, E, N, K, 1, c, 2)
+    ws = torch.empty(need + 256, dtype=torch.uint8, device="cuda")
+    wp = -ws.data_ptr() % 256 + ws.data_ptr()
+    rc = lib.kq_gather_qmm(xt.data_ptr(), wd.data_ptr(), lhs.data_ptr(), rhs.data_ptr(), buf[offset:].data_ptr(), P, 1, E, N, K, K,
+                           wd[0].numel(), 1, 0, c, 2, wp, need, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.kq_last_error()
+    got = dev_to_bits(buf)
+    want = O.gather_qmm(xb, w, codec, np.arange(P), idx[:, 0], True, "bfloat16")
+    assert rel_l2(got[offset:offset + P * N].reshape(P, 1, N), want, "bfloat16") <= TOL
+    assert (got[:offset] == 0x40e0).all() and (got[offset + P * N:] == 0x40e0).all()
