@@ -115,10 +115,12 @@ int kq_qmv_bias(const void* x_dev, const void* w_dev, const void* bias_dev, void
  * column tile, 1025 = the 128 x 256 form of that kernel (q6_k only; other codecs fall back to automatic); for
  * q8_0 / q4_0 / q4_1 / q5_0 / q5_1 / iq4_nl / mxfp4 / nvfp4 and the codebook codecs (iq1 / iq2 / iq3), 1024 / 1025 force the 256- / 128-row form of their tall-tile kernels on any
  * shape of 128 rows or more and 64 keeps them on the any-codec kernel; 32 = the streamed kernel of 9 ... 512 activation
- * rows wherever it can run (every other forced shape switches it off);
- * anything else restores the automatic choice (q4_k / q5_k / q6_k with 256 rows or more: the 256 x 256 kernel on the
- * column tiles that fill whole rounds of one workgroup per CU, a 128 x 256 kernel on the rest; q6_k matrices of
- * few tiles stay on the 64-row kernel).
+ * rows wherever it can run; 33 = the kernel of 128-weight-row tiles (33 rows and more, K a multiple of 256 from 512 to 32768)
+ * wherever it can run (every other forced shape switches these two off);
+ * anything else restores the automatic choice: that kernel where it is ahead of the other two, else the streamed kernel for few rows,
+ * else the codec's tall tiles where they fill the chip (q4_k / q5_k / q6_k with 256 rows or more: the 256 x 256 kernel on
+ * the column tiles that fill whole rounds of one workgroup per CU, a 128 x 256 kernel on the rest; q6_k matrices of
+ * few tiles stay on the 64-row kernel), else the any-codec kernel.
  * Process-wide, not thread-safe. */
 void kq_set_gemm_tile_rows(int rows);
 /* Tuning hook without a counterpart in the reference: which skinny-M kernel dense calls use.
@@ -142,7 +144,7 @@ int kq_moe_segment_rows(int T, int R, int E, int N, int K, int glu, int codec);
  * skipped by the batched path and must not occur).  `rhs_sorted` != 0 promises rhs is
  * non-decreasing.  With a workspace of kq_gather_qmm_workspace_size bytes and more than 16 output
  * rows (B * M) the entries are grouped by expert on the device, so an expert's wire bytes are
- * streamed once per 32 rows instead of once per entry; without one every entry is computed on its own.
+ * streamed once per 32 rows (up to 96: kq_moe_segment_rows) instead of once per entry; without one every entry is computed on its own.
  * Replaces KQuantGatherQMM::eval_cpu, reference src/kquant_gather.cpp:470-746
  * (kquant_qmm_cpu_batch, src/kquant_cpu_decode.cpp:1361-1527). */
 size_t kq_gather_qmm_workspace_size(int B, int M, int E, int N, int K, int transpose, int codec, int dtype);
@@ -219,7 +221,8 @@ int kq_moe_glu_gather_shexp(const void* x_dev, const void* gate_w_dev, const voi
  * shexp_w_dev != NULL: idx is [T, S - 1], slot S - 1 multiplies the shared expert's single matrix (codec
  * `shexp_codec`: the expert codec, or q6_k / q8_0) -- op gather_qmv_mix_kq; shexp_w_dev == NULL: idx is
  * [T, S] and every slot gathers from the stack -- op gather_qmv_mix_ns_kq (pass shexp_codec = -1 to the
- * size query).  Decode-sized calls (one token; up to three with a shared expert; S <= 32) run as one kernel and
+ * size query).  Decode-sized calls (one token; up to three with a shared expert; S <= 32) run as one kernel, sum f32 products
+ * of the activations as they are and the decoded weights, and
  * need no workspace (the size query returns 0, any pointer is accepted); larger calls need the 256-byte aligned
  * workspace.  Entries whose expert id is >= E add nothing.
  * Replaces KQuantGatherQMVMixKQ / KQuantGatherQMVMixNSKQ, reference src/kquant_moe_glu.cpp:1274-1364. */

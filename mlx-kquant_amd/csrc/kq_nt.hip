@@ -745,7 +745,7 @@ int nt_ranges(int M, int N, int K, bool tall) {
 // 128-row tiles two run per CU, each half a step per 32 rows, and a last round evens out but for a quarter.  Measured / by this,
 // 256-row over 128-row kernel, middle of eight codecs, rows, reduction x outputs: 1800 4096 x 4096 0.73 / 0.96, 512 4096 x 4096 0.89 / 1.09,
 // 600 8192 x 2048 0.85 / 1.09, 768 4096 x 4096 0.87 / 1.13, 1024 2048 x 6144 0.88 / 1.18, 1500 2048 x 8192 1.08 / 1.20, 1400 4096 x 4096 0.97 /
-// 1.25, 8192 x 8192 1.05 / 1.25, 600 4096 x 4096 1.02 / 1.37, 4096 x 14336 1.09 / 1.52; the codecs lie within 5 % of that.  Ranges of
+// 1.25, 8192 x 8192 1.05 / 1.25, 600 4096 x 4096 1.02 / 1.37, 4096 x 14336 1.09 / 1.52; the codecs lie within 5 % of that (q3_k 8 % above at 600 rows of 4096 x 14336).  Ranges of
 // fewer than eight steps hardly leave the filling of the pipeline (2048 rows of 1024 x 1024, four steps, 1.09 / 1.33) and keep to 5 %, q2_k
 // and q4_1 to -5 %.  Never for the codebook codecs, whose table reads from eight waves decoding together make the 256-row
 // kernel 1.3 - 1.5 times the other (1.1 where it is best; both before activations went through LDS).

@@ -18,6 +18,12 @@
 // rows of 28672 x 8192 a pair of steps of all eight waves takes 5.2 us = 0.8 PFLOP/s; taking out the
 // activation loads, the wire loads, the LDS reads or the decode (timing only) gives 14, 7, 4 and 3 %: the stages add up.  A
 // workgroup's fixed cost is 8 us at NB = 4 (11 with 2-byte stores and row scales loaded between them).
+// Precision: exact f16 terms of the weights, f32 sums per scale block and of those.  Results that are not the correctly rounded ones,
+// bf16, 1024 rows of 2048 x 4096 N(0, 1) activations (any-codec kernel / tall tiles that had the calls): q3_k 0.02 % (0.23 / -), q4_1 and q5_1 0.025 (0.031 /
+// 0.049), q2_k 0.013 (0.034), mxfp4 0.006 (0.006 / 0.007), nvfp4 0.012 (0.010 / 0.013); q8_0, iq4_xs, iq3_s, iq1_m 0.01 - 0.02 (0.4 - 0.5).  A minimum's
+// products cancel against the codes' where activations have a mean: of 0.3, q4_1 / q5_1 0.07 (0.03 / 0.05), q2_k 0.04 (0.03).  Activations
+// are f16 under their row's power of two; of a bf16 row that does not count as wide one value in 4096 may have lost bits below 2^-31 of
+// its largest (RowRange of kq_mma.h; N(0, 1): one in 10^9), which the any-codec kernel keeps.
 #include <algorithm>
 #include <cmath>
 
