@@ -5,10 +5,13 @@
 //
 // What bounds it.  K-quants: the vector ALU.  A sub-block's fit tries 37 (scale, min) or 19 scale candidates, and the
 // order of its sums is part of the result, so a candidate is one lane's serial work: 15 (8) instructions per weight and
-// candidate that cannot be fused.  16.8 M weights of q4_k are 1.5e8 wave instructions = 240 us at the chip's issue rate,
-// against 32 us of memory traffic.  One lane per sub-block (8 or 16 per superblock) keeps all three arrays of a fit in
-// registers; one thread per superblock, the form this replaced, kept them in 2.4 KB of scratch per lane.  4096 x 4096
-// f32: q4_k 3527 -> 222 us (q5_k 261, q2_k 338, q3_k 82, q6_k 78).
+// candidate that cannot be fused.  The (scale, min) codecs evaluate one or two of the 37 and rule the others out by a bound
+// (fit_scale_min below): 210 instead of 660 instructions a weight, the SIMDs 95 % busy issuing them.  One lane per
+// sub-block (8 or 16 per superblock) keeps all three arrays of a fit in registers.  4096 x 4096 f32, all candidates ->
+// bounded, with the launch: q4_k 241 -> 118 us, q5_k 260 -> 121, q2_k 345 -> 181 (q3_k 82, q6_k 78: 19 candidates, no
+// bound); 300 x 4096 q4_k 42 -> 25; 128 x 1024, where one wave's latency counts, 23.4 -> 24.5.  Every-candidate kernels
+// shared the candidates of a small matrix between lanes; the bounded scan is as fast there without.  Blocks narrow and far
+// above zero, whose least-squares systems are near singular, keep more candidates: q4_k 251 -> 230, q5_k 275 -> 280.
 // Legacy codecs: memory.  Eight lanes per block, 16-byte loads, wire bytes assembled in LDS and stored as dwords
 // (4096 x 4096 f32 to q8_0: 20 us, 4.2 TB/s).
 #include "kq_common.h"
@@ -24,6 +27,15 @@ __device__ __forceinline__ float clamp_level(float v, float lo, float hi) {  // 
 // makes it the lower bound.  (With lo = 0 both are 0.)
 __device__ __forceinline__ float clamp_level_signed(float v, float lo, float hi) {
   return v == v ? clamp_level(v, lo, hi) : 0.f;
+}
+
+// rint(a / b) for a quotient that is clamped to a few hundred levels afterwards, from v_rcp_f32 (1 ulp): the product is
+// within 4e-7 of its size of the quotient, so it rounds like the quotient unless it lies that close to a half.  `sure` is
+// cleared then, and for every quotient that is not finite; the caller divides instead.
+__device__ __forceinline__ float rint_quotient(float a, float rcp_b, bool& sure) {
+  const float q = a * rcp_b, l = __builtin_rintf(q);
+  sure &= std::fabs(q - l) < 0.4999f;
+  return l;
 }
 
 // four weights at element i (a multiple of four) of w, widened exactly
@@ -126,46 +138,63 @@ __global__ __launch_bounds__(LEG_THREADS) void encode_legacy_kernel(const void* 
 }
 
 // ------------------------------------------------------------------ K-quant superblocks
-// One wave per workgroup.  Lane = (superblock, sub-block j, part s): S lanes share a sub-block's candidates.  S > 1 is
-// for matrices whose sub-blocks are too few to fill the chip; the lanes of a sub-block redo everything outside the
-// candidate scan, so it costs instructions where they are not short of waves.
+// One wave per workgroup, lane = (superblock, sub-block j).
 template <int C>
 struct KGeom {
   static constexpr int SUBS = C == KQ_Q4_K || C == KQ_Q5_K ? 8 : 16, N = 256 / SUBS;
   static constexpr int NMAX = C == KQ_Q2_K ? 3 : C == KQ_Q4_K ? 15 : 31;  // of the (scale, min) codecs
 };
 
-// kqenc::fit_scale_min.  A candidate replaces the best one if its error is strictly smaller, so the scan's result is the
-// earliest candidate of least error whatever order they are tried in: part s tries steps s, s + S, ... and the parts
-// are compared afterwards.
-template <int N, int NMAX, int S>
-__device__ __forceinline__ float fit_scale_min(const float (&x)[N], const float (&wt)[N], int part, float& neg_min) {
-  float vmin = x[0], vmax = x[0], sw = wt[0], swx = sw * x[0];
+// kqenc::fit_scale_min, with most of its 37 candidates ruled out before they are evaluated.  A candidate's levels decide
+// everything about it, and from one candidate to the next few levels change: level i is the rounded product of an inverse
+// scale that grows with the step and a distance d_i >= 0 from the minimum, so it climbs by less than two over all steps.
+//   1. For each weight the steps at which its level climbs are found (estimated, then settled by the level's own rounded
+//      expression at the estimate), and what the climb adds to the sums of w l, w l^2 and w l d is added to that step's
+//      bins.  The weights of the bins are 16-bit whole numbers w' <= w: the first two sums are exact, the third to 2^-53.
+//   2. Running sums over the steps give each candidate's least possible error E = min over (s, m <= 0) of
+//      sum w' (s l + m - x)^2 in closed form.  The rounded error of the candidate cannot be below
+//      (sqrt(E) - r X sqrt(sum w))^2 (1 - 1e-5), r = 2^-24 (10 + 2.2 cond): rounding moves each of its terms s l + m - x by
+//      at most 2^-24 (2 X + 3 |term| + |m|) and d by 2^-24 2 X, X the largest |x|, and |m| <= 2.2 cond X where
+//      sum w sum w l^2 <= cond det and cond <= 8000 (the rounded determinant is then within 7 % of det).
+//      The grid from minimum to maximum has the levels of step 18 and a known (s, m): its error follows the same way, with
+//      |m| <= X and 2^-24 3 X for the rounding of s.
+//   3. The candidate of least E is evaluated as the sequential code does it, then what else has a bound that does not
+//      exceed the best error so far, except candidates with the levels of the step before (the same result, tried earlier).
+// What wins is the earliest candidate of least rounded error, as in the sequential scan.  Sub-blocks outside the ranges
+// for which the bound is derived (negative, huge or vanishing weights, not-finite values, errors near underflow) evaluate
+// every candidate, the others those whose system is too near singular.  On normally distributed weights a lane evaluates 1.0 - 1.1 candidates, the
+// slowest of 64 about two.
+// The steps are taken in two halves, each of which a level climbs in at most once (0.9 of a level where the distance is the
+// whole range): half the bins, so that two waves share a SIMD.
+constexpr int STEPS = 37, HALF = 18;
+
+struct FitBins {  // [step of the half][lane], eight bytes a lane: conflict-free
+  unsigned long long wl[HALF][64];  // low half: sum of w' and, from bit 24, the number of climbs; high half: growth of w' l^2
+  double wld[HALF][64];             // of w' d
+};
+
+__device__ __forceinline__ float step_numerator(float step, int nmax) { return -0.9f + 0.05f * step + float(nmax); }
+
+template <int N, int NMAX>
+__device__ __forceinline__ float fit_scale_min(float (&x)[N], float (&wt)[N], FitBins& bins, int lane,
+                                               float& neg_min) {
+  float vmin = x[0], vmax = x[0], sw = wt[0], swx = sw * x[0], wmin = wt[0], wmax = wt[0];
 #pragma unroll
   for (int i = 1; i < N; i++) {
     if (x[i] < vmin) vmin = x[i];
     if (x[i] > vmax) vmax = x[i];
     sw += wt[i];
     swx += wt[i] * x[i];
+    wmin = fminf(wmin, wt[i]);
+    wmax = fmaxf(wmax, wt[i]);
   }
   if (vmin > 0.f) vmin = 0.f;
   const bool flat = vmax <= vmin;
   const float range = vmax - vmin;
-  float scale, best_min = vmin, best_err = 0.f;
-  {
-    const float inv = float(NMAX) / range;
-    scale = 1.0f / inv;
-#pragma unroll
-    for (int i = 0; i < N; i++) {
-      const float l = clamp_level(inv * (x[i] - vmin), 0.f, float(NMAX));
-      const float e = scale * l + vmin - x[i];
-      best_err += wt[i] * e * e;
-    }
-  }
-  int best_step = -1;
-#pragma unroll 1
-  for (int step = part; step <= 36; step += S) {
-    const float inv_s = (-0.9f + 0.05f * float(step) + float(NMAX)) / range;
+  float scale = 0.f, best_min = vmin, best_err = INFINITY;
+  int best_step = STEPS;
+  auto evaluate = [&](int step) {
+    const float inv_s = step_numerator(float(step), NMAX) / range;
     float lv[N], sl = 0.f, sl2 = 0.f, sxl = 0.f;
 #pragma unroll
     for (int i = 0; i < N; i++) {
@@ -187,23 +216,162 @@ __device__ __forceinline__ float fit_scale_min(const float (&x)[N], const float 
       const float e = s * lv[i] + m - x[i];
       err += wt[i] * e * e;
     }
-    if (det > 0.f && err < best_err) {
+    if (det > 0.f && (err < best_err || (err == best_err && step < best_step))) {
       best_err = err;
       scale = s;
       best_min = m;
       best_step = step;
     }
-  }
+  };
+
+  unsigned long long todo = flat ? 0 : (1ull << STEPS) - 1;
+  bool grid = true;
+  if (range >= 1e-9f && range <= 1e9f && vmax <= 1e9f && vmin >= -1e9f && wmin >= 0.f && wmax >= 1e-9f && wmax <= 1e9f &&
+      sw == sw && swx == swx) {
+    const float ws = 65535.0f / wmax, inv0 = step_numerator(0.f, NMAX) / range;
+    const float rr = 1.0f / range;  // correctly rounded: two corrections of n * rr give n / range so
+    const float per_step = 20.f * range, zero_step = -(float(NMAX) - 0.9f) * 20.f - 1e-3f;
+    auto over_range = [&](float num) {  // num / range
+      float v = num * rr;
+      v = __builtin_fmaf(__builtin_fmaf(-v, range, num), rr, v);
+      return __builtin_fmaf(__builtin_fmaf(-v, range, num), rr, v);
+    };
+    uint32_t W = 0, sl = 0, sl2 = 0;
+    double sd = 0.0, sdd = 0.0, sdl = 0.0;
 #pragma unroll
-  for (int m = 1; m < S; m <<= 1) {
-    const float oe = __shfl_xor(best_err, m), os = __shfl_xor(scale, m), om = __shfl_xor(best_min, m);
-    const int ost = __shfl_xor(best_step, m);
-    if (oe < best_err || (oe == best_err && ost < best_step)) {
-      best_err = oe;
-      scale = os;
-      best_min = om;
-      best_step = ost;
+    for (int i = 0; i < N; i++) {
+      const float d = x[i] - vmin, l0 = __builtin_rintf(inv0 * d);
+      const uint32_t w = (uint32_t)(wt[i] * ws), l = (uint32_t)l0, wl = __umul24(w, l);
+      const double wd = double(w) * double(d);
+      W += w;
+      sl += wl;
+      sl2 += __umul24(wl, l);
+      sd += wd;
+      sdd = __builtin_fma(wd, double(d), sdd);
+      sdl = __builtin_fma(wd, double(l0), sdl);
     }
+    const double Wd = double(W), sddc = __builtin_fma(Wd, sdd, -sd * sd);
+    const float unit = 1.0f / (ws * float(W));
+    float least = INFINITY, det_least = INFINITY;
+    const float reach = fmaxf(vmax, -vmin) * std::sqrt(sw);
+    int first = 0;
+    auto bound_of = [&](auto at_zero, int c, bool same) {
+      const double sld = double(sl), sl2d = double(sl2);
+      const double det = __builtin_fma(Wd, sl2d, -sld * sld), cross = __builtin_fma(Wd, sdl, -sd * sld);
+      const float detf = float(det);
+      float e = float(__builtin_fma(sddc, det, -cross * cross)) * __builtin_amdgcn_rcpf(detf) * unit;
+      if constexpr (decltype(at_zero)::value) {  // the minimum may be held at zero: where m would be positive, it is zero
+        const float e0 = float(__builtin_fma(sdd, sl2d, -sdl * sdl)) * __builtin_amdgcn_rcpf(float(sl2) * ws);
+        e = vmin == 0.f && sl2d * sd > sld * sdl ? e0 : e;
+        // such lanes may have levels almost all alike at some steps (narrow blocks far from zero): cond by the step, and no
+        // bound where it is too large
+        const float cond = float(W) * (float(sl2) + float(N * NMAX * NMAX)) * __builtin_amdgcn_rcpf(detf);
+        if (!(cond <= 8000.f)) return same ? INFINITY : -INFINITY;
+        const float root = fmaxf(std::sqrt(e) - (2.2f * 5.98e-8f) * cond * reach, 0.f);
+        e = root * root;
+      } else {
+        det_least = fminf(det_least, detf);
+      }
+      e = same ? INFINITY : e;
+      if (e < least) {
+        least = e;
+        first = c;
+      }
+      return e;
+    };
+    float bound0 = bound_of(std::true_type{}, 0, false), bound[HALF], bound_lo[HALF], grid_bound = 0.f;
+#pragma unroll 1
+    for (int base = 0; base < 2 * HALF; base += HALF) {
+#pragma unroll
+      for (int c = 0; c < HALF; c++) {
+        bins.wl[c][lane] = 0;
+        bins.wld[c][lane] = 0.0;
+      }
+      // what the loop below derives from x and wt is not to be kept from one half to the next: that would be 150 registers
+#pragma unroll
+      for (int i = 0; i < N; i++) asm volatile("" : "+v"(x[i]), "+v"(wt[i]));
+      const float inv_b = over_range(step_numerator(float(base), NMAX));
+#pragma unroll
+      for (int g = 0; g < N; g += 8) {
+        unsigned at[8], l[8];
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+          const float d = x[g + t] - vmin, lb = __builtin_rintf(inv_b * d);
+          // The real step at which the product passes lb + 1/2, off by less than 1e-3: every rounding on the way, here and in
+          // the level's own expression, is 2^-24 of at most 20 (NMAX + 1) steps.  d = 0: no step.
+          const float q = __builtin_amdgcn_rcpf(std::fabs(d)) * per_step;
+          const float n = fminf(__builtin_ceilf(__builtin_fmaf(lb + 0.5f, q, zero_step)), 64.f);
+          const float inv_s = over_range(step_numerator(n, NMAX));
+          at[t] = unsigned(int(n)) - unsigned(base) - (__builtin_rintf(inv_s * d) > lb ? 1u : 0u);
+          l[t] = (uint32_t)lb;
+        }
+#pragma unroll
+        for (int t = 0; t < 8; t++)
+          if (at[t] < unsigned(HALF) && l[t] < unsigned(NMAX)) {
+            const uint32_t w = (uint32_t)(wt[g + t] * ws);
+            __builtin_assume(w < 1u << 16);
+            const unsigned long long v = (unsigned long long)__umul24(w, 2 * l[t] + 1) << 32 | w | 1u << 24;
+            const double wd = double(w) * double(x[g + t] - vmin);
+            __hip_atomic_fetch_add(&bins.wl[at[t]][lane], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_fetch_add(&bins.wld[at[t]][lane], wd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          }
+      }
+      auto steps = [&](auto at_zero) {
+#pragma unroll
+        for (int c = 0; c < HALF; c++) {
+          const unsigned long long v = bins.wl[c][lane];
+          sl += (uint32_t)v & 0xffffff;
+          sl2 += (uint32_t)(v >> 32);
+          sdl += bins.wld[c][lane];
+          bound[c] = bound_of(at_zero, base + c + 1, (uint32_t)v == 0);
+        }
+      };
+      if (__builtin_amdgcn_ballot_w64(vmin == 0.f)) steps(std::true_type{});
+      else steps(std::false_type{});
+      if (base == 0) {
+        const float s = range / float(NMAX);  // the grid's levels are those of step 18
+        grid_bound = float(__builtin_fma(double(s), __builtin_fma(double(s), double(sl2), -2.0 * sdl), sdd)) / ws;
+#pragma unroll
+        for (int c = 0; c < HALF; c++) bound_lo[c] = bound[c];
+      }
+    }
+    evaluate(first);
+    const float cond = float(W) * (float(sl2) + float(N * NMAX * NMAX)) / det_least;
+    if (cond <= 8000.f && det_least > 0.f && best_err >= 1e-28f) {
+      const float r = (10.f + 2.2f * cond) * 5.97e-8f;
+      const float root = std::sqrt(best_err) * 1.00001f + r * reach, lim = root * root * 1.00001f;
+      uint32_t lo = 0, hi = 0;
+#pragma unroll
+      for (int c = 0; c < HALF; c++) {
+        lo |= bound_lo[c] > lim ? 0 : 2u << c;
+        hi |= bound[c] > lim ? 0 : 2u << c;
+      }
+      todo = ((unsigned long long)hi << HALF | lo | (bound0 > lim ? 0 : 1)) & ~(1ull << first);
+      grid = !(grid_bound > lim);
+    } else {
+      best_err = INFINITY;
+    }
+  }
+  if (grid && !flat) {
+    const float inv = float(NMAX) / range, s = 1.0f / inv;
+    float err = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const float l = clamp_level(inv * (x[i] - vmin), 0.f, float(NMAX));
+      const float e = s * l + vmin - x[i];
+      err += wt[i] * e * e;
+    }
+    if (!(err > best_err)) {  // first of all in the sequential order (where a NaN stays)
+      best_err = err;
+      scale = s;
+      best_min = vmin;
+      best_step = -1;
+    }
+  }
+  while (todo) {
+    const int step = __builtin_ctzll(todo);
+    todo &= todo - 1;
+    evaluate(step);
   }
   neg_min = flat ? -vmin : -best_min;
   return flat ? 0.f : scale;
@@ -251,65 +419,64 @@ __device__ __forceinline__ float fit_signed16(const float (&x)[16], const float 
   return apeak < 1e-30f ? 0.f : scale;
 }
 
-// kqenc::fit_positive of the sub-block scales (which = 0) and of the minima (1): both arrays lie in LDS.  The nine-point
-// scan takes one candidate per lane of an octet (again the earliest of least error wins); the refinement, whose steps
-// depend on each other, runs on the even lanes for the scales and on the odd ones for the minima.  Returns the factor
-// of the lane's array and leaves its levels in lv.
+// kqenc::fit_positive of the sub-block scales (even lanes) and of the minima (odd ones): both arrays lie in LDS.  The four
+// lanes of an octet that share an array take two candidates each of the nine-point scan (again the earliest of least error
+// wins) and all do the refinement, whose steps depend on each other.  Returns the factor of the lane's array and leaves its
+// levels in lv.
 template <int N, int NMAX>
 __device__ __forceinline__ float fit_positive_pair(const float* sc, const float* mn, const float* sw, int lane,
                                                    int (&lv)[N]) {
-  float wt[N], inv_of[2];
+  const float* src = lane & 1 ? mn : sc;
+  float wt[N], x[N], vmax = 0.f;
 #pragma unroll
-  for (int i = 0; i < N; i++) wt[i] = sw[i];
-  float x[N];
-#pragma unroll
-  for (int which = 0; which < 2; which++) {
-    const float* src = which ? mn : sc;
-    float vmax = 0.f;
-#pragma unroll
-    for (int i = 0; i < N; i++) {
-      x[i] = src[i];
-      if (x[i] > vmax) vmax = x[i];
-    }
-    float inv = float(NMAX) / vmax, best = 0.f;
-    {
-      const float s = 1.0f / inv;
-#pragma unroll
-      for (int i = 0; i < N; i++) {
-        const int l = (uint8_t)kqenc::clampi(kqenc::rne(inv * x[i]), 0, NMAX);
-        const float e = x[i] - s * float(l);
-        best += wt[i] * e * e;
-      }
-    }
-    const int c = lane & 7, k = c < 4 ? c - 4 : c - 3;
-    float inv_k = (0.1f * float(k) + float(NMAX)) / vmax, err = 0.f;
-    const float s_k = 1.0f / inv_k;
-#pragma unroll
-    for (int i = 0; i < N; i++) {
-      const int l = min(NMAX, kqenc::rne(inv_k * x[i]));
-      const float e = x[i] - s_k * float(l);
-      err += wt[i] * e * e;
-    }
-    int order = c;
-#pragma unroll
-    for (int m = 1; m < 8; m <<= 1) {
-      const float oe = __shfl_xor(err, m), oi = __shfl_xor(inv_k, m);
-      const int oo = __shfl_xor(order, m);
-      if (oe < err || (oe == err && oo < order) || !(err == err)) {
-        err = oe;
-        inv_k = oi;
-        order = oo;
-      }
-    }
-    inv_of[which] = vmax < 1e-30f ? -1.f : err < best ? inv_k : inv;
+  for (int i = 0; i < N; i++) {
+    wt[i] = sw[i];
+    x[i] = src[i];
+    if (x[i] > vmax) vmax = x[i];
   }
-  const bool odd = lane & 1;
-  const float inv = odd ? inv_of[1] : inv_of[0];
-  const float* src = odd ? mn : sc;
+  float inv = float(NMAX) / vmax, best = 0.f;
+  {
+    const float s = 1.0f / inv;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const int l = (uint8_t)kqenc::clampi(kqenc::rne(inv * x[i]), 0, NMAX);
+      const float e = x[i] - s * float(l);
+      best += wt[i] * e * e;
+    }
+  }
+  float err = NAN, inv_k = 0.f;
+  int order = 0;
+#pragma unroll
+  for (int half = 0; half < 2; half++) {
+    const int c = ((lane >> 1) & 3) + 4 * half, k = half ? c - 3 : c - 4;
+    const float inv_c = (0.1f * float(k) + float(NMAX)) / vmax, s_c = 1.0f / inv_c;
+    float err_c = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const int l = min(NMAX, kqenc::rne(inv_c * x[i]));
+      const float e = x[i] - s_c * float(l);
+      err_c += wt[i] * e * e;
+    }
+    if (err_c < err || !(err == err)) {
+      err = err_c;
+      inv_k = inv_c;
+      order = c;
+    }
+  }
+#pragma unroll
+  for (int m = 2; m < 8; m <<= 1) {
+    const float oe = __shfl_xor(err, m), oi = __shfl_xor(inv_k, m);
+    const int oo = __shfl_xor(order, m);
+    if (oe < err || (oe == err && oo < order) || !(err == err)) {
+      err = oe;
+      inv_k = oi;
+      order = oo;
+    }
+  }
+  inv = vmax < 1e-30f ? -1.f : err < best ? inv_k : inv;
   float slx = 0.f, sl2 = 0.f;
 #pragma unroll
   for (int i = 0; i < N; i++) {
-    x[i] = src[i];
     const int l = min(NMAX, kqenc::rne(inv * x[i]));
     lv[i] = (uint8_t)l;
     slx += wt[i] * x[i] * float(l);
@@ -323,7 +490,11 @@ __device__ __forceinline__ float fit_positive_pair(const float* sc, const float*
       const float w = wt[i];
       float a = slx - w * x[i] * float(lv[i]);
       float b = sl2 - w * float(lv[i]) * float(lv[i]);
-      const int nl = min(NMAX, kqenc::rne(x[i] * b / a));
+      const float xb = x[i] * b;
+      bool sure = true;
+      float r = rint_quotient(xb, __builtin_amdgcn_rcpf(a), sure);
+      if (!sure) r = std::rint(xb / a);
+      const int nl = min(NMAX, int(r));
       if (a > 0.f && b > 0.f && nl != lv[i]) {
         a += w * x[i] * float(nl);
         b += w * float(nl) * float(nl);
@@ -345,26 +516,38 @@ __device__ __forceinline__ float fit_positive_pair(const float* sc, const float*
   return sl2 > 0.f ? slx / sl2 : 0.f;
 }
 
-template <int C, int S>
-__global__ __launch_bounds__(64) void encode_k_kernel(const void* __restrict__ w, int dtype,
+template <int C>
+__global__ __launch_bounds__(64, 2) void encode_k_kernel(const void* __restrict__ w, int dtype,
                                                       const float* __restrict__ imatrix, uint8_t* __restrict__ wire,
                                                       int64_t nblocks, int64_t blocks_per_row, bool aligned) {
   constexpr int BPB = kq_geom(C).bpb, SUBS = KGeom<C>::SUBS, N = KGeom<C>::N;
-  constexpr int GROUP = SUBS * S, NSB = 64 / GROUP;  // lanes per superblock, superblocks per wave
+  constexpr int GROUP = SUBS, NSB = 64 / GROUP;      // lanes per superblock, superblocks per wave
   constexpr int XS = 256 + 4;                        // floats between superblocks in LDS: eight of them in eight banks
   constexpr bool kMin = C == KQ_Q2_K || C == KQ_Q4_K || C == KQ_Q5_K;
-  __shared__ __attribute__((aligned(16))) float xs[NSB * XS];
+  // One buffer for what lives one after the other: the staged weights, the bins of the (scale, min) fit, and the levels and
+  // wire bytes (a workgroup of less than 20 KiB lets a CU hold eight, two per SIMD).
+  constexpr size_t BUF = NSB * XS * sizeof(float);
+  __shared__ __attribute__((aligned(16))) uint8_t buf[kMin ? sizeof(FitBins) : BUF];
+  static_assert(BUF >= NSB * 256 + NSB * BPB && sizeof(FitBins) >= BUF, "buffer");
+  float* xs = reinterpret_cast<float*>(buf);
+  auto* s_lv = reinterpret_cast<uint8_t(*)[256]>(buf);
+  uint8_t* out = buf + NSB * 256;
   __shared__ float s_sc[NSB][SUBS], s_mn[NSB][SUBS], s_sw[NSB][SUBS];
-  __shared__ __attribute__((aligned(16))) uint8_t s_lv[NSB][256];
   __shared__ int s_ls[NSB][SUBS], s_lm[NSB][SUBS];
-  __shared__ __attribute__((aligned(16))) uint8_t out[NSB * BPB];
-  const int lane = threadIdx.x, sb = lane / GROUP, gl = lane % GROUP, j = gl / S, part = gl % S;
-  const int64_t blk0 = (int64_t)blockIdx.x * NSB;
-  for (int i = lane; i < NSB * 64; i += 64) {
-    // superblocks past the end redo the last one; their bytes are not stored
-    const int64_t blk = min(blk0 + (i >> 6), nblocks - 1);
-    *reinterpret_cast<float4*>(xs + (i >> 6) * XS + 4 * (i & 63)) = load4_any(w, dtype, blk * 256 + 4 * (i & 63), aligned);
-  }
+  const int lane = threadIdx.x, sb = lane / GROUP, gl = lane % GROUP, j = gl;
+  // superblocks past the end redo the last one; their bytes are not stored
+  const int64_t blk0 = (int64_t)blockIdx.x * NSB, last = min(blk0 + NSB, nblocks) - 1;
+  auto stage = [&](int dt, bool al) {  // all loads first: few waves are there to cover their latency
+    float4 v[NSB];
+#pragma unroll
+    for (int i = 0; i < NSB; i++) v[i] = load4_any(w, dt, min(blk0 + i, last) * 256 + 4 * lane, al);
+#pragma unroll
+    for (int i = 0; i < NSB; i++) *reinterpret_cast<float4*>(xs + i * XS + 4 * lane) = v[i];
+  };
+  if (!aligned) stage(dtype, false);
+  else if (dtype == KQ_F32) stage(KQ_F32, true);
+  else if (dtype == KQ_F16) stage(KQ_F16, true);
+  else stage(KQ_BF16, true);
   __syncthreads();
   const float* xb = xs + sb * XS;
   float x[N], wt[N];
@@ -373,14 +556,19 @@ __global__ __launch_bounds__(64) void encode_k_kernel(const void* __restrict__ w
 
   // importance weights (kqenc::importance; q6_k weights by the matrix itself, q3_k and q6_k by x^2 without one)
   const float* im = nullptr;
-  if (imatrix) im = imatrix + (min(blk0 + sb, nblocks - 1) % blocks_per_row) * 256 + N * j;
+  if (imatrix) im = imatrix + (min(blk0 + sb, last) % blocks_per_row) * 256 + N * j;
   if (C == KQ_Q6_K || (C == KQ_Q3_K && !im)) {
 #pragma unroll
     for (int i = 0; i < N; i++) wt[i] = im ? im[i] : x[i] * x[i];
   } else {
+    __syncthreads();
+    float* sq = xs + sb * XS;
+#pragma unroll
+    for (int i = 0; i < N; i++) sq[N * j + i] = x[i] * x[i];
+    __syncthreads();
     float total = 0.f;
-#pragma unroll 16
-    for (int i = 0; i < 256; i++) total += xb[i] * xb[i];
+#pragma unroll 32
+    for (int i = 0; i < 256; i++) total += sq[i];
     const float sigma2 = (C == KQ_Q2_K ? 1.0f : 2.0f) * total / 256.0f, av = std::sqrt(sigma2);
     if (im) {
 #pragma unroll
@@ -391,17 +579,36 @@ __global__ __launch_bounds__(64) void encode_k_kernel(const void* __restrict__ w
     }
   }
 
+  __syncthreads();  // the weights have been read from buf
   uint8_t* b = out + sb * BPB;
+  // levels of the lane's weights, four to a word: level(i, rint((x + add) / by)).  (A sum with a zero changes no quotient.)
+  auto store_levels = [&](auto level, float add, float by) {
+    const float rcp = __builtin_amdgcn_rcpf(by);
+    bool sure = true;
+    uint32_t packed[N / 4];
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const uint32_t l = level(i, rint_quotient(x[i] + add, rcp, sure));
+      packed[i / 4] = i % 4 ? packed[i / 4] | l << (8 * (i % 4)) : l;
+    }
+    if (!sure) {
+#pragma unroll
+      for (int i = 0; i < N; i++) {
+        const uint32_t l = level(i, __builtin_rintf((x[i] + add) / by));
+        packed[i / 4] = i % 4 ? packed[i / 4] | l << (8 * (i % 4)) : l;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < N / 4; i++) reinterpret_cast<uint32_t*>(s_lv[sb])[N / 4 * j + i] = packed[i];
+  };
   if constexpr (kMin) {
     float sw = 0.f, neg_min;
 #pragma unroll
     for (int i = 0; i < N; i++) sw += wt[i];
-    const float sc = fit_scale_min<N, KGeom<C>::NMAX, S>(x, wt, part, neg_min);
-    if (part == 0) {
-      s_sc[sb][j] = sc;
-      s_mn[sb][j] = neg_min;
-      s_sw[sb][j] = sw;
-    }
+    const float sc = fit_scale_min<N, KGeom<C>::NMAX>(x, wt, *reinterpret_cast<FitBins*>(buf), lane, neg_min);
+    s_sc[sb][j] = sc;
+    s_mn[sb][j] = neg_min;
+    s_sw[sb][j] = sw;
     __syncthreads();
     constexpr int LMAX = C == KQ_Q2_K ? 15 : 63, DOFF = C == KQ_Q2_K ? 80 : 0;
     int lv[SUBS];
@@ -413,10 +620,8 @@ __global__ __launch_bounds__(64) void encode_k_kernel(const void* __restrict__ w
     }
     __syncthreads();
     const float ds = kqenc::get_f16(b + DOFF) * float(s_ls[sb][j]), dm = kqenc::get_f16(b + DOFF + 2) * float(s_lm[sb][j]);
-#pragma unroll
-    for (int i = 0; i < N; i++)
-      if (i % S == part)
-        s_lv[sb][N * j + i] = ds == 0.f ? 0 : (uint8_t)(int)clamp_level((x[i] + dm) / ds, 0.f, float(KGeom<C>::NMAX));
+    store_levels([&](int i, float q) { return ds == 0.f ? 0 : (uint8_t)(int)__builtin_amdgcn_fmed3f(q, 0.f, float(KGeom<C>::NMAX)); },
+                 dm, ds);
   } else {
     constexpr int NMAX = C == KQ_Q6_K ? 32 : 4;
     bool finite = true;
@@ -450,10 +655,9 @@ __global__ __launch_bounds__(64) void encode_k_kernel(const void* __restrict__ w
       __syncthreads();
       de = kqenc::get_f16(b + 108) * float(l - 32);
     }
-#pragma unroll
-    for (int i = 0; i < N; i++)
-      s_lv[sb][N * j + i] =
-          de == 0.f ? NMAX : (uint8_t)((int)clamp_level_signed(x[i] / de, -float(NMAX), float(NMAX - 1)) + NMAX);
+    store_levels([&](int i, float q) {
+      return de == 0.f ? NMAX : (uint8_t)((q == q ? (int)__builtin_amdgcn_fmed3f(q, -float(NMAX), float(NMAX - 1)) : 0) + NMAX);
+    }, 0.f, de);
   }
   __syncthreads();
 
@@ -512,8 +716,7 @@ __global__ __launch_bounds__(64) void encode_k_kernel(const void* __restrict__ w
     }
   }
   __syncthreads();
-  const int64_t left = nblocks - blk0;
-  store_wire(wire + blk0 * BPB, out, (int)(left < NSB ? left : NSB) * BPB, lane, 64);
+  store_wire(wire + blk0 * BPB, out, (int)(last + 1 - blk0) * BPB, lane, 64);
 }
 
 // four elements per load need the tensor's address to be a multiple of them
@@ -531,27 +734,15 @@ int launch_legacy(const void* w, int dtype, uint8_t* wire, int64_t nblocks, hipS
   return KQ_OK;
 }
 
-template <int C, int S>
-int launch_k_split(const void* w, int dtype, const float* im, uint8_t* wire, int64_t nblocks, int64_t bpr, hipStream_t s) {
-  constexpr int NSB = 64 / (KGeom<C>::SUBS * S);
+template <int C>
+int launch_k(const void* w, int dtype, const float* im, uint8_t* wire, int64_t nblocks, int64_t bpr, hipStream_t s) {
+  constexpr int NSB = 64 / KGeom<C>::SUBS;
   const int64_t wgs = (nblocks + NSB - 1) / NSB;
   if (wgs > 0x7fffffff) return kq_set_error(KQ_ERR_INVALID, "quantize: tensor too large for one launch");
-  hipLaunchKernelGGL((encode_k_kernel<C, S>), dim3((unsigned)wgs), dim3(64), 0, s, w, dtype, im, wire, nblocks, bpr,
+  hipLaunchKernelGGL(encode_k_kernel<C>, dim3((unsigned)wgs), dim3(64), 0, s, w, dtype, im, wire, nblocks, bpr,
                      four_aligned(w, dtype));
   KQ_HIP_CHECK(hipGetLastError());
   return KQ_OK;
-}
-
-// Below this many waves of whole sub-blocks (one per SIMD) four lanes share one's candidates.  One lane / four lanes,
-// us: q4_k 16384 superblocks 70 / 87, 8192 (1024 waves) 50 / 49, 4096 49 / 30, 2048 49 / 23; q2_k 8192 (2048 waves)
-// 53 / 65, 4096 37 / 40, 2048 37 / 27.
-constexpr int64_t SPLIT_WAVES = 1024;
-
-template <int C>
-int launch_k(const void* w, int dtype, const float* im, uint8_t* wire, int64_t nblocks, int64_t bpr, hipStream_t s) {
-  if constexpr (C == KQ_Q2_K || C == KQ_Q4_K || C == KQ_Q5_K)
-    if (nblocks * KGeom<C>::SUBS < 64 * SPLIT_WAVES) return launch_k_split<C, 4>(w, dtype, im, wire, nblocks, bpr, s);
-  return launch_k_split<C, 1>(w, dtype, im, wire, nblocks, bpr, s);
 }
 
 }  // namespace

@@ -164,3 +164,51 @@ def test_device_encoder_nonfinite_weights_keep_their_bytes(kq, codec):
             got = kq.quantize(w, codec, imat)[0].cpu().numpy()
             bad = np.argwhere((got != gold[key]).any(axis=1)).ravel().tolist()
             assert not bad, (key, bad)
+
+
+# rows of each kind for the encoders that rule out candidates by a bound: lattices whose levels sit on ties, one-sided and
+# narrow blocks (the least-squares system near singular, the minimum held at zero), blocks that few levels fit exactly, a
+# few outliers, scales near the ends of the float range and outside those for which the bound is derived
+_FIT_ROWS = {
+    "normal": lambda r, n: r.standard_normal(n) * 0.02,
+    "bytes": lambda r, n: r.integers(-127, 128, n) * 0.0007,
+    "few levels": lambda r, n: r.integers(-3, 4, n) * 0.01,
+    "two values": lambda r, n: r.choice([-0.5, 0.25], n),
+    "16 levels": lambda r, n: r.integers(0, 16, n) * 0.125 - 1.0,
+    "one-sided": lambda r, n: np.abs(r.standard_normal(n)),
+    "narrow": lambda r, n: 1.0 + r.standard_normal(n) * 0.02,
+    "narrow below": lambda r, n: -1.0 + r.standard_normal(n) * 1e-4,
+    "outliers": lambda r, n: r.standard_normal(n) * np.where(r.random(n) < 0.03, 50.0, 0.01),
+    "peaked": lambda r, n: r.random(n) ** 8 * r.standard_normal(n),
+    "sparse": lambda r, n: r.standard_normal(n) * (r.random(n) < 0.1),
+    "tiny": lambda r, n: r.standard_normal(n) * 1e-8,
+    "vanishing": lambda r, n: r.standard_normal(n) * 1e-22,
+    "huge": lambda r, n: r.standard_normal(n) * 3e9,
+}
+_FIT_WEIGHTS = {
+    "none": None,
+    "squares": lambda r, n: r.standard_normal(n) ** 2 + 0.05,
+    "wide": lambda r, n: 10.0 ** r.uniform(-9, 3, n),
+    "zeros": lambda r, n: r.random(n) * (r.random(n) < 0.5),
+    "negative": lambda r, n: r.standard_normal(n),
+    "tiny": lambda r, n: r.random(n) * 1e-20,
+}
+
+
+@pytest.mark.parametrize("weights", sorted(_FIT_WEIGHTS))
+@pytest.mark.parametrize("codec", KCODECS)
+def test_device_encoder_fit_bytes_over_kinds_of_rows(kq, codec, weights):
+    """Bytes equal the host's for every kind of row, kinds alternating by row and, in the last rows, by sub-block."""
+    rng = np.random.default_rng(31 + O.codec_id(codec))
+    K = 1024
+    w = np.stack([f(rng, K) for f in _FIT_ROWS.values() for _ in range(8)])
+    mixed = np.stack([np.concatenate([w[rng.integers(len(w)), 16 * j:16 * j + 16] for j in range(K // 16)])
+                      for _ in range(16)])
+    w = torch.from_numpy(np.concatenate([w, mixed]).astype(np.float32))
+    make = _FIT_WEIGHTS[weights]
+    im = None if make is None else torch.from_numpy(make(rng, K).astype(np.float32))
+    host = kq.quantize(w, codec, im)[0].numpy()
+    dev = kq.quantize(w.cuda(), codec, None if im is None else im.cuda())[0].cpu().numpy()
+    bad = np.argwhere((dev != host).any(axis=1)).ravel().tolist()
+    kinds = list(_FIT_ROWS)
+    assert not bad, sorted({kinds[b // 8] if b < 8 * len(kinds) else "mixed" for b in bad})
