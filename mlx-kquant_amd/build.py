@@ -32,6 +32,7 @@ SOURCES = [
     ("kq_gemm3f.hip", ["-Wno-inline-asm"]),
     ("kq_gemm3i.hip", ["-Wno-inline-asm", "-ffp-contract=off"]),
     ("kq_mid.hip", []),
+    ("kq_heads.hip", ["-Wno-inline-asm"]),
     # one source, an object per tile height
     ("kq_tile.hip", ["-Wno-inline-asm", "-DKQ_TILE_NB=2"], "kq_tile_2"),
     ("kq_tile.hip", ["-Wno-inline-asm", "-DKQ_TILE_NB=3"], "kq_tile_3"),

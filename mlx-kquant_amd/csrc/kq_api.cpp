@@ -311,12 +311,19 @@ int kq_gather_qmm(const void* x_dev, const void* w_dev, const uint32_t* lhs_idx_
     return kq_launch_gather_nt_generic(x_dev, static_cast<const uint8_t*>(w_dev), lhs_idx_dev, rhs_idx_dev, out_dev, B,
                                        M, E, N, K, x_batch_stride, w_expert_stride_bytes, codec, dtype, s);
   }
-  // many output rows: gather them into a dense matrix and run the expert-grouped kernels
   int64_t P;
-  if (workspace_dev && gather_batched_shape(B, M, E, N, K, transpose, codec, &P) &&
-      !per_entry_route(P, M, false, 0, 0, codec, E, N, K,
-                       kq_gather_stream_takes(x_dev, w_dev, nullptr, (int)(P > 0x7fffffff ? 0x7fffffff : P), N, K, true,
-                                              x_batch_stride, w_expert_stride_bytes, false, codec)) &&
+  const bool batched = gather_batched_shape(B, M, E, N, K, transpose, codec, &P);
+  const bool by_entry = per_entry_route(P, M, false, 0, 0, codec, E, N, K,
+                                        kq_gather_stream_takes(x_dev, w_dev, nullptr, (int)(P > 0x7fffffff ? 0x7fffffff : P), N, K,
+                                                               true, x_batch_stride, w_expert_stride_bytes, false, codec));
+  // short contractions over few rows per expert: one launch
+  if (!by_entry) {
+    const int rch = kq_launch_heads(x_dev, static_cast<const uint8_t*>(w_dev), lhs_idx_dev, rhs_idx_dev, out_dev, B, M, E, N, K,
+                                    x_batch_stride, w_expert_stride_bytes, codec, dtype, s);
+    if (rch != KQ_ERR_UNSUPPORTED) return rch;
+  }
+  // many output rows: gather them into a dense matrix and run the expert-grouped kernels
+  if (workspace_dev && batched && !by_entry &&
       !(reinterpret_cast<uintptr_t>(workspace_dev) & 255) && !(reinterpret_cast<uintptr_t>(x_dev) & 15) &&
       !(x_batch_stride & 7)) {
     const size_t need = kq_gather_qmm_workspace_size(B, M, E, N, K, transpose, codec, dtype);

@@ -26,7 +26,7 @@ struct MidGeom {
   static constexpr int BYTES = CK_STEP / WPB * BPB;
   static constexpr int PIECES = (BYTES + 15) / 16, LP = PIECES | 1, LROW = 16 * LP;
   static constexpr int LOADS = (32 * LP + 63) / 64;
-  // activation order (see mid_prepass_kernel) and sum fragments per step
+  // activation order (store_frags) and sum fragments per step
   static constexpr int ORD = C == KQ_Q4_K || C == KQ_Q5_K || C == KQ_Q6_K                       ? 0
                              : C == KQ_IQ4_NL || C == KQ_IQ4_XS || C == KQ_MXFP4 ? 2
                              : C == KQ_NVFP4                                     ? 3
@@ -40,6 +40,57 @@ template <int C>
 constexpr int mid_table_bytes() {
   if constexpr (k_quant<C>() || fp4<C>()) return 0;
   else return CodeGeom<C>::GROUPED_GRID_BYTES + CodeGeom<C>::SPREAD_BYTES;
+}
+
+// Eight consecutive activations h (8-group pc of a row's step) to the step's fragments, 1 KiB each of [lane = 32 kg + row][8
+// halves]; `step` is the step's first fragment plus 16 bytes per row of the block of 32.
+// ORD 0 (q4_k / q5_k / q6_k): fragment 2 j + s, half kg = weights 32 j + 16 kg + 8 s .. of the step; ORD 1: fragment J,
+// half kg = weights 16 J + 8 kg ..; both k0 k2 k1 k3 k4 k6 k5 k7 inside the eight; ORD 2: as ORD 1 with the positions of
+// x[j], x[j + 16] interleaved over every 32 (ORD 3: x[j], x[j + 8] over every 16).  NSUM 1: fragment 16 = sums of the eight 32-wide blocks, kg 0 the f16 part hi,
+// kg 1 the remainder lo, X = 32 (hi + lo); NSUM 2: fragments 16 / 17 = hi / lo of the sixteen 16-wide sums, X = 16 (hi + lo).
+// Whole octets of lanes call together, lane by lane consecutive groups.  SWZ, for fragments in LDS: row r of half kg of fragment
+// J < 16 lies in place r ^ (2 J + kg), so that the 32 groups of a row, written by 32 lanes at once, meet 32 different places.
+template <int ORD, int NSUM, bool SWZ = false>
+__device__ __forceinline__ void store_frags(uint8_t* step, int pc, const _Float16 (&h)[8], int row = 0) {
+  auto at = [&](int q) { return step + 512 * q + (SWZ ? 16 * (row ^ q) - 16 * row : 0); };  // q = 2 J + kg
+  if constexpr (ORD >= 2) {
+    uint32_t own[4], par[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      own[e] = (uint32_t)__builtin_bit_cast(uint16_t, h[2 * e]) | ((uint32_t)__builtin_bit_cast(uint16_t, h[2 * e + 1]) << 16);
+      // the neighbour two (ORD 3: one) groups on: quad_perm [2,3,0,1] or [1,0,3,2]
+      par[e] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)own[e], ORD == 2 ? 0x4E : 0xB1, 0xf, 0xf, true);
+    }
+    const bool high = (pc & (ORD == 2 ? 2 : 1)) != 0;
+    const uint32_t a0 = high ? par[2] : own[0], a1 = high ? par[3] : own[1];
+    const uint32_t b0 = high ? own[2] : par[0], b1 = high ? own[3] : par[1];
+    const u32x4 o = {(a0 & 0xffffu) | (b0 << 16), (a0 >> 16) | (b0 & 0xffff0000u), (a1 & 0xffffu) | (b1 << 16),
+                     (a1 >> 16) | (b1 & 0xffff0000u)};
+    const int pos = ORD == 2 ? 4 * (pc >> 2) + 2 * (pc & 1) + (high ? 1 : 0) : pc;
+    *reinterpret_cast<u32x4*>(at(pos)) = o;
+  } else {
+    const int J = ORD == 0 ? 2 * (pc >> 2) + (pc & 1) : pc >> 1, kg = ORD == 0 ? (pc >> 1) & 1 : pc & 1;
+    *reinterpret_cast<f16x8*>(at(2 * J + kg)) = f16x8{h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
+  }
+  if constexpr (NSUM > 0) {
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; e++) s += (float)h[e];
+    s += __shfl_xor(s, 1);
+    if constexpr (NSUM == 1) s += __shfl_xor(s, 2);
+    constexpr float unit = NSUM == 1 ? 32.0f : 16.0f;
+    const _Float16 hi = (_Float16)(s * (1.0f / unit)), lo = (_Float16)((s - unit * (float)hi) * (1.0f / unit));
+    if constexpr (NSUM == 1) {
+      if ((pc & 3) == 0) {
+        *reinterpret_cast<_Float16*>(step + 16 * 1024 + 2 * (pc >> 2)) = hi;
+        *reinterpret_cast<_Float16*>(step + 16 * 1024 + 512 + 2 * (pc >> 2)) = lo;
+      }
+    } else if ((pc & 1) == 0) {
+      const int sb = pc >> 1;
+      *reinterpret_cast<_Float16*>(step + 16 * 1024 + 512 * (sb >> 3) + 2 * (sb & 7)) = hi;
+      *reinterpret_cast<_Float16*>(step + 17 * 1024 + 512 * (sb >> 3) + 2 * (sb & 7)) = lo;
+    }
+  }
 }
 
 // Row bytes of a step from LDS into registers (codes of kq_codes.h).  The long blocks come in two halves, to leave
@@ -105,6 +156,79 @@ __device__ __forceinline__ f16x8 fp4_frag(const R& row, int kg) {
     for (int e = 0; e < 4; e++) p[e] *= sp;
   }
   return f16x8{p[0][0], p[0][1], p[1][0], p[1][1], p[2][0], p[2][1], p[3][0], p[3][1]};
+}
+
+// acc += (32 weight rows of the step in LDS at b_lane) . (32 activation rows in the fragments a)
+template <int C>
+__device__ __forceinline__ void mid_step(const uint8_t* b_lane, int kg, const f16x8 (&a)[MidGeom<C>::NF], const Tables& tabs,
+                                         const kqfrag::KMasks& masks, int kvalid, f32x16& acc) {
+  if constexpr (k_quant<C>()) {
+    kqfrag::KRow<C> row;
+    row.load(b_lane, kg);
+    f32x16 part = f32x16{0};
+    StaticFor<16>::run([&](auto jc) {
+      constexpr int J = decltype(jc)::value;
+      f16x8 b[2];
+      row.template frag<J>(kg, masks, b);
+      part = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[J], b[0], part, 0, 0, 0);
+      if constexpr (kqfrag::KRow<C>::TERMS == 2) part = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[J], b[1], part, 0, 0, 0);
+    });
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[i] = fmaf(row.d, part[i], acc[i]);
+    if constexpr (kqfrag::KRow<C>::NSUM > 0) {
+      const f16x8 m = row.template min_frag<0>(kg);
+      part = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[16], m, f32x16{0}, 0, 0, 0);
+      if constexpr (kqfrag::KRow<C>::NSUM == 2) part = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[17], m, part, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[i] = fmaf(row.dm, part[i], acc[i]);
+    }
+  } else {
+    using G = CodeGeom<C>;
+    constexpr int MPS = G::SB / 16, PARTS = row_parts<C>(), JP = 16 / PARTS;
+    auto run = [&](auto full_c) {
+      constexpr bool FULL = decltype(full_c)::value;
+      f32x16 part[2];
+      f16x8 mins = {};
+      StaticFor<PARTS>::run([&](auto pc) {
+        constexpr int P = decltype(pc)::value;
+        RowPart<C, P> row;
+        row.load(b_lane);
+        StaticFor<JP>::run([&](auto jc) {
+          constexpr int J = P * JP + decltype(jc)::value;
+          if (FULL || 16 * J < kvalid) {  // uniform
+            if constexpr (C == KQ_NVFP4) {
+              acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[J], fp4_frag<C, J>(row, kg), acc, 0, 0, 0);
+              return;
+            }
+            f16x8 b;
+            if constexpr (C == KQ_MXFP4) b = fp4_frag<C, J>(row, kg);
+            else b = codes<C, J>(row, kg, tabs);
+            constexpr int sbi = J / MPS, slot = sbi & 1;
+            if constexpr (J % MPS == 0)
+              part[slot] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[J], b, f32x16{0}, 0, 0, 0);
+            else
+              part[slot] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[J], b, part[slot], 0, 0, 0);
+            if constexpr (J % MPS == MPS - 1) {
+              float mn;
+              const float sc = block_scale<C, sbi>(row, mn);
+#pragma unroll
+              for (int i = 0; i < 16; i++) acc[i] = fmaf(sc, part[slot][i], acc[i]);
+              if constexpr (G::HAS_MIN) mins[sbi] = (_Float16)mn;  // the f16 it came from
+            }
+          }
+        });
+      });
+      if constexpr (G::HAS_MIN) {  // blocks past the end of K: minimum 0 on sums of zeros
+        part[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[16], mins, f32x16{0}, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[i] = fmaf(32.0f, part[0][i], acc[i]);
+      }
+    };
+    if (kvalid >= CK_STEP)
+      run(std::true_type{});
+    else
+      run(std::false_type{});
+  }
 }
 
 // The step of a block that holds a row of wide range: bf16 activations as they are, weights by the reference-order decoder

@@ -1,0 +1,99 @@
+"""GPU parity of the one-launch gather_qmm of short contractions (K of one or two 256-weight steps, few rows per expert):
+every codec, tiles of weight rows that end inside the matrix, experts without entries, with one row, with more than the 32 rows
+of a round and more rounds than workgroups, ids outside the stack, rows of very different size, strided stacks."""
+import numpy as np
+import pytest
+import torch
+
+import kq
+import oracle_lib as O
+from gpu_util import bits_to_dev, dev_to_bits, rel_l2, wire_to_dev
+from test_gpu_moe import TOL, _idx_dev, _stack
+
+pytestmark = pytest.mark.gpu
+CODECS = sorted(kq.CODEC_GEOMETRY)
+
+
+def _case(codec, E, N, K, B, M, L, dtype, ids, seed):
+    w = _stack(codec, E, N, K, seed=seed)
+    rng = np.random.default_rng(seed + 1)
+    lhs = rng.integers(0, L, B)
+    x = rng.standard_normal((L, M, K)) * 10.0 ** rng.uniform(-3, 3 if dtype == "bfloat16" else 0, (L, M, 1))
+    xb = O.f32_to_bits(x.astype(np.float32), dtype)
+    return w, lhs, xb, bits_to_dev(xb, dtype)
+
+
+def _per_row(got, want, dtype):
+    """Largest relative error of a row: rows differ in size by powers of ten."""
+    g, w = got.reshape(-1, got.shape[-1]), want.reshape(-1, want.shape[-1])
+    return max(rel_l2(a, b, dtype) for a, b in zip(g, w))
+
+
+# a row of 24 ... 300 bf16 / f16 results: each off by half a unit in the last place at most beside sums in another order
+ROW_TOL = {"bfloat16": 2.0 ** -8, "float16": 2.0 ** -11}
+
+
+@pytest.mark.parametrize("codec", CODECS)
+@pytest.mark.parametrize("N,K,B,M,dtype", [(24, 256, 23, 1, "bfloat16"), (72, 512, 30, 3, "float16"), (136, 512, 9, 2, "bfloat16"),
+                                           (296, 256, 40, 5, "bfloat16"), (40, 512, 22, 70, "float16")])
+def test_few_rows_per_expert(codec, N, K, B, M, dtype):
+    E = 11
+    rng = np.random.default_rng(77)
+    rhs = rng.integers(0, E - 2, B)  # two experts without entries
+    rhs[0] = E - 1
+    w, lhs, xb, xt = _case(codec, E, N, K, B, M, 7, dtype, rhs, 501)
+    got = dev_to_bits(kq.gather_qmm(xt, wire_to_dev(w), None, codec, lhs_indices=_idx_dev(lhs), rhs_indices=_idx_dev(rhs)))
+    want = O.gather_qmm(xb, w, codec, lhs, rhs, True, dtype)
+    assert rel_l2(got, want, dtype) <= TOL, codec
+    assert _per_row(got, want, dtype) <= ROW_TOL[dtype], codec
+
+
+@pytest.mark.parametrize("codec", ["q4_k", "q8_0", "iq4_xs", "iq2_xs"])
+@pytest.mark.parametrize("B,M", [(1024, 1), (200, 7), (33, 1)])
+def test_most_entries_on_one_expert(codec, B, M):
+    E, N, K, dtype = 64, 40, 512, "bfloat16"
+    rng = np.random.default_rng(78)
+    rhs = np.where(rng.random(B) < 0.95, 5, rng.integers(0, E, B))
+    w, lhs, xb, xt = _case(codec, E, N, K, B, M, 9, dtype, rhs, 511)
+    got = dev_to_bits(kq.gather_qmm(xt, wire_to_dev(w), None, codec, lhs_indices=_idx_dev(lhs), rhs_indices=_idx_dev(rhs)))
+    want = O.gather_qmm(xb, w, codec, lhs, rhs, True, dtype)
+    assert _per_row(got, want, dtype) <= ROW_TOL[dtype], codec
+
+
+@pytest.mark.parametrize("codec", ["q6_k", "q8_0"])
+def test_strided_stack_and_repeated_replays(codec):
+    """Every second expert of a larger stack; the same call captured and replayed with other activations."""
+    E, N, K, B, dtype = 6, 48, 512, 24, "bfloat16"
+    rhs = np.arange(B) % E
+    w, lhs, xb, xt = _case(codec, 2 * E, N, K, B, 2, 5, dtype, rhs, 521)
+    wd, li, ri = wire_to_dev(w)[::2], _idx_dev(lhs), _idx_dev(rhs)
+    kq.gather_qmm(xt, wd, None, codec, lhs_indices=li, rhs_indices=ri)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y = kq.gather_qmm(xt, wd, None, codec, lhs_indices=li, rhs_indices=ri)
+    for k in range(3):
+        bits = O.f32_to_bits(np.random.default_rng(530 + k).standard_normal((5, 2, K)).astype(np.float32), dtype)
+        xt.copy_(bits_to_dev(bits, dtype))
+        g.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(dev_to_bits(y), O.gather_qmm(bits, w[::2], codec, lhs, rhs, True, dtype), dtype) <= TOL
+
+
+def test_ids_outside_the_stack_write_nothing():
+    E, N, K, B, codec, dtype = 5, 40, 256, 20, "q8_0", "bfloat16"
+    rhs = np.arange(B) % E
+    w, lhs, xb, xt = _case(codec, E, N, K, B, 1, 5, dtype, rhs, 541)
+    bad = rhs.copy()
+    bad[[3, 17]] = [E, 2 ** 31 - 1]
+    out = torch.full((B, 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    wd, li, ri = wire_to_dev(w), _idx_dev(lhs).to(torch.int32), _idx_dev(bad).to(torch.int32)
+    lib = kq._load()
+    rc = lib.kq_gather_qmm(xt.data_ptr(), wd.data_ptr(), li.data_ptr(), ri.data_ptr(), out.data_ptr(), B, 1, E, N, K, K,
+                           wd.stride(0), 1, 0, O.codec_id(codec), kq._DT[torch.bfloat16], None, 0, None)
+    assert rc == 0
+    torch.cuda.synchronize()
+    want = O.gather_qmm(xb, w, codec, lhs, rhs, True, dtype)
+    keep = [i for i in range(B) if i not in (3, 17)]
+    assert rel_l2(dev_to_bits(out)[keep], want[keep], dtype) <= TOL
+    assert bool((out[[3, 17]] == 7.0).all())
