@@ -34,7 +34,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32_a1 __attribute__((aligned(1)));  // the hardware serves unaligned dword loads
 
 constexpr int NT_WAVES = 4, NT_THREADS = 64 * NT_WAVES;
-constexpr int NT_KSTEP = 32, NT_COLS = 128;
+constexpr int NT_KSTEP = 32, NT_COLS = 128, NT_MERGE_ENTRIES = 1024;
 // Codecs whose 32-row form does not fit 256 registers (it spills up to 248 bytes per lane) take 64-row tiles on one
 // wave per SIMD beyond 32 rows (q6_k 4096 x 4096, 512 rows: 292 -> 146 us); for the others the 64-row form measured
 // level or slower (q8_0 93 -> 111 us).
@@ -51,7 +51,7 @@ struct NtArgs {
   void* y;
   const uint32_t* lhs;
   const uint32_t* rhs;
-  int M, N, K, E;
+  int M, N, K, E, B;
   int64_t x_batch_stride, w_expert_stride;
   int x_vec;  // activation rows can be read 16 bytes at a time (K % 8 == 0, aligned base and stride)
   // dense calls with few tiles: grid z cuts the K steps into ksplit ranges whose f32 partial sums go to `part`
@@ -88,10 +88,11 @@ struct NtGeom {
 
 // MR = 16-row groups of activations per workgroup (1: up to 16 rows, 2: 32, 4: 64 rows on one wave per SIMD, for
 // calls of many rows: every decoded weight then feeds four MFMAs)
-// MERGE (gathered calls of up to eight rows per entry that name some expert more than once): the workgroup of every
-// G-th entry of an expert, G = 16 / M, multiplies the rows of G entries in one tile, those of the entries between leave.
-// Which they are, every wave finds by itself in the entry list (512 ids a round of loads).  128 heads of 128 -> 512
-// q8_0, four sequences, 512 entries: the kernel 23 us before; with the opposite orientation of the same heads 41 -> 32 us.
+// MERGE (gathered calls of few rows per entry that name the experts more than once): grid z counts experts, and a workgroup
+// multiplies the rows of all entries of its expert, 16 MR at a time (grid y of them at once).  It asks for its first wire
+// bytes before it looks for the entries in the id list.  128 heads of 128 -> 512, us, 4 x 1 / 8 x 1 / 8 x 4 (sequences x rows), against
+// a workgroup per entry that looked for the others of its expert: q8_0 12.8 / 26.4 / 32.7 -> 8.4 / 8.6 / 11.5, q4_k 14.2 / 27.7 /
+// 34.5 -> 9.0 / 9.5 / 11.6, q6_k 15.9 / 29.5 / 37.6 -> 10.4 / 10.8 / 13.2.
 template <int C, int DT, int MR, bool MERGE = false>
 __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kernel(NtArgs a, const uint8_t* __restrict__ grids) {
   using G = NtGeom<C>;
@@ -101,37 +102,13 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
   float* red = reinterpret_cast<float*>(lds);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, h = lane >> 4;
-  const int item = a.ksplit > 1 ? 0 : blockIdx.z, split = a.ksplit > 1 ? blockIdx.z : 0;
-  const uint32_t e = a.rhs ? a.rhs[item] : 0u;
+  const int item = a.ksplit > 1 || MERGE ? 0 : blockIdx.z, split = a.ksplit > 1 ? blockIdx.z : 0;
+  const uint32_t e = MERGE ? blockIdx.z : a.rhs ? a.rhs[item] : 0u;
   if (e >= (uint32_t)a.E) return;  // the whole workgroup leaves: the entry's output rows stay untouched
-  static_assert(!MERGE || MR == 1, "merged entries share one 16-row tile");
-  __shared__ int entry[MERGE ? 16 : 1];
-  int nent = 1;
-  if constexpr (MERGE) {
-    // every wave writes the same values
-    const int per = 16 / a.M, B = gridDim.z;
-    int before = 0;
-    nent = 0;
-    for (int c0 = 0; c0 < B; c0 += 512) {
-      uint32_t id[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) id[u] = a.rhs[c0 + 64 * u + lane < B ? c0 + 64 * u + lane : 0];
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const int j0 = c0 + 64 * u, j = j0 + lane;
-        const uint64_t same = __builtin_amdgcn_ballot_w64(j < B && id[u] == e);
-        const uint64_t ahead = j0 + 64 <= item ? ~0ull : j0 > item ? 0ull : (1ull << (item - j0)) - 1;
-        before += __builtin_popcountll(same & ahead);
-        const uint64_t mine = same & ~ahead;
-        const int rank = nent + __builtin_popcountll(mine & ((1ull << lane) - 1));
-        if (((mine >> lane) & 1) && rank < per) entry[rank] = j;
-        nent += __builtin_popcountll(mine);
-      }
-    }
-    if (before % per != 0) return;  // uniform: an earlier workgroup has this entry
-    nent = nent < per ? nent : per;
-    __syncthreads();
-  }
+  static_assert(!MERGE || MR <= 2, "rows of a round");
+  __shared__ int entry_of[MERGE ? NT_MERGE_ENTRIES : 1];
+  __shared__ uint32_t lhs_of[MERGE ? NT_MERGE_ENTRIES : 1];
+  __shared__ int64_t x_off[MERGE ? 16 * MR : 1], y_row[MERGE ? 16 * MR : 1];
   const int tile = blockIdx.x;
   const int ngroups = a.N / 8;
   const int gi = tile * 16 + c;  // this lane's 8-column group
@@ -146,38 +123,27 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
   uint8_t* stage = lds + wave * NT_KSTEP * STRIDE;
   const uint8_t* blk = stage + (gp / GPB) * BPB;
   const int g = gp % GPB, klast = a.K - 1;
-  const int m0 = blockIdx.y * 16 * MR;
-  const int rows = MERGE ? nent * a.M : a.M;
   const uint16_t* xr[MR];
-#pragma unroll
-  for (int q = 0; q < MR; q++) {
-    int mrow = m0 + 16 * q + c < rows ? m0 + 16 * q + c : rows - 1;  // rows past the last repeat it, never stored
-    int it = item;
-    if constexpr (MERGE) it = entry[mrow / a.M], mrow %= a.M;
-    xr[q] = static_cast<const uint16_t*>(a.x) + (a.lhs ? (size_t)a.lhs[it] * (size_t)a.x_batch_stride : 0) +
-            (size_t)mrow * a.K;
-  }
-
-  f32x4 acc[MR][8];
-#pragma unroll
-  for (int q = 0; q < MR; q++)
-#pragma unroll
-    for (int t = 0; t < 8; t++) acc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-
   uint32_t wreg[NDW], xreg[MR][4];
   // Rows past K repeat the last row (their activations are zero).  No branch stands between the loads, so they are
   // all in flight together: a lane past the end of the step or of a short piece reads a clamped address, and the
   // last bytes of a piece come out of the dword that ends with the piece, shifted (never a byte past a row's end).
-  auto fetch = [&](int st) {
+  auto fetch_w = [&](int st) {
+    int l = lane;
+    // the addresses are not kept from one use to the next: most merged waves have one step, and 27 addresses of q6_k spilled 76
+    // registers over the loop of rounds
+    if constexpr (MERGE) asm volatile("" : "+v"(l));
 #pragma unroll
     for (int j = 0; j < NDW; j++) {
-      const int idx = lane + 64 * j < NT_KSTEP * PDW ? lane + 64 * j : NT_KSTEP * PDW - 1;
+      const int idx = l + 64 * j < NT_KSTEP * PDW ? l + 64 * j : NT_KSTEP * PDW - 1;
       const int row = idx / PDW, boff = 4 * (idx - row * PDW);
       const int eoff = boff < piece_here - 4 ? boff : piece_here - 4;
       const int k = NT_KSTEP * st + row < a.K ? NT_KSTEP * st + row : klast;
       const uint32_t v = *reinterpret_cast<const u32_a1*>(wt + (size_t)k * row_bytes + eoff);
       wreg[j] = v >> (8 * ((boff - eoff) & 3));
     }
+  };
+  auto fetch_x = [&](int st) {
     const int k0 = NT_KSTEP * st + 8 * h;
 #pragma unroll
     for (int q = 0; q < MR; q++) {
@@ -198,122 +164,203 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
   const int steps_all = (a.K + NT_KSTEP - 1) / NT_KSTEP;
   const int st_begin = split * a.steps_per_split;
   const int nsteps = st_begin + a.steps_per_split < steps_all ? st_begin + a.steps_per_split : steps_all;
-  if (st_begin + wave < nsteps) fetch(st_begin + wave);
-  for (int st = st_begin + wave; st < nsteps; st += NT_WAVES) {
+  int rows = a.M, m0 = MERGE ? 0 : blockIdx.y * 16 * MR;
+  if constexpr (MERGE) {
+    if (blockIdx.y == 0 && st_begin + wave < nsteps) fetch_w(st_begin + wave);
+    // places in the order of the list, the same in every workgroup of the expert
+    constexpr int NU = NT_MERGE_ENTRIES / NT_THREADS;
+    __shared__ __attribute__((aligned(16))) int counts[NU][NT_WAVES];
+    const int tid = threadIdx.x, B = a.B;
+    uint32_t id[NU], lh[NU];
+    uint64_t hit[NU];
 #pragma unroll
-    for (int j = 0; j < NDW; j++) {
-      const int idx = lane + 64 * j;
-      if (idx < NT_KSTEP * PDW) *reinterpret_cast<uint32_t*>(stage + 4 * idx) = wreg[j];
+    for (int u = 0; u < NU; u++) {
+      if (NT_THREADS * u >= B) break;  // uniform
+      const int j = tid + NT_THREADS * u;
+      id[u] = j < B ? a.rhs[j] : ~0u;
+      lh[u] = j < B ? a.lhs[j] : 0u;
     }
-    bf16x8 ah[MR], al[MR];
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      if (NT_THREADS * u >= B) break;
+      hit[u] = __builtin_amdgcn_ballot_w64(id[u] == e);
+      if (lane == 0) counts[u][wave] = __builtin_popcountll(hit[u]);
+    }
+    __syncthreads();
+    int count = 0;
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      if (NT_THREADS * u >= B) break;
+      const int4 n = *reinterpret_cast<const int4*>(counts[u]);
+      const int before = (wave > 0 ? n.x : 0) + (wave > 1 ? n.y : 0) + (wave > 2 ? n.z : 0);
+      if ((hit[u] >> lane) & 1) {
+        const int place = count + before + __builtin_popcountll(hit[u] & ((1ull << lane) - 1));
+        entry_of[place] = tid + NT_THREADS * u;
+        lhs_of[place] = lh[u];
+      }
+      count += n.x + n.y + n.z + n.w;
+    }
+    rows = count * a.M;
+    m0 = 16 * MR * blockIdx.y;
+    if (m0 >= rows) return;  // uniform
+  }
+  bool first = MERGE && blockIdx.y == 0;
+#pragma unroll 1
+  for (;;) {  // MERGE: rounds of 16 MR rows; once otherwise
+    if constexpr (MERGE) {
+      __syncthreads();
+      if ((int)threadIdx.x < 16 * MR) {  // rows past the last repeat it, never stored
+        const int r = m0 + (int)threadIdx.x < rows ? m0 + (int)threadIdx.x : rows - 1, place = r / a.M, m = r - place * a.M;
+        x_off[threadIdx.x] = (int64_t)lhs_of[place] * a.x_batch_stride + (int64_t)m * a.K;
+        y_row[threadIdx.x] = (int64_t)entry_of[place] * a.M + m;
+      }
+      __syncthreads();
+    }
 #pragma unroll
     for (int q = 0; q < MR; q++) {
-      if constexpr (DT == KQ_BF16) {
-        ah[q] = __builtin_bit_cast(bf16x8, make_uint4(xreg[q][0], xreg[q][1], xreg[q][2], xreg[q][3]));
+      if constexpr (MERGE) {
+        xr[q] = static_cast<const uint16_t*>(a.x) + x_off[16 * q + c];
       } else {
-        uint32_t hi[4], lo[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const float f0 = kq::h2f((uint16_t)(xreg[q][j] & 0xffffu)), f1 = kq::h2f((uint16_t)(xreg[q][j] >> 16));
-          hi[j] = pack_hi(f0, f1);
-          lo[j] = pack_hi(f0 - trunc_bf16(f0), f1 - trunc_bf16(f1));  // exact: 11 significant bits in all
-        }
-        ah[q] = __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
-        al[q] = __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+        const int mrow = m0 + 16 * q + c < a.M ? m0 + 16 * q + c : a.M - 1;  // rows past the last repeat it, never stored
+        xr[q] = static_cast<const uint16_t*>(a.x) + (a.lhs ? (size_t)a.lhs[item] * (size_t)a.x_batch_stride : 0) + (size_t)mrow * a.K;
       }
     }
-    if (st + NT_WAVES < nsteps) fetch(st + NT_WAVES);
-    // weights: rows 8h ... 8h + 7 of the step, column group of this lane, split into bf16 hi / lo and regrouped by
-    // column
-    uint32_t bh[8][4], bl[8][4];
+    f32x4 acc[MR][8];
 #pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-      float w0[8], w1[8];
-      kq::decode8<C>(blk + (8 * h + i) * STRIDE, g, grids, w0);
-      kq::decode8<C>(blk + (8 * h + i + 1) * STRIDE, g, grids, w1);
+    for (int q = 0; q < MR; q++)
 #pragma unroll
-      for (int t = 0; t < 8; t++) {
-        bh[t][i >> 1] = pack_hi(w0[t], w1[t]);
-        bl[t][i >> 1] = pack_rne(w0[t] - trunc_bf16(w0[t]), w1[t] - trunc_bf16(w1[t]));
-      }
+      for (int t = 0; t < 8; t++) acc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (st_begin + wave < nsteps) {
+      if (!first) fetch_w(st_begin + wave);
+      fetch_x(st_begin + wave);
     }
+    first = false;
+    for (int st = st_begin + wave; st < nsteps; st += NT_WAVES) {
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
-      const bf16x8 wh = __builtin_bit_cast(bf16x8, make_uint4(bh[t][0], bh[t][1], bh[t][2], bh[t][3]));
-      const bf16x8 wl = __builtin_bit_cast(bf16x8, make_uint4(bl[t][0], bl[t][1], bl[t][2], bl[t][3]));
+      for (int j = 0; j < NDW; j++) {
+        const int idx = lane + 64 * j;
+        if (idx < NT_KSTEP * PDW) *reinterpret_cast<uint32_t*>(stage + 4 * idx) = wreg[j];
+      }
+      bf16x8 ah[MR], al[MR];
 #pragma unroll
       for (int q = 0; q < MR; q++) {
-        acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[q], wh, acc[q][t], 0, 0, 0);
-        acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[q], wl, acc[q][t], 0, 0, 0);
-        if constexpr (DT == KQ_F16) acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[q], wh, acc[q][t], 0, 0, 0);
+        if constexpr (DT == KQ_BF16) {
+          ah[q] = __builtin_bit_cast(bf16x8, make_uint4(xreg[q][0], xreg[q][1], xreg[q][2], xreg[q][3]));
+        } else {
+          uint32_t hi[4], lo[4];
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const float f0 = kq::h2f((uint16_t)(xreg[q][j] & 0xffffu)), f1 = kq::h2f((uint16_t)(xreg[q][j] >> 16));
+            hi[j] = pack_hi(f0, f1);
+            lo[j] = pack_hi(f0 - trunc_bf16(f0), f1 - trunc_bf16(f1));  // exact: 11 significant bits in all
+          }
+          ah[q] = __builtin_bit_cast(bf16x8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+          al[q] = __builtin_bit_cast(bf16x8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+        }
+      }
+      if (st + NT_WAVES < nsteps) {
+        fetch_w(st + NT_WAVES);
+        fetch_x(st + NT_WAVES);
+      }
+      // weights: rows 8h ... 8h + 7 of the step, column group of this lane, split into bf16 hi / lo and regrouped by
+      // column
+      uint32_t bh[8][4], bl[8][4];
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) {
+        float w0[8], w1[8];
+        kq::decode8<C>(blk + (8 * h + i) * STRIDE, g, grids, w0);
+        kq::decode8<C>(blk + (8 * h + i + 1) * STRIDE, g, grids, w1);
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+          bh[t][i >> 1] = pack_hi(w0[t], w1[t]);
+          bl[t][i >> 1] = pack_rne(w0[t] - trunc_bf16(w0[t]), w1[t] - trunc_bf16(w1[t]));
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 8; t++) {
+        const bf16x8 wh = __builtin_bit_cast(bf16x8, make_uint4(bh[t][0], bh[t][1], bh[t][2], bh[t][3]));
+        const bf16x8 wl = __builtin_bit_cast(bf16x8, make_uint4(bl[t][0], bl[t][1], bl[t][2], bl[t][3]));
+#pragma unroll
+        for (int q = 0; q < MR; q++) {
+          acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[q], wh, acc[q][t], 0, 0, 0);
+          acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[q], wl, acc[q][t], 0, 0, 0);
+          if constexpr (DT == KQ_F16) acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[q], wh, acc[q][t], 0, 0, 0);
+        }
       }
     }
-  }
 
-  if (nsteps - st_begin > 1) {  // uniform over the workgroup: waves 2, 3 -> waves 0, 1, then wave 1 -> wave 0
-    constexpr int NACC = 32 * MR;
-    __syncthreads();  // every wave is done with its staging area
-    float* mine = red + (size_t)(wave & 1) * NACC * 64 + lane;
-    auto put = [&](float* dst) {
+    if (nsteps - st_begin > 1) {  // uniform over the workgroup: waves 2, 3 -> waves 0, 1, then wave 1 -> wave 0
+      constexpr int NACC = 32 * MR;
+      __syncthreads();  // every wave is done with its staging area
+      float* mine = red + (size_t)(wave & 1) * NACC * 64 + lane;
+      auto put = [&](float* dst) {
 #pragma unroll
-      for (int q = 0; q < MR; q++)
+        for (int q = 0; q < MR; q++)
 #pragma unroll
-        for (int t = 0; t < 8; t++)
+          for (int t = 0; t < 8; t++)
 #pragma unroll
-          for (int r = 0; r < 4; r++) dst[((q * 8 + t) * 4 + r) * 64] = acc[q][t][r];
-    };
-    auto add = [&](const float* src) {
+            for (int r = 0; r < 4; r++) dst[((q * 8 + t) * 4 + r) * 64] = acc[q][t][r];
+      };
+      auto add = [&](const float* src) {
 #pragma unroll
-      for (int q = 0; q < MR; q++)
+        for (int q = 0; q < MR; q++)
 #pragma unroll
-        for (int t = 0; t < 8; t++)
+          for (int t = 0; t < 8; t++)
 #pragma unroll
-          for (int r = 0; r < 4; r++) acc[q][t][r] += src[((q * 8 + t) * 4 + r) * 64];
-    };
-    if (wave >= 2) put(mine);
-    __syncthreads();
-    if (wave < 2) add(mine);
-    __syncthreads();
-    if (wave == 1) put(red + lane);
-    __syncthreads();
-    if (wave == 0) add(red + lane);
-  }
-  if (wave != 0 || !col_ok) return;
-  if (a.ksplit > 1) {
-    float* pb = a.part + (size_t)split * a.M * a.N + 8 * (size_t)gi;
+            for (int r = 0; r < 4; r++) acc[q][t][r] += src[((q * 8 + t) * 4 + r) * 64];
+      };
+      if (wave >= 2) put(mine);
+      __syncthreads();
+      if (wave < 2) add(mine);
+      __syncthreads();
+      if (wave == 1) put(red + lane);
+      __syncthreads();
+      if (wave == 0) add(red + lane);
+    }
+    if constexpr (!MERGE) {
+      if (wave != 0 || !col_ok) return;
+    }
+    if (!MERGE && a.ksplit > 1) {
+      float* pb = a.part + (size_t)split * a.M * a.N + 8 * (size_t)gi;
+#pragma unroll
+      for (int q = 0; q < MR; q++) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int m = m0 + 16 * q + 4 * h + r;
+          if (m < a.M) {
+            float4* o = reinterpret_cast<float4*>(pb + (size_t)m * a.N);
+            o[0] = make_float4(acc[q][0][r], acc[q][1][r], acc[q][2][r], acc[q][3][r]);
+            o[1] = make_float4(acc[q][4][r], acc[q][5][r], acc[q][6][r], acc[q][7][r]);
+          }
+        }
+      }
+      return;
+    }
+    uint16_t* yb = static_cast<uint16_t*>(a.y) + 8 * (size_t)gi;
+    if (wave == 0 && col_ok)
 #pragma unroll
     for (int q = 0; q < MR; q++) {
 #pragma unroll
       for (int r = 0; r < 4; r++) {
         const int m = m0 + 16 * q + 4 * h + r;
-        if (m < a.M) {
-          float4* o = reinterpret_cast<float4*>(pb + (size_t)m * a.N);
-          o[0] = make_float4(acc[q][0][r], acc[q][1][r], acc[q][2][r], acc[q][3][r]);
-          o[1] = make_float4(acc[q][4][r], acc[q][5][r], acc[q][6][r], acc[q][7][r]);
+        if (m < rows) {
+          uint32_t o[4];
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const float v0 = acc[q][2 * j][r], v1 = acc[q][2 * j + 1][r];
+            const uint16_t lo = DT == KQ_F16 ? kq::f2f16(v0) : kq::f2bf16(v0);
+            const uint16_t hi = DT == KQ_F16 ? kq::f2f16(v1) : kq::f2bf16(v1);
+            o[j] = (uint32_t)lo | ((uint32_t)hi << 16);
+          }
+          const size_t row = MERGE ? (size_t)y_row[m - m0] : (size_t)item * a.M + m;
+          *reinterpret_cast<uint4*>(yb + row * a.N) = make_uint4(o[0], o[1], o[2], o[3]);
         }
       }
     }
-    return;
-  }
-  uint16_t* yb = static_cast<uint16_t*>(a.y) + 8 * (size_t)gi;
-#pragma unroll
-  for (int q = 0; q < MR; q++) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      const int m = m0 + 16 * q + 4 * h + r;
-      if (m < rows) {
-        uint32_t o[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const float v0 = acc[q][2 * j][r], v1 = acc[q][2 * j + 1][r];
-          const uint16_t lo = DT == KQ_F16 ? kq::f2f16(v0) : kq::f2bf16(v0);
-          const uint16_t hi = DT == KQ_F16 ? kq::f2f16(v1) : kq::f2bf16(v1);
-          o[j] = (uint32_t)lo | ((uint32_t)hi << 16);
-        }
-        const size_t row = MERGE ? (size_t)entry[m / a.M] * a.M + m % a.M : (size_t)item * a.M + m;
-        *reinterpret_cast<uint4*>(yb + row * a.N) = make_uint4(o[0], o[1], o[2], o[3]);
-      }
-    }
+    if constexpr (!MERGE) return;
+    m0 += 16 * MR * gridDim.y;
+    if (m0 >= rows) return;
+    __syncthreads();  // the sums have been read: the staging areas may be filled again
   }
 }
 
@@ -765,9 +812,15 @@ bool nt_tall(int codec, int M, int N, int K, bool cut, int entries) {
   return tall <= (steps / st < 8 ? codec == KQ_Q2_K || codec == KQ_Q4_1 ? 0.95 : 1.05 : 1.19) * wide;
 }
 
-// Entries of one expert share tiles: two or more fit a tile, an expert comes twice on average, and the list is short enough
-// to be searched by every workgroup (1024 ids: two rounds of loads, about 1 us beside the 5 us a workgroup works).
-bool nt_merge(int M, int B, int E, bool gathered) { return gathered && M <= 8 && B >= 2 * E && B <= 1024; }
+// Entries of one expert share tiles (gathered calls in which an expert comes twice on average, of a list short enough to be
+// searched by every workgroup): where the rows of an entry fill half a tile at most, or a tile and the unmerged workgroups would
+// be more than two rounds of two per CU, or 32 rows of the codec that spills without.  Merged / not, us, entries of 16 rows,
+// four sequences: 128 heads of 128 x 512 q8_0 21.8 / 24.2, q4_k 22.6 / 27.9, 64 of 192 x 512 13.6 / 16.7, 16.4 / 21.0, but 32 of
+// 128 x 256 8.6 / 6.3, 8.9 / 6.8; of 32 rows, two sequences, 128 heads q8_0 21.3 / 18.5, q6_k 25.0 / 30.1.
+bool nt_merge(int M, int B, int E, int N, int codec, bool gathered) {
+  if (!gathered || B < 2 * E || B > NT_MERGE_ENTRIES || E > 65535) return false;
+  return M <= 8 || (M <= 16 && (int64_t)B * ((N + NT_COLS - 1) / NT_COLS) >= 4 * kq_num_cus()) || (M <= 32 && nt_wide(codec));
+}
 
 template <int C>
 struct NtRun {
@@ -781,6 +834,10 @@ struct NtRun {
   template <int DT, int MR, bool MERGE = false>
   static void go(const NtArgs& a, int B, const uint8_t* grids, hipStream_t s) {
     dim3 grid((a.N + NT_COLS - 1) / NT_COLS, (a.M + 16 * MR - 1) / (16 * MR), a.ksplit > 1 ? a.ksplit : B);
+    if (MERGE) {  // rounds of an expert that run at once: what it has on average
+      grid.y = (unsigned)(((int64_t)B * a.M + 16 * MR * a.E - 1) / (16 * MR * a.E));
+      grid.z = a.E;
+    }
     hipLaunchKernelGGL((gemm_nt_mfma_kernel<C, DT, MR, MERGE>), grid, dim3(NT_THREADS), 0, s, a, grids);
     reduce<DT>(a, s);
   }
@@ -808,8 +865,11 @@ struct NtRun {
   static int run(const NtArgs& a, int B, int dt, const uint8_t* grids, hipStream_t s) {
     if (a.M >= NT_SHARED_ROWS) {
       dt == KQ_F16 ? many_rows<KQ_F16>(a, B, grids, s) : many_rows<KQ_BF16>(a, B, grids, s);
-    } else if (nt_merge(a.M, B, a.E, a.rhs != nullptr)) {
-      dt == KQ_F16 ? go<KQ_F16, 1, true>(a, B, grids, s) : go<KQ_BF16, 1, true>(a, B, grids, s);
+    } else if (nt_merge(a.M, B, a.E, a.N, C, a.rhs != nullptr)) {
+      if ((int64_t)B * a.M <= 16 * (int64_t)a.E)
+        dt == KQ_F16 ? go<KQ_F16, 1, true>(a, B, grids, s) : go<KQ_BF16, 1, true>(a, B, grids, s);
+      else
+        dt == KQ_F16 ? go<KQ_F16, 2, true>(a, B, grids, s) : go<KQ_BF16, 2, true>(a, B, grids, s);
     } else if (a.M <= 16) {
       dt == KQ_F16 ? go<KQ_F16, 1>(a, B, grids, s) : go<KQ_BF16, 1>(a, B, grids, s);
     } else if (nt_wide(C) && a.M > 32) {
@@ -857,7 +917,7 @@ int kq_launch_nt_mfma(const void* x, const uint8_t* w, const uint32_t* lhs, cons
   if (reinterpret_cast<uintptr_t>(out) & 15) return KQ_ERR_UNSUPPORTED;
   const uint8_t* grids = kq_device_grids();
   if (!grids) return KQ_ERR_HIP;
-  NtArgs a{x, w, out, lhs, rhs, M, N, K, E, x_batch_stride, w_expert_stride, 0, 1, 0, nullptr, false};
+  NtArgs a{x, w, out, lhs, rhs, M, N, K, E, B, x_batch_stride, w_expert_stride, 0, 1, 0, nullptr, false};
   a.x_vec = !(K & 7) && !(reinterpret_cast<uintptr_t>(x) & 15) && !(x_batch_stride & 7);
   // K is cut into the ranges that kq_nt_workspace_bytes was asked for, into what fits where unaligned activations turn the call
   // to the 128-row kernel, or not at all

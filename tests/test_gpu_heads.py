@@ -97,3 +97,23 @@ def test_ids_outside_the_stack_write_nothing():
     keep = [i for i in range(B) if i not in (3, 17)]
     assert rel_l2(dev_to_bits(out)[keep], want[keep], dtype) <= TOL
     assert bool((out[[3, 17]] == 7.0).all())
+
+
+@pytest.mark.parametrize("codec", ["q8_0", "q4_k", "q6_k", "iq3_s", "q5_1", "nvfp4"])
+@pytest.mark.parametrize("K,M,B,dtype", [(96, 1, 40, "bfloat16"), (130, 3, 31, "float16"), (64, 8, 200, "bfloat16"),
+                                         (192, 16, 30, "bfloat16"), (100, 24, 23, "bfloat16")])
+def test_other_orientation_merges_entries(codec, K, M, B, dtype):
+    """transpose=False, entries of one expert in shared tiles: most of them on one expert (several rounds), experts without any,
+    rows that cannot be read 16 bytes at a time, a last step of K that is not whole, a last column tile that is not."""
+    E, N, L = 11, 768 if codec in ("q4_k", "q6_k", "iq3_s") else 320, 9
+    rng = np.random.default_rng(79)
+    rhs = np.where(rng.random(B) < 0.7, 4, rng.integers(0, E - 2, B))
+    w = _stack(codec, E, K, N, seed=551)  # K wire rows of N weights
+    lhs = rng.integers(0, L, B)
+    xb = O.f32_to_bits((rng.standard_normal((L, M, K)) * 10.0 ** rng.uniform(-2, 2, (L, M, 1))).astype(np.float32), dtype)
+    xt = bits_to_dev(xb, dtype)
+    got = dev_to_bits(kq.gather_qmm(xt, wire_to_dev(w), None, codec, lhs_indices=_idx_dev(lhs), rhs_indices=_idx_dev(rhs),
+                                    transpose=False))
+    want = O.gather_qmm(xb, w, codec, lhs, rhs, False, dtype)
+    assert rel_l2(got, want, dtype) <= TOL, codec
+    assert _per_row(got, want, dtype) <= ROW_TOL[dtype], codec
