@@ -914,7 +914,7 @@ __device__ __forceinline__ void q6k_unit(const uint8_t* __restrict__ bl, float d
 template <int MB>
 constexpr int st_xch() { return MB > 4 ? 2 : MB; }  // activation rows staged at a time
 
-// XU = units (superblocks) a wave handles per tile at most: 4 or 8, i.e. K ranges of up to 16 or 32 superblocks
+// XU = units (superblocks) a wave handles per tile at most: 4 or 8, i.e. K ranges of up to 4 NW or 8 NW superblocks
 // per workgroup (the A registers of all of them stay resident).
 // NW = waves per workgroup (4 or 8): wave w owns superblocks sb_begin + w + NW u of the workgroup's K range.
 // GM = 0: dense.  GM = 1: gathered, one tile of one entry per workgroup.  GM = 2: gathered gate / up pair: a
@@ -1586,25 +1586,45 @@ constexpr int st_nw8_rows() {
   return st_lds_bytes<C, 4, 2, 4, 8>() <= 160 * 1024 ? 4 : st_lds_bytes<C, 2, 2, 4, 8>() <= 160 * 1024 ? 2 :
          st_lds_bytes<C, 1, 2, 4, 8>() <= 160 * 1024 ? 1 : 0;
 }
-int st_max_sb(int codec, int M) {
-  if (!g_st_nw8) return 16;
-  int rows = 0;
+// and rows up to which an eight-wave workgroup of eight units per wave (K ranges of up to 64 superblocks) fits
+template <int C>
+constexpr int st_long_rows() {
+  // (one row's codebook tables are the larger ones: iq3_s and iq2_xxs fit with neither)
+  return st_lds_bytes<C, 1, 2, 8, 8>() > 160 * 1024 ? 0 : st_lds_bytes<C, 2, 2, 8, 8>() <= 160 * 1024 ? 2 : 1;
+}
+struct StRows {
+  int nw8, lng;
+};
+template <int C>
+constexpr StRows st_rows_of() {
+  return StRows{st_nw8_rows<C>(), st_long_rows<C>()};
+}
+StRows st_rows(int codec) {
   switch (codec) {
-    case KQ_Q2_K: rows = st_nw8_rows<KQ_Q2_K>(); break;
-    case KQ_Q3_K: rows = st_nw8_rows<KQ_Q3_K>(); break;
-    case KQ_Q4_K: rows = st_nw8_rows<KQ_Q4_K>(); break;
-    case KQ_Q5_K: rows = st_nw8_rows<KQ_Q5_K>(); break;
-    case KQ_Q6_K: rows = st_nw8_rows<KQ_Q6_K>(); break;
-    case KQ_IQ4_XS: rows = st_nw8_rows<KQ_IQ4_XS>(); break;
-    case KQ_IQ2_XXS: rows = st_nw8_rows<KQ_IQ2_XXS>(); break;
-    case KQ_IQ3_S: rows = st_nw8_rows<KQ_IQ3_S>(); break;
-    case KQ_Q8_0: rows = st_nw8_rows<KQ_Q8_0>(); break;
-    case KQ_IQ4_NL: rows = st_nw8_rows<KQ_IQ4_NL>(); break;
-    case KQ_Q4_0: rows = st_nw8_rows<KQ_Q4_0>(); break;
-    case KQ_MXFP4: rows = st_nw8_rows<KQ_MXFP4>(); break;
-    case KQ_NVFP4: rows = st_nw8_rows<KQ_NVFP4>(); break;
+    case KQ_Q2_K: return st_rows_of<KQ_Q2_K>();
+    case KQ_Q3_K: return st_rows_of<KQ_Q3_K>();
+    case KQ_Q4_K: return st_rows_of<KQ_Q4_K>();
+    case KQ_Q5_K: return st_rows_of<KQ_Q5_K>();
+    case KQ_Q6_K: return st_rows_of<KQ_Q6_K>();
+    case KQ_IQ4_XS: return st_rows_of<KQ_IQ4_XS>();
+    case KQ_IQ2_XXS: return st_rows_of<KQ_IQ2_XXS>();
+    case KQ_IQ3_S: return st_rows_of<KQ_IQ3_S>();
+    case KQ_Q8_0: return st_rows_of<KQ_Q8_0>();
+    case KQ_IQ4_NL: return st_rows_of<KQ_IQ4_NL>();
+    case KQ_Q4_0: return st_rows_of<KQ_Q4_0>();
+    case KQ_MXFP4: return st_rows_of<KQ_MXFP4>();
+    case KQ_NVFP4: return st_rows_of<KQ_NVFP4>();
   }
-  return M <= rows ? 32 : 16;
+  return StRows{0, 0};
+}
+int st_max_sb(int codec, int M) { return g_st_nw8 && M <= st_rows(codec).nw8 ? 32 : 16; }
+// longest row (superblocks) up to which matrices of at most CUs / 2 tiles take short tiles, below which a split is slower:
+// q4_k, two rows, 4096 x 11008 9.4 -> 9.1 but x 14336 10.1 against 10.5; q2_k 9.3 -> 8.1 and 9.3 against 9.5, two rows 9.5 ->
+// 8.6 at 8448 and 9.3 against 9.5 at 11008
+int st_long_max(int codec, int M) {
+  if (codec == KQ_Q4_K) return M == 1 ? 64 : 48;
+  if (codec == KQ_Q2_K) return M == 1 ? 48 : 40;
+  return 0;
 }
 StSplit st_split_plan(int M, int N, int K, int codec, int cus) {
   const int nsb = K >> 8, tiles = (N + ST_ROWS - 1) / ST_ROWS, maxsb = st_max_sb(codec, M);
@@ -1623,6 +1643,17 @@ StSplit st_split_plan(int M, int N, int K, int codec, int cus) {
     int r = (N + cus - 1) / cus;
     if (r < 8) r = 8;
     if (r < ST_ROWS) return StSplit{1, nsb > 16 ? nsb : 17, r};  // sb_per_split > 16 selects the eight-wave kernel
+  }
+  // 33 .. 64 superblocks: the same with eight units per wave.  Its time depends on K alone (a unit takes as long for 16 rows as
+  // for 32), the split's on the matrix: two splits are one round of workgroups up to cus / 2 tiles and two from there on, so
+  // beyond that the short tiles win for every codec (5120 x 13824, one row, us with the host, split before: q4_k 12.4 -> 9.3,
+  // q5_k 15.5 -> 12.4, q6_k 20.3 -> 16.7, iq4_xs 13.6 -> 12.5, nvfp4 15.0 -> 13.8).  Below, only the codecs of few instructions
+  // per unit do, up to st_long_max superblocks (q4_k, 4096 x 8448: 9.4 -> 7.0, 4096 x 14336: 9.8 -> 9.1; q6_k 13.0 against 13.5).
+  if (g_st_short_tiles && nsb > 32 && nsb <= 64 && M <= st_rows(codec).lng && tiles < cus &&
+      (2 * tiles > cus || nsb <= st_long_max(codec, M))) {
+    int r = (N + cus - 1) / cus;
+    if (r < 8) r = 8;
+    if (r < ST_ROWS) return StSplit{1, nsb, r};
   }
   int per = (nsb + want - 1) / want;
   if (per > maxsb) per = maxsb;
@@ -1667,6 +1698,12 @@ int st_launch_one(StArgs a, int splits, hipStream_t s) {
 template <int C, int DT>
 int st_launch_m(const StArgs& a, int splits, hipStream_t s) {
   constexpr int D = 2;  // units in LDS per wave; 3 and 4 measured slower for every codec
+  if (a.sb_per_split > 32) {
+    if constexpr (st_long_rows<C>() >= 1)
+      if (a.M == 1) return st_launch_one<C, DT, 1, D, 8, 8>(a, splits, s);
+    if constexpr (st_long_rows<C>() >= 2) return st_launch_one<C, DT, 2, D, 8, 8>(a, splits, s);
+    return KQ_ERR_UNSUPPORTED;
+  }
   if (a.sb_per_split > 16) {
     // K ranges of 17 .. 32 superblocks: eight waves of four units (st_max_sb allows this for up to four rows).
     // Four waves of eight units, the alternative without more waves, took 9.0 instead of 7.1 us on q2_k 8192^2.

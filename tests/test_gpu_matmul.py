@@ -142,6 +142,25 @@ def test_qmm_streamed_kernel_shapes(kq, codec, dtype):
         assert rel_l2(dev_to_bits(got), want, dtype) <= TOL, (codec, dtype, M, N, K)
 
 
+@pytest.mark.parametrize("codec", ["q4_k", "q5_k", "q6_k", "q2_k", "q3_k", "iq4_xs", "q4_0", "mxfp4", "nvfp4"])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+def test_qmm_streamed_kernel_long_rows_in_short_tiles(kq, codec, dtype):
+    """33 to 64 superblocks in one workgroup (eight units per wave) instead of a K split: the first and the last length, waves of
+    unequal unit counts, the least height that every codec takes (17 rows, the last tile ragged), the largest (31 rows), a K
+    that ends inside a unit, and 8-row tiles of the codecs that take matrices of any height."""
+    shapes = [(1, 4100, 33 * 256), (1, 7930, 37 * 256), (2, 4200, 41 * 256), (1, 4097, 64 * 256), (2, 7900, 64 * 256)]
+    if codec in ("q4_0", "mxfp4"):
+        shapes.append((1, 4111, 40 * 256 + 96))
+    if codec in ("q4_k", "q2_k"):
+        shapes += [(1, 100, 48 * 256), (2, 1001, 40 * 256), (1, 2050, 33 * 256)]
+    for M, N, K in shapes:
+        wire = _wire(codec, N, K, seed=45)
+        xb, xt = make_x((M, K), dtype, seed=46)
+        got = kq.quantized_matmul(xt, wire_to_dev(wire), None, codec)
+        want = O.qmm(xb, wire, codec, True, dtype)
+        assert rel_l2(dev_to_bits(got), want, dtype) <= TOL, (codec, dtype, M, N, K)
+
+
 @pytest.mark.parametrize("codec", ["mxfp4", "q4_0", "iq4_nl", "q8_0"])
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
 def test_qmm_streamed_kernel_k_ends_inside_a_unit(kq, codec, dtype):
