@@ -37,16 +37,23 @@ using kqmma::RowRange;
 // rs[m] is negative for a wide row (RowRange).
 constexpr int MP_THREADS = 512, MP_REGS = 4;
 
+// Row of a workgroup.  Eight neighbouring rows write the 16-byte eighths of the same 128-byte lines, and workgroups go to the
+// eight XCDs in turn: rows are dealt so that those eight meet in one L2, which then writes back whole lines.
+__device__ __forceinline__ int prepass_row_of(int b) { return 64 * (b >> 6) + 8 * (b & 7) + ((b >> 3) & 7); }
+constexpr int prepass_grid(int M) { return (M + 63) & ~63; }
+
 template <int DT, int ORD, int NSUM>
 __global__ __launch_bounds__(MP_THREADS) void mid_prepass_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ xf,
-                                                                 float* __restrict__ rs, int K, int nsteps,
+                                                                 float* __restrict__ rs, int M, int K, int nsteps,
                                                                  int* __restrict__ counters, int ncounters) {
   constexpr int NF = 16 + NSUM;
   __shared__ float red[MP_THREADS / 64];
   __shared__ uint32_t range_lds[MP_THREADS / 64 + 2];
-  const int m = blockIdx.x, tid = threadIdx.x;
+  const int tid = threadIdx.x;
   // arrival counters of the main kernel's cut tiles
-  for (int i = m * MP_THREADS + tid; i < ncounters; i += gridDim.x * MP_THREADS) counters[i] = 0;
+  for (int i = blockIdx.x * MP_THREADS + tid; i < ncounters; i += gridDim.x * MP_THREADS) counters[i] = 0;
+  const int m = prepass_row_of(blockIdx.x);
+  if (m >= M) return;
   const uint16_t* xi = x + (size_t)m * K;
   const int ngroups = 32 * nsteps;  // 8-weight groups, the step K ends in zero-filled
   auto fetch = [&](int g) -> u32x4 {
@@ -354,8 +361,8 @@ MidPlan mid_plan(int M, int N, int K) {
 template <int C, int DT>
 int launch_prepass(const void* x, uint8_t* xf, float* rs, int* counters, int ncounters, int M, int K, hipStream_t s) {
   using G = MidGeom<C>;
-  hipLaunchKernelGGL((mid_prepass_kernel<DT, G::ORD, G::NSUM>), dim3(M), dim3(MP_THREADS), 0, s,
-                     static_cast<const uint16_t*>(x), xf, rs, K, (K + CK_STEP - 1) / CK_STEP, counters, ncounters);
+  hipLaunchKernelGGL((mid_prepass_kernel<DT, G::ORD, G::NSUM>), dim3(prepass_grid(M)), dim3(MP_THREADS), 0, s,
+                     static_cast<const uint16_t*>(x), xf, rs, M, K, (K + CK_STEP - 1) / CK_STEP, counters, ncounters);
   KQ_HIP_CHECK(hipGetLastError());
   return KQ_OK;
 }
