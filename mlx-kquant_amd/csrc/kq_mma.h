@@ -106,22 +106,25 @@ struct RowRange {
 //   xhl  f16 [Mpad][K/256][16]    per superblock: hi_j (8) then lo_j (8) with X_j = 32 (hi_j + lo_j)
 //        S16: [Mpad][K/256][32]   sums of the 16-weight sub-blocks: hi_s (16) then lo_s (16), X_s = 16 (hi_s + lo_s)
 //   rs   f32 [Mpad]               2^e[m]
-// `red` = 4 floats of LDS; every thread of the workgroup must call (one barrier inside for bf16 input).
+// `red` = 4 floats of LDS; every thread of the workgroup must call (one barrier inside for bf16 input).  THREADS = 64: a wave
+// does the row, `red` is not used and there is no barrier.
 constexpr int PP_THREADS = 256;
 
 // IL16: xh keeps x[j], x[j + 16] interleaved over every 32 values instead (a byte of an iq4 block holds weights j
 // and j + 16 of its sub-block).
-template <int DT, bool S16 = false, bool IL16 = false>
+template <int DT, bool S16 = false, bool IL16 = false, int THREADS = PP_THREADS>
 __device__ __forceinline__ void prepass_row(const uint16_t* __restrict__ x, _Float16* __restrict__ xh,
                                             _Float16* __restrict__ xhl, float* __restrict__ rs, int M, int K, int m,
                                             int tid, float* red, KqRowSource src = KQ_PLAIN_ROWS) {
+  static_assert(THREADS == PP_THREADS || THREADS == 64, "`red` holds the maxima of four waves");
+  constexpr int UNROLL = THREADS > 64 ? 1 : 4;  // a single wave has several loads of its row in flight
   const int ngroups = K >> 3;
   constexpr int HPS = S16 ? 32 : 16;  // halves per superblock in xhl
   _Float16* xo = xh + (size_t)m * K;
   _Float16* ho = xhl + (size_t)m * (K >> 8) * HPS;
   if (m >= M) {
-    for (int g = tid; g < ngroups; g += PP_THREADS) *reinterpret_cast<u32x4*>(xo + 8 * g) = u32x4{0, 0, 0, 0};
-    for (int i = tid; i < (K >> 8) * HPS; i += PP_THREADS) ho[i] = (_Float16)0.f;
+    for (int g = tid; g < ngroups; g += THREADS) *reinterpret_cast<u32x4*>(xo + 8 * g) = u32x4{0, 0, 0, 0};
+    for (int i = tid; i < (K >> 8) * HPS; i += THREADS) ho[i] = (_Float16)0.f;
     if (tid == 0) rs[m] = 0.f;
     return;
   }
@@ -129,7 +132,8 @@ __device__ __forceinline__ void prepass_row(const uint16_t* __restrict__ x, _Flo
   float inv = 1.f, scale = 1.f;
   if constexpr (DT == KQ_BF16) {
     float amax = 0.f;
-    for (int g = tid; g < ngroups; g += PP_THREADS) {
+#pragma unroll UNROLL
+    for (int g = tid; g < ngroups; g += THREADS) {
       const u32x4 v = *reinterpret_cast<const u32x4*>(xi + 8 * g);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
@@ -139,9 +143,11 @@ __device__ __forceinline__ void prepass_row(const uint16_t* __restrict__ x, _Flo
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
-    if ((tid & 63) == 0) red[tid >> 6] = amax;
-    __syncthreads();
-    amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    if constexpr (THREADS > 64) {
+      if ((tid & 63) == 0) red[tid >> 6] = amax;
+      __syncthreads();
+      amax = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    }
     const uint32_t eb = (__builtin_bit_cast(uint32_t, amax) >> 23) & 0xff;
     if (eb != 0 && eb != 0xff) {
       int e = (int)eb - 127 - 14;  // largest magnitude lands in [2^14, 2^15)
@@ -151,7 +157,8 @@ __device__ __forceinline__ void prepass_row(const uint16_t* __restrict__ x, _Flo
     }
   }
   if (tid == 0) rs[m] = scale;
-  for (int g = tid; g < ngroups; g += PP_THREADS) {  // ngroups is a multiple of 32: whole quads stay together
+#pragma unroll UNROLL
+  for (int g = tid; g < ngroups; g += THREADS) {  // ngroups is a multiple of 32: whole quads stay together
     const u32x4 v = *reinterpret_cast<const u32x4*>(xi + 8 * g);
     _Float16 h[8];
 #pragma unroll

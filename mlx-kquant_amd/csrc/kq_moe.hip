@@ -68,6 +68,30 @@ __global__ __launch_bounds__(PP_THREADS) void moe_prologue_kernel(const uint16_t
     prepass_row<DT>(x, xh, xhl, rs, rows, K, blockIdx.x - 1, threadIdx.x, red, src);
 }
 
+// The same with workgroups of 1024 threads, four rows each, or sixteen (a wave per row, WAVE_ROWS).  What bounds the prologue of
+// many pairs is the sort: one workgroup whose LDS atomics come back one wave at a time.  With 1024 threads up to 8192 pairs stay in
+// registers and are counted once; 256 hold 2048 and count the others twice.  A wave per row suits short rows: 768 values are 96
+// 16-byte groups for 256 threads.
+template <int DT, bool WAVE_ROWS>
+__global__ __launch_bounds__(SORT_THREADS) void moe_prologue_wide_kernel(const uint16_t* __restrict__ x, _Float16* __restrict__ xh,
+                                                                         _Float16* __restrict__ xhl, float* __restrict__ rs,
+                                                                         int rows, int K, const uint32_t* __restrict__ idx, int P,
+                                                                         int E, int* __restrict__ order,
+                                                                         Segment* __restrict__ segs, int* __restrict__ nseg_out,
+                                                                         int seg_rows, KqRowSource src) {
+  constexpr int RT = WAVE_ROWS ? 64 : PP_THREADS, RPW = SORT_THREADS / RT;
+  __shared__ int cnt[SORT_MAX_E];
+  __shared__ int scan_p[SORT_THREADS / 64], scan_s[SORT_THREADS / 64];
+  __shared__ float red[SORT_THREADS / 64];
+  if (blockIdx.x == 0) {
+    moe_sort_body<SORT_THREADS>(idx, P, E, order, segs, nseg_out, cnt, scan_p, scan_s, seg_rows, src.rows_per_entry ? src.rows_per_entry : 1);
+    return;
+  }
+  const int q = threadIdx.x / RT, m = ((int)blockIdx.x - 1) * RPW + q;
+  // the last workgroup's spare rows: the last row again (the same values), so that its barrier has every wave
+  prepass_row<DT, false, false, RT>(x, xh, xhl, rs, rows, K, m < rows ? m : rows - 1, threadIdx.x % RT, red + q * (RT / 64), src);
+}
+
 // ------------------------------------------------------------------ row gather (batched gather_qmm)
 // One workgroup per output row p = b*M + m: copies the K 16-bit activations of x[lhs[b]][m] to
 // xg[p] and notes the row's expert, so that the grouped kernels below see a plain [P, K] matrix.
@@ -530,6 +554,22 @@ int launch_grouped_any(const MoeArgs& a, int P, int E, int codec, int dtype, hip
                          : launch_grouped<KQ_Q6_K, KQ_BF16, GLU>(a, P, E, s);
 }
 
+template <int DT>
+void launch_prologue(const void* x, const MoeWorkspace& m, int rows, int K, const uint32_t* idx, int P, int E, int seg_rows,
+                     hipStream_t s, KqRowSource src) {
+  const uint16_t* xi = static_cast<const uint16_t*>(x);
+  // beyond the pairs that 256 threads keep in registers; rows of up to four groups per lane go to a wave each
+  if (P <= 8 * PP_THREADS)
+    hipLaunchKernelGGL(moe_prologue_kernel<DT>, dim3(rows + 1), dim3(PP_THREADS), 0, s, xi, m.xh, m.xhl, m.rs, rows, K, idx, P, E,
+                       m.order, m.segs, m.nseg, seg_rows, src);
+  else if (K <= 2048)
+    hipLaunchKernelGGL((moe_prologue_wide_kernel<DT, true>), dim3((rows + 15) / 16 + 1), dim3(SORT_THREADS), 0, s, xi, m.xh, m.xhl,
+                       m.rs, rows, K, idx, P, E, m.order, m.segs, m.nseg, seg_rows, src);
+  else
+    hipLaunchKernelGGL((moe_prologue_wide_kernel<DT, false>), dim3((rows + 3) / 4 + 1), dim3(SORT_THREADS), 0, s, xi, m.xh, m.xhl,
+                       m.rs, rows, K, idx, P, E, m.order, m.segs, m.nseg, seg_rows, src);
+}
+
 }  // namespace
 
 int kq_launch_moe_sort(const uint32_t* idx, int P, int E, void* order, void* segs, void* nseg, hipStream_t s, int per_id) {
@@ -629,11 +669,9 @@ int kq_launch_moe_grouped(const void* x, const uint8_t* w, const uint8_t* w2, co
   const bool tile = moe_tile_takes(P, P / std::max(rows, 1), E, N, glu != 0, codec);
   const int seg_rows = tile ? KQ_MOE_TILE_SEG : SEG_M;
   if (dtype == KQ_F16)
-    hipLaunchKernelGGL(moe_prologue_kernel<KQ_F16>, dim3(rows + 1), dim3(PP_THREADS), 0, s, static_cast<const uint16_t*>(x),
-                       m.xh, m.xhl, m.rs, rows, K, idx, P, E, m.order, m.segs, m.nseg, seg_rows, src);
+    launch_prologue<KQ_F16>(x, m, rows, K, idx, P, E, seg_rows, s, src);
   else
-    hipLaunchKernelGGL(moe_prologue_kernel<KQ_BF16>, dim3(rows + 1), dim3(PP_THREADS), 0, s, static_cast<const uint16_t*>(x),
-                       m.xh, m.xhl, m.rs, rows, K, idx, P, E, m.order, m.segs, m.nseg, seg_rows, src);
+    launch_prologue<KQ_BF16>(x, m, rows, K, idx, P, E, seg_rows, s, src);
   KQ_HIP_CHECK(hipGetLastError());
   MoeArgs a{};
   a.xh = m.xh;

@@ -85,3 +85,28 @@ def test_results_stored_one_by_one(codec, N, offset):
     want = O.gather_qmm(xb, w, codec, np.arange(P), idx[:, 0], True, "bfloat16")
     assert rel_l2(got[offset:offset + P * N].reshape(P, 1, N), want, "bfloat16") <= TOL
     assert (got[:offset] == 0x40e0).all() and (got[offset + P * N:] == 0x40e0).all()
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("T,R,K,glu", [
+    (2048, 1, 256, 0),   # the last count of the narrow prologue
+    (2049, 1, 256, 0),   # a wave per row from here: one row in the last workgroup
+    (1025, 2, 2048, 1),  # the longest such rows, fewer rows than pairs
+    (2063, 1, 2304, 0),  # four rows a workgroup, three in the last
+    (2731, 3, 256, 0),   # 8193 pairs: the sort counts twice
+])
+def test_prologue_of_many_pairs(T, R, K, glu, dtype):
+    codec, E, N = "q4_k", 5, 40
+    idx = np.random.default_rng(20).integers(0, E, (T, R))
+    w, w2 = _stack(codec, E, N, K, 21), _stack(codec, E, N, K, 22)
+    if glu:
+        xb, xt = make_x((T, K), dtype, seed=23, scale=0.05)
+        got = dev_to_bits(kq.moe_glu_gather_kq(xt, wire_to_dev(w), wire_to_dev(w2), codec, _idx_dev(idx), "silu"))
+        want = O.moe_glu_gather(xb, w, w2, codec, idx, "silu", dtype=dtype)
+    else:
+        xb, xt = make_x((T * R, 1, K), dtype, seed=23, scale=0.05)
+        got = dev_to_bits(kq.gather_qmv_kq(xt, wire_to_dev(w), codec, _idx_dev(idx.reshape(-1, 1))))[:, 0]
+        want = O.gather_qmv_mix(xb, w, None, codec, None, idx.reshape(-1, 1), np.ones((T * R, 1), np.float32), dtype)
+    assert rel_l2(got, want, dtype) <= TOL
+    # the rows at the ends one by one
+    assert rel_l2(got[:1], want[:1], dtype) <= 3 * TOL and rel_l2(got[-1:], want[-1:], dtype) <= 3 * TOL
