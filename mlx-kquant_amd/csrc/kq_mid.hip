@@ -38,7 +38,8 @@ using kqmma::RowRange;
 constexpr int MP_THREADS = 512, MP_REGS = 4;
 
 // Row of a workgroup.  Eight neighbouring rows write the 16-byte eighths of the same 128-byte lines, and workgroups go to the
-// eight XCDs in turn: rows are dealt so that those eight meet in one L2, which then writes back whole lines.
+// eight XCDs in turn: rows are dealt so that those eight meet in one L2, which then writes back whole lines.  K = 4096, us in a
+// trace, row m on workgroup m before: 32 rows 3.2 -> 2.4, 333 rows 5.2 -> 4.5, 1024 rows 10.2 -> 6.7.
 __device__ __forceinline__ int prepass_row_of(int b) { return 64 * (b >> 6) + 8 * (b & 7) + ((b >> 3) & 7); }
 constexpr int prepass_grid(int M) { return (M + 63) & ~63; }
 

@@ -72,6 +72,7 @@ __global__ __launch_bounds__(PP_THREADS) void moe_prologue_kernel(const uint16_t
 // many pairs is the sort: one workgroup whose LDS atomics come back one wave at a time.  With 1024 threads up to 8192 pairs stay in
 // registers and are counted once; 256 hold 2048 and count the others twice.  A wave per row suits short rows: 768 values are 96
 // 16-byte groups for 256 threads.
+// 128 experts, us in a trace, before -> with it: 1000 rows of 2048, 8000 pairs 12.2 -> 8.9; 8000 rows of 768 12.9 -> 10.8.
 template <int DT, bool WAVE_ROWS>
 __global__ __launch_bounds__(SORT_THREADS) void moe_prologue_wide_kernel(const uint16_t* __restrict__ x, _Float16* __restrict__ xh,
                                                                          _Float16* __restrict__ xhl, float* __restrict__ rs,
