@@ -117,7 +117,6 @@ __device__ __forceinline__ void prepass_row(const uint16_t* __restrict__ x, _Flo
                                             _Float16* __restrict__ xhl, float* __restrict__ rs, int M, int K, int m,
                                             int tid, float* red, KqRowSource src = KQ_PLAIN_ROWS) {
   static_assert(THREADS == PP_THREADS || THREADS == 64, "`red` holds the maxima of four waves");
-  constexpr int UNROLL = THREADS > 64 ? 1 : 4;  // a single wave has several loads of its row in flight
   const int ngroups = K >> 3;
   constexpr int HPS = S16 ? 32 : 16;  // halves per superblock in xhl
   _Float16* xo = xh + (size_t)m * K;
@@ -132,14 +131,19 @@ __device__ __forceinline__ void prepass_row(const uint16_t* __restrict__ x, _Flo
   float inv = 1.f, scale = 1.f;
   if constexpr (DT == KQ_BF16) {
     float amax = 0.f;
-#pragma unroll UNROLL
-    for (int g = tid; g < ngroups; g += THREADS) {
+    auto take = [&](int g) {
       const u32x4 v = *reinterpret_cast<const u32x4*>(xi + 8 * g);
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] << 16)));
         amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] & 0xffff0000u)));
       }
+    };
+    if constexpr (THREADS > 64) {
+      for (int g = tid; g < ngroups; g += THREADS) take(g);
+    } else {  // a single wave has several loads of its row in flight
+#pragma unroll 4
+      for (int g = tid; g < ngroups; g += THREADS) take(g);
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
@@ -157,8 +161,7 @@ __device__ __forceinline__ void prepass_row(const uint16_t* __restrict__ x, _Flo
     }
   }
   if (tid == 0) rs[m] = scale;
-#pragma unroll UNROLL
-  for (int g = tid; g < ngroups; g += THREADS) {  // ngroups is a multiple of 32: whole quads stay together
+  auto convert = [&](int g) {  // ngroups is a multiple of 32: whole quads stay together
     const u32x4 v = *reinterpret_cast<const u32x4*>(xi + 8 * g);
     _Float16 h[8];
 #pragma unroll
@@ -186,7 +189,7 @@ __device__ __forceinline__ void prepass_row(const uint16_t* __restrict__ x, _Flo
       const u32x4 o = {(a0 & 0xffffu) | (b0 << 16), (a0 >> 16) | (b0 & 0xffff0000u), (a1 & 0xffffu) | (b1 << 16),
                        (a1 >> 16) | (b1 & 0xffff0000u)};
       *reinterpret_cast<u32x4*>(xo + 32 * (g >> 2) + 16 * (g & 1) + (high ? 8 : 0)) = o;
-      continue;
+      return;
     }
     const f16x8 o = {h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
     *reinterpret_cast<f16x8*>(xo + 8 * g) = o;
@@ -202,7 +205,7 @@ __device__ __forceinline__ void prepass_row(const uint16_t* __restrict__ x, _Flo
         ho[(j >> 4) * 32 + (j & 15)] = hi;
         ho[(j >> 4) * 32 + 16 + (j & 15)] = lo;
       }
-      continue;
+      return;
     }
     s += __shfl_xor(s, 2);  // 4 threads = one 32-wide sub-block
     if ((tid & 3) == 0) {
@@ -212,6 +215,12 @@ __device__ __forceinline__ void prepass_row(const uint16_t* __restrict__ x, _Flo
       ho[(j >> 3) * 16 + (j & 7)] = hi;
       ho[(j >> 3) * 16 + 8 + (j & 7)] = lo;
     }
+  };
+  if constexpr (THREADS > 64) {
+    for (int g = tid; g < ngroups; g += THREADS) convert(g);
+  } else {
+#pragma unroll 4
+    for (int g = tid; g < ngroups; g += THREADS) convert(g);
   }
 }
 
