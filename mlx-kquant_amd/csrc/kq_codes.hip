@@ -397,73 +397,75 @@ struct CgArgs {
 constexpr int CG_THREADS = 256;
 
 // Activation prepass of the grouped kernel: what every workgroup used to redo for its 32 slots at every step (bf16 ->
-// f16 with an exact power-of-two scale per (row, step), staging order, block sums) is done once per row.  One
-// workgroup per row; 32 threads per step, eight steps at a time.  Steps are zero-filled past K.  The pair sort is workgroup 0 of
-// the same launch where it keeps its pairs in registers (SORT), and rows are read where the call has them: 128 heads of 128 x 512
-// q8_0, four entries each, row gather + sort + prepass as three launches 9.9 us, as one 3.6.
-template <int DT, bool PAIR, bool SUMS, bool SORT>
-__global__ __launch_bounds__(256) void codes_prepass_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ xh,
-                                                            float* __restrict__ xsc, float* __restrict__ xsum, int K,
-                                                            int nsteps, KqRowSource src, const uint32_t* __restrict__ idx, int P, int E,
-                                                            int* __restrict__ order, Segment* __restrict__ segs,
-                                                            int* __restrict__ nseg_out) {
-  if constexpr (SORT) {
-    __shared__ int cnt[kqsort::SORT_MAX_E];
-    __shared__ int scan_p[256], scan_s[256];
-    if (blockIdx.x == 0) {
-      kqsort::moe_sort_body<256>(idx, P, E, order, segs, nseg_out, cnt, scan_p, scan_s, kqsort::SEG_M,
-                                 src.rows_per_entry ? src.rows_per_entry : 1);
-      return;
+// f16 with an exact power-of-two scale per (row, step), staging order, block sums) is done once per row.  32 threads per
+// (row, step), whatever row it belongs to: rows of three steps leave no thread idle.  Steps are zero-filled past K.
+// The pair sort is workgroup 0 of the same launch, and rows are read where the call has them: 128 heads of 128 x 512 q8_0, four
+// entries each, row gather + sort + prepass as three launches 9.9 us, as one 3.6.  THREADS: the sort keeps eight pairs per thread in
+// registers and counts the others twice, so more than 2048 pairs take 1024 threads.  A pass of 8000 pairs over 128 experts of 2048 <-> 768,
+// against a sort launch of its own and a workgroup per row: q8_0 440 -> 432 us, iq3_s 407 -> 398; 2056 pairs 203 -> 197, 180 -> 174; level
+// below 2048.
+template <int DT, bool PAIR, bool SUMS, int THREADS>
+__global__ __launch_bounds__(THREADS) void codes_prepass_kernel(const uint16_t* __restrict__ x, uint8_t* __restrict__ xh,
+                                                                float* __restrict__ xsc, float* __restrict__ xsum, int K, int rows,
+                                                                int nsteps, KqRowSource src, const uint32_t* __restrict__ idx, int P,
+                                                                int E, int* __restrict__ order, Segment* __restrict__ segs,
+                                                                int* __restrict__ nseg_out) {
+  __shared__ int cnt[kqsort::SORT_MAX_E];
+  __shared__ int scan_p[THREADS / 64], scan_s[THREADS / 64];
+  if (blockIdx.x == 0) {
+    kqsort::moe_sort_body<THREADS>(idx, P, E, order, segs, nseg_out, cnt, scan_p, scan_s, kqsort::SEG_M,
+                                   src.rows_per_entry ? src.rows_per_entry : 1);
+    return;
+  }
+  const int tid = threadIdx.x, pc = tid & 31;
+  const int64_t item = (int64_t)(blockIdx.x - 1) * (THREADS / 32) + (tid >> 5);
+  const int row = (int)(item / nsteps), st = (int)(item - (int64_t)row * nsteps);
+  if (row >= rows) return;
+  const uint16_t* xi = src.row(x, row, K);
+  const int k0 = CK_STEP * st + 8 * pc;
+  u32x4 v = {0, 0, 0, 0};
+  if (k0 < K) v = *reinterpret_cast<const u32x4*>(xi + k0);
+  float xscale = 1.f;
+  _Float16 h[8];
+  if constexpr (DT == KQ_BF16) {
+    float amax = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] << 16)));
+      amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] & 0xffff0000u)));
+    }
+#pragma unroll
+    for (int off = 16; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));  // the step's 32 lanes
+    float inv = 1.f;
+    const uint32_t eb = (__builtin_bit_cast(uint32_t, amax) >> 23) & 0xff;
+    if (eb != 0 && eb != 0xff) {
+      int e = (int)eb - 127 - 14;  // the largest magnitude lands in [2^14, 2^15)
+      if (e < -100) e = -100;
+      xscale = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
+      inv = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      h[2 * e] = (_Float16)(__builtin_bit_cast(float, v[e] << 16) * inv);
+      h[2 * e + 1] = (_Float16)(__builtin_bit_cast(float, v[e] & 0xffff0000u) * inv);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      h[2 * e] = __builtin_bit_cast(_Float16, (uint16_t)(v[e] & 0xffff));
+      h[2 * e + 1] = __builtin_bit_cast(_Float16, (uint16_t)(v[e] >> 16));
     }
   }
-  const int row = (int)blockIdx.x - (SORT ? 1 : 0), tid = threadIdx.x, pc = tid & 31;
-  const uint16_t* xi = src.row(x, row, K);
-  for (int st = tid >> 5; st < nsteps; st += 8) {
-    const int k0 = CK_STEP * st + 8 * pc;
-    u32x4 v = {0, 0, 0, 0};
-    if (k0 < K) v = *reinterpret_cast<const u32x4*>(xi + k0);
-    float xscale = 1.f;
-    _Float16 h[8];
-    if constexpr (DT == KQ_BF16) {
-      float amax = 0.f;
+  const size_t rs = (size_t)row * nsteps + st;
+  stage_group<PAIR>(xh + rs * 512, pc, h);
+  if (pc == 0) xsc[rs] = xscale;
+  if constexpr (SUMS) {
+    float sum = 0.f;
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] << 16)));
-        amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] & 0xffff0000u)));
-      }
-#pragma unroll
-      for (int off = 16; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));  // the step's 32 lanes
-      float inv = 1.f;
-      const uint32_t eb = (__builtin_bit_cast(uint32_t, amax) >> 23) & 0xff;
-      if (eb != 0 && eb != 0xff) {
-        int e = (int)eb - 127 - 14;  // the largest magnitude lands in [2^14, 2^15)
-        if (e < -100) e = -100;
-        xscale = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
-        inv = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23);
-      }
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        h[2 * e] = (_Float16)(__builtin_bit_cast(float, v[e] << 16) * inv);
-        h[2 * e + 1] = (_Float16)(__builtin_bit_cast(float, v[e] & 0xffff0000u) * inv);
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        h[2 * e] = __builtin_bit_cast(_Float16, (uint16_t)(v[e] & 0xffff));
-        h[2 * e + 1] = __builtin_bit_cast(_Float16, (uint16_t)(v[e] >> 16));
-      }
-    }
-    const size_t rs = (size_t)row * nsteps + st;
-    stage_group<PAIR>(xh + rs * 512, pc, h);
-    if (pc == 0) xsc[rs] = xscale;
-    if constexpr (SUMS) {
-      float sum = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; e++) sum += (float)h[e];
-      sum += __shfl_xor(sum, 1);
-      sum += __shfl_xor(sum, 2);  // 4 lanes = one 32-weight block
-      if ((pc & 3) == 0) xsum[rs * 8 + (pc >> 2)] = sum;
-    }
+    for (int e = 0; e < 8; e++) sum += (float)h[e];
+    sum += __shfl_xor(sum, 1);
+    sum += __shfl_xor(sum, 2);  // 4 lanes = one 32-weight block
+    if ((pc & 3) == 0) xsum[rs * 8 + (pc >> 2)] = sum;
   }
 }
 
@@ -719,11 +721,9 @@ size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 }  // namespace
 
-// kq_moe.hip
 // The three launcher groups below can be compiled into separate objects (KQ_CODES_PART = 1 dense, 2 gathered,
 // 3 grouped; unset = all) so that the build instantiates their kernels in parallel.
 #if !defined(KQ_CODES_PART) || KQ_CODES_PART == 3
-int kq_launch_moe_sort(const uint32_t* idx, int P, int E, void* order, void* segs, void* nseg, hipStream_t s, int per_id = 1);
 
 bool kq_codes_moe_supported(int P, int E, int N, int K, int codec) {
   // nvfp4 (a scale per 16 weights: 16 x 16 scalings per step) does not fit the register file here and
@@ -753,11 +753,6 @@ int kq_launch_codes_moe(const void* x, const uint8_t* w, const uint8_t* w2, cons
   int* order = reinterpret_cast<int*>(p);
   Segment* segs = reinterpret_cast<Segment*>(p + align256((size_t)P * 4));
   int* nseg = reinterpret_cast<int*>(p + align256((size_t)P * 4) + align256(((size_t)E + P / 32 + 1) * sizeof(Segment)));
-  const bool sort_inside = P <= 8 * 256;
-  if (!sort_inside) {
-    const int rc = kq_launch_moe_sort(idx, P, E, order, segs, nseg, s, src.rows_per_entry ? src.rows_per_entry : 1);
-    if (rc) return rc;
-  }
   const int rows = glu ? P / (x_div < 1 ? 1 : x_div) : P, nsteps = (K + CK_STEP - 1) / CK_STEP;
   const size_t rs = (size_t)rows * nsteps;
   uint8_t* xh = reinterpret_cast<uint8_t*>(nseg) + 256;
@@ -768,12 +763,13 @@ int kq_launch_codes_moe(const void* x, const uint8_t* w, const uint8_t* w2, cons
     const uint16_t* xi = static_cast<const uint16_t*>(x);
 #define KQ_PRE(DTV, PV, SV)                                                                                                       \
   do {                                                                                                                          \
-    if (sort_inside)                                                                                                            \
-      hipLaunchKernelGGL((codes_prepass_kernel<DTV, PV, SV, true>), dim3(rows + 1), dim3(256), 0, s, xi, xh, xsc, xsum, K, nsteps, \
-                         src, idx, P, E, order, segs, nseg);                                                                    \
+    constexpr int narrow = 256, wide = 1024;                                                                                    \
+    if (P <= 8 * narrow)                                                                                                        \
+      hipLaunchKernelGGL((codes_prepass_kernel<DTV, PV, SV, narrow>), dim3((unsigned)((rs + 7) / 8 + 1)), dim3(narrow), 0, s, xi, xh, xsc,  \
+                         xsum, K, rows, nsteps, src, idx, P, E, order, segs, nseg);                                             \
     else                                                                                                                        \
-      hipLaunchKernelGGL((codes_prepass_kernel<DTV, PV, SV, false>), dim3(rows), dim3(256), 0, s, xi, xh, xsc, xsum, K, nsteps,    \
-                         src, idx, P, E, order, segs, nseg);                                                                    \
+      hipLaunchKernelGGL((codes_prepass_kernel<DTV, PV, SV, wide>), dim3((unsigned)((rs + 31) / 32 + 1)), dim3(wide), 0, s, xi, xh, xsc,    \
+                         xsum, K, rows, nsteps, src, idx, P, E, order, segs, nseg);                                             \
   } while (0)
     if (dtype == KQ_F16) {
       if (pair) KQ_PRE(KQ_F16, true, false);

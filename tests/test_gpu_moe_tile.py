@@ -87,6 +87,7 @@ def test_results_stored_one_by_one(codec, N, offset):
     assert (got[:offset] == 0x40e0).all() and (got[offset + P * N:] == 0x40e0).all()
 
 
+@pytest.mark.parametrize("codec", ["q4_k", "q8_0", "q4_1", "iq4_xs"])  # the last three: the code-level kernel, its sums and pairs
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
 @pytest.mark.parametrize("T,R,K,glu", [
     (2048, 1, 256, 0),   # the last count of the narrow prologue
@@ -95,8 +96,8 @@ def test_results_stored_one_by_one(codec, N, offset):
     (2063, 1, 2304, 0),  # four rows a workgroup, three in the last
     (2731, 3, 256, 0),   # 8193 pairs: the sort counts twice
 ])
-def test_prologue_of_many_pairs(T, R, K, glu, dtype):
-    codec, E, N = "q4_k", 5, 40
+def test_prologue_of_many_pairs(T, R, K, glu, dtype, codec):
+    E, N = 5, 40
     idx = np.random.default_rng(20).integers(0, E, (T, R))
     w, w2 = _stack(codec, E, N, K, 21), _stack(codec, E, N, K, 22)
     if glu:
