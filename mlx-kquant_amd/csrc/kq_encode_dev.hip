@@ -250,14 +250,18 @@ __device__ __forceinline__ float fit_scale_min(float (&x)[N], float (&wt)[N], Fi
       sdd = __builtin_fma(wd, double(d), sdd);
       sdl = __builtin_fma(wd, double(l0), sdl);
     }
-    const double Wd = double(W), sddc = __builtin_fma(Wd, sdd, -sd * sd);
-    const float unit = 1.0f / (ws * float(W));
+    // The distances of the closed form are taken in units of 2^k next to the range: its numerators, about W^4 times the square
+    // of a distance, leave the floats otherwise (from a range of 1e7 on).  A power of two: the same digits.
+    const uint32_t rexp = __builtin_bit_cast(uint32_t, range) >> 23;
+    const double dunit = double(__builtin_bit_cast(float, (254u - rexp) << 23)), range_unit2 = 1.0 / (dunit * dunit);
+    const double Wd = double(W), sddc = __builtin_fma(Wd, sdd, -sd * sd) * (dunit * dunit), Wu = Wd * dunit, sdu = sd * dunit;
+    const float unit = float(range_unit2 / (double(ws) * Wd));
     float least = INFINITY, det_least = INFINITY;
     const float reach = fmaxf(vmax, -vmin) * std::sqrt(sw);
     int first = 0;
     auto bound_of = [&](auto at_zero, int c, bool same) {
       const double sld = double(sl), sl2d = double(sl2);
-      const double det = __builtin_fma(Wd, sl2d, -sld * sld), cross = __builtin_fma(Wd, sdl, -sd * sld);
+      const double det = __builtin_fma(Wd, sl2d, -sld * sld), cross = __builtin_fma(Wu, sdl, -sdu * sld);
       const float detf = float(det);
       float e = float(__builtin_fma(sddc, det, -cross * cross)) * __builtin_amdgcn_rcpf(detf) * unit;
       if constexpr (decltype(at_zero)::value) {  // the minimum may be held at zero: where m would be positive, it is zero

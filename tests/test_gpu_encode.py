@@ -212,3 +212,27 @@ def test_device_encoder_fit_bytes_over_kinds_of_rows(kq, codec, weights):
     bad = np.argwhere((dev != host).any(axis=1)).ravel().tolist()
     kinds = list(_FIT_ROWS)
     assert not bad, sorted({kinds[b // 8] if b < 8 * len(kinds) else "mixed" for b in bad})
+
+
+@pytest.mark.parametrize("codec", ["q2_k", "q4_k", "q5_k"])
+def test_device_encoder_fit_up_to_the_ends_of_the_bound(kq, codec):
+    """Rows whose ranges run up to the largest and down to the smallest for which candidates are ruled out by a bound: the
+    bound's own products must hold them.  Weights times 2^s with importance times 2^(-5 s / 3), which keeps every product of the
+    scales' own fit in range, have the same scale bytes: the host's at s = 0 (where the f16 factors behind them overflow, the
+    quotients that give the levels are not finite, and host and device convert those differently).  And without importance all
+    bytes are the host's as far as the factors stay finite."""
+    rng = np.random.default_rng(61 + O.codec_id(codec))
+    K, bpb = 1024, O.geometry(codec)[1]
+    scales = slice(0, 16) if codec == "q2_k" else slice(4, 16)
+    w = torch.from_numpy(np.concatenate([rng.random((12, K)), 2 * rng.random((12, K)) - 1, np.clip(rng.standard_normal((8, K)) / 4, -1, 1),
+                                         rng.integers(0, 9, (4, K)) / 8]).astype(np.float32))
+    for im in (np.ones(K), rng.random(K), 10.0 ** rng.uniform(-6, 0, K)):
+        im = torch.from_numpy(im.astype(np.float32))
+        host = kq.quantize(w, codec, im)[0].numpy().reshape(len(w), -1, bpb)
+        for s in (-27, -12, 15, 18, 21, 24, 27, 30):
+            dev = kq.quantize((w * 2.0 ** s).cuda(), codec, (im * 2.0 ** (-5 * s // 3)).cuda())[0].cpu().numpy().reshape(host.shape)
+            bad = np.argwhere((dev[:, :, scales] != host[:, :, scales]).any(axis=(1, 2))).ravel().tolist()
+            assert not bad, (s, bad)
+    for s in range(14, {"q2_k": 21, "q4_k": 25, "q5_k": 26}[codec] + 1):  # rows from 0: the minima stay finite
+        big = w[:12] * 2.0 ** s
+        assert torch.equal(kq.quantize(big.cuda(), codec)[0].cpu(), kq.quantize(big, codec)[0]), s
