@@ -8,8 +8,9 @@
 // (a list of at most 1024 ids, read by every workgroup at once); then one load of the activations, which it converts itself.
 //   * Workgroup = 4 waves; wave = one 32-row weight tile x one 256-weight step (mid_step of kq_mid.h, wire bytes through LDS),
 //     so a workgroup covers four tiles or two; the steps of a tile meet in LDS at the end.
-//   * Activations: up to 32 rows at a time as f16 fragments in LDS under a power of two per row and step, exact like the
-//     prepass kernels'.  More rows than that take further rounds on the same wire bytes.
+//   * Activations: up to 32 rows at a time as f16 fragments in LDS under a power of two per row and step.  A row with a nonzero
+//     value that this does not hold (2^-31 of the step's largest, bf16), or with an infinity, is done in f32 instead.
+//     More rows than 32 take further rounds on the same wire bytes.
 // 128 heads of 128 x 512, 4 / 16 / 32 rows each, us: q8_0 12.3 / 14.2 / 22.2 -> 6.3 / 7.0 / 9.3, q4_k 10.2 / 11.4 / 14.7 -> 5.6 / 6.7 / 9.5,
 // q6_k 11.3 / 12.7 / 16.0 -> 6.3 / 7.2 / 9.4, the empty launch 2.4; 64 / 128 rows q8_0 31 / 61 -> 10.6 / 20.6, q4_k 28 / 45 -> 11.0 / 21.7.
 #include <algorithm>
@@ -33,6 +34,46 @@ struct HeadArgs {
   int64_t x_batch_stride, w_expert_stride;
 };
 
+// The rows of a round that f16 does not hold, in f32 on the reference-order weights from global memory (the order of the sums
+// aside, the arithmetic of the kernels that go entry by entry).  Rare, so small code rather than speed: a weight is decoded once
+// for eight rows.
+template <int C, int DT>
+__device__ __forceinline__ void wide_rows_f32(const HeadArgs& a, uint32_t expert, uint32_t wide, const int64_t* x_off,
+                                              const int64_t* y_row, int tid) {
+  using G = MidGeom<C>;
+  const int lg = a.K > CK_STEP ? 2 : 1, parts = 1 << lg;  // threads per weight row: 32 HD_WAVES / steps rows a workgroup
+  const int part = tid & (parts - 1), n = (HD_THREADS >> lg) * (int)blockIdx.x + (tid >> lg);
+  const bool live = n < a.N;
+  const uint8_t* w = a.w + (size_t)expert * (size_t)a.w_expert_stride + (size_t)(live ? n : 0) * (size_t)(a.K / G::WPB) * G::BPB;
+#pragma unroll 1
+  for (int r0 = 0; r0 < 32; r0 += 8) {
+    if (!((wide >> r0) & 0xff)) continue;  // uniform
+    float sum[8] = {};
+#pragma unroll 1
+    for (int g = part; g < a.K / 8; g += parts) {
+      float f[8];
+      kq::decode8<C>(w + (size_t)(8 * g / G::WPB) * G::BPB, 8 * g % G::WPB / 8, a.grids, f);
+#pragma unroll
+      for (int r = 0; r < 8; r++) {
+        if (!((wide >> (r0 + r)) & 1)) continue;  // uniform
+        const u32x4 v = *reinterpret_cast<const u32x4*>(a.x + x_off[r0 + r] + 8 * g);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const uint16_t lo = (uint16_t)(v[e] & 0xffffu), hi = (uint16_t)(v[e] >> 16);
+          sum[r] = fmaf(DT == KQ_BF16 ? kq::bf162f(lo) : kq::h2f(lo), f[2 * e], sum[r]);
+          sum[r] = fmaf(DT == KQ_BF16 ? kq::bf162f(hi) : kq::h2f(hi), f[2 * e + 1], sum[r]);
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+      if (!((wide >> (r0 + r)) & 1)) continue;
+      for (int m = 1; m < parts; m <<= 1) sum[r] += __shfl_xor(sum[r], m);
+      if (live && part == 0) a.y[(size_t)y_row[r0 + r] * a.N + n] = DT == KQ_F16 ? kq::f2f16(sum[r]) : kq::f2bf16(sum[r]);
+    }
+  }
+}
+
 template <int C, int DT>
 __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
   using G = MidGeom<C>;
@@ -43,6 +84,7 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
   __shared__ uint32_t lhs_of[HD_MAX_ENTRIES];
   __shared__ float xs[HD_STEPS][32];
   __shared__ int64_t x_off[32], y_row[32];
+  __shared__ uint32_t wide_rows;  // rows of the round that f16 under a power of two does not hold, by bit
   const int N = a.N, K = a.K, nsteps = K / CK_STEP;
   uint8_t* slots = smem + mid_table_bytes<C>();
   uint8_t* frags = slots + HD_WAVES * SLOT;  // [step][fragment][lane][16]; the sums of the waves afterwards
@@ -131,16 +173,21 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
   auto lo_f = [](uint32_t v) { return DT == KQ_BF16 ? __builtin_bit_cast(float, v << 16) : kq::h2f((uint16_t)(v & 0xffffu)); };
   auto hi_f = [](uint32_t v) { return DT == KQ_BF16 ? __builtin_bit_cast(float, v & 0xffff0000u) : kq::h2f((uint16_t)(v >> 16)); };
   for (int r0 = 32 * blockIdx.z; r0 < rows; r0 += 32 * gridDim.z) {
+    // what is rare takes its lane from here: nothing of it is computed ahead of the loop
+    int cold_tid = tid;
+    asm volatile("" : "+v"(cold_tid));
     const int here = rows - r0 < 32 ? rows - r0 : 32;
     if (tid < here) {
       const int place = (r0 + tid) / a.M, m = r0 + tid - place * a.M;
       x_off[tid] = (int64_t)lhs_of[place] * a.x_batch_stride + (int64_t)m * K;
       y_row[tid] = (int64_t)entry_of[place] * a.M + m;
     }
+    if (tid == 0) wide_rows = 0;
     lds_barrier();
     // ---- activations: 32 lanes per (row, step), eight rows of a step at a time, the loads of four such blocks in flight
     const int pc = tid & 31, rblocks = (here + 7) / 8, nblocks = rblocks * nsteps;
     const int per_block = rblocks == 1 ? 32 : rblocks == 2 ? 16 : rblocks == 3 ? 11 : 8;  // b / rblocks = b per_block / 32
+    uint32_t lost_rows = 0;  // of the lane's, by bit
     for (int b0 = 0; b0 < nblocks; b0 += HD_AHEAD) {
       u32x4 v[HD_AHEAD];
 #pragma unroll
@@ -164,6 +211,16 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
           scale = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
           inv = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23);
         }
+        // values below 2^-17 in the step's unit lose bits (RowRange of kq_mma.h); an infinity leaves the others unscaled
+        bool lost = eb == 0xff;
+        if constexpr (DT == KQ_BF16) {
+          const uint32_t cut = ((__builtin_bit_cast(uint32_t, scale) >> 23) - 17) << 7;
+          u16x2 low = {0xffff, 0xffff};
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            low = __builtin_elementwise_min(low, (u16x2)(__builtin_bit_cast(u16x2, v[u][e] & 0x7fff7fffu) - (uint16_t)1));
+          lost |= (uint32_t)(low[0] < low[1] ? low[0] : low[1]) < cut - 1;
+        }
         _Float16 h[8];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
@@ -171,12 +228,15 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
           h[2 * e + 1] = (_Float16)(hi_f(v[u][e]) * inv);
         }
         if (row >= here) continue;  // 32 lanes at a time
+        lost_rows |= lost ? 1u << row : 0u;
         store_frags<G::ORD, G::NSUM, true>(frags + s * (G::NF * 1024) + 16 * row, pc, h, row);
         if (pc == 0) xs[s][row] = scale;
       }
     }
+    if (__builtin_expect(lost_rows != 0, 0)) atomicOr(&wide_rows, lost_rows);
     vmwait<0>();  // the wire bytes
     lds_barrier();
+    const uint32_t rows_here = here == 32 ? ~0u : (1u << here) - 1, wide = __builtin_amdgcn_readfirstlane(wide_rows) & rows_here;
     f32x16 acc = f32x16{0};
     if (live) {
       // places past the last row hold whatever lies there: their results are not stored
@@ -209,12 +269,14 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
       }
     }
     if (live && st == 0 && l32 < nrows) {
+      const uint32_t mine = (rows_here & ~wide) >> (4 * kg);
 #pragma unroll
       for (int i = 0; i < 16; i++) {
-        const int r = 8 * (i >> 2) + 4 * kg + (i & 3);
-        if (r < here) a.y[(size_t)y_row[r] * N + row0 + l32] = DT == KQ_F16 ? kq::f2f16(acc[i]) : kq::f2bf16(acc[i]);
+        const int r0 = 8 * (i >> 2) + (i & 3);
+        if ((mine >> r0) & 1) a.y[(size_t)y_row[r0 + 4 * kg] * N + row0 + l32] = DT == KQ_F16 ? kq::f2f16(acc[i]) : kq::f2bf16(acc[i]);
       }
     }
+    if (__builtin_expect(wide != 0, 0)) wide_rows_f32<C, DT>(a, expert, wide, x_off, y_row, cold_tid);
     lds_barrier();  // before the next rows' fragments
   }
 }

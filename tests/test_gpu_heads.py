@@ -1,6 +1,7 @@
 """GPU parity of the one-launch gather_qmm of short contractions (K of one or two 256-weight steps, few rows per expert):
 every codec, tiles of weight rows that end inside the matrix, experts without entries, with one row, with more than the 32 rows
-of a round and more rounds than workgroups, ids outside the stack, rows of very different size, strided stacks."""
+of a round and more rounds than workgroups, ids outside the stack, rows of very different size, rows of wide range, infinities,
+strided stacks."""
 import numpy as np
 import pytest
 import torch
@@ -78,6 +79,75 @@ def test_strided_stack_and_repeated_replays(codec):
         g.replay()
         torch.cuda.synchronize()
         assert rel_l2(dev_to_bits(y), O.gather_qmm(bits, w[::2], codec, lhs, rhs, True, dtype), dtype) <= TOL
+
+
+def _zero_first_weights(w, codec):
+    """The first weights of every row made zero: the sub-block's scale (and minimum) inside the first block, or the whole of it."""
+    wpb, bpb = O.geometry(codec)
+    b = w.reshape(-1, w.shape[-1] // bpb, bpb)[:, 0]
+    if codec == "q2_k":
+        b[:, 0] = 0
+    elif codec == "q3_k":  # six bits less 32
+        b[:, 96] &= 0xf0
+        b[:, 104] = (b[:, 104] & 0xfc) | 2
+    elif codec in ("q4_k", "q5_k"):
+        b[:, [4, 8]] &= 0xc0
+    elif codec == "q6_k":
+        b[:, 192] = 0
+    elif codec == "nvfp4":
+        b[:, 0] = 0
+    elif codec == "iq4_xs":  # six bits less 32
+        b[:, 4] &= 0xf0
+        b[:, 2] = (b[:, 2] & 0xfc) | 2
+    else:
+        b[:] = 0
+    rows = O.dequantize(w.reshape(-1, w.shape[-1]), codec).reshape(-1, w.shape[-1] // bpb * wpb)
+    assert not rows[:, :16].any()
+
+
+@pytest.mark.parametrize("codec", CODECS)
+@pytest.mark.parametrize("K,B,M", [(256, 30, 1), (512, 12, 9)])
+def test_rows_of_wide_range(codec, K, B, M):
+    """Large values on zero weights beside small ones that are the result: every row on its own; with and without a workspace."""
+    if O.geometry(codec)[0] == 256 and K == 256 and codec.startswith("iq") and codec != "iq4_xs":
+        pytest.skip("zero weights of this codec fill a step")
+    E, N, L, dtype = 5, 136, 6, "bfloat16"
+    w = _stack(codec, E, N, K, seed=561)
+    _zero_first_weights(w, codec)
+    rng = np.random.default_rng(562)
+    x = rng.standard_normal((L, M, K)).astype(np.float32)
+    x[0, :, 3], x[1, 0, 0], x[2, :, 1] = -3e38, 7e12, 1e30
+    x[2, :, 16:] *= 1e-12
+    x[3, M - 1] *= 1e-35
+    xb = O.f32_to_bits(x, dtype)
+    lhs, rhs = rng.integers(0, L, B), rng.integers(0, E, B)
+    xt, wd, li, ri = bits_to_dev(xb, dtype), wire_to_dev(w), _idx_dev(lhs).to(torch.int32), _idx_dev(rhs).to(torch.int32)
+    want = O.gather_qmm(xb, w, codec, lhs, rhs, True, dtype)
+    got = dev_to_bits(kq.gather_qmm(xt, wd, None, codec, lhs_indices=li, rhs_indices=ri))
+    assert _per_row(got, want, dtype) <= ROW_TOL[dtype], codec
+    out = torch.zeros((B, M, N), dtype=torch.bfloat16, device="cuda")
+    assert kq._load().kq_gather_qmm(xt.data_ptr(), wd.data_ptr(), li.data_ptr(), ri.data_ptr(), out.data_ptr(), B, M, E, N, K, M * K,
+                                    wd.stride(0), 1, 0, O.codec_id(codec), kq._DT[torch.bfloat16], None, 0, None) == 0
+    torch.cuda.synchronize()
+    assert _per_row(dev_to_bits(out), want, dtype) <= ROW_TOL[dtype], codec
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("codec", ["q2_k", "q3_k", "q4_k", "q8_0", "nvfp4", "iq2_xs"])
+def test_rows_with_an_infinity(codec, dtype):
+    """Infinite where the products say so; the other rows of the round are the ordinary ones."""
+    E, N, K, B, M, L = 5, 72, 512, 20, 2, 6
+    w, lhs, xb, _ = _case(codec, E, N, K, B, M, L, dtype, None, 571)
+    rhs = np.arange(B) % E
+    xb = xb.copy()
+    xb[2, 1, 300] = 0x7f80 if dtype == "bfloat16" else 0x7c00
+    xb[4, 0, 7] = 0xff80 if dtype == "bfloat16" else 0xfc00
+    got, want = (O.bits_to_f32(b, dtype) for b in (
+        dev_to_bits(kq.gather_qmm(bits_to_dev(xb, dtype), wire_to_dev(w), None, codec, lhs_indices=_idx_dev(lhs), rhs_indices=_idx_dev(rhs))),
+        O.gather_qmm(xb, w, codec, lhs, rhs, True, dtype)))
+    fin = np.isfinite(want)
+    assert np.array_equal(got[~fin], want[~fin], equal_nan=True) and np.isfinite(got[fin]).all()
+    assert np.linalg.norm(got[fin] - want[fin]) <= ROW_TOL[dtype] * np.linalg.norm(want[fin])
 
 
 def test_ids_outside_the_stack_write_nothing():
