@@ -301,7 +301,7 @@ int launch_heads(const HeadArgs& a, int E, hipStream_t s) {
 
 bool kq_heads_supported(int B, int M, int E, int N, int K, int codec) {
   if (codec < 0 || codec >= KQ_NUM_CODECS || B <= 0 || M <= 0 || E <= 0 || E > 65535 || N <= 0 || B > HD_MAX_ENTRIES) return false;
-  if (K % CK_STEP || K > HD_STEPS * CK_STEP || K % kq_geom(codec).wpb) return false;
+  if (K <= 0 || K % CK_STEP || K > HD_STEPS * CK_STEP || K % kq_geom(codec).wpb) return false;
   const int64_t row_bytes = (int64_t)(K / kq_geom(codec).wpb) * kq_geom(codec).bpb;
   if (row_bytes & 1) return false;  // the direct-to-LDS loads take 2-byte aligned addresses
   // Up to 16 rows the streamed kernel goes entry by entry (16 heads of 64 x 512: 3.4 us q4_k, 4.1 q8_0; here 4.4, 5.0).

@@ -818,7 +818,7 @@ bool nt_tall(int codec, int M, int N, int K, bool cut, int entries) {
 // four sequences: 128 heads of 128 x 512 q8_0 21.8 / 24.2, q4_k 22.6 / 27.9, 64 of 192 x 512 13.6 / 16.7, 16.4 / 21.0, but 32 of
 // 128 x 256 8.6 / 6.3, 8.9 / 6.8; of 32 rows, two sequences, 128 heads q8_0 21.3 / 18.5, q6_k 25.0 / 30.1.
 bool nt_merge(int M, int B, int E, int N, int codec, bool gathered) {
-  if (!gathered || B < 2 * E || B > NT_MERGE_ENTRIES || E > 65535) return false;
+  if (!gathered || E < 1 || B < 2 * E || B > NT_MERGE_ENTRIES) return false;
   return M <= 8 || (M <= 16 && (int64_t)B * ((N + NT_COLS - 1) / NT_COLS) >= 4 * kq_num_cus()) || (M <= 32 && nt_wide(codec));
 }
 

@@ -169,6 +169,28 @@ def test_ids_outside_the_stack_write_nothing():
     assert bool((out[[3, 17]] == 7.0).all())
 
 
+@pytest.mark.parametrize("codec", ["q8_0", "q4_k"])
+def test_empty_contraction_and_empty_stack(codec):
+    """K = 0: sums of nothing.  No experts: every id is outside the stack and nothing is written, in either orientation."""
+    E, N, B, M = 5, 256, 40, 2
+    lib, x = kq._load(), torch.ones(B * M * 256, dtype=torch.bfloat16, device="cuda")
+    w = torch.zeros(1024, dtype=torch.uint8, device="cuda")
+    ids = torch.arange(B, device="cuda", dtype=torch.int32) % E
+
+    def call(out, e, k, transpose):
+        rc = lib.kq_gather_qmm(x.data_ptr(), w.data_ptr(), ids.data_ptr(), ids.data_ptr(), out.data_ptr(), B, M, e, N, k, M * k, 0,
+                               transpose, 0, O.codec_id(codec), kq._DT[torch.bfloat16], None, 0, None)
+        torch.cuda.synchronize()
+        return rc
+
+    out = torch.full((B, M, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    for transpose in (0, 1):
+        assert call(out, 0, 256, transpose) == 0 and bool((out == 7.0).all())
+    for transpose in (0, 1):
+        out.fill_(7.0)
+        assert call(out, E, 0, transpose) == 0 and bool((out == 0.0).all())
+
+
 @pytest.mark.parametrize("codec", ["q8_0", "q4_k", "q6_k", "iq3_s", "q5_1", "nvfp4"])
 @pytest.mark.parametrize("K,M,B,dtype", [(96, 1, 40, "bfloat16"), (130, 3, 31, "float16"), (64, 8, 200, "bfloat16"),
                                          (192, 16, 30, "bfloat16"), (100, 24, 23, "bfloat16")])
