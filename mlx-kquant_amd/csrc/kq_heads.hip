@@ -15,13 +15,15 @@
 // q6_k 11.3 / 12.7 / 16.0 -> 6.3 / 7.2 / 9.4, the empty launch 2.4; 64 / 128 rows q8_0 31 / 61 -> 10.6 / 20.6, q4_k 28 / 45 -> 11.0 / 21.7.
 #include <algorithm>
 
+#include "kq_entries.h"
 #include "kq_mid.h"
 
 namespace {
 
 using namespace kqmid;
+using kqentries::MAX_ENTRIES;
 
-constexpr int HD_WAVES = 4, HD_THREADS = 64 * HD_WAVES, HD_MAX_ENTRIES = 1024, HD_AHEAD = 4, HD_STEPS = 2;
+constexpr int HD_WAVES = 4, HD_THREADS = 64 * HD_WAVES, HD_AHEAD = 4, HD_STEPS = 2;
 
 struct HeadArgs {
   const uint16_t* x;
@@ -79,9 +81,8 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
   using G = MidGeom<C>;
   constexpr int SLOT = mid_slot_bytes<C>();
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  __shared__ __attribute__((aligned(16))) int counts[HD_MAX_ENTRIES / HD_THREADS][HD_WAVES];
-  __shared__ int entry_of[HD_MAX_ENTRIES];
-  __shared__ uint32_t lhs_of[HD_MAX_ENTRIES];
+  static_assert(HD_THREADS == kqentries::THREADS, "the search of the id list");
+  __shared__ kqentries::Places places;
   __shared__ float xs[HD_STEPS][32];
   __shared__ int64_t x_off[32], y_row[32];
   __shared__ uint32_t wide_rows;  // rows of the round that f16 under a power of two does not hold, by bit
@@ -112,14 +113,8 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
   if (blockIdx.z == 0) request();
 
   // ---- the expert's entries
-  uint32_t id[HD_MAX_ENTRIES / HD_THREADS], lhs[HD_MAX_ENTRIES / HD_THREADS];
-#pragma unroll
-  for (int u = 0; u < HD_MAX_ENTRIES / HD_THREADS; u++) {
-    if (HD_THREADS * u >= a.B) break;  // uniform
-    const int j = tid + HD_THREADS * u;
-    id[u] = j < a.B ? a.rhs[j] : ~0u;
-    lhs[u] = j < a.B ? a.lhs[j] : 0u;
-  }
+  kqentries::Ids ids;
+  ids.load(a.rhs, a.lhs, a.B, tid);
   kqfrag::KMasks masks;
   masks.init<C>();
   Tables tabs{smem, smem, 2};
@@ -128,28 +123,7 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
     build_tables<C, HD_THREADS, true>(smem, spread, a.grids, tid);
     tabs = Tables{CodeGeom<C>::PAIR_LUT ? smem + 4 * l32 : smem, spread, 7};
   }
-  // places in the order of the list, the same in every workgroup of the expert
-  uint64_t hit[HD_MAX_ENTRIES / HD_THREADS];
-#pragma unroll
-  for (int u = 0; u < HD_MAX_ENTRIES / HD_THREADS; u++) {
-    if (HD_THREADS * u >= a.B) break;  // uniform
-    hit[u] = __builtin_amdgcn_ballot_w64(id[u] == expert);
-    if (lane == 0) counts[u][wave] = __builtin_popcountll(hit[u]);
-  }
-  lds_barrier();
-  int count = 0;
-#pragma unroll
-  for (int u = 0; u < HD_MAX_ENTRIES / HD_THREADS; u++) {
-    if (HD_THREADS * u >= a.B) break;
-    const int4 c = *reinterpret_cast<const int4*>(counts[u]);
-    const int before = (wave > 0 ? c.x : 0) + (wave > 1 ? c.y : 0) + (wave > 2 ? c.z : 0);
-    if ((hit[u] >> lane) & 1) {
-      const int place = count + before + __builtin_popcountll(hit[u] & ((1ull << lane) - 1));
-      entry_of[place] = tid + HD_THREADS * u;
-      lhs_of[place] = lhs[u];
-    }
-    count += c.x + c.y + c.z + c.w;
-  }
+  const int count = ids.find(expert, a.B, tid, wave, places, [] { lds_barrier(); });
   lds_barrier();
   const int rows = count * a.M;
   if (32 * (int)blockIdx.z >= rows) {  // uniform; nothing may be on its way into LDS when the workgroup ends
@@ -179,8 +153,8 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
     const int here = rows - r0 < 32 ? rows - r0 : 32;
     if (tid < here) {
       const int place = (r0 + tid) / a.M, m = r0 + tid - place * a.M;
-      x_off[tid] = (int64_t)lhs_of[place] * a.x_batch_stride + (int64_t)m * K;
-      y_row[tid] = (int64_t)entry_of[place] * a.M + m;
+      x_off[tid] = (int64_t)places.lhs_of[place] * a.x_batch_stride + (int64_t)m * K;
+      y_row[tid] = (int64_t)places.entry_of[place] * a.M + m;
     }
     if (tid == 0) wide_rows = 0;
     lds_barrier();
@@ -300,7 +274,7 @@ int launch_heads(const HeadArgs& a, int E, hipStream_t s) {
 }  // namespace
 
 bool kq_heads_supported(int B, int M, int E, int N, int K, int codec) {
-  if (codec < 0 || codec >= KQ_NUM_CODECS || B <= 0 || M <= 0 || E <= 0 || E > 65535 || N <= 0 || B > HD_MAX_ENTRIES) return false;
+  if (codec < 0 || codec >= KQ_NUM_CODECS || B <= 0 || M <= 0 || E <= 0 || E > 65535 || N <= 0 || B > MAX_ENTRIES) return false;
   if (K <= 0 || K % CK_STEP || K > HD_STEPS * CK_STEP || K % kq_geom(codec).wpb) return false;
   const int64_t row_bytes = (int64_t)(K / kq_geom(codec).wpb) * kq_geom(codec).bpb;
   if (row_bytes & 1) return false;  // the direct-to-LDS loads take 2-byte aligned addresses

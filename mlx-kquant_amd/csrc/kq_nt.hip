@@ -26,6 +26,7 @@
 
 #include "kq_decode.h"
 #include "kq_dma.h"
+#include "kq_entries.h"
 
 namespace {
 
@@ -34,7 +35,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32_a1 __attribute__((aligned(1)));  // the hardware serves unaligned dword loads
 
 constexpr int NT_WAVES = 4, NT_THREADS = 64 * NT_WAVES;
-constexpr int NT_KSTEP = 32, NT_COLS = 128, NT_MERGE_ENTRIES = 1024;
+constexpr int NT_KSTEP = 32, NT_COLS = 128;
 // Codecs whose 32-row form does not fit 256 registers (it spills up to 248 bytes per lane) take 64-row tiles on one
 // wave per SIMD beyond 32 rows (q6_k 4096 x 4096, 512 rows: 292 -> 146 us); for the others the 64-row form measured
 // level or slower (q8_0 93 -> 111 us).
@@ -106,8 +107,8 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
   const uint32_t e = MERGE ? blockIdx.z : a.rhs ? a.rhs[item] : 0u;
   if (e >= (uint32_t)a.E) return;  // the whole workgroup leaves: the entry's output rows stay untouched
   static_assert(!MERGE || MR <= 2, "rows of a round");
-  __shared__ int entry_of[MERGE ? NT_MERGE_ENTRIES : 1];
-  __shared__ uint32_t lhs_of[MERGE ? NT_MERGE_ENTRIES : 1];
+  static_assert(!MERGE || NT_THREADS == kqentries::THREADS, "the search of the id list");
+  __shared__ std::conditional_t<MERGE, kqentries::Places, int> places;
   __shared__ int64_t x_off[MERGE ? 16 * MR : 1], y_row[MERGE ? 16 * MR : 1];
   const int tile = blockIdx.x;
   const int ngroups = a.N / 8;
@@ -167,39 +168,9 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
   int rows = a.M, m0 = MERGE ? 0 : blockIdx.y * 16 * MR;
   if constexpr (MERGE) {
     if (blockIdx.y == 0 && st_begin + wave < nsteps) fetch_w(st_begin + wave);
-    // places in the order of the list, the same in every workgroup of the expert
-    constexpr int NU = NT_MERGE_ENTRIES / NT_THREADS;
-    __shared__ __attribute__((aligned(16))) int counts[NU][NT_WAVES];
-    const int tid = threadIdx.x, B = a.B;
-    uint32_t id[NU], lh[NU];
-    uint64_t hit[NU];
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-      if (NT_THREADS * u >= B) break;  // uniform
-      const int j = tid + NT_THREADS * u;
-      id[u] = j < B ? a.rhs[j] : ~0u;
-      lh[u] = j < B ? a.lhs[j] : 0u;
-    }
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-      if (NT_THREADS * u >= B) break;
-      hit[u] = __builtin_amdgcn_ballot_w64(id[u] == e);
-      if (lane == 0) counts[u][wave] = __builtin_popcountll(hit[u]);
-    }
-    __syncthreads();
-    int count = 0;
-#pragma unroll
-    for (int u = 0; u < NU; u++) {
-      if (NT_THREADS * u >= B) break;
-      const int4 n = *reinterpret_cast<const int4*>(counts[u]);
-      const int before = (wave > 0 ? n.x : 0) + (wave > 1 ? n.y : 0) + (wave > 2 ? n.z : 0);
-      if ((hit[u] >> lane) & 1) {
-        const int place = count + before + __builtin_popcountll(hit[u] & ((1ull << lane) - 1));
-        entry_of[place] = tid + NT_THREADS * u;
-        lhs_of[place] = lh[u];
-      }
-      count += n.x + n.y + n.z + n.w;
-    }
+    kqentries::Ids ids;
+    ids.load(a.rhs, a.lhs, a.B, threadIdx.x);
+    const int count = ids.find(e, a.B, threadIdx.x, wave, places, [] { __syncthreads(); });
     rows = count * a.M;
     m0 = 16 * MR * blockIdx.y;
     if (m0 >= rows) return;  // uniform
@@ -211,8 +182,8 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
       __syncthreads();
       if ((int)threadIdx.x < 16 * MR) {  // rows past the last repeat it, never stored
         const int r = m0 + (int)threadIdx.x < rows ? m0 + (int)threadIdx.x : rows - 1, place = r / a.M, m = r - place * a.M;
-        x_off[threadIdx.x] = (int64_t)lhs_of[place] * a.x_batch_stride + (int64_t)m * a.K;
-        y_row[threadIdx.x] = (int64_t)entry_of[place] * a.M + m;
+        x_off[threadIdx.x] = (int64_t)places.lhs_of[place] * a.x_batch_stride + (int64_t)m * a.K;
+        y_row[threadIdx.x] = (int64_t)places.entry_of[place] * a.M + m;
       }
       __syncthreads();
     }
@@ -818,7 +789,7 @@ bool nt_tall(int codec, int M, int N, int K, bool cut, int entries) {
 // four sequences: 128 heads of 128 x 512 q8_0 21.8 / 24.2, q4_k 22.6 / 27.9, 64 of 192 x 512 13.6 / 16.7, 16.4 / 21.0, but 32 of
 // 128 x 256 8.6 / 6.3, 8.9 / 6.8; of 32 rows, two sequences, 128 heads q8_0 21.3 / 18.5, q6_k 25.0 / 30.1.
 bool nt_merge(int M, int B, int E, int N, int codec, bool gathered) {
-  if (!gathered || E < 1 || B < 2 * E || B > NT_MERGE_ENTRIES) return false;
+  if (!gathered || E < 1 || B < 2 * E || B > kqentries::MAX_ENTRIES) return false;
   return M <= 8 || (M <= 16 && (int64_t)B * ((N + NT_COLS - 1) / NT_COLS) >= 4 * kq_num_cus()) || (M <= 32 && nt_wide(codec));
 }
 
