@@ -10,7 +10,8 @@
 //     so a workgroup covers four tiles or two; the steps of a tile meet in LDS at the end.
 //   * Activations: up to 32 rows at a time as f16 fragments in LDS under a power of two per row and step.  A row with a nonzero
 //     value that this does not hold (2^-31 of the step's largest, bf16), or with an infinity, is done in f32 instead.
-//     More rows than 32 take further rounds on the same wire bytes.
+//     More rows than 32 are further rounds, of other workgroups (kq_entries.h): 1024 entries of 8 rows on one of 64 experts
+//     243 -> 31 us against rounds in series on the expert's own, 512 of one row on one of 128 100 -> 18.4, even shares 6.7 -> 6.8 (q8_0).
 // 128 heads of 128 x 512, 4 / 16 / 32 rows each, us: q8_0 12.3 / 14.2 / 22.2 -> 6.3 / 7.0 / 9.3, q4_k 10.2 / 11.4 / 14.7 -> 5.6 / 6.7 / 9.5,
 // q6_k 11.3 / 12.7 / 16.0 -> 6.3 / 7.2 / 9.4, the empty launch 2.4; 64 / 128 rows q8_0 31 / 61 -> 10.6 / 20.6, q4_k 28 / 45 -> 11.0 / 21.7.
 #include <algorithm>
@@ -83,6 +84,7 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   static_assert(HD_THREADS == kqentries::THREADS, "the search of the id list");
   __shared__ kqentries::Places places;
+  __shared__ kqentries::Share share;
   __shared__ float xs[HD_STEPS][32];
   __shared__ int64_t x_off[32], y_row[32];
   __shared__ uint32_t wide_rows;  // rows of the round that f16 under a power of two does not hold, by bit
@@ -92,7 +94,7 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, kg = lane >> 5;
-  const uint32_t expert = blockIdx.y;
+  uint32_t expert = blockIdx.y;
 
   // ---- this wave's wire bytes
   const int tpw = HD_WAVES / nsteps, t = wave / nsteps, st = wave - t * nsteps;
@@ -110,27 +112,11 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
       if (r < nrows) dma16(base, (uint32_t)r * row_bytes + (uint32_t)off, l0 + 1024 * T);
     });
   };
-  if (blockIdx.z == 0) request();
-
-  // ---- the expert's entries
-  kqentries::Ids ids;
-  ids.load(a.rhs, a.lhs, a.B, tid);
   kqfrag::KMasks masks;
   masks.init<C>();
   Tables tabs{smem, smem, 2};
-  if constexpr (mid_table_bytes<C>() > 0) {
-    uint8_t* spread = smem + CodeGeom<C>::GROUPED_GRID_BYTES;
-    build_tables<C, HD_THREADS, true>(smem, spread, a.grids, tid);
-    tabs = Tables{CodeGeom<C>::PAIR_LUT ? smem + 4 * l32 : smem, spread, 7};
-  }
-  const int count = ids.find(expert, a.B, tid, wave, places, [] { lds_barrier(); });
-  lds_barrier();
-  const int rows = count * a.M;
-  if (32 * (int)blockIdx.z >= rows) {  // uniform; nothing may be on its way into LDS when the workgroup ends
-    vmwait<0>();
-    return;
-  }
-  if (blockIdx.z != 0) request();
+  uint8_t* spread = smem + CodeGeom<C>::GROUPED_GRID_BYTES;
+  if constexpr (mid_table_bytes<C>() > 0) tabs = Tables{CodeGeom<C>::PAIR_LUT ? smem + 4 * l32 : smem, spread, 7};
 
   // largest magnitude over the lane's 32, as the half's bits
   auto magnitude = [](u32x4 v) {
@@ -146,10 +132,13 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
   };
   auto lo_f = [](uint32_t v) { return DT == KQ_BF16 ? __builtin_bit_cast(float, v << 16) : kq::h2f((uint16_t)(v & 0xffffu)); };
   auto hi_f = [](uint32_t v) { return DT == KQ_BF16 ? __builtin_bit_cast(float, v & 0xffff0000u) : kq::h2f((uint16_t)(v >> 16)); };
-  for (int r0 = 32 * blockIdx.z; r0 < rows; r0 += 32 * gridDim.z) {
-    // what is rare takes its lane from here: nothing of it is computed ahead of the loop
-    int cold_tid = tid;
-    asm volatile("" : "+v"(cold_tid));
+  uint32_t* entries = reinterpret_cast<uint32_t*>(frags + nsteps * (G::NF * 1024));  // per expert
+  const int E = gridDim.y, Z = gridDim.z;
+  auto barrier = [] { lds_barrier(); };
+  auto round = [&](int r0, int rows) __attribute__((always_inline)) {  // rows r0 ... of the expert whose places and wire bytes are in LDS or on the way
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    lds_barrier();
     const int here = rows - r0 < 32 ? rows - r0 : 32;
     if (tid < here) {
       const int place = (r0 + tid) / a.M, m = r0 + tid - place * a.M;
@@ -250,9 +239,38 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
         if ((mine >> r0) & 1) a.y[(size_t)y_row[r0 + 4 * kg] * N + row0 + l32] = DT == KQ_F16 ? kq::f2f16(acc[i]) : kq::f2bf16(acc[i]);
       }
     }
-    if (__builtin_expect(wide != 0, 0)) wide_rows_f32<C, DT>(a, expert, wide, x_off, y_row, cold_tid);
-    lds_barrier();  // before the next rows' fragments
+    if (__builtin_expect(wide != 0, 0)) wide_rows_f32<C, DT>(a, expert, wide, x_off, y_row, tid);
+  };
+  // A round of the workgroup's own expert, if it has one for it, then one that another expert leaves over.  The second is written
+  // out: a loop around both kept the addresses of the first alive in it (172 registers where this takes 127, even shares 10 % longer).
+  if (blockIdx.z == 0) request();
+  const int r0 = 32 * blockIdx.z;
+  int own_rows;
+  {
+    kqentries::Ids ids;
+    ids.load(a.rhs, a.lhs, a.B, tid);
+    if constexpr (mid_table_bytes<C>() > 0) build_tables<C, HD_THREADS, true>(smem, spread, a.grids, tid);
+    own_rows = kqentries::find_and_count<32>(ids, expert, a.B, a.M, E, Z, tid, wave, places, entries, share, barrier) * a.M;
   }
+  if (__builtin_expect(r0 < own_rows, 1)) {  // uniform
+    if (blockIdx.z != 0) request();
+    round(r0, own_rows);
+    if (__builtin_expect(!share.left || !kqentries::shares_rounds<32>(own_rows, a.B, a.M, E, Z), 1)) return;
+  } else {
+    vmwait<0>();  // nothing may be on its way into LDS when the workgroup ends
+    lds_barrier();
+    if (!share.left) return;
+  }
+  const uint32_t next = kqentries::share_rounds<32>(a.B, a.M, E, Z, blockIdx.y, blockIdx.z, tid, entries, share, barrier);
+  if (next == kqentries::NO_ROUND) return;
+  expert = next & (kqentries::MAX_EXPERTS - 1);
+  request();
+  int cold_tid = tid;
+  asm volatile("" : "+v"(cold_tid));
+  kqentries::Ids ids;
+  ids.load(a.rhs, a.lhs, a.B, cold_tid);
+  const int rows = ids.find(expert, a.B, cold_tid, wave, places, barrier) * a.M;
+  round(32 * (int)(next >> kqentries::EXPERT_BITS), rows);
 }
 
 template <int C, int DT>
@@ -260,13 +278,14 @@ int launch_heads(const HeadArgs& a, int E, hipStream_t s) {
   using G = MidGeom<C>;
   const int nsteps = a.K / CK_STEP, cols = 32 * (HD_WAVES / nsteps);
   constexpr size_t fixed = (size_t)mid_table_bytes<C>() + HD_WAVES * mid_slot_bytes<C>();
-  static_assert(fixed + HD_STEPS * G::NF * 1024 + 9 * 1024 <= 160 * 1024, "LDS of a CU");
-  // an expert's rows beyond the first 32 spread over up to eight workgroups, two of them should most entries name few experts
+  static_assert(fixed + HD_STEPS * G::NF * 1024 + kqentries::count_bytes(kqentries::MAX_EXPERTS) + 9 * 1024 <= 160 * 1024, "LDS of a CU");
+  // workgroups for the rounds of an average expert, and for more in long lists of random ids: those without one leave early
   const int64_t P = (int64_t)a.B * a.M;
-  const int z = (int)std::min<int64_t>(8, std::max<int64_t>(1 + P / 1024, (P + 32 * E - 1) / (32 * E)));
+  const int z = (int)std::min<int64_t>(8, std::max<int64_t>(1 + P / 2048, (P + 32 * E - 1) / (32 * E)));
+  const size_t lds = fixed + (size_t)nsteps * G::NF * 1024 + kqentries::count_bytes(E);
   auto kern = heads_kernel<C, DT>;
-  KQ_SET_MAX_LDS_ONCE((kern), fixed + HD_STEPS * G::NF * 1024);
-  hipLaunchKernelGGL(kern, dim3((a.N + cols - 1) / cols, E, z), dim3(HD_THREADS), fixed + (size_t)nsteps * G::NF * 1024, s, a);
+  KQ_SET_MAX_LDS_ONCE((kern), fixed + HD_STEPS * G::NF * 1024 + kqentries::count_bytes(kqentries::MAX_EXPERTS));
+  hipLaunchKernelGGL(kern, dim3((a.N + cols - 1) / cols, E, z), dim3(HD_THREADS), lds, s, a);
   KQ_HIP_CHECK(hipGetLastError());
   return KQ_OK;
 }
@@ -274,7 +293,7 @@ int launch_heads(const HeadArgs& a, int E, hipStream_t s) {
 }  // namespace
 
 bool kq_heads_supported(int B, int M, int E, int N, int K, int codec) {
-  if (codec < 0 || codec >= KQ_NUM_CODECS || B <= 0 || M <= 0 || E <= 0 || E > 65535 || N <= 0 || B > MAX_ENTRIES) return false;
+  if (codec < 0 || codec >= KQ_NUM_CODECS || B <= 0 || M <= 0 || E <= 0 || E > kqentries::MAX_EXPERTS || N <= 0 || B > MAX_ENTRIES) return false;
   if (K <= 0 || K % CK_STEP || K > HD_STEPS * CK_STEP || K % kq_geom(codec).wpb) return false;
   const int64_t row_bytes = (int64_t)(K / kq_geom(codec).wpb) * kq_geom(codec).bpb;
   if (row_bytes & 1) return false;  // the direct-to-LDS loads take 2-byte aligned addresses

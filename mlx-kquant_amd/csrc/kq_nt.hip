@@ -90,10 +90,12 @@ struct NtGeom {
 // MR = 16-row groups of activations per workgroup (1: up to 16 rows, 2: 32, 4: 64 rows on one wave per SIMD, for
 // calls of many rows: every decoded weight then feeds four MFMAs)
 // MERGE (gathered calls of few rows per entry that name the experts more than once): grid z counts experts, and a workgroup
-// multiplies the rows of all entries of its expert, 16 MR at a time (grid y of them at once).  It asks for its first wire
-// bytes before it looks for the entries in the id list.  128 heads of 128 -> 512, us, 4 x 1 / 8 x 1 / 8 x 4 (sequences x rows), against
-// a workgroup per entry that looked for the others of its expert: q8_0 12.8 / 26.4 / 32.7 -> 8.4 / 8.6 / 11.5, q4_k 14.2 / 27.7 /
-// 34.5 -> 9.0 / 9.5 / 11.6, q6_k 15.9 / 29.5 / 37.6 -> 10.4 / 10.8 / 13.2.
+// multiplies 16 MR rows of its expert's entries (grid y of them), then some that a larger expert leaves over (kq_entries.h).  It
+// asks for its first wire bytes before it looks for the entries in the id list.  128 heads of 128 -> 512, us, 4 x 1 / 8 x 1 / 8 x 4
+// (sequences x rows), against a workgroup per entry that looked for the others of its expert: q8_0 12.8 / 26.4 / 32.7 ->
+// 8.8 / 9.1 / 12.0, q4_k 14.2 / 27.7 / 34.5 -> 9.6 / 9.9 / 12.1, q6_k 15.9 / 29.5 / 37.6 -> 10.9 / 11.3 / 13.9.  1024 entries of 8
+// rows, 64 experts, q8_0: all on one 66 -> 33 (427 with its rounds in series on its own workgroups), half of them 54 -> 34, random
+// ids 53 -> 31; of one row 46 -> 16, 32 -> 16, 30 -> 16 (in series 276, 140, 12).
 template <int C, int DT, int MR, bool MERGE = false>
 __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kernel(NtArgs a, const uint8_t* __restrict__ grids) {
   using G = NtGeom<C>;
@@ -109,6 +111,8 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
   static_assert(!MERGE || MR <= 2, "rows of a round");
   static_assert(!MERGE || NT_THREADS == kqentries::THREADS, "the search of the id list");
   __shared__ std::conditional_t<MERGE, kqentries::Places, int> places;
+  __shared__ std::conditional_t<MERGE, kqentries::Share, int> share;
+  __shared__ uint32_t entries[MERGE ? kqentries::count_bytes(kqentries::MAX_ENTRIES / 2) / 4 : 1];  // per expert (nt_merge)
   __shared__ int64_t x_off[MERGE ? 16 * MR : 1], y_row[MERGE ? 16 * MR : 1];
   const int tile = blockIdx.x;
   const int ngroups = a.N / 8;
@@ -118,7 +122,7 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
   const int pi = G::SUPER ? tile >> 1 : tile;  // row piece the tile reads
   // group inside the piece; lanes past the last column decode the last group and store nothing
   const int gp = (col_ok ? gi : ngroups - 1) - pi * (G::PCOLS / 8);
-  const uint8_t* wt = a.w + (size_t)e * (size_t)a.w_expert_stride + (size_t)pi * G::PIECE;
+  const uint8_t* wt = a.w + (size_t)e * (size_t)a.w_expert_stride + (size_t)pi * G::PIECE;  // MERGE: of the round's expert
   const int cols_here = a.N - G::PCOLS * pi < G::PCOLS ? a.N - G::PCOLS * pi : G::PCOLS;
   const int piece_here = cols_here / G::WPB * BPB;  // the last piece of a 32-weight codec may be shorter
   uint8_t* stage = lds + wave * NT_KSTEP * STRIDE;
@@ -165,25 +169,43 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
   const int steps_all = (a.K + NT_KSTEP - 1) / NT_KSTEP;
   const int st_begin = split * a.steps_per_split;
   const int nsteps = st_begin + a.steps_per_split < steps_all ? st_begin + a.steps_per_split : steps_all;
-  int rows = a.M, m0 = MERGE ? 0 : blockIdx.y * 16 * MR;
+  int rows = a.M, m0 = 16 * MR * blockIdx.y;
   if constexpr (MERGE) {
     if (blockIdx.y == 0 && st_begin + wave < nsteps) fetch_w(st_begin + wave);
     kqentries::Ids ids;
     ids.load(a.rhs, a.lhs, a.B, threadIdx.x);
-    const int count = ids.find(e, a.B, threadIdx.x, wave, places, [] { __syncthreads(); });
-    rows = count * a.M;
-    m0 = 16 * MR * blockIdx.y;
-    if (m0 >= rows) return;  // uniform
-  }
-  bool first = MERGE && blockIdx.y == 0;
-#pragma unroll 1
-  for (;;) {  // MERGE: rounds of 16 MR rows; once otherwise
-    if constexpr (MERGE) {
+    rows = kqentries::find_and_count<16 * MR>(ids, e, a.B, a.M, a.E, gridDim.y, threadIdx.x, wave, places, entries, share,
+                                              [] { __syncthreads(); }) * a.M;
+    if (m0 >= rows) {  // uniform
       __syncthreads();
-      if ((int)threadIdx.x < 16 * MR) {  // rows past the last repeat it, never stored
-        const int r = m0 + (int)threadIdx.x < rows ? m0 + (int)threadIdx.x : rows - 1, place = r / a.M, m = r - place * a.M;
-        x_off[threadIdx.x] = (int64_t)places.lhs_of[place] * a.x_batch_stride + (int64_t)m * a.K;
-        y_row[threadIdx.x] = (int64_t)places.entry_of[place] * a.M + m;
+      if (!share.left) return;
+    }
+  }
+  // MERGE: a round of the workgroup's own expert, if it has one for it, then one that another expert leaves over
+  bool fetched = MERGE && blockIdx.y == 0, own = !MERGE || m0 < rows, others = false;
+#pragma unroll 1
+  for (;;) {
+    int tid = threadIdx.x;
+    if constexpr (MERGE) {
+      if (__builtin_expect(!own, 0)) {
+        asm volatile("" : "+v"(tid));  // what the search derives from it is not kept from one round to the next
+        const uint32_t next = kqentries::share_rounds<16 * MR>(a.B, a.M, a.E, gridDim.y, e, blockIdx.y, tid, entries, share,
+                                                               [] { __syncthreads(); });
+        if (next == kqentries::NO_ROUND) return;
+        others = true;
+        const uint32_t expert = next & (kqentries::MAX_EXPERTS - 1);
+        m0 = 16 * MR * (int)(next >> kqentries::EXPERT_BITS);
+        wt = a.w + (size_t)expert * (size_t)a.w_expert_stride + (size_t)pi * G::PIECE;
+        kqentries::Ids ids;
+        ids.load(a.rhs, a.lhs, a.B, tid);
+        rows = ids.find(expert, a.B, tid, wave, places, [] { __syncthreads(); }) * a.M;
+        fetched = false;
+      }
+      __syncthreads();
+      if (tid < 16 * MR) {  // rows past the last repeat it, never stored
+        const int r = m0 + tid < rows ? m0 + tid : rows - 1, place = r / a.M, m = r - place * a.M;
+        x_off[tid] = (int64_t)places.lhs_of[place] * a.x_batch_stride + (int64_t)m * a.K;
+        y_row[tid] = (int64_t)places.entry_of[place] * a.M + m;
       }
       __syncthreads();
     }
@@ -202,10 +224,9 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
 #pragma unroll
       for (int t = 0; t < 8; t++) acc[q][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (st_begin + wave < nsteps) {
-      if (!first) fetch_w(st_begin + wave);
+      if (!fetched) fetch_w(st_begin + wave);
       fetch_x(st_begin + wave);
     }
-    first = false;
     for (int st = st_begin + wave; st < nsteps; st += NT_WAVES) {
 #pragma unroll
       for (int j = 0; j < NDW; j++) {
@@ -328,10 +349,13 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
         }
       }
     }
-    if constexpr (!MERGE) return;
-    m0 += 16 * MR * gridDim.y;
-    if (m0 >= rows) return;
-    __syncthreads();  // the sums have been read: the staging areas may be filled again
+    if constexpr (!MERGE) {
+      return;
+    } else {
+      if (others || !share.left || !kqentries::shares_rounds<16 * MR>(rows, a.B, a.M, a.E, gridDim.y)) return;
+      own = false;
+      __syncthreads();  // the sums have been read: the staging areas may be filled again
+    }
   }
 }
 
@@ -805,8 +829,10 @@ struct NtRun {
   template <int DT, int MR, bool MERGE = false>
   static void go(const NtArgs& a, int B, const uint8_t* grids, hipStream_t s) {
     dim3 grid((a.N + NT_COLS - 1) / NT_COLS, (a.M + 16 * MR - 1) / (16 * MR), a.ksplit > 1 ? a.ksplit : B);
-    if (MERGE) {  // rounds of an expert that run at once: what it has on average
-      grid.y = (unsigned)(((int64_t)B * a.M + 16 * MR * a.E - 1) / (16 * MR * a.E));
+    if (MERGE) {
+      // workgroups for the rounds of an average expert; half as many again for random ids where they all run at once
+      const int64_t rows = (int64_t)B * a.M, more = (3 * rows / 2 + 16 * MR * a.E - 1) / (16 * MR * a.E);
+      grid.y = (unsigned)(grid.x * a.E * more <= kq_num_cus() ? more : (rows + 16 * MR * a.E - 1) / (16 * MR * a.E));
       grid.z = a.E;
     }
     hipLaunchKernelGGL((gemm_nt_mfma_kernel<C, DT, MR, MERGE>), grid, dim3(NT_THREADS), 0, s, a, grids);

@@ -61,6 +61,36 @@ def test_most_entries_on_one_expert(codec, B, M):
     assert _per_row(got, want, dtype) <= ROW_TOL[dtype], codec
 
 
+@pytest.mark.parametrize("transpose", [True, False])
+@pytest.mark.parametrize("E,B,M", [(1, 256, 1), (3, 96, 8), (64, 1024, 8), (300, 1000, 1), (511, 1024, 5), (700, 1024, 7), (8, 17, 120)])
+@pytest.mark.parametrize("spread", ["one", "two", "half", "ramp", "all but one", "outside"])
+def test_rounds_that_experts_leave_over(E, B, M, spread, transpose):
+    """Experts with more rows than their workgroups do: every row is done, once (the output starts as NaN), whoever takes it."""
+    N, K = (64, 256) if transpose else (128, 32)
+    rng = np.random.default_rng(E + B)
+    rhs = {"one": np.full(B, E // 2), "two": np.where(np.arange(B) % 3 == 0, 0, E - 1),
+           "half": np.where(np.arange(B) % 2 == 0, E // 3, rng.integers(0, E, B)),
+           "ramp": np.sort((rng.random(B) ** 3 * E).astype(np.int64)), "all but one": np.arange(B) % max(E - 1, 1),
+           "outside": np.where(rng.random(B) < 0.5, E + 5, E - 1)}[spread]
+    w = _stack("q8_0", E, *((N, K) if transpose else (K, N)), seed=541)
+    lhs = rng.integers(0, 9, B)
+    xb = O.f32_to_bits(rng.standard_normal((9, M, K)).astype(np.float32), "bfloat16")
+    xt, wd, li, ri = bits_to_dev(xb, "bfloat16"), wire_to_dev(w), _idx_dev(lhs).to(torch.int32), _idx_dev(rhs).to(torch.int32)
+    out = torch.full((B, M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    assert kq._load().kq_gather_qmm(xt.data_ptr(), wd.data_ptr(), li.data_ptr(), ri.data_ptr(), out.data_ptr(), B, M, E, N, K, M * K,
+                                    wd.stride(0), int(transpose), 0, O.codec_id("q8_0"), kq._DT[torch.bfloat16], None, 0, None) == 0
+    torch.cuda.synchronize()
+    inside = rhs < E
+    assert bool(out[torch.from_numpy(~inside).cuda()].isnan().all())
+    want = O.bits_to_f32(xb, "bfloat16").astype(np.float64)[lhs[inside]]
+    mats = O.dequantize(w.reshape(-1, w.shape[-1]), "q8_0").reshape(E, -1, K if transpose else N).astype(np.float64)
+    mats = mats.transpose(0, 2, 1) if transpose else mats
+    want = np.stack([x @ mats[e] for x, e in zip(want, rhs[inside])])
+    got = out[torch.from_numpy(inside).cuda()].float().cpu().numpy().astype(np.float64)
+    err = np.linalg.norm(got - want, axis=-1) / np.linalg.norm(want, axis=-1)
+    assert err.max() <= ROW_TOL["bfloat16"]
+
+
 @pytest.mark.parametrize("codec", ["q6_k", "q8_0"])
 def test_strided_stack_and_repeated_replays(codec):
     """Every second expert of a larger stack; the same call captured and replayed with other activations."""
