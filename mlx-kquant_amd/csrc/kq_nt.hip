@@ -808,13 +808,13 @@ bool nt_tall(int codec, int M, int N, int K, bool cut, int entries) {
 }
 
 // Entries of one expert share tiles (gathered calls in which an expert comes twice on average, of a list short enough to be
-// searched by every workgroup): where the rows of an entry fill half a tile at most, or a tile and the unmerged workgroups would
-// be more than two rounds of two per CU, or 32 rows of the codec that spills without.  Merged / not, us, entries of 16 rows,
+// searched by every workgroup): where the rows of an entry fill half a tile at most, or a tile (two of the codec that spills
+// without) and the unmerged workgroups would be more than two rounds of two per CU.  Merged / not, us, entries of 16 rows,
 // four sequences: 128 heads of 128 x 512 q8_0 21.8 / 24.2, q4_k 22.6 / 27.9, 64 of 192 x 512 13.6 / 16.7, 16.4 / 21.0, but 32 of
-// 128 x 256 8.6 / 6.3, 8.9 / 6.8; of 32 rows, two sequences, 128 heads q8_0 21.3 / 18.5, q6_k 25.0 / 30.1.
+// 128 x 256 8.6 / 6.3, 8.9 / 6.8, 16 of 192 x 512 q6_k 12.8 / 11.3; of 32 rows, two sequences, 128 heads q8_0 21.3 / 18.5, q6_k 25.0 / 30.1.
 bool nt_merge(int M, int B, int E, int N, int codec, bool gathered) {
   if (!gathered || E < 1 || B < 2 * E || B > kqentries::MAX_ENTRIES) return false;
-  return M <= 8 || (M <= 16 && (int64_t)B * ((N + NT_COLS - 1) / NT_COLS) >= 4 * kq_num_cus()) || (M <= 32 && nt_wide(codec));
+  return M <= 8 || ((M <= 16 || (M <= 32 && nt_wide(codec))) && (int64_t)B * ((N + NT_COLS - 1) / NT_COLS) >= 4 * kq_num_cus());
 }
 
 template <int C>
