@@ -1124,58 +1124,70 @@ __global__ __launch_bounds__(64 * NW, WGS) void stream_gemv_kernel(StArgsOf<GM> 
   if constexpr (IQ2_COP > 1) SFor<8>::run([&](auto ii) { tie_v2(gq[decltype(ii)::value]); });
 
   // ---- activations -> f16 fragments (+ sums) in the wave's LDS, then this lane's A registers
-  float xscale = 1.0f, inv = 1.0f;
+  // A power of two covers four units of the wave at most, as in the ranges of a K split: a dense wave of eight has two, for units
+  // 0 .. 3 and 4 .. 7.  (Values below 2^-31 of the largest that shares it lose bits.)
+  constexpr int NS = GM == 0 && XU == 8 ? 2 : 1;
+  float xscale_of[NS], inv_of[NS];
   bool wide = false;  // mixed: activations that f16 under one power of two does not hold
-  if constexpr (DT == KQ_BF16) {
-    // largest magnitude: bf16 magnitudes order like their bit patterns, two per packed integer maximum
-    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-    u16x2 am2 = {0, 0};
-    const uint32_t absmask = opaque_sgpr(0x7fff7fffu);
-    SFor<MB * XL>::run([&](auto t) {
-      const u32x4 v = xreg[decltype(t)::value];
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const uint32_t mag = v[e] & absmask;
-        am2 = __builtin_elementwise_max(am2, __builtin_bit_cast(u16x2, mag));
-      }
-    });
-    float amax = __builtin_bit_cast(float, (uint32_t)(am2[0] > am2[1] ? am2[0] : am2[1]) << 16);
-    amax = wave_max_nonneg(amax);
-    if (((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xff) == 0xff) {
-      // an infinity or a NaN among the activations (their patterns order above every finite one): the largest
-      // finite-or-infinite magnitude the floating-point maximum finds, which ignores NaNs
-      amax = 0.f;
+  SFor<NS>::run([&](auto half) {
+    constexpr int HALF = decltype(half)::value;
+    constexpr auto covers = [](int t) { return NS == 1 || t % XL / 2 == HALF; };
+    float& xscale = xscale_of[HALF];
+    float& inv = inv_of[HALF];
+    xscale = inv = 1.0f;
+    if constexpr (DT == KQ_BF16) {
+      // largest magnitude: bf16 magnitudes order like their bit patterns, two per packed integer maximum
+      typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+      u16x2 am2 = {0, 0};
+      const uint32_t absmask = opaque_sgpr(0x7fff7fffu);
       SFor<MB * XL>::run([&](auto t) {
+        if constexpr (!covers(decltype(t)::value)) return;
         const u32x4 v = xreg[decltype(t)::value];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] << 16)));
-          amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] & 0xffff0000u)));
+          const uint32_t mag = v[e] & absmask;
+          am2 = __builtin_elementwise_max(am2, __builtin_bit_cast(u16x2, mag));
         }
       });
+      float amax = __builtin_bit_cast(float, (uint32_t)(am2[0] > am2[1] ? am2[0] : am2[1]) << 16);
       amax = wave_max_nonneg(amax);
-    }
-    // bring the largest magnitude into [2^14, 2^15): exact power-of-two scaling
-    const uint32_t eb = (__builtin_bit_cast(uint32_t, amax) >> 23) & 0xff;
-    if (eb != 0 && eb != 0xff) {
-      int e = (int)eb - 127 - 14;
-      if (e < -100) e = -100;
-      xscale = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
-      inv = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23);
-    }
-    if constexpr (GM == 3) {
-      // a value below 2^-17 in the scaled unit loses bits of its own, and beside weights of zero it may be the result
-      const uint32_t cut = eb == 0xff || eb == 0 ? 0x8000u : ((__builtin_bit_cast(uint32_t, xscale) >> 23) - 17) << 7;
-      u16x2 low = {0xffff, 0xffff};
-      SFor<MB * XL>::run([&](auto t) {
-        const u32x4 v = xreg[decltype(t)::value];
+      if (((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xff) == 0xff) {
+        // an infinity or a NaN among the activations (their patterns order above every finite one): the largest
+        // finite-or-infinite magnitude the floating-point maximum finds, which ignores NaNs
+        amax = 0.f;
+        SFor<MB * XL>::run([&](auto t) {
+          if constexpr (!covers(decltype(t)::value)) return;
+          const u32x4 v = xreg[decltype(t)::value];
 #pragma unroll
-        for (int e = 0; e < 4; e++)
-          low = __builtin_elementwise_min(low, (u16x2)(__builtin_bit_cast(u16x2, v[e] & absmask) - (uint16_t)1));
-      });
-      wide = __builtin_amdgcn_ballot_w64((int)(low[0] < low[1] ? low[0] : low[1]) < (int)cut - 1) != 0;
+          for (int e = 0; e < 4; e++) {
+            amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] << 16)));
+            amax = fmaxf(amax, fabsf(__builtin_bit_cast(float, v[e] & 0xffff0000u)));
+          }
+        });
+        amax = wave_max_nonneg(amax);
+      }
+      // bring the largest magnitude into [2^14, 2^15): exact power-of-two scaling
+      const uint32_t eb = (__builtin_bit_cast(uint32_t, amax) >> 23) & 0xff;
+      if (eb != 0 && eb != 0xff) {
+        int e = (int)eb - 127 - 14;
+        if (e < -100) e = -100;
+        xscale = __builtin_bit_cast(float, (uint32_t)(127 + e) << 23);
+        inv = __builtin_bit_cast(float, (uint32_t)(127 - e) << 23);
+      }
+      if constexpr (GM == 3) {
+        // a value below 2^-17 in the scaled unit loses bits of its own, and beside weights of zero it may be the result
+        const uint32_t cut = eb == 0xff || eb == 0 ? 0x8000u : ((__builtin_bit_cast(uint32_t, xscale) >> 23) - 17) << 7;
+        u16x2 low = {0xffff, 0xffff};
+        SFor<MB * XL>::run([&](auto t) {
+          const u32x4 v = xreg[decltype(t)::value];
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            low = __builtin_elementwise_min(low, (u16x2)(__builtin_bit_cast(u16x2, v[e] & absmask) - (uint16_t)1));
+        });
+        wide = __builtin_amdgcn_ballot_w64((int)(low[0] < low[1] ? low[0] : low[1]) < (int)cut - 1) != 0;
+      }
     }
-  }
+  });
   // A registers.  Lane (kg, fa, fi) keeps, for every row group, unit and register pair, the four activations of
   // row 4 g + fi that MFMA block fa needs.
   //   q4_k / q5_k: pair pc, block 2 e + h  -> k = 128 kg + 32 (2 (pc / 2) + h) + 16 (pc % 2) + 4 e
@@ -1192,6 +1204,7 @@ __global__ __launch_bounds__(64 * NW, WGS) void stream_gemv_kernel(StArgsOf<GM> 
       constexpr int ml = T / XL, m = c * XCH + ml, s = T % XL;
       const int gi = lane + 64 * s, uu = gi >> 5, grp = gi & 31;
       const u32x4 v = xreg[m * XL + s];
+      const float inv = inv_of[NS == 1 ? 0 : s / 2];
       _Float16 h[8];
       typedef _Float16 f16x2p __attribute__((ext_vector_type(2)));
       f16x2p hp[4];
@@ -1430,6 +1443,7 @@ __global__ __launch_bounds__(64 * NW, WGS) void stream_gemv_kernel(StArgsOf<GM> 
         const uint8_t* slot = wb + cslot * U::SLOT;
         const uint8_t* bl = slot + crow * G::LBPB;
         constexpr int us = u / UPS;  // the wave's superblock this unit belongs to
+        const float xscale = xscale_of[NS == 1 ? 0 : us / 4];
         float* acc = (GM == 2 && (u & 1)) ? acc_b : acc_a;
         float unit_sum[GM == 3 ? R : 1];
         if constexpr (GM == 3) {

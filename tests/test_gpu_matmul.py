@@ -161,6 +161,27 @@ def test_qmm_streamed_kernel_long_rows_in_short_tiles(kq, codec, dtype):
         assert rel_l2(dev_to_bits(got), want, dtype) <= TOL, (codec, dtype, M, N, K)
 
 
+@pytest.mark.parametrize("codec", ["q4_k", "q5_k", "q6_k", "q2_k", "q3_k"])
+@pytest.mark.parametrize("M", [1, 2])
+def test_qmm_streamed_kernel_long_rows_of_wide_range(kq, codec, M):
+    """A large value on weights that are zero leaves the other half of the row its bits, whichever half it lies in: waves take every
+    eighth superblock, so no power of two is shared between the first 32 and the others."""
+    N, K = 4200, 64 * 256
+    wire = _wire(codec, N, K, seed=47)
+    blocks = wire.reshape(N, K // 256, -1)
+    for big in (5, 40):
+        w = blocks.copy()
+        w[:, big] = 0  # scales (and for q3_k / q6_k codes) of zero: weights of zero
+        x = np.random.default_rng(48).standard_normal((M, K)).astype(np.float32) * 1e-4
+        x[:, :8192] *= big >= 32
+        x[:, 8192:] *= big < 32
+        x[:, 256 * big + 7] = 1e12
+        xb = O.f32_to_bits(x, "bfloat16")
+        w = w.reshape(wire.shape)
+        got = kq.quantized_matmul(bits_to_dev(xb, "bfloat16"), wire_to_dev(w), None, codec)
+        assert rel_l2(dev_to_bits(got), O.qmm(xb, w, codec, True, "bfloat16"), "bfloat16") <= TOL, big
+
+
 @pytest.mark.parametrize("codec", ["mxfp4", "q4_0", "iq4_nl", "q8_0"])
 @pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
 def test_qmm_streamed_kernel_k_ends_inside_a_unit(kq, codec, dtype):
