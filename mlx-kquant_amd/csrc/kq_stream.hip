@@ -1632,13 +1632,17 @@ StRows st_rows(int codec) {
   return StRows{0, 0};
 }
 int st_max_sb(int codec, int M) { return g_st_nw8 && M <= st_rows(codec).nw8 ? 32 : 16; }
-// longest row (superblocks) up to which matrices of at most CUs / 2 tiles take short tiles, below which a split is slower:
-// q4_k, two rows, 4096 x 11008 9.4 -> 9.1 but x 14336 10.1 against 10.5; q2_k 9.3 -> 8.1 and 9.3 against 9.5, two rows 9.5 ->
-// 8.6 at 8448 and 9.3 against 9.5 at 11008
-int st_long_max(int codec, int M) {
-  if (codec == KQ_Q4_K) return M == 1 ? 64 : 48;
-  if (codec == KQ_Q2_K) return M == 1 ? 48 : 40;
-  return 0;
+// Longest row (superblocks) that q4_k and q2_k, the codecs of few instructions per unit, bring into short tiles where the matrix
+// has at most CUs / 2 tiles (a split is ahead for the others).  us, split / short tiles, matrices of 64 ... 2048, 3072 and 4096 rows:
+//   q4_k, one row, 40 superblocks   in a graph 6.7 - 7.8, 9.3, 7.2 / 7.5 - 8.0, 8.0, 8.0   launched one by one 8.6 - 8.8, 9.4, 8.7 / 7.4 - 7.8, 7.5, 7.5
+//                   33              6.2 - 7.6, 9.2, 7.0 / 7.0 - 7.5, 7.4, 7.3                                  8.6 - 9.1, 9.6, 8.9 / 7.0, 7.1, 7.0
+//                   56              6.8 - 8.9, 11.1, 8.7 / 9.1 - 9.7, 9.5, 9.6                                 8.6 - 8.9, 10.8, 8.9 / 8.9 - 9.3, 9.2, 9.2
+//   two rows        40              6.8 - 8.9, 9.9, 7.7 / 8.9 - 9.5, 9.4, 9.3                                  8.6 - 9.1, 9.9, 8.7 / 8.8 - 9.2, 9.0, 8.9
+// (q2_k the same within 0.4).  Between CUs / 4 and CUs / 2 tiles the split fills a part of a second round of workgroups, hence the 3072.
+int st_long_max(int codec, int M, int tiles, int cus) {
+  if (codec != KQ_Q4_K && codec != KQ_Q2_K) return 0;
+  const bool part_round = 4 * tiles > cus && 2 * tiles < cus;
+  return M == 1 ? (part_round ? 48 : 40) : part_round ? 40 : 0;
 }
 StSplit st_split_plan(int M, int N, int K, int codec, int cus) {
   const int nsb = K >> 8, tiles = (N + ST_ROWS - 1) / ST_ROWS, maxsb = st_max_sb(codec, M);
@@ -1662,9 +1666,9 @@ StSplit st_split_plan(int M, int N, int K, int codec, int cus) {
   // for 32), the split's on the matrix: two splits are one round of workgroups up to cus / 2 tiles and two from there on, so
   // beyond that the short tiles win for every codec (5120 x 13824, one row, us with the host, split before: q4_k 12.4 -> 9.3,
   // q5_k 15.5 -> 12.4, q6_k 20.3 -> 16.7, iq4_xs 13.6 -> 12.5, nvfp4 15.0 -> 13.8).  Below, only the codecs of few instructions
-  // per unit do, up to st_long_max superblocks (q4_k, 4096 x 8448: 9.4 -> 7.0, 4096 x 14336: 9.8 -> 9.1; q6_k 13.0 against 13.5).
+  // per unit do, up to st_long_max superblocks.
   if (g_st_short_tiles && nsb > 32 && nsb <= 64 && M <= st_rows(codec).lng && tiles < cus &&
-      (2 * tiles > cus || nsb <= st_long_max(codec, M))) {
+      (2 * tiles > cus || nsb <= st_long_max(codec, M, tiles, cus))) {
     int r = (N + cus - 1) / cus;
     if (r < 8) r = 8;
     if (r < ST_ROWS) return StSplit{1, nsb, r};

@@ -153,6 +153,7 @@ def test_qmm_streamed_kernel_long_rows_in_short_tiles(kq, codec, dtype):
         shapes.append((1, 4111, 40 * 256 + 96))
     if codec in ("q4_k", "q2_k"):
         shapes += [(1, 100, 48 * 256), (2, 1001, 40 * 256), (1, 2050, 33 * 256)]
+        shapes += [(1, 64, 40 * 256), (1, 3071, 48 * 256), (2, 2081, 40 * 256)]
     for M, N, K in shapes:
         wire = _wire(codec, N, K, seed=45)
         xb, xt = make_x((M, K), dtype, seed=46)
