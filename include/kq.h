@@ -148,6 +148,10 @@ int kq_moe_segment_rows(int T, int R, int E, int N, int K, int glu, int codec);
  * Replaces KQuantGatherQMM::eval_cpu, reference src/kquant_gather.cpp:470-746
  * (kquant_qmm_cpu_batch, src/kquant_cpu_decode.cpp:1361-1527). */
 size_t kq_gather_qmm_workspace_size(int B, int M, int E, int N, int K, int transpose, int codec, int dtype);
+/* What of it a call with these addresses and strides uses: that size, or 0 (short contractions over few rows per expert run in one
+ * launch). */
+size_t kq_gather_qmm_workspace_used(const void* x_dev, const void* w_dev, int B, int M, int E, int N, int K, int64_t x_batch_stride,
+                                    int64_t w_expert_stride_bytes, int transpose, int codec, int dtype);
 int kq_gather_qmm(const void* x_dev, const void* w_dev, const uint32_t* lhs_idx_dev,
                   const uint32_t* rhs_idx_dev, void* out_dev, int B, int M, int E, int N, int K,
                   int64_t x_batch_stride, int64_t w_expert_stride_bytes, int transpose, int rhs_sorted,

@@ -288,6 +288,23 @@ static int try_moe_grouped(const char* op, const void* x, const void* w, const v
 static bool per_entry_route(int64_t P, int entry_rows, bool has_bias, int glu, int act, int codec, int E, int N, int K,
                             bool stream_takes);
 
+// Whether a transposed call runs entry by entry; the others are kq_launch_heads' if it takes them, else the grouped kernels'
+static bool gather_by_entry(const void* x, const void* w, int64_t P, int M, int E, int N, int K, int64_t x_batch_stride,
+                            int64_t w_expert_stride, int codec) {
+  return per_entry_route(P, M, false, 0, 0, codec, E, N, K,
+                         kq_gather_stream_takes(x, w, nullptr, (int)(P > 0x7fffffff ? 0x7fffffff : P), N, K, true, x_batch_stride,
+                                                w_expert_stride, false, codec));
+}
+
+size_t kq_gather_qmm_workspace_used(const void* x_dev, const void* w_dev, int B, int M, int E, int N, int K, int64_t x_batch_stride,
+                                    int64_t w_expert_stride_bytes, int transpose, int codec, int dtype) {
+  const size_t size = kq_gather_qmm_workspace_size(B, M, E, N, K, transpose, codec, dtype);
+  if (!size || gather_by_entry(x_dev, w_dev, (int64_t)B * M, M, E, N, K, x_batch_stride, w_expert_stride_bytes, codec) ||
+      kq_heads_takes(x_dev, w_dev, B, M, E, N, K, x_batch_stride, w_expert_stride_bytes, codec))
+    return 0;
+  return size;
+}
+
 int kq_gather_qmm(const void* x_dev, const void* w_dev, const uint32_t* lhs_idx_dev, const uint32_t* rhs_idx_dev,
                   void* out_dev, int B, int M, int E, int N, int K, int64_t x_batch_stride,
                   int64_t w_expert_stride_bytes, int transpose, int rhs_sorted, int codec, int dtype,
@@ -313,9 +330,7 @@ int kq_gather_qmm(const void* x_dev, const void* w_dev, const uint32_t* lhs_idx_
   }
   int64_t P;
   const bool batched = gather_batched_shape(B, M, E, N, K, transpose, codec, &P);
-  const bool by_entry = per_entry_route(P, M, false, 0, 0, codec, E, N, K,
-                                        kq_gather_stream_takes(x_dev, w_dev, nullptr, (int)(P > 0x7fffffff ? 0x7fffffff : P), N, K,
-                                                               true, x_batch_stride, w_expert_stride_bytes, false, codec));
+  const bool by_entry = gather_by_entry(x_dev, w_dev, P, M, E, N, K, x_batch_stride, w_expert_stride_bytes, codec);
   // short contractions over few rows per expert: one launch
   if (!by_entry) {
     const int rch = kq_launch_heads(x_dev, static_cast<const uint8_t*>(w_dev), lhs_idx_dev, rhs_idx_dev, out_dev, B, M, E, N, K,

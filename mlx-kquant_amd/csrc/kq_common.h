@@ -182,7 +182,8 @@ inline size_t kq_redo_bytes(int M, int N) { return ((size_t)M + (size_t)((N + 31
 KqRedo kq_tall_redo(void* ws, int M, int N, int K);
 int kq_launch_anymma_redo(const void* x, const uint8_t* w, void* y, int M, int N, int K, int codec, int dtype, KqRedo redo,
                           hipStream_t s);
-bool kq_heads_supported(int B, int M, int E, int N, int K, int codec);
+bool kq_heads_takes(const void* x, const void* w, int B, int M, int E, int N, int K, int64_t x_batch_stride,
+                    int64_t w_expert_stride, int codec);
 int kq_launch_heads(const void* x, const uint8_t* w, const uint32_t* lhs, const uint32_t* rhs, void* out, int B, int M, int E,
                     int N, int K, int64_t x_batch_stride, int64_t w_expert_stride, int codec, int dtype, hipStream_t s);
 bool kq_mid_supported(int M, int N, int K, int codec);

@@ -292,7 +292,7 @@ int launch_heads(const HeadArgs& a, int E, hipStream_t s) {
 
 }  // namespace
 
-bool kq_heads_supported(int B, int M, int E, int N, int K, int codec) {
+static bool heads_shape(int B, int M, int E, int N, int K, int codec) {
   if (codec < 0 || codec >= KQ_NUM_CODECS || B <= 0 || M <= 0 || E <= 0 || E > kqentries::MAX_EXPERTS || N <= 0 || B > MAX_ENTRIES) return false;
   if (K <= 0 || K % CK_STEP || K > HD_STEPS * CK_STEP || K % kq_geom(codec).wpb) return false;
   const int64_t row_bytes = (int64_t)(K / kq_geom(codec).wpb) * kq_geom(codec).bpb;
@@ -307,12 +307,16 @@ bool kq_heads_supported(int B, int M, int E, int N, int K, int codec) {
   return P <= 32 * (int64_t)E || N <= 256 || !kq_moe_grouped_supported((int)P, E, N, K, codec);
 }
 
+bool kq_heads_takes(const void* x, const void* w, int B, int M, int E, int N, int K, int64_t x_batch_stride, int64_t w_expert_stride,
+                    int codec) {
+  return heads_shape(B, M, E, N, K, codec) && !(reinterpret_cast<uintptr_t>(x) & 15) && !(x_batch_stride & 7) &&
+         !(reinterpret_cast<uintptr_t>(w) & 1) && !(w_expert_stride & 1);
+}
+
 // KQ_ERR_UNSUPPORTED: nothing launched
 int kq_launch_heads(const void* x, const uint8_t* w, const uint32_t* lhs, const uint32_t* rhs, void* out, int B, int M, int E,
                     int N, int K, int64_t x_batch_stride, int64_t w_expert_stride, int codec, int dtype, hipStream_t s) {
-  if (!kq_heads_supported(B, M, E, N, K, codec) || (reinterpret_cast<uintptr_t>(x) & 15) || (x_batch_stride & 7) ||
-      (reinterpret_cast<uintptr_t>(w) & 1) || (w_expert_stride & 1))
-    return KQ_ERR_UNSUPPORTED;
+  if (!kq_heads_takes(x, w, B, M, E, N, K, x_batch_stride, w_expert_stride, codec)) return KQ_ERR_UNSUPPORTED;
   HeadArgs a{static_cast<const uint16_t*>(x), w, static_cast<uint16_t*>(out), lhs, rhs, kq_device_grids(), B, M, N, K,
              x_batch_stride, w_expert_stride};
   if (!a.grids) return KQ_ERR_HIP;

@@ -27,7 +27,7 @@ struct Abi {
   KQ_FN(kq_dequantize);
   KQ_FN(kq_qmm_workspace_size);
   KQ_FN(kq_qmm);
-  KQ_FN(kq_gather_qmm_workspace_size);
+  KQ_FN(kq_gather_qmm_workspace_used);
   KQ_FN(kq_gather_qmm);
   KQ_FN(kq_moe_workspace_size);
   KQ_FN(kq_moe_glu_gather);
@@ -211,7 +211,8 @@ PyObject* op_gather_qmm(PyObject* const* a) {  // x, w, codec, lhs, rhs, transpo
   size.push_back(M);
   size.push_back(N);
   at::Tensor out = c.empty(size, x.scalar_type());
-  const Workspace ws(c, abi.kq_gather_qmm_workspace_size(B, M, E, N, K, tr, codec, dt));
+  const Workspace ws(c, abi.kq_gather_qmm_workspace_used(x.data_ptr(), w.data_ptr(), B, M, E, N, K, (int64_t)M * K,
+                                                           w.size(1) * w.size(2), tr, codec, dt));
   void* s = c.stream();
   int rc;
   {
@@ -444,7 +445,7 @@ PyObject* init(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return nullptr;                                                          \
   }
   KQ_FN(kq_last_error) KQ_FN(kq_codec_get) KQ_FN(kq_dequantize) KQ_FN(kq_qmm_workspace_size) KQ_FN(kq_qmm)
-  KQ_FN(kq_gather_qmm_workspace_size) KQ_FN(kq_gather_qmm) KQ_FN(kq_moe_workspace_size) KQ_FN(kq_moe_glu_gather)
+  KQ_FN(kq_gather_qmm_workspace_used) KQ_FN(kq_gather_qmm) KQ_FN(kq_moe_workspace_size) KQ_FN(kq_moe_glu_gather)
   KQ_FN(kq_gather_qmv) KQ_FN(kq_moe_glu_gather_shexp_workspace_size) KQ_FN(kq_moe_glu_gather_shexp)
   KQ_FN(kq_gather_qmv_mix_workspace_size) KQ_FN(kq_gather_qmv_mix) KQ_FN(kq_moe_router_topk)
   KQ_FN(kq_quantize_dev_supported) KQ_FN(kq_quantize_dev)

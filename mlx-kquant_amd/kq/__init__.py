@@ -80,6 +80,8 @@ def _load():
     lib.kq_moe_router_topk.argtypes = [vp, i, i, i, i, i, i, vp, vp, i, C.c_float, vp, vp, vp]
     lib.kq_gather_qmm_workspace_size.restype = sz
     lib.kq_gather_qmm_workspace_size.argtypes = [i, i, i, i, i, i, i, i]
+    lib.kq_gather_qmm_workspace_used.restype = sz
+    lib.kq_gather_qmm_workspace_used.argtypes = [vp, vp, i, i, i, i, i, i64, i64, i, i, i]
     lib.kq_gather_qmm.argtypes = [vp, vp, vp, vp, vp, i, i, i, i, i, i64, i64, i, i, i, i, vp, sz, vp]
     lib.kq_moe_workspace_size.restype = sz
     lib.kq_moe_workspace_size.argtypes = [i, i, i, i, i, i, i, i]
@@ -409,7 +411,8 @@ def _gather_qmm_impl(x, w, kquant_type, lhs_indices, rhs_indices, transpose, sor
     right_sorted = bool(sorted_indices) and lhs_indices is None
     lib = _load()
     with torch.cuda.device(x.device):
-        ws_bytes = lib.kq_gather_qmm_workspace_size(B, M, E, N, K, int(bool(transpose)), cid, _DT[out_type])
+        ws_bytes = lib.kq_gather_qmm_workspace_used(x_c.data_ptr(), w3.data_ptr(), B, M, E, N, K, M * K, estride,
+                                                    int(bool(transpose)), cid, _DT[out_type])
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
         _check(lib.kq_gather_qmm(x_c.data_ptr(), w3.data_ptr(), lhs.data_ptr(), rhs.data_ptr(), out.data_ptr(), B, M, E,
                                  N, K, M * K, estride, int(bool(transpose)), int(right_sorted), cid, _DT[out_type],

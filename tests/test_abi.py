@@ -177,3 +177,20 @@ def test_mix_of_one_token_needs_no_workspace(lib, codec, S, N, K):
     assert f(2, S, 64, N, K, c, -1, 2) > 0
     assert f(4, S, 64, N, K, c, c, 2) > 0
     assert f(1, 33, 64, N, K, c, -1, 2) > 0
+
+
+@pytest.mark.parametrize("codec,K", [("q8_0", 512), ("q4_k", 256), ("nvfp4", 512)])
+def test_gather_of_short_rows_uses_no_workspace(lib, codec, K):
+    """128 heads, four tokens each, run in one launch; not from activations or weights that its loads cannot take, nor longer rows."""
+    size, used = lib.kq_gather_qmm_workspace_size, lib.kq_gather_qmm_workspace_used
+    size.restype = used.restype = C.c_size_t
+    c = lib.kq_codec_id(codec.encode())
+
+    def call(x=4096, w=8192, B=512, K=K, transpose=1):
+        return used(C.c_void_p(x), C.c_void_p(w), B, 1, 128, 128, K, C.c_int64(K), C.c_int64(1 << 16), transpose, c, 2)
+
+    assert size(512, 1, 128, 128, K, 1, c, 2) > 0 and call() == 0
+    assert call(w=8193) == call(x=4098) == size(512, 1, 128, 128, K, 1, c, 2)
+    assert call(K=2048) == size(512, 1, 128, 128, 2048, 1, c, 2) > 0
+    assert call(B=16) == call(transpose=0) == 0
+    assert call(B=24) == 0  # entry by entry, or the one launch
