@@ -9,9 +9,8 @@
 // (fit_scale_min below): 210 instead of 660 instructions a weight, the SIMDs 95 % busy issuing them.  One lane per
 // sub-block (8 or 16 per superblock) keeps all three arrays of a fit in registers.  4096 x 4096 f32, all candidates ->
 // bounded, with the launch: q4_k 241 -> 118 us, q5_k 260 -> 121, q2_k 345 -> 181 (q3_k 82, q6_k 78: 19 candidates, no
-// bound); 300 x 4096 q4_k 42 -> 25; 128 x 1024, where one wave's latency counts, 23.4 -> 24.5.  Every-candidate kernels
-// shared the candidates of a small matrix between lanes; the bounded scan is as fast there without.  Blocks narrow and far
-// above zero, whose least-squares systems are near singular, keep more candidates: q4_k 251 -> 230, q5_k 275 -> 280.
+// bound); 300 x 4096 q4_k 42 -> 25; small matrices, where one wave's latency counts, share all candidates of a sub-block between four
+// lanes (launch_k).  Blocks narrow and far above zero, whose least-squares systems are near singular, keep more candidates.
 // Legacy codecs: memory.  Eight lanes per block, 16-byte loads, wire bytes assembled in LDS and stored as dwords
 // (4096 x 4096 f32 to q8_0: 20 us, 4.2 TB/s).
 #include "kq_common.h"
@@ -175,8 +174,8 @@ struct FitBins {  // [step of the half][lane], eight bytes a lane: conflict-free
 
 __device__ __forceinline__ float step_numerator(float step, int nmax) { return -0.9f + 0.05f * step + float(nmax); }
 
-template <int N, int NMAX>
-__device__ __forceinline__ float fit_scale_min(float (&x)[N], float (&wt)[N], FitBins& bins, int lane,
+template <int N, int NMAX, int S>
+__device__ __forceinline__ float fit_scale_min(float (&x)[N], float (&wt)[N], FitBins* bins_lds, int lane, int part,
                                                float& neg_min) {
   float vmin = x[0], vmax = x[0], sw = wt[0], swx = sw * x[0], wmin = wt[0], wmax = wt[0];
 #pragma unroll
@@ -226,8 +225,13 @@ __device__ __forceinline__ float fit_scale_min(float (&x)[N], float (&wt)[N], Fi
 
   unsigned long long todo = flat ? 0 : (1ull << STEPS) - 1;
   bool grid = true;
-  if (range >= 1e-9f && range <= 1e9f && vmax <= 1e9f && vmin >= -1e9f && wmin >= 0.f && wmax >= 1e-9f && wmax <= 1e9f &&
+  if constexpr (S > 1) {
+    unsigned long long every = 0;
+    for (int step = 0; step < STEPS; step += S) every |= 1ull << step;
+    todo &= every << part;
+  } else if (range >= 1e-9f && range <= 1e9f && vmax <= 1e9f && vmin >= -1e9f && wmin >= 0.f && wmax >= 1e-9f && wmax <= 1e9f &&
       sw == sw && swx == swx) {
+    FitBins& bins = *bins_lds;
     const float ws = 65535.0f / wmax, inv0 = step_numerator(0.f, NMAX) / range;
     const float rr = 1.0f / range;  // correctly rounded: two corrections of n * rr give n / range so
     const float per_step = 20.f * range, zero_step = -(float(NMAX) - 0.9f) * 20.f - 1e-3f;
@@ -377,6 +381,17 @@ __device__ __forceinline__ float fit_scale_min(float (&x)[N], float (&wt)[N], Fi
     todo &= todo - 1;
     evaluate(step);
   }
+#pragma unroll
+  for (int m = 1; m < S; m <<= 1) {  // of equal errors the earliest
+    const float oe = __shfl_xor(best_err, m), os = __shfl_xor(scale, m), om = __shfl_xor(best_min, m);
+    const int ost = __shfl_xor(best_step, m);
+    if (oe < best_err || (oe == best_err && ost < best_step)) {
+      best_err = oe;
+      scale = os;
+      best_min = om;
+      best_step = ost;
+    }
+  }
   neg_min = flat ? -vmin : -best_min;
   return flat ? 0.f : scale;
 }
@@ -520,25 +535,25 @@ __device__ __forceinline__ float fit_positive_pair(const float* sc, const float*
   return sl2 > 0.f ? slx / sl2 : 0.f;
 }
 
-template <int C>
+template <int C, int S>
 __global__ __launch_bounds__(64, 2) void encode_k_kernel(const void* __restrict__ w, int dtype,
                                                       const float* __restrict__ imatrix, uint8_t* __restrict__ wire,
                                                       int64_t nblocks, int64_t blocks_per_row, bool aligned) {
   constexpr int BPB = kq_geom(C).bpb, SUBS = KGeom<C>::SUBS, N = KGeom<C>::N;
-  constexpr int GROUP = SUBS, NSB = 64 / GROUP;      // lanes per superblock, superblocks per wave
+  constexpr int GROUP = SUBS * S, NSB = 64 / GROUP;  // lanes per superblock, superblocks per wave
   constexpr int XS = 256 + 4;                        // floats between superblocks in LDS: eight of them in eight banks
   constexpr bool kMin = C == KQ_Q2_K || C == KQ_Q4_K || C == KQ_Q5_K;
   // One buffer for what lives one after the other: the staged weights, the bins of the (scale, min) fit, and the levels and
   // wire bytes (a workgroup of less than 20 KiB lets a CU hold eight, two per SIMD).
   constexpr size_t BUF = NSB * XS * sizeof(float);
-  __shared__ __attribute__((aligned(16))) uint8_t buf[kMin ? sizeof(FitBins) : BUF];
+  __shared__ __attribute__((aligned(16))) uint8_t buf[kMin && S == 1 ? sizeof(FitBins) : BUF];
   static_assert(BUF >= NSB * 256 + NSB * BPB && sizeof(FitBins) >= BUF, "buffer");
   float* xs = reinterpret_cast<float*>(buf);
   auto* s_lv = reinterpret_cast<uint8_t(*)[256]>(buf);
   uint8_t* out = buf + NSB * 256;
   __shared__ float s_sc[NSB][SUBS], s_mn[NSB][SUBS], s_sw[NSB][SUBS];
   __shared__ int s_ls[NSB][SUBS], s_lm[NSB][SUBS];
-  const int lane = threadIdx.x, sb = lane / GROUP, gl = lane % GROUP, j = gl;
+  const int lane = threadIdx.x, sb = lane / GROUP, gl = lane % GROUP, j = gl / S, part = gl % S;
   // superblocks past the end redo the last one; their bytes are not stored
   const int64_t blk0 = (int64_t)blockIdx.x * NSB, last = min(blk0 + NSB, nblocks) - 1;
   auto stage = [&](int dt, bool al) {  // all loads first: few waves are there to cover their latency
@@ -603,16 +618,19 @@ __global__ __launch_bounds__(64, 2) void encode_k_kernel(const void* __restrict_
       }
     }
 #pragma unroll
-    for (int i = 0; i < N / 4; i++) reinterpret_cast<uint32_t*>(s_lv[sb])[N / 4 * j + i] = packed[i];
+    for (int i = 0; i < N / 4; i++)
+      if (i % S == part) reinterpret_cast<uint32_t*>(s_lv[sb])[N / 4 * j + i] = packed[i];
   };
   if constexpr (kMin) {
     float sw = 0.f, neg_min;
 #pragma unroll
     for (int i = 0; i < N; i++) sw += wt[i];
-    const float sc = fit_scale_min<N, KGeom<C>::NMAX>(x, wt, *reinterpret_cast<FitBins*>(buf), lane, neg_min);
-    s_sc[sb][j] = sc;
-    s_mn[sb][j] = neg_min;
-    s_sw[sb][j] = sw;
+    const float sc = fit_scale_min<N, KGeom<C>::NMAX, S>(x, wt, reinterpret_cast<FitBins*>(buf), lane, part, neg_min);
+    if (part == 0) {
+      s_sc[sb][j] = sc;
+      s_mn[sb][j] = neg_min;
+      s_sw[sb][j] = sw;
+    }
     __syncthreads();
     constexpr int LMAX = C == KQ_Q2_K ? 15 : 63, DOFF = C == KQ_Q2_K ? 80 : 0;
     int lv[SUBS];
@@ -738,15 +756,27 @@ int launch_legacy(const void* w, int dtype, uint8_t* wire, int64_t nblocks, hipS
   return KQ_OK;
 }
 
-template <int C>
-int launch_k(const void* w, int dtype, const float* im, uint8_t* wire, int64_t nblocks, int64_t bpr, hipStream_t s) {
-  constexpr int NSB = 64 / KGeom<C>::SUBS;
+template <int C, int S>
+int launch_k_shared(const void* w, int dtype, const float* im, uint8_t* wire, int64_t nblocks, int64_t bpr, hipStream_t s) {
+  constexpr int NSB = 64 / (KGeom<C>::SUBS * S);
   const int64_t wgs = (nblocks + NSB - 1) / NSB;
   if (wgs > 0x7fffffff) return kq_set_error(KQ_ERR_INVALID, "quantize: tensor too large for one launch");
-  hipLaunchKernelGGL(encode_k_kernel<C>, dim3((unsigned)wgs), dim3(64), 0, s, w, dtype, im, wire, nblocks, bpr,
+  hipLaunchKernelGGL((encode_k_kernel<C, S>), dim3((unsigned)wgs), dim3(64), 0, s, w, dtype, im, wire, nblocks, bpr,
                      four_aligned(w, dtype));
   KQ_HIP_CHECK(hipGetLastError());
   return KQ_OK;
+}
+
+// Up to this many waves of four lanes to a sub-block (one per SIMD) they share its candidates: latency counts, and it hardly depends
+// on the weights.  us, four lanes / one and the bound, normally distributed, in [0, 1), 1000 + normal: q4_k 512 superblocks 22, 22,
+// 20 / 24, 30, 70; 2048 22, 22, 20 / 25, 32, 84; 4096 30, 30, 29 / 25, 32, 84; q2_k 1024 21, 21, 17 / 22, 27, 41.
+constexpr int64_t SHARED_WAVES = 1024;
+
+template <int C>
+int launch_k(const void* w, int dtype, const float* im, uint8_t* wire, int64_t nblocks, int64_t bpr, hipStream_t s) {
+  if constexpr (C == KQ_Q2_K || C == KQ_Q4_K || C == KQ_Q5_K)
+    if (nblocks * KGeom<C>::SUBS * 4 <= 64 * SHARED_WAVES) return launch_k_shared<C, 4>(w, dtype, im, wire, nblocks, bpr, s);
+  return launch_k_shared<C, 1>(w, dtype, im, wire, nblocks, bpr, s);
 }
 
 }  // namespace
