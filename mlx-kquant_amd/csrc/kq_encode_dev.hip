@@ -187,6 +187,9 @@ __device__ __forceinline__ float fit_scale_min(float (&x)[N], float (&wt)[N], Fi
     wmin = fminf(wmin, wt[i]);
     wmax = fmaxf(wmax, wt[i]);
   }
+  // Blocks this narrow and far above zero have all levels alike at most steps and no bound there: a wave of them does not look for
+  // one (1000 + normal, 4096 x 4096: q4_k 341 -> 281 us, q2_k 402 -> 262; 222 and 289 before there was a bound).
+  const bool alike = __builtin_amdgcn_ballot_w64(!((vmax - vmin) * float(NMAX) < 0.1f * vmax)) == 0;
   if (vmin > 0.f) vmin = 0.f;
   const bool flat = vmax <= vmin;
   const float range = vmax - vmin;
@@ -230,7 +233,7 @@ __device__ __forceinline__ float fit_scale_min(float (&x)[N], float (&wt)[N], Fi
     for (int step = 0; step < STEPS; step += S) every |= 1ull << step;
     todo &= every << part;
   } else if (range >= 1e-9f && range <= 1e9f && vmax <= 1e9f && vmin >= -1e9f && wmin >= 0.f && wmax >= 1e-9f && wmax <= 1e9f &&
-      sw == sw && swx == swx) {
+      sw == sw && swx == swx && !alike) {
     FitBins& bins = *bins_lds;
     const float ws = 65535.0f / wmax, inv0 = step_numerator(0.f, NMAX) / range;
     const float rr = 1.0f / range;  // correctly rounded: two corrections of n * rr give n / range so
