@@ -75,28 +75,32 @@ struct Share {
 constexpr size_t count_bytes(int E) { return (size_t)(E + 1) / 2 * 4; }
 __device__ __forceinline__ int count_of(const uint32_t* cnt, int e) { return (int)((cnt[e >> 1] >> (16 * (e & 1))) & 0xffffu); }
 
-// Ids::find for the workgroup's own expert, and the counts of all; after the caller's next barrier share.left is known too.
-template <int ROWS, class Barrier>
-__device__ __forceinline__ int find_and_count(const Ids& ids, uint32_t expert, int B, int M, int E, int cap, int tid, int wave,
-                                              Places& p, uint32_t* cnt, Share& share, Barrier barrier) {
+// Ids::find for the workgroup's own expert, and the counts of all, complete after the caller's next barrier.
+template <class Barrier>
+__device__ __forceinline__ int find_and_count(const Ids& ids, uint32_t expert, int B, int E, int tid, int wave, Places& p,
+                                              uint32_t* cnt, Share& share, Barrier barrier) {
 #pragma unroll 1
   for (int i = tid; i < (E + 1) / 2; i += THREADS) cnt[i] = 0;
   if (tid == 0) {
     share.left = 0;
     share.round = NO_ROUND;
   }
-  barrier();
+  const int count = ids.find(expert, B, tid, wave, p, barrier);
 #pragma unroll
   for (int u = 0; u < PER_THREAD; u++) {
     if (THREADS * u >= B) break;
     if (ids.id[u] < (uint32_t)E) atomicAdd(&cnt[ids.id[u] >> 1], 1u << (16 * (ids.id[u] & 1)));
   }
-  const int count = ids.find(expert, B, tid, wave, p, barrier);
+  return count;
+}
+
+// share.left, known after the caller's next barrier: where the workgroup waits for loads
+template <int ROWS>
+__device__ __forceinline__ void note_left(int M, int E, int cap, int tid, const uint32_t* cnt, Share& share) {
   bool left = false;
 #pragma unroll 1
   for (int e = tid; e < E; e += THREADS) left |= count_of(cnt, e) * M > ROWS * cap;
   if (left) share.left = 1;
-  return count;
 }
 
 // Whether a workgroup that has done its own round takes one of those left over: its expert leaves some, or has fewer rows than

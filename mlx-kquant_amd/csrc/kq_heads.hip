@@ -135,7 +135,7 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
   uint32_t* entries = reinterpret_cast<uint32_t*>(frags + nsteps * (G::NF * 1024));  // per expert
   const int E = gridDim.y, Z = gridDim.z;
   auto barrier = [] { lds_barrier(); };
-  auto round = [&](int r0, int rows) __attribute__((always_inline)) {  // rows r0 ... of the expert whose places and wire bytes are in LDS or on the way
+  auto round = [&](int r0, int rows, auto own) __attribute__((always_inline)) {  // rows r0 ... of the expert whose places and wire bytes are in LDS or on the way
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     lds_barrier();
@@ -197,6 +197,7 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
       }
     }
     if (__builtin_expect(lost_rows != 0, 0)) atomicOr(&wide_rows, lost_rows);
+    if constexpr (decltype(own)::value) kqentries::note_left<32>(a.M, E, Z, tid, entries, share);
     vmwait<0>();  // the wire bytes
     lds_barrier();
     const uint32_t rows_here = here == 32 ? ~0u : (1u << here) - 1, wide = __builtin_amdgcn_readfirstlane(wide_rows) & rows_here;
@@ -250,14 +251,16 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
     kqentries::Ids ids;
     ids.load(a.rhs, a.lhs, a.B, tid);
     if constexpr (mid_table_bytes<C>() > 0) build_tables<C, HD_THREADS, true>(smem, spread, a.grids, tid);
-    own_rows = kqentries::find_and_count<32>(ids, expert, a.B, a.M, E, Z, tid, wave, places, entries, share, barrier) * a.M;
+    own_rows = kqentries::find_and_count(ids, expert, a.B, E, tid, wave, places, entries, share, barrier) * a.M;
   }
   if (__builtin_expect(r0 < own_rows, 1)) {  // uniform
     if (blockIdx.z != 0) request();
-    round(r0, own_rows);
+    round(r0, own_rows, std::true_type{});
     if (__builtin_expect(!share.left || !kqentries::shares_rounds<32>(own_rows, a.B, a.M, E, Z), 1)) return;
   } else {
     vmwait<0>();  // nothing may be on its way into LDS when the workgroup ends
+    lds_barrier();
+    kqentries::note_left<32>(a.M, E, Z, tid, entries, share);
     lds_barrier();
     if (!share.left) return;
   }
@@ -270,7 +273,7 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
   kqentries::Ids ids;
   ids.load(a.rhs, a.lhs, a.B, cold_tid);
   const int rows = ids.find(expert, a.B, cold_tid, wave, places, barrier) * a.M;
-  round(32 * (int)(next >> kqentries::EXPERT_BITS), rows);
+  round(32 * (int)(next >> kqentries::EXPERT_BITS), rows, std::false_type{});
 }
 
 template <int C, int DT>

@@ -174,9 +174,10 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
     if (blockIdx.y == 0 && st_begin + wave < nsteps) fetch_w(st_begin + wave);
     kqentries::Ids ids;
     ids.load(a.rhs, a.lhs, a.B, threadIdx.x);
-    rows = kqentries::find_and_count<16 * MR>(ids, e, a.B, a.M, a.E, gridDim.y, threadIdx.x, wave, places, entries, share,
-                                              [] { __syncthreads(); }) * a.M;
+    rows = kqentries::find_and_count(ids, e, a.B, a.E, threadIdx.x, wave, places, entries, share, [] { __syncthreads(); }) * a.M;
     if (m0 >= rows) {  // uniform
+      __syncthreads();
+      kqentries::note_left<16 * MR>(a.M, a.E, gridDim.y, threadIdx.x, entries, share);
       __syncthreads();
       if (!share.left) return;
     }
@@ -226,6 +227,9 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
     if (st_begin + wave < nsteps) {
       if (!fetched) fetch_w(st_begin + wave);
       fetch_x(st_begin + wave);
+    }
+    if constexpr (MERGE) {
+      if (own) kqentries::note_left<16 * MR>(a.M, a.E, gridDim.y, tid, entries, share);
     }
     for (int st = st_begin + wave; st < nsteps; st += NT_WAVES) {
 #pragma unroll
@@ -352,9 +356,9 @@ __global__ __launch_bounds__(NT_THREADS, MR == 4 ? 1 : 2) void gemm_nt_mfma_kern
     if constexpr (!MERGE) {
       return;
     } else {
+      __syncthreads();  // the sums have been read: the staging areas may be filled again; share.left is known
       if (others || !share.left || !kqentries::shares_rounds<16 * MR>(rows, a.B, a.M, a.E, gridDim.y)) return;
       own = false;
-      __syncthreads();  // the sums have been read: the staging areas may be filled again
     }
   }
 }
