@@ -20,7 +20,7 @@
 #include "kq_epilogue.h"
 
 // kq_moe.hip
-int kq_launch_moe_sort(const uint32_t* idx, int P, int E, void* order, void* segs, void* nseg, hipStream_t s, int per_id = 1);
+int kq_launch_moe_sort(const uint32_t* idx, int P, int E, void* order, void* segs, void* nseg, hipStream_t s);
 
 namespace {
 

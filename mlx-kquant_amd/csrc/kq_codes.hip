@@ -364,7 +364,7 @@ int launch_codes_dt(const CkArgs& a, int dtype, hipStream_t s) {
 }
 
 // ------------------------------------------------------------------ grouped kernel (batched MoE)
-// Pairs sorted by expert and cut into segments of at most 32 pairs of one expert (moe_sort_kernel).  A
+// Pairs sorted by expert and cut into segments of at most 32 pairs of one expert (codes_prepass_kernel).  A
 // workgroup multiplies a segment's gathered activation rows (the MFMA's 32 rows) by a 128-row slab of that
 // expert's wire: 4 waves x 32 weight rows, one 256-weight step at a time, wire bytes and activations
 // fetched one step ahead and parked in LDS.  GLU: the slab is 64 gate rows + the same 64 up rows (waves

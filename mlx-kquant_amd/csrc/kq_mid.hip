@@ -370,7 +370,6 @@ int launch_prepass(const void* x, uint8_t* xf, float* rs, int* counters, int nco
 
 template <int C, int DT>
 int launch_mid(const void* x, MidArgs a, uint8_t* xf, float* rs, hipStream_t s) {
-  using G = MidGeom<C>;
   constexpr size_t lds = (size_t)mid_table_bytes<C>() + (size_t)MID_WAVES * 2 * mid_slot_bytes<C>() + 64;
   static_assert(lds <= 160 * 1024, "the ring does not fit the LDS of a CU");
   const MidPlan p = mid_plan(a.M, a.N, a.K);

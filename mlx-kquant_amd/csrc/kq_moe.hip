@@ -43,10 +43,10 @@ constexpr int SORT_THREADS = 1024;
 
 __global__ __launch_bounds__(SORT_THREADS) void moe_sort_kernel(const uint32_t* __restrict__ idx, int P, int E,
                                                                int* __restrict__ order, Segment* __restrict__ segs,
-                                                               int* __restrict__ nseg_out, int per_id) {
+                                                               int* __restrict__ nseg_out) {
   __shared__ int cnt[SORT_MAX_E];     // pairs per expert, then the running cursor
-  __shared__ int scan_p[SORT_THREADS], scan_s[SORT_THREADS];
-  moe_sort_body<SORT_THREADS>(idx, P, E, order, segs, nseg_out, cnt, scan_p, scan_s, SEG_M, per_id);
+  __shared__ int scan_p[SORT_THREADS / 64], scan_s[SORT_THREADS / 64];
+  moe_sort_body<SORT_THREADS>(idx, P, E, order, segs, nseg_out, cnt, scan_p, scan_s);
 }
 
 // The pair sort and the activation prepass of one grouped launch in ONE kernel: workgroup 0 sorts the pairs, workgroups
@@ -573,10 +573,10 @@ void launch_prologue(const void* x, const MoeWorkspace& m, int rows, int K, cons
 
 }  // namespace
 
-int kq_launch_moe_sort(const uint32_t* idx, int P, int E, void* order, void* segs, void* nseg, hipStream_t s, int per_id) {
+int kq_launch_moe_sort(const uint32_t* idx, int P, int E, void* order, void* segs, void* nseg, hipStream_t s) {
   if (E > SORT_MAX_E) return KQ_ERR_UNSUPPORTED;
   hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(SORT_THREADS), 0, s, idx, P, E, static_cast<int*>(order),
-                     static_cast<Segment*>(segs), static_cast<int*>(nseg), per_id);
+                     static_cast<Segment*>(segs), static_cast<int*>(nseg));
   KQ_HIP_CHECK(hipGetLastError());
   return KQ_OK;
 }

@@ -223,7 +223,8 @@ def test_empty_contraction_and_empty_stack(codec):
 
 @pytest.mark.parametrize("codec", ["q8_0", "q4_k", "q6_k", "iq3_s", "q5_1", "nvfp4"])
 @pytest.mark.parametrize("K,M,B,dtype", [(96, 1, 40, "bfloat16"), (130, 3, 31, "float16"), (64, 8, 200, "bfloat16"),
-                                         (192, 16, 30, "bfloat16"), (100, 24, 23, "bfloat16")])
+                                         (192, 16, 30, "bfloat16"), (100, 24, 23, "bfloat16"),
+                                         (64, 16, 350, "bfloat16"), (40, 24, 180, "float16")])
 def test_other_orientation_merges_entries(codec, K, M, B, dtype):
     """transpose=False, entries of one expert in shared tiles: most of them on one expert (several rounds), experts without any,
     rows that cannot be read 16 bytes at a time, a last step of K that is not whole, a last column tile that is not."""
