@@ -7,10 +7,11 @@
 // order of its sums is part of the result, so a candidate is one lane's serial work: 15 (8) instructions per weight and
 // candidate that cannot be fused.  The (scale, min) codecs evaluate one or two of the 37 and rule the others out by a bound
 // (fit_scale_min below): 210 instead of 660 instructions a weight, the SIMDs 95 % busy issuing them.  One lane per
-// sub-block (8 or 16 per superblock) keeps all three arrays of a fit in registers.  4096 x 4096 f32, all candidates ->
-// bounded, with the launch: q4_k 241 -> 118 us, q5_k 260 -> 121, q2_k 345 -> 181 (q3_k 82, q6_k 78: 19 candidates, no
-// bound); 300 x 4096 q4_k 42 -> 25; small matrices, where one wave's latency counts, share all candidates of a sub-block between four
-// lanes (launch_k).  Blocks narrow and far above zero, whose least-squares systems are near singular, keep more candidates.
+// sub-block (8 or 16 per superblock) keeps all three arrays of a fit in registers.  4096 x 4096 f32, normally distributed,
+// all candidates -> bounded: q4_k 225 -> 112 us, q5_k 254 -> 116, q2_k 296 -> 161 (q3_k 82, q6_k 78: 19 candidates, no
+// bound); 300 x 4096 q4_k 41 -> 26; small matrices, where one wave's latency counts, share all candidates of a sub-block between four
+// lanes (launch_k).  Blocks narrow and far above zero, whose least-squares systems are near singular, keep more candidates
+// (50 + normal: q4_k 223 -> 215, q5_k 252 -> 275; 100 + normal 222 -> 157, 252 -> 320; 1000 + normal 222 -> 281, 251 -> 219).
 // Legacy codecs: memory.  Eight lanes per block, 16-byte loads, wire bytes assembled in LDS and stored as dwords
 // (4096 x 4096 f32 to q8_0: 20 us, 4.2 TB/s).
 #include "kq_common.h"

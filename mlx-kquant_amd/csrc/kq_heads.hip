@@ -12,8 +12,8 @@
 //     value that this does not hold (2^-31 of the step's largest, bf16), or with an infinity, is done in f32 instead.
 //     More rows than 32 are further rounds, of other workgroups (kq_entries.h): 1024 entries of 8 rows on one of 64 experts
 //     243 -> 31 us against rounds in series on the expert's own, 512 of one row on one of 128 100 -> 18.4, even shares 6.7 -> 6.8 (q8_0).
-// 128 heads of 128 x 512, 4 / 16 / 32 rows each, us: q8_0 12.3 / 14.2 / 22.2 -> 6.3 / 7.0 / 9.3, q4_k 10.2 / 11.4 / 14.7 -> 5.6 / 6.7 / 9.5,
-// q6_k 11.3 / 12.7 / 16.0 -> 6.3 / 7.2 / 9.4, the empty launch 2.4; 64 / 128 rows q8_0 31 / 61 -> 10.6 / 20.6, q4_k 28 / 45 -> 11.0 / 21.7.
+// 128 heads of 128 x 512, 4 / 16 / 32 rows each, us: q8_0 12.6 / 14.6 / 22.4 -> 6.8 / 7.8 / 10.0, q4_k 10.3 / 11.7 / 15.4 -> 6.5 / 7.7 / 10.3,
+// q6_k 11.9 / 12.9 / 16.9 -> 7.0 / 7.9 / 9.9, the empty launch 2.4; 64 / 128 rows q8_0 28 / 61 -> 12.9 / 23.3, q4_k 22 / 45 -> 13.5 / 24.1.
 #include <algorithm>
 
 #include "kq_entries.h"
@@ -304,7 +304,7 @@ static bool heads_shape(int B, int M, int E, int N, int K, int codec) {
   // Stacks of more weights than a few per lane and long rows are no matter of latency, and a workgroup of one tile converts its
   // activations for few products: 1000 random pairs, here / the grouped kernels, us: 128 x 2048 x 768 q4_k 109 / 37, q8_0 199 / 62,
   // 128 x 768 x 1024 86 / 24, 86 / 40; but 16 x 512 x 512 14 / 12, 14 / 17, 8 x 4096 x 256 19 / 16, 20 / 29, 128 x 128 x 512 7.8 / 11.2,
-  // 8.1 / 13.9.  256 rows on each expert: 128 x 128 x 512 44 / 80, 42 / 109, 16 x 512 x 512 23 / 24, 22 / 31.
+  // 8.1 / 13.9.  256 rows on each expert: 128 x 128 x 512 43 / 78, 41 / 108, 16 x 512 x 512 20 / 23, 22 / 30.
   const int64_t P = (int64_t)B * M;
   if ((int64_t)E * N * K > (int64_t)1 << 24 || P <= 16 || P > 256 * (int64_t)E) return false;
   return P <= 32 * (int64_t)E || N <= 256 || !kq_moe_grouped_supported((int)P, E, N, K, codec);
