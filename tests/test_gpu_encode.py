@@ -151,6 +151,17 @@ def test_device_encoder_both_lane_splits_and_ragged_ends(kq, codec, dtype):
             assert torch.equal(dev.cpu(), host), (codec, rows, K, off)
 
 
+def _device_bytes(kq, w, codec, im):
+    """w encoded as it is (a small matrix: four lanes share a sub-block's candidates) and, repeated until it is no small one, by the
+    kernel that rules candidates out: the bytes of both, rows of w by bytes."""
+    w, im = w.cuda(), None if im is None else im.cuda()
+    times = 2049 * 256 // w.numel() + 1
+    yield kq.quantize(w, codec, im)[0].cpu().numpy()
+    many = kq.quantize(w.repeat(times, 1), codec, im)[0].reshape(times, len(w), -1)
+    assert torch.equal(many, many[:1].expand_as(many))
+    yield many[0].cpu().numpy()
+
+
 @pytest.mark.parametrize("codec", DEV_CODECS)
 def test_device_encoder_nonfinite_weights_keep_their_bytes(kq, codec):
     """NaN, infinite and f16-overflowing weights: the bytes that the sequential block encoders write when compiled for the
@@ -161,9 +172,9 @@ def test_device_encoder_nonfinite_weights_keep_their_bytes(kq, codec):
     w, im = torch.from_numpy(gold["w"]).cuda(), torch.from_numpy(gold["imatrix"]).cuda()
     for key, imat in ((codec, None), (codec + "_im", im)):
         if key in gold:
-            got = kq.quantize(w, codec, imat)[0].cpu().numpy()
-            bad = np.argwhere((got != gold[key]).any(axis=1)).ravel().tolist()
-            assert not bad, (key, bad)
+            for got in _device_bytes(kq, w, codec, imat):
+                bad = np.argwhere((got != gold[key]).any(axis=1)).ravel().tolist()
+                assert not bad, (key, bad)
 
 
 # rows of each kind for the encoders that rule out candidates by a bound: lattices whose levels sit on ties, one-sided and
@@ -208,10 +219,25 @@ def test_device_encoder_fit_bytes_over_kinds_of_rows(kq, codec, weights):
     make = _FIT_WEIGHTS[weights]
     im = None if make is None else torch.from_numpy(make(rng, K).astype(np.float32))
     host = kq.quantize(w, codec, im)[0].numpy()
-    dev = kq.quantize(w.cuda(), codec, None if im is None else im.cuda())[0].cpu().numpy()
-    bad = np.argwhere((dev != host).any(axis=1)).ravel().tolist()
     kinds = list(_FIT_ROWS)
-    assert not bad, sorted({kinds[b // 8] if b < 8 * len(kinds) else "mixed" for b in bad})
+    for dev in _device_bytes(kq, w, codec, im):
+        bad = np.argwhere((dev != host).any(axis=1)).ravel().tolist()
+        assert not bad, sorted({kinds[b // 8] if b < 8 * len(kinds) else "mixed" for b in bad})
+
+
+@pytest.mark.parametrize("codec", ["q2_k", "q4_k", "q5_k"])
+def test_device_encoder_fit_of_blocks_far_above_zero(kq, codec):
+    """Waves of nothing but blocks without a bound, of some, and of none; weights of one size and of many."""
+    rng = np.random.default_rng(91 + O.codec_id(codec))
+    K = 1024
+    w = np.concatenate([c + rng.standard_normal((16, K)) for c in (1000.0, 300.0, 100.0, 30.0, 5.0)] +
+                       [np.where(np.arange(K) // 64 % 2, 1000.0, 0.0) + rng.standard_normal((16, K))])
+    w = torch.from_numpy(w.astype(np.float32))
+    for im in (None, torch.ones(K), torch.from_numpy((10.0 ** rng.uniform(-6, 0, K)).astype(np.float32))):
+        host = kq.quantize(w, codec, im)[0].numpy()
+        for dev in _device_bytes(kq, w, codec, im):
+            bad = np.argwhere((dev != host).any(axis=1)).ravel().tolist()
+            assert not bad, bad
 
 
 @pytest.mark.parametrize("codec", ["q2_k", "q4_k", "q5_k"])
@@ -230,9 +256,10 @@ def test_device_encoder_fit_up_to_the_ends_of_the_bound(kq, codec):
         im = torch.from_numpy(im.astype(np.float32))
         host = kq.quantize(w, codec, im)[0].numpy().reshape(len(w), -1, bpb)
         for s in (-27, -12, 15, 18, 21, 24, 27, 30):
-            dev = kq.quantize((w * 2.0 ** s).cuda(), codec, (im * 2.0 ** (-5 * s // 3)).cuda())[0].cpu().numpy().reshape(host.shape)
-            bad = np.argwhere((dev[:, :, scales] != host[:, :, scales]).any(axis=(1, 2))).ravel().tolist()
-            assert not bad, (s, bad)
+            for dev in _device_bytes(kq, w * 2.0 ** s, codec, im * 2.0 ** (-5 * s // 3)):
+                bad = np.argwhere((dev.reshape(host.shape)[:, :, scales] != host[:, :, scales]).any(axis=(1, 2))).ravel().tolist()
+                assert not bad, (s, bad)
     for s in range(14, {"q2_k": 21, "q4_k": 25, "q5_k": 26}[codec] + 1):  # rows from 0: the minima stay finite
         big = w[:12] * 2.0 ** s
-        assert torch.equal(kq.quantize(big.cuda(), codec)[0].cpu(), kq.quantize(big, codec)[0]), s
+        for dev in _device_bytes(kq, big, codec, None):
+            assert np.array_equal(dev, kq.quantize(big, codec)[0].numpy()), s
