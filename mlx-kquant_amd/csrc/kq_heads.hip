@@ -159,6 +159,9 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
         const int row = 8 * (b - s * rblocks) + (tid >> 5);
         v[u] = *reinterpret_cast<const u32x4*>(a.x + x_off[row < here ? row : here - 1] + CK_STEP * s + 8 * pc);
       }
+      if constexpr (decltype(own)::value) {
+        if (b0 == 0) kqentries::note_left<32>(a.M, E, Z, tid, entries, share);
+      }
 #pragma unroll
       for (int u = 0; u < HD_AHEAD; u++) {
         const int b = b0 + u, s = b * per_block >> 5, row = 8 * (b - s * rblocks) + (tid >> 5);
@@ -197,7 +200,6 @@ __global__ __launch_bounds__(HD_THREADS, 2) void heads_kernel(HeadArgs a) {
       }
     }
     if (__builtin_expect(lost_rows != 0, 0)) atomicOr(&wide_rows, lost_rows);
-    if constexpr (decltype(own)::value) kqentries::note_left<32>(a.M, E, Z, tid, entries, share);
     vmwait<0>();  // the wire bytes
     lds_barrier();
     const uint32_t rows_here = here == 32 ? ~0u : (1u << here) - 1, wide = __builtin_amdgcn_readfirstlane(wide_rows) & rows_here;
