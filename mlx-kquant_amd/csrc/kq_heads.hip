@@ -11,9 +11,9 @@
 //   * Activations: up to 32 rows at a time as f16 fragments in LDS under a power of two per row and step.  A row with a nonzero
 //     value that this does not hold (2^-31 of the step's largest, bf16), or with an infinity, is done in f32 instead.
 //     More rows than 32 are further rounds, of other workgroups (kq_entries.h): 1024 entries of 8 rows on one of 64 experts
-//     243 -> 31 us against rounds in series on the expert's own, 512 of one row on one of 128 100 -> 18.4, even shares 6.7 -> 6.8 (q8_0).
-// 128 heads of 128 x 512, 4 / 16 / 32 rows each, us: q8_0 12.6 / 14.6 / 22.4 -> 6.8 / 7.8 / 10.0, q4_k 10.3 / 11.7 / 15.4 -> 6.5 / 7.7 / 10.3,
-// q6_k 11.9 / 12.9 / 16.9 -> 7.0 / 7.9 / 9.9, the empty launch 2.4; 64 / 128 rows q8_0 28 / 61 -> 12.9 / 23.3, q4_k 22 / 45 -> 13.5 / 24.1.
+//     243 -> 31 us against rounds in series on the expert's own, 512 of one row on one of 128 100 -> 18.4, even shares 6.7 -> 6.7 (q8_0).
+// 128 heads of 128 x 512, 4 / 16 / 32 rows each, us: q8_0 12.6 / 14.6 / 22.4 -> 6.7 / 7.7 / 9.8, q4_k 10.3 / 11.7 / 15.4 -> 6.3 / 7.4 / 10.0,
+// q6_k 11.9 / 12.9 / 16.9 -> 6.9 / 7.8 / 9.8, the empty launch 2.4; 64 / 128 rows q8_0 28 / 61 -> 12.7 / 23.0, q4_k 22 / 45 -> 13.1 / 24.1.
 #include <algorithm>
 
 #include "kq_entries.h"
